@@ -54,7 +54,7 @@ class PlanInfo(ctypes.Structure):
         ("tiledGrouped", ctypes.c_int), ("superM", ctypes.c_int), ("superK", ctypes.c_int),
         ("tiledAligned", ctypes.c_int), ("itemOrder", ctypes.c_int),
         ("numPieces", ctypes.c_int), ("numShapes", ctypes.c_int), ("wideOffsets", ctypes.c_int),
-        ("tileDigits", ctypes.c_char * 192),
+        ("tileDigits", ctypes.c_char * 192), ("rowGather", ctypes.c_int),
     ]
 
     @property

@@ -32,6 +32,7 @@
 #include "hip_layer.h"
 #include "mbar_decode.h"
 #include "packed_items.h"
+#include "row_blocks.h"
 #include "tile_order.h"
 
 using namespace cutt;
@@ -163,6 +164,23 @@ __global__ __launch_bounds__(kTileThreads) void countTiledCopyKernel(const cuttH
   flush(c, total);
 }
 
+// Mirrors rowGatherKernel writing to a line-aligned buffer (row_blocks.h: locateRows, rowInputOffset).
+__global__ __launch_bounds__(kRowThreads) void countRowsKernel(const cuttHipRowArgs a, unsigned long long* total) {
+  RowBlock b;
+  if (!locateRows(a, 0, b)) return;
+  const uint32_t es = (uint32_t)a.elemSize, lane = threadIdx.x & 63;
+  LaneCounts c = {};
+  for (int j = 0; j < kRowElems; j++) {
+    const uint32_t slot = threadIdx.x + kRowThreads * j, i = min(slot, b.hi - 1), p = b.col0 + i;
+    const uint32_t r = fastDivide(p, a.rowDiv.mul, a.rowDiv.shift, a.rowDiv.add);
+    const bool idle = slot - lane >= b.hi;  // the wavefront's first lane is already beyond the tensor
+    countAccess(c, false, idle, (uint64_t)rowInputOffset(a, b.row0 + r) + (p - r * a.rowLen), es);
+    countAccess(c, true, idle, (uint64_t)b.first + i, es);
+  }
+  if (threadIdx.x == 0) c.v[kWrPartial] += partialEnds((uint64_t)b.first, b.hi, es);
+  flush(c, total);
+}
+
 // Mirrors packedKernel: the work items a workgroup takes and where they lie (all three work-item
 // orders), and the lanes' offsets inside a staged block, come from the functions that kernel uses
 // (packed_items.h: packedItems, packedLocate, packedInElem, packedOutElem); E elements per lane.
@@ -252,6 +270,10 @@ extern "C" int cuttHipCountTiled(const cuttHipTiledArgs* a, cuttHipStreamCounts*
 
 extern "C" int cuttHipCountTiledCopy(const cuttHipTiledCopyArgs* a, cuttHipStreamCounts* out, void* stream) {
   if (int v = cuttHipValidateTiledCopy(a); v != 0) return v;
+  if (a->rowGather)
+    return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
+      return launchCount(countRowsKernel, dim3((uint32_t)cuttHipRowGrid(&a->rows)), dim3(kRowThreads), s, a->rows, d);
+    });
   const long long blocks = cuttHipTiledCopyGrid(a);
   if (blocks < 1) return (int)hipErrorInvalidConfiguration;
   return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {

@@ -86,7 +86,7 @@ std::string planKey(int deviceID, int force, int rank, const int* dim, const int
   for (int i = 0; i < rank; i++) put(perm[i]);
   for (const char* name : {"CUTT_TILED_ORDER", "CUTT_XCD_AWARE", "CUTT_ELEMS_PER_THREAD", "CUTT_PACKED_ROUNDS",
                            "CUTT_MAX_ITEMS", "CUTT_ITEM_ORDER", "CUTT_PAD_SHIFT", "CUTT_CACHE_POLICY", "CUTT_WIDE_OFFSETS", "CUTT_MBAR_ORDER",
-                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
+                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
     const char* e = std::getenv(name);
     k += e ? e : "-";
     k += ';';
@@ -176,13 +176,19 @@ bool currentDevice(int& deviceID, cuttHipDeviceProps& props) {
   return true;
 }
 
+int cachePolicyOf(const Plan& p) {
+  if (p.method == kTiled) return p.tiled.cachePolicy;
+  if (p.method == kTiledCopy) return p.tcopy.rowGather ? p.tcopy.rows.cachePolicy : p.tcopy.cachePolicy;
+  return p.packed.cachePolicy;
+}
+
 void fillInfo(const Plan& p, cuttPlanInfo& o) {
   std::memset(&o, 0, sizeof(o));
   o.method = p.method;
   o.fromReduced = p.fromReduced;
   o.rank = p.pb.rank;
   o.numMm = p.split.numMm;
-  o.numMk = p.split.numMk;
+  o.numMk = p.method == kTiledCopy && p.tcopy.rowGather ? 1 : p.split.numMk;  // (gathered rows have no second tile axis)
   o.splitRank = p.split.splitRank[0];
   o.splitDim = p.split.splitDim[0];
   o.numSplit = p.split.numSplit[0];
@@ -211,11 +217,11 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.wrSectors = p.model.wrSectors;
   o.ldsCycles = p.model.ldsCycles;
   o.blocksPerCU = p.model.blocksPerCU;
-  o.cachePolicy = p.method == kTiled ? p.tiled.cachePolicy
-                                      : (p.method == kTiledCopy ? p.tcopy.cachePolicy : p.packed.cachePolicy);
+  o.cachePolicy = cachePolicyOf(p);
   o.elemsPerThread = p.packed.elemsPerThread;
   o.tiledGrouped = p.method == kTiled ? p.tiled.grouped : 0;
   o.tiledAligned = p.method == kTiled ? p.tiled.alignedStores : 0;
+  o.rowGather = p.method == kTiledCopy ? p.tcopy.rowGather : 0;
   o.itemOrder = (p.method == kPacked || p.method == kPackedSplit) ? p.packed.itemOrder : 0;
   o.numPieces = 1;
   o.numShapes = 1;
@@ -235,15 +241,10 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
 }
 
 void setCachePolicy(Plan& p, int policy) {
+  if (p.method == kTiledCopy && p.tcopy.rowGather) return;  // chosen with the row gathering (plan.cpp: setupRows)
   p.tiled.cachePolicy = policy;
   p.tcopy.cachePolicy = policy;
   p.packed.cachePolicy = policy;
-}
-
-int cachePolicyOf(const Plan& p) {
-  if (p.method == kTiled) return p.tiled.cachePolicy;
-  if (p.method == kTiledCopy) return p.tcopy.cachePolicy;
-  return p.packed.cachePolicy;
 }
 
 // Cache policy from the model's sampled address stream.  Streaming loads give up the L2 copy of a
@@ -413,9 +414,10 @@ PlannerOptions plannerOptions(int forceMethod) {
   if (const char* e = std::getenv("CUTT_PAD_SHIFT")) opt.padShift = std::min(31, std::max(1, std::atoi(e)));
   if (const char* e = std::getenv("CUTT_ITEM_ORDER")) opt.itemOrder = std::min(2, std::max(0, std::atoi(e)));
   if (const char* e = std::getenv("CUTT_MAX_ITEMS")) opt.maxItemsPerBlock = std::max(1, std::atoi(e));
+  if (const char* e = std::getenv("CUTT_ROW_GATHER")) opt.rowGather = std::atoi(e) != 0;
   if (const char* e = std::getenv("CUTT_CACHE_POLICY")) {
     const int v = std::atoi(e);
-    if (v == 0 || v == 1 || v == 3) opt.cachePolicy = v;
+    if (v == 0 || v == 1 || v == 3) opt.cachePolicy = opt.rowPolicy = v;
   }
   if (const char* e = std::getenv("CUTT_WIDE_OFFSETS")) opt.wideOffsets = std::atoi(e) != 0;
   if (const char* e = std::getenv("CUTT_MBAR_ORDER")) opt.mbarOrder = std::atoi(e);
@@ -746,10 +748,11 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   // per workgroup, order of the Mbar ranks, cache policy); a setting that measures faster is kept
   // for the knobs that follow.
   if (!failed && best >= 0 && plans[best].method != kTrivial) {
-    const bool tiled = plans[best].method == kTiled || plans[best].method == kTiledCopy;
+    const bool rowGather = plans[best].method == kTiledCopy && plans[best].tcopy.rowGather;
+    const bool tiled = !rowGather && (plans[best].method == kTiled || plans[best].method == kTiledCopy);
     // options that reproduce the winner as it stands
     PlannerOptions cur = plannerOptions(force);
-    cur.cachePolicy = cachePolicyOf(plans[best]);
+    if (!rowGather) cur.cachePolicy = cachePolicyOf(plans[best]);
     if (tiled) {
       const bool t = plans[best].method == kTiled;
       cur.tiledOrder = t ? plans[best].tiled.order : plans[best].tcopy.order;
@@ -760,7 +763,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         cur.tileDigits = formatTileDigits(t ? plans[best].tiled.digits : plans[best].tcopy.digits);
         cur.tiledOrder = -1;
       }
-    } else {
+    } else if (!rowGather) {
       cur.maxItemsPerBlock = plans[best].packed.itemsPerBlock;
       cur.itemOrder = plans[best].packed.itemOrder;
       // (a winner whose work items are numbered by address bits keeps that through the variants: the order is
@@ -791,7 +794,23 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       return true;
     };
 
-    if (tiled) {
+    if (rowGather) {
+      // groups of blocks per XCD, non-temporal accesses
+      for (int g : {0, 4, 7, 9}) {
+        if (failed) break;
+        if (g == plans[best].tcopy.rows.xcdGroup) continue;
+        PlannerOptions v = cur;
+        v.rowGroup = g;
+        if (tryVariant(v, false)) cur = v;
+      }
+      for (int pol : {0, 2, 3}) {
+        if (failed || std::getenv("CUTT_CACHE_POLICY")) break;
+        if (pol == plans[best].tcopy.rows.cachePolicy) continue;
+        PlannerOptions v = cur;
+        v.rowPolicy = pol;
+        if (tryVariant(v, false)) cur = v;
+      }
+    } else if (tiled) {
       // patches of several shapes instead of strips (small patches walked for all Mbar positions in
       // turn make long sequential streams of a batched 2-D transpose: C2 +4...7 %), rows of tiles
       // along Mm / along Mk, strips per Mbar position / for all Mbar positions in turn
@@ -850,7 +869,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     // the order in which consecutive work items (or strips of tiles) walk the Mbar ranks decides
     // which partly used lines neighbouring workgroups share in the L2; it can move the time by 20 %
     for (int order : {0, 1, 2}) {
-      if (failed || std::getenv("CUTT_MBAR_ORDER")) break;
+      if (failed || rowGather || std::getenv("CUTT_MBAR_ORDER")) break;
       if (order == start.mbarOrder) continue;
       PlannerOptions v = cur;
       v.mbarOrder = order;
@@ -858,14 +877,14 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     }
     // workgroup b at logical position b (the XCDs then interleave instead of walking a chunk each):
     // rarely better, but then by 5-10 % (measured on PackedSplit plans with long runs)
-    if (!failed && !std::getenv("CUTT_XCD_AWARE") && cur.xcdAware) {
+    if (!failed && !rowGather && !std::getenv("CUTT_XCD_AWARE") && cur.xcdAware) {
       PlannerOptions v = cur;
       v.xcdAware = false;
       if (tryVariant(v, false)) cur = v;
     }
     // ... and the other cache policies of the global accesses
     for (int pol : {0, 1, 3}) {
-      if (failed || std::getenv("CUTT_CACHE_POLICY")) break;
+      if (failed || rowGather || std::getenv("CUTT_CACHE_POLICY")) break;
       if (pol == start.cachePolicy) continue;
       PlannerOptions v = cur;
       v.cachePolicy = pol;

@@ -184,6 +184,34 @@ typedef struct cuttHipTiledArgs {
 } cuttHipTiledArgs;
 
 /*
+ * Rows gathered into a dense output (TiledCopy method, the usual kernel): rank 0 keeps its place, so the
+ * output is the sequence of numRows rows of rowLen contiguous elements, and row o of it lies
+ * sum_k ((o / prod_{j<k} extent_j) % extent_k) * stride_k elements into the input (ranks 1, 2, ... of the
+ * output, fastest first).  A workgroup writes CUTT_ROW_BLOCK consecutive output elements that start on
+ * a 128-byte line, whatever rows they belong to.
+ */
+typedef struct cuttHipRowRank {
+  uint32_t extent, stride;
+  uint32_t mul, ctl;      /* division by extent (cuttHipMakeDivisor): shift | add << 8 */
+} cuttHipRowRank;
+
+#define CUTT_ROW_BLOCK 1024
+#define CUTT_ROW_TABLE 256  /* rows one workgroup can meet: rowLen >= 5 */
+typedef struct cuttHipRowArgs {
+  int elemSize;
+  uint32_t rowLen, numRows, volume;  /* volume = rowLen * numRows < 2^32 */
+  cuttHipDivisor rowDiv;             /* division by rowLen */
+  int cachePolicy;    /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
+  int xcdGroup;       /* 0: workgroup b writes block b; g >= 1: XCD b % 8 takes groups of 2^(g-1) neighbouring blocks */
+  int n;              /* ranks below */
+  cuttHipRowRank rank[CUTT_MAX_RANK];
+} cuttHipRowArgs;
+
+/* Workgroups of a row-gathering launch, 0 if there is no valid grid.  (A buffer that starts inside a 128-byte
+ * line has its blocks moved down to the line, which may take one more.) */
+uint64_t cuttHipRowGrid(const cuttHipRowArgs* a);
+
+/*
  * TiledCopy method: rank 0 keeps its place, so rows along rank 0 (extent
  * volMm) are copied; the second output rank (extent volMk, input stride
  * strideInK, output stride strideOutK) is the other tile axis.  No LDS.
@@ -199,6 +227,8 @@ typedef struct cuttHipTiledCopyArgs {
   uint32_t xcdChunk;
   uint32_t superM, superK;
   int cachePolicy;
+  int rowGather;            /* 1: the launch takes `rows` (dense tensors with rows of 64 bytes and more); 0: 64x64 tiles */
+  cuttHipRowArgs rows;
   cuttHipTileDigits digits; /* order 7 only */
   cuttHipMbar mbar;
 } cuttHipTiledCopyArgs;

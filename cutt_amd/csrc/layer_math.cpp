@@ -43,6 +43,15 @@ extern "C" int cuttHipFinishMbar(cuttHipMbar* mb) {
   return 0;
 }
 
+extern "C" uint64_t cuttHipRowGrid(const cuttHipRowArgs* a) {
+  uint64_t blocks = ((uint64_t)a->volume + 128 / a->elemSize - 1 + CUTT_ROW_BLOCK - 1) / CUTT_ROW_BLOCK;
+  if (a->xcdGroup) {
+    const uint64_t unit = 8ull << (a->xcdGroup - 1);  // a group per XCD
+    blocks = (blocks + unit - 1) / unit * unit;
+  }
+  return blocks <= 0x7fffffffull && blocks * 256 <= CUTT_HIP_MAX_GRID_LANES ? blocks : 0;
+}
+
 static int finishTileDigits(cuttHipTileDigits* dg, const cuttHipMbar* mb);
 
 extern "C" int cuttHipFinishTileDigits(cuttHipTileDigits* dg, const cuttHipMbar* mb) {

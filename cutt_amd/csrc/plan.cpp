@@ -1068,6 +1068,35 @@ int64_t addressBitOrder(const Problem& pb, const Split& sp, const cuttHipMbar& m
   return logical <= 0x7fffffffll ? logical : 0;
 }
 
+// Arguments of the row-gathering kernel for a problem whose leading rank stays; false where the 64x64 copy tiles
+// have to do: pieces of a larger tensor (their output has gaps) and rows of less than 64 bytes.
+bool setupRows(const Problem& pb, const PlannerOptions& opt, cuttHipRowArgs& a) {
+  std::memset(&a, 0, sizeof(a));
+  if (!pb.dense || pb.rank < 2 || pb.perm[0] != 0 || (int64_t)pb.dim[0] * pb.elemSize < 64 || pb.volume > 0xffffffffll) return false;
+  a.elemSize = pb.elemSize;
+  a.rowLen = (uint32_t)pb.dim[0];
+  a.rowDiv = cuttHipMakeDivisor(a.rowLen);
+  a.numRows = (uint32_t)(pb.volume / pb.dim[0]);
+  a.volume = (uint32_t)pb.volume;
+  for (int j = 1; j < pb.rank; j++) {
+    const int r = pb.perm[j];
+    const cuttHipDivisor dv = cuttHipMakeDivisor((uint32_t)pb.dim[r]);
+    a.rank[a.n++] = cuttHipRowRank{(uint32_t)pb.dim[r], (uint32_t)pb.strideIn[r], dv.mul, dv.shift | dv.add << 8};
+  }
+  // Non-temporal stores always (the lines are written whole).  Non-temporal loads only for long rows of 8-byte
+  // elements beyond the caches: 4-21 % faster there ((533853,15,5)/(0,2,1) 105 -> 94 us, (159,140130,2)/(0,2,1)
+  // 117 -> 107 us), but rows share the lines at their ends, and those are read again: rows of 216-720 bytes ran
+  // 6-20 % slower, cache-sized tensors 15-30 %, 4-byte elements 0-4 %.
+  const int64_t rowBytes = (int64_t)a.rowLen * pb.elemSize, bytes = pb.volume * pb.elemSize;
+  a.cachePolicy = opt.rowPolicy >= 0 ? opt.rowPolicy : (pb.elemSize == 8 && rowBytes >= 800 && bytes >= ((int64_t)96 << 20) ? 3 : 2);
+  // Every XCD takes groups of 64 neighbouring blocks, so that the row two blocks share is read into one L2: 0-2 %
+  // faster than single blocks dealt out in turn on 40 random tensors, 15-20 % where rows are 64-150 bytes long.
+  // Below 8192 blocks (32 MB of 4-byte elements) the last round of groups would leave XCDs idle.
+  const int64_t blocks = ceilDiv(pb.volume, (int64_t)CUTT_ROW_BLOCK);
+  a.xcdGroup = opt.rowGroup >= 0 ? opt.rowGroup : (blocks >= 8192 ? 7 : 0);
+  return true;
+}
+
 bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt) {
   const Split& sp = plan.split;
   const Problem& pb = plan.pb;
@@ -1233,7 +1262,13 @@ void addTiled(const Problem& red, const cuttHipDeviceProps& props, const Planner
     p.split.update(1, 2, red);
     if (!allowed(opt, p.method)) return;
     if (!setupTiled(p, props, opt)) return;
-    if (!exists(p.split, plans)) plans.push_back(std::move(p));
+    // ... or gather the rows in output order, which needs no second tile axis (unless the options pin a tile order)
+    if (opt.rowGather && opt.tiledOrder < 0 && opt.tileDigits.empty()) {
+      Plan q = p.clone();
+      q.tcopy.rowGather = setupRows(red, opt, q.tcopy.rows) ? 1 : 0;
+      if (q.tcopy.rowGather) plans.push_back(std::move(q));
+    }
+    plans.push_back(std::move(p));
     return;
   }
   if (!allowed(opt, kTiled)) return;
@@ -1438,7 +1473,9 @@ bool rebuildPlan(const Plan& src, const cuttHipDeviceProps& props, const Planner
   switch (src.method) {
     case kTiled:
     case kTiledCopy:
-      return setupTiled(out, props, opt);
+      if (!setupTiled(out, props, opt)) return false;
+      if (src.method == kTiledCopy && src.tcopy.rowGather) out.tcopy.rowGather = setupRows(out.pb, opt, out.tcopy.rows) ? 1 : 0;
+      return true;
     case kPacked:
     case kPackedSplit:
       return setupPacked(out, props, opt);
@@ -1602,7 +1639,10 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
 
 int Plan::activate() {
   if (method == kTiled) return launchable ? 0 : ((launchable = cuttHipValidateTiled(&tiled) == 0) ? 0 : -1);
-  if (method == kTiledCopy) return launchable ? 0 : ((launchable = cuttHipValidateTiledCopy(&tcopy) == 0) ? 0 : -1);
+  if (method == kTiledCopy) {
+    if (tcopy.rowGather) numBlocks = (int64_t)cuttHipRowGrid(&tcopy.rows);
+    return launchable ? 0 : ((launchable = cuttHipValidateTiledCopy(&tcopy) == 0) ? 0 : -1);
+  }
   if (method != kPacked && method != kPackedSplit) {
     launchable = method == kTrivial;
     return launchable ? 0 : -1;

@@ -173,6 +173,8 @@ struct PlannerOptions {
   int mbarOrder = 2;        // order of the Mbar ranks: 0 = input order, 1 = output order,
                             // 2 = first input rank outside Mmk, then output order
   bool wideOffsets = false; // Packed/PackedSplit: 64-bit address arithmetic also below 4 GB (tests)
+  bool rowGather = true;    // TiledCopy: gather the rows of dense tensors in output order instead of copying tiles
+  int rowPolicy = -1, rowGroup = -1;  // ... its cache policy and XCD grouping, -1 = planner's choice
   bool xcdAware = true;     // give every XCD (private L2) a contiguous chunk of the workgroup sequence
 };
 

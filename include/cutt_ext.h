@@ -49,7 +49,7 @@ typedef struct cuttPlanInfo {
   /* planning statistics of the call that made the plan */
   int numCandidates;
   double planMs;
-  int cachePolicy;      /* 0 default, 1 non-temporal loads, 3 non-temporal loads and stores */
+  int cachePolicy;      /* 0 default, 1 non-temporal loads, 2 non-temporal stores, 3 both */
   int elemsPerThread;   /* Packed/PackedSplit */
   /* cost model: work items between the accesses to the two parts of a line shared by neighbouring
    * runs, on the read and on the write side (0 = no such neighbour) */
@@ -69,6 +69,8 @@ typedef struct cuttPlanInfo {
                            syntax of CUTT_TILE_DIGITS ("m2@1,k2@1,b3@64,..." = coordinate, radix, weight);
                            Packed/PackedSplit whose work items are numbered by digits (m, k = slab of the
                            first, second cut rank; b = Mbar position): those digits; else empty */
+  int rowGather;        /* TiledCopy: 1 if the rows are gathered in output order (dense tensors), 0 if 64x64 tiles are
+                           copied */
 } cuttPlanInfo;
 
 /* Describe an existing plan. */
