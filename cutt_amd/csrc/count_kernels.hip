@@ -6,8 +6,7 @@
  * They take the same arguments and the same grid as the kernel they mirror and derive every
  * address with the device functions that kernel itself calls (tile_order.h: tile order, tile geometry and
  * row addresses; packed_items.h: work-item orders, item offsets, run tables; mbar_decode.h), but issue
- * no load or store of tensor data (the instance of the Tiled kernel with line-aligned stores has no
- * counting kernel: cuttHipCountTiled refuses it); the counts of all wavefronts are added up
+ * no load or store of tensor data; the counts of all wavefronts are added up
  * with atomics.  A test compares them with the host model's walk over the same plan.  Counterpart
  * of the reference's model-validation kernels (src/cuttGpuModelKernel.cu:246-646, countTiled,
  * countPacked, countPackedSplit, countTiledCopy, and the driver :686-782), redone for 64-lane
@@ -30,6 +29,7 @@
 #include <type_traits>
 
 #include "hip_layer.h"
+#include "line_windows.h"
 #include "mbar_decode.h"
 #include "packed_items.h"
 #include "row_blocks.h"
@@ -134,6 +134,36 @@ __global__ __launch_bounds__(kTileThreads) void countTiledKernel(const cuttHipTi
     if (row <= t.wM && lane == 0) c.v[kWrPartial] += partialEnds(elem, t.wK + 1, es);
   }
   // the partial-line counts sit in lane 0 already; the per-instruction counts are wave-uniform
+  flush(c, total);
+}
+
+// Mirrors tiledLinesKernel writing to a line-aligned buffer (line_windows.h: lineTile, lineElem, lineRowIn, lineRowOut).
+// The bank-conflict degree is that of the column reads.
+template <typename T, int TH>
+__global__ __launch_bounds__(TH) void countLinesKernel(const cuttHipTiledArgs a, unsigned long long* total) {
+  constexpr uint32_t ES = sizeof(T);
+  uint32_t tm, tk, offIn, offOut;
+  if (!locateTile(a, tm, tk, offIn, offOut)) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const LineTile t = lineTile<T>(a, tm, tk, offOut);
+  if (t.rows == 0) return;
+  LaneCounts c = {};
+  const uint32_t n = t.rows * t.width;
+  for (uint32_t p0 = 0; p0 < n; p0 += TH) {
+    uint32_t r, col;
+    lineElem(a, t, min(p0 + tid, n - 1), r, col);
+    countAccess(c, false, p0 + (tid & ~63u) >= n, offIn + t.m0 + col + lineRowIn<true>(a, (uint32_t)t.kLo + r), ES);
+  }
+  for (uint32_t r = tid >> 6; r < t.width; r += TH / 64) {
+    const uint32_t rowStart = offOut + lineRowOut<true>(a, t.m0 + r);
+    const int32_t s = (int32_t)(rowStart & (kLineElems<T> - 1));
+    const int32_t lo = max(t.kWin - s, 0), hi = min(t.kWin - s + kWindow, (int32_t)a.volMk);
+    const int32_t k = t.kWin - s + (int32_t)lane, kc = min(max(k, lo), hi - 1);
+    countAccess(c, true, hi <= lo, rowStart + (uint32_t)kc, ES);
+    if (hi <= lo) continue;
+    c.maxDegree = max(c.maxDegree, waveMaxMultiplicity((((uint32_t)(kc - t.kLo) * t.pitch + r) * (ES / 4)) & 63, __ballot(k == kc)));
+    if (lane == 0) c.v[kWrPartial] += partialEnds(rowStart + (uint32_t)lo, (uint32_t)(hi - lo), ES);
+  }
   flush(c, total);
 }
 
@@ -258,9 +288,15 @@ int runCount(cuttHipStreamCounts* out, void* stream, F&& launch) {
 
 extern "C" int cuttHipCountTiled(const cuttHipTiledArgs* a, cuttHipStreamCounts* out, void* stream) {
   if (int v = cuttHipValidateTiled(a); v != 0) return v;
-  if (a->alignedStores) return (int)hipErrorNotSupported;
   const long long blocks = cuttHipTiledGrid(a);
   if (blocks < 1) return (int)hipErrorInvalidConfiguration;
+  if (a->alignedStores)
+    return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
+      const int threads = cuttHipLinesThreads(a->elemSize, a->tileWidth);
+      if (a->elemSize == 8) return launchCount(countLinesKernel<uint64_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, d);
+      return threads == 512 ? launchCount(countLinesKernel<uint32_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, d)
+                            : launchCount(countLinesKernel<uint32_t, 256>, dim3((uint32_t)blocks), dim3(256), s, *a, d);
+    });
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
   return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
     return fused ? launchCount(countTiledKernel<true>, dim3((uint32_t)blocks), dim3(kTileThreads), s, *a, d)

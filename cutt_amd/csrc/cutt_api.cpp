@@ -247,41 +247,46 @@ void setCachePolicy(Plan& p, int policy) {
   p.packed.cachePolicy = policy;
 }
 
-// Cache policy from the model's sampled address stream.  Streaming loads give up the L2 copy of a
-// line, so they pay off only when a workgroup uses (nearly) whole lines of what it reads;
-// streaming stores only when no written line is left partly covered by a workgroup.
-// (Not applied when CUTT_CACHE_POLICY pins the policy.)
+PlannerOptions plannerOptions(int forceMethod);
+
+// Cache policy of a plan's global accesses, from its size and the model's sampled address stream.  (Not applied when
+// CUTT_CACHE_POLICY pins the policy.)  Timed on 120 random tensors of 0.14-1.6 GB per buffer, buffers in rotation and
+// the same ones again and again:
+//  - input and output inside the memory-side cache together: ordinary accesses (non-temporal ones go past it);
+//  - outputs written in whole lines - at most one line in a hundred left partly covered by a workgroup -:
+//    non-temporal stores, 2-10 % faster than ordinary ones ((37,59,7,16,6,30) 146 -> 132 us, (985024,28,4) 345 ->
+//    317 us); from 3 partial lines in a hundred on they lose (4-byte rows of 9 KB: 188 -> 207 us).  Where the reads
+//    are whole lines too and nothing fits the cache the loads go past it as well (another 1-2 %);
+//  - line-aligned stores: the same, with ordinary loads (neighbouring tiles read the fringe rows again; non-temporal
+//    loads cost them 3-30 %);
+//  - everything else beyond one cache size per buffer: ordinary accesses, 1-12 % faster than non-temporal loads on 61
+//    of 66 tensors (C5-like (621,1489,116)/(1,2,0), 8 bytes: 389 -> 347 us);
+//  - up to one cache size per buffer non-temporal loads leave the cache to the output: 10-28 % faster when the same
+//    buffers are used again, 0-7 % slower when they are not - unless the plan requests each line of data more than
+//    1.7 times (1.5 for the 256-byte rows of 4-byte tiles), when the re-reads must hit.
 void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
   if (std::getenv("CUTT_CACHE_POLICY")) return;
-  // The memory-side cache decides for small and medium tensors (measured on random tensors of
-  // 4M-200M elements): while input and output fit it together, ordinary accesses are best
-  // (non-temporal ones go past it: 65-72 % of memcpy instead of 80-89 %); up to about 3.5 times
-  // its size per buffer, streaming the reads and letting the cache merge the writes wins clearly
-  // (at one cache size per buffer 99 % against 81 %); beyond that it no longer matters.
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
   const double cache = (double)props.infinityCacheBytes;
   if (cache > 0 && 2.0 * bytes <= cache) {
     setCachePolicy(p, 0);
     return;
   }
-  const double lines = bytes / 128.0;
-  if (cache > 0 && bytes <= 3.5 * cache) {
-    // ... unless the plan reads each line from several requests (more than ~1.7 lines requested
-    // per line of data): then the re-reads must find the line in the caches (0.85-0.97 x).
-    // A Tiled plan's 256-byte rows of 4-byte elements share every third line with the neighbouring
-    // tile: there the limit is 1.5, except between 0.8 and 1.8 cache sizes per buffer, where it is
-    // 1.6 (at 1.56 lines per line of data: ordinary loads +10 % at 0.75 cache sizes and +7...+15 %
-    // at 2.1-3.1, streaming loads +9...+18 % at 0.88-1.56), and a plan that keeps four rows per
-    // lane in flight always streams its reads (+2...+24 % over ordinary loads at 1-3.4 cache sizes).
-    const bool narrowTiles = (p.method == kTiled || p.method == kTiledCopy) && p.pb.elemSize == 4;
-    const double limit = narrowTiles ? (bytes >= 0.8 * cache && bytes < 1.8 * cache ? 1.6 : 1.5) : 1.7;
-    const bool grouped = p.method == kTiled && p.tiled.grouped;
-    setCachePolicy(p, grouped || p.model.rdLines < limit * lines ? 1 : 0);
+  if (p.method == kTiled && p.tiled.alignedStores) {
+    setCachePolicy(p, 2);
     return;
   }
-  const bool wholeReads = p.model.rdLines <= 1.15 * lines;
-  const bool wholeWrites = p.model.wrPartialLines == 0.0;
-  setCachePolicy(p, wholeReads ? (wholeWrites ? 3 : 1) : 0);
+  const double lines = bytes / 128.0;
+  if (p.method == kTrivial) {
+    setCachePolicy(p, bytes <= 3.5 * cache ? 1 : 3);
+    return;
+  }
+  if (p.model.wrPartialLines <= 0.01 * lines) {
+    setCachePolicy(p, bytes > cache && p.model.rdLines <= 1.02 * lines ? 3 : 2);
+    return;
+  }
+  const bool narrowTiles = (p.method == kTiled || p.method == kTiledCopy) && p.pb.elemSize == 4;
+  setCachePolicy(p, bytes <= cache && p.model.rdLines < (narrowTiles ? 1.5 : 1.7) * lines ? 1 : 0);
 }
 
 // Runs f(0) .. f(n-1) on up to eight host threads (CUTT_PLAN_THREADS caps the number; 1 = the
@@ -337,10 +342,55 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (grouped) p.model.usPredicted *= 0.96;
 }
 
+// Whether a Tiled plan stores its rows in line-aligned windows (kernels.hip: tiledLinesKernel): output rows that start
+// off the line grid, long enough that the lines cut at the run's ends do not count, of a tensor beyond the memory-side
+// cache.  Against ordinary tiles on 60 such tensors of 0.14-1.7 GB per buffer, both widths: 3-18 % faster (23425 x 8538,
+// 8 bytes: 674 -> 603 us; (50,7,13,43610)/(3,1,2,0) 656 -> 617; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 361 ->
+// 316 us).  Runs of 1.4 KB lose 5 %, so do batches of separate matrices with runs of 2 KB (those break even at 4 KB);
+// with tiles of less than 256 bytes along Mm the fringe rows, read twice, cost more than the stores gain ((7,4,99,4,...),
+// 28 columns: 247 -> 298 us).  Tensors inside the cache: 24 MB +20 % time, 120 MB -1 %, left to the ordinary tiles.
+bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
+  if (p.method != kTiled || p.tiled.alignedStores) return false;
+  const Problem& pb = p.pb;
+  const int64_t runBytes = p.split.volMk * pb.elemSize;
+  const double bytes = (double)pb.volume * pb.elemSize;
+  const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
+  // batches of separate matrices: the Mbar ranks are slowest on both sides
+  bool offGrid = false, batch = p.split.volMbar > 1;
+  for (int r = 0; r < pb.rank; r++) {
+    if (pb.inv[r] < p.split.numMk) continue;
+    offGrid = offGrid || (pb.dim[r] > 1 && pb.strideOut[r] * pb.elemSize % 128 != 0);
+    if (!p.split.inMmk[r]) batch = batch && pb.strideIn[r] >= p.split.volMm * p.split.volMk && pb.strideOut[r] >= p.split.volMm * p.split.volMk;
+  }
+  if (2.0 * bytes <= cache || p.split.volMm * pb.elemSize < 256 || runBytes < (batch ? 4096 : 2048)) return false;
+  if (!offGrid) return false;
+  const PlannerOptions opt = plannerOptions(0);  // options that pin the plain kernel's variants leave the plan as it is
+  return opt.tiledOrder < 0 && opt.superAuto && opt.tileDigits.empty() && opt.tiledGrouped < 0 && opt.tiledAligned < 0 && opt.digitLanes < 0;
+}
+
+// What is left to decide about a plan that is going to be used: line-aligned stores and the cache policy.
+void finishPlan(Plan& p, const cuttHipDeviceProps& props) {
+  if (lineWindowsPay(p, props)) {
+    PlannerOptions opt = plannerOptions(0);
+    opt.tiledAligned = 1;
+    opt.tiledGrouped = p.tiled.grouped;
+    Plan q;
+    if (rebuildPlan(p, props, opt, q)) {
+      q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
+      if (estimatePlan(q, props, 10)) {
+        q.model.usPredicted = p.model.usPredicted;
+        p = std::move(q);
+      }
+    }
+  }
+  chooseCachePolicy(p, props);
+}
+
 // The model's estimate of a candidate and the launch details that follow from it.
 bool estimateAndTune(Plan& p, const cuttHipDeviceProps& props) {
   if (!estimatePlan(p, props, 10)) return false;
   chooseTiledGrouping(p, props);
+  if (lineWindowsPay(p, props)) p.model.usPredicted *= 0.92;
   return true;
 }
 
@@ -352,8 +402,6 @@ bool estimateAll(std::vector<Plan>& plans, const cuttHipDeviceProps& props) {
   });
   return ran && ok;
 }
-
-PlannerOptions plannerOptions(int forceMethod);
 
 // The order in which consecutive work items walk the Mbar ranks decides whether the lines shared
 // by neighbouring runs meet in the L2 on the read side or on the write side.  For the few
@@ -417,7 +465,7 @@ PlannerOptions plannerOptions(int forceMethod) {
   if (const char* e = std::getenv("CUTT_ROW_GATHER")) opt.rowGather = std::atoi(e) != 0;
   if (const char* e = std::getenv("CUTT_CACHE_POLICY")) {
     const int v = std::atoi(e);
-    if (v == 0 || v == 1 || v == 3) opt.cachePolicy = opt.rowPolicy = v;
+    if (v >= 0 && v <= 3) opt.cachePolicy = opt.rowPolicy = v;
   }
   if (const char* e = std::getenv("CUTT_WIDE_OFFSETS")) opt.wideOffsets = std::atoi(e) != 0;
   if (const char* e = std::getenv("CUTT_MBAR_ORDER")) opt.mbarOrder = std::atoi(e);
@@ -508,7 +556,7 @@ static cuttResult decideHeuristically(int rank, int* dim, int* permutation, size
   refineMbarOrder(plans, props, force);
   const int best = chooseHeuristic(plans);
   if (best < 0) return CUTT_INTERNAL_ERROR;
-  chooseCachePolicy(plans[best], props);
+  finishPlan(plans[best], props);
   if (useCache) planCacheInsert(key, plans[best], (int)plans.size());
   numCandidates = (int)plans.size();
   chosen = std::move(plans[best]);
@@ -566,7 +614,7 @@ static cuttResult planLarge(cuttHandle* handle, int rank, int* dim, int* permuta
       refineMbarOrder(plans, props, force);
       const int best = chooseHeuristic(plans);
       if (best < 0) return CUTT_INTERNAL_ERROR;
-      chooseCachePolicy(plans[best], props);
+      finishPlan(plans[best], props);
       if (s == 0) numCandidates = (int)plans.size();
       parts[s] = std::move(plans[best]);
     }
@@ -674,7 +722,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   if (!createPlans(orig, red, props, plannerOptions(force), plans)) return CUTT_INTERNAL_ERROR;
   if (plans.empty()) return CUTT_INTERNAL_ERROR;
   if (!estimateAll(plans, props)) return CUTT_INTERNAL_ERROR;
-  for (Plan& p : plans) chooseCachePolicy(p, props);
+  for (Plan& p : plans) finishPlan(p, props);
 
   // Candidates the model puts more than twice behind its best are not timed when there are many (the
   // model's worst recorded errors: classes of plans that ran 1.3-1.4 times their estimate, a pick at 0.6 of
@@ -802,7 +850,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         v.rowGroup = g;
         if (tryVariant(v, false)) cur = v;
       }
-      for (int pol : {0, 2, 3}) {
+      for (int pol : {0, 1, 2, 3}) {
         if (failed || std::getenv("CUTT_CACHE_POLICY")) break;
         if (pol == plans[best].tcopy.rows.cachePolicy) continue;
         PlannerOptions v = cur;
@@ -835,14 +883,12 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         v.tiledGrouped = 1 - cur.tiledGrouped;
         if (tryVariant(v, false)) cur = v;
       }
-      // every tile row storing its own line-aligned window (measured: +2...+4 % on some 8-byte
-      // tensors with output runs off the 128-byte grid, -5...-15 % on others, so only by trial)
+      // line-aligned stores the other way (lineWindowsPay)
       if (!failed && plans[best].method == kTiled && !std::getenv("CUTT_TILED_ALIGNED") &&
           ((int64_t)plans[best].tiled.volMk * plans[best].pb.elemSize % 128 != 0 ||
            (int64_t)plans[best].tiled.strideOutM * plans[best].pb.elemSize % 128 != 0)) {
         PlannerOptions v = cur;
-        v.tiledAligned = 1;
-        v.tiledGrouped = 0;
+        v.tiledAligned = 1 - cur.tiledAligned;
         if (tryVariant(v, false)) cur = v;
       }
     } else {
@@ -882,7 +928,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       if (tryVariant(v, false)) cur = v;
     }
     // ... and the other cache policies of the global accesses
-    for (int pol : {0, 1, 3}) {
+    for (int pol : {0, 1, 2, 3}) {
       if (failed || rowGather || std::getenv("CUTT_CACHE_POLICY")) break;
       if (pol == start.cachePolicy) continue;
       PlannerOptions v = cur;
@@ -903,7 +949,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       refineMbarOrder(again, props, force);
       const int h = chooseHeuristic(again);
       if (h >= 0 && again[h].method != kTrivial) {
-        chooseCachePolicy(again[h], props);
+        finishPlan(again[h], props);
         Plan heur = std::move(again[h]);
         double tw = 1e300, th = 1e300;
         for (int round = 0; round < 2 && !failed; round++) {

@@ -159,7 +159,7 @@ typedef struct cuttHipTiledArgs {
   int volMm, volMk;
   uint32_t strideInK;
   uint32_t strideOutM;
-  int tilesM, tilesK; /* ceil(volMm/64), ceil(volMk/64) */
+  int tilesM, tilesK; /* ceil(volMm/64), ceil(volMk/64); see alignedStores for the other geometry */
   int volMbar;
   int order;          /* logical numbering of the workgroups: 0 = Mbar fastest, 1 = tiles along Mm
                          fastest, 2 = tiles along Mk fastest, 3 / 4 = superM x superK super-tiles with the
@@ -171,16 +171,19 @@ typedef struct cuttHipTiledArgs {
   uint32_t xcdChunk;  /* 0: workgroup b is logical position b; else (b % 8)*xcdChunk + b/8, and the
                          grid has 8*xcdChunk workgroups */
   uint32_t superM, superK;
-  int cachePolicy;    /* 0 = default, 1 = non-temporal loads, 3 = non-temporal loads and stores */
+  int cachePolicy;    /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
   int grouped;        /* 0: a lane has all 16 rows of its tile in flight at once; 1: four at a time
                          (each group of 16 tile rows is waited for before the next is requested) */
   int alignedStores;  /* 1: every tile row stores its own 64-element window of the output run, shifted
                          so that it starts on a 128-byte line; tilesK is then
-                         ceil((volMk + 128/elemSize - 1) / 64) and grouped must be 0 */
+                         ceil((volMk + 128/elemSize - 1) / 64), a tile is tileWidth elements wide along Mm
+                         (tilesM = ceil(volMm/tileWidth)), and grouped has no effect */
   cuttHipRowRadix rowsK; /* Mk index -> input offset (n == 0: index * strideInK) */
   cuttHipRowRadix rowsM; /* Mm index -> output offset (n == 0: index * strideOutM) */
   cuttHipTileDigits digits; /* order 7 only */
   cuttHipMbar mbar;
+  int tileWidth;           /* alignedStores only: 1 ... cuttHipLinesMaxWidth(elemSize) */
+  cuttHipDivisor widthDiv; /* division by tileWidth (cuttHipMakeDivisor) */
 } cuttHipTiledArgs;
 
 /*
@@ -295,7 +298,7 @@ typedef struct cuttHipPackedArgs {
   int maxVol;          /* largest class volume */
   uint32_t xcdChunk;   /* 0: workgroup b is logical block b; else logical block = (b % 8)*xcdChunk + b/8
                           and the grid has 8*xcdChunk workgroups */
-  int cachePolicy;     /* 0 = default, 1 = non-temporal loads, 3 = non-temporal loads and stores */
+  int cachePolicy;     /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
   long long volume;    /* elements from the first to the last one of the tensor, on its wider side (bounds every offset) */
   int wideOffsets;     /* 0: the tensor is below 4 GB and the kernel keeps 32-bit byte offsets;
                           1: element offsets with 64-bit address arithmetic (required from 4 GB on) */
@@ -345,6 +348,11 @@ const char* cuttHipErrorString(int err);
 int cuttHipValidateTiled(const cuttHipTiledArgs* args);
 int cuttHipValidateTiledCopy(const cuttHipTiledCopyArgs* args);
 int cuttHipValidatePacked(const cuttHipPackedArgs* args);
+#define CUTT_LINE_WIDTH 68
+/* Tiled with line-aligned stores: the widest tile along Mm, lanes per workgroup and bytes of LDS for a tile width. */
+int cuttHipLinesMaxWidth(int elemSize);
+int cuttHipLinesThreads(int elemSize, int tileWidth);
+size_t cuttHipLinesLdsBytes(int elemSize, int tileWidth);
 /* Workgroups of a tiled launch with these arguments (padding workgroups included), 0 if they have no valid grid. */
 long long cuttHipTiledGrid(const cuttHipTiledArgs* args);
 long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* args);

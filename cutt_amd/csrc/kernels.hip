@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "hip_layer.h"
+#include "line_windows.h"
 #include "mbar_decode.h"
 #include "packed_items.h"
 #include "row_blocks.h"
@@ -159,96 +160,73 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
 }
 
 // ---------------------------------------------------------------------------
-// Tiled with line-aligned stores.  When the output rows (runs along Mk) start off the 128-byte
-// grid, the 64-wide store of a tile row covers three lines, two of them partly, and the tile next
-// door along Mk completes them later.  Here every row of a tile takes its own window of 64
-// elements along Mk: row m, whose output run starts s_m elements past a line boundary, stores the
-// elements [64 tk - s_m, 64 tk - s_m + 64) of its run, so every store of a wave is two whole lines
-// (except at the two ends of a run).  The windows of the rows of a tile differ by up to one line,
-// so the workgroup reads up to 64 + (elements per line - 1) rows along Mk into a taller LDS tile;
-// the rows in the fringe are also read by the tile next door (from the L2).  The grid has
-// ceil((volMk + elements per line - 1) / 64) tiles along Mk.
-template <typename T>
-constexpr int kLineElems = 128 / (int)sizeof(T);
-template <typename T>
-constexpr int kAlignedRows = kTile + kLineElems<T> - 1;  // rows along Mk that a workgroup may need
+// Tiled with line-aligned stores.
+// ---------------------------------------------------------------------------
+// Bound by memory bandwidth.  When the output rows (runs along Mk) start off the 128-byte grid, the 64-wide store
+// of a tile row covers the lines at its two ends partly, and the tile next door completes them later.  Here every
+// row of a tile takes its own window of 64 elements along Mk: row m, whose output run starts s_m elements past a
+// line boundary, stores the elements [64 tk - s_m, 64 tk - s_m + 64) of its run, so a store of a wave is whole
+// lines (except at the two ends of a run) and can go past the caches.  The windows of the rows of a tile differ by
+// up to one line, so the workgroup reads up to 64 + (elements per line - 1) rows along Mk into a taller LDS tile;
+// the rows in the fringe are also read by the tile next door, from the L2, which is why the loads are temporal.
+//
+// 23425 x 8538, 8 bytes: 674 us with ordinary tiles (4.75 TB/s) -> 603 us (5.3 TB/s); 16411 x 9377, 4 bytes: 285 ->
+// 242 us; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 357 -> 316 us.  The same windows with ordinary stores gain
+// half of that, ordinary tiles with non-temporal stores lose 20-40 % (their partial lines go to memory twice).
+// 512 lanes for 8-byte elements keep 11 loads per lane in flight, 256 for
+// narrow tiles of 4-byte ones 26; twice the lanes with half the loads each are 1-2 % slower, four times 10-60 %.
+//
+// A tile is tileWidth columns wide along Mm (plan.cpp: lineTileWidth): its elements are read in order of rows and
+// columns, so that a width of 33 or 66 leaves no lane of a request idle.
+template <typename T, int TH>
+constexpr int kLineLoads = sizeof(T) == 8 ? 11 : 26;  // per lane: rows * width / TH, rounded up
 
-template <typename T, int NT>
-__global__ __launch_bounds__(kTileThreads) void tiledAlignedKernel(const cuttHipTiledArgs a,
-                                                                   const T* __restrict__ in,
-                                                                   T* __restrict__ out) {
-  constexpr int LE = kLineElems<T>;
-  constexpr int ROWS = kAlignedRows<T>;
-  constexpr int RD = (ROWS + kWaves - 1) / kWaves;  // rows a wave reads at most
-  __shared__ T tile[ROWS][kTile + 1];
+template <typename T, int TH, int NT, bool FUSED>
+__global__ __launch_bounds__(TH) void tiledLinesKernel(const cuttHipTiledArgs a, const T* __restrict__ in, T* __restrict__ out) {
+  constexpr uint32_t LE = kLineElems<T>;
+  constexpr int LOADS = kLineLoads<T, TH>;
+  static_assert(kLineRows<T> * (TH == 256 ? CUTT_LINE_WIDTH : kLineMaxWidth<T>) <= LOADS * TH, "the loads reach every element of a tile");
+  extern __shared__ __align__(16) unsigned char ldsRaw[];
+  __shared__ uint32_t rowIn[FUSED ? kLineRows<T> : 1], rowOut[FUSED ? TH : 1];
+  T* const tile = reinterpret_cast<T*>(ldsRaw);
 
   uint32_t tm, tk, offIn, offOut;
-  if (!locateTile(a, tm, tk, offIn, offOut)) return;
-
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = threadIdx.x >> 6;
-  const uint32_t m0 = tm * kTile;
-  const int32_t kBase = (int32_t)(tk * kTile) - (LE - 1);  // first row along Mk the tile may need
-  const uint32_t volMm = a.volMm, volMk = a.volMk;
-  const uint32_t wM = min((uint32_t)kTile, volMm - m0) - 1;
-  const uint32_t groupsM = (wM >> 4) + 1;
-
-  // Misalignment of output row m in elements (the low bits of its element address).  Over the
-  // rows of a tile it takes the values c + j g (mod LE), g = gcd(strideOutM, LE): the rows along
-  // Mk that some row of the tile needs are kBase + [LE - 1 - sMax, LE - 1 - sMin + 64).
+  if (!locateTile<true>(a, tm, tk, offIn, offOut)) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t outWord = (uint32_t)(reinterpret_cast<uintptr_t>(out) / sizeof(T)) + offOut;
-  const uint32_t g = min((uint32_t)LE, a.strideOutM & (0u - a.strideOutM));  // lowest set bit, capped
-  const uint32_t sMin = (outWord + m0 * a.strideOutM) & (g - 1);
-  const uint32_t sMax = sMin + (LE - g);
-  const uint32_t rowLo = (LE - 1) - sMax, rowHi = (LE - 1) - sMin + kTile;  // [rowLo, rowHi)
-
-  // Read: lanes run along input rank 0, rows along Mk (clamped to the rank's ends).
+  const LineTile t = lineTile<T>(a, tm, tk, outWord);
+  if (t.rows == 0) return;
+  if constexpr (FUSED) {
+    if (tid < t.rows) rowIn[tid] = lineRowIn<true>(a, (uint32_t)t.kLo + tid);
+    if (tid < t.width) rowOut[tid] = lineRowOut<true>(a, t.m0 + tid);
+    __syncthreads();
+  }
   {
-    const uint32_t cx = min(lane, wM);
-    const T* src = in + (offIn + m0 + cx);
-    T v[RD];
+    const uint32_t n = t.rows * t.width;
+    const uint32_t base = offIn + t.m0 + (FUSED ? 0u : (uint32_t)t.kLo * a.strideInK);
+    T v[LOADS];
+    uint32_t slot[LOADS];
 #pragma unroll
-    for (int j = 0; j < RD; j++) {
-      const uint32_t row = wave + kWaves * j;
-      if (row >= rowLo && row < rowHi) {  // uniform over the wave
-        const int32_t k = min(max(kBase + (int32_t)row, 0), (int32_t)volMk - 1);
-        v[j] = ldg<NT>(src + (uint32_t)k * a.strideInK);
+    for (int j = 0; j < LOADS; j++) {
+      if ((uint32_t)(j * TH) < n) {  // uniform over the workgroup
+        uint32_t r, c;
+        lineElem(a, t, min(tid + j * TH, n - 1), r, c);
+        slot[j] = r * t.pitch + c;
+        v[j] = ldg<NT>(in + (base + (FUSED ? rowIn[r] : r * a.strideInK) + c));
       }
     }
 #pragma unroll
-    for (int j = 0; j < RD; j++) {
-      const uint32_t row = wave + kWaves * j;
-      if (row >= rowLo && row < rowHi) tile[row][cx] = v[j];
-    }
+    for (int j = 0; j < LOADS; j++)
+      if ((uint32_t)(j * TH) < n) tile[slot[j]] = v[j];
   }
   __syncthreads();
   // Write: lanes run along Mk inside the row's own window.
-  {
-    T v[kTileRows];
-    uint32_t dstOff[kTileRows];
-#pragma unroll
-    for (int gI = 0; gI < kRowGroups; gI++) {
-      if ((uint32_t)gI < groupsM) {
-#pragma unroll
-        for (int j = gI * kGroupRows; j < (gI + 1) * kGroupRows; j++) {
-          const uint32_t r = min(wave + kWaves * j, wM);
-          const uint32_t rowStart = offOut + (m0 + r) * a.strideOutM;
-          const uint32_t sRow = (outWord - offOut + rowStart) & (LE - 1);
-          const int32_t k = min(max((int32_t)(tk * kTile) - (int32_t)sRow + (int32_t)lane, 0), (int32_t)volMk - 1);
-          // (a window that lies wholly beyond the run's end repeats the run's last element, which
-          // every LDS row from rowLo on holds in that case)
-          v[j] = tile[max(k - kBase, (int32_t)rowLo)][r];
-          dstOff[j] = rowStart + (uint32_t)k;
-        }
-      }
-    }
-#pragma unroll
-    for (int gI = 0; gI < kRowGroups; gI++) {
-      if ((uint32_t)gI < groupsM) {
-#pragma unroll
-        for (int j = gI * kGroupRows; j < (gI + 1) * kGroupRows; j++) stg<NT>(out + dstOff[j], v[j]);
-      }
-    }
+#pragma unroll 8
+  for (uint32_t r = tid >> 6; r < t.width; r += TH / 64) {
+    const uint32_t rowStart = offOut + (FUSED ? rowOut[r] : (t.m0 + r) * a.strideOutM);
+    const uint32_t s = (outWord - offOut + rowStart) & (LE - 1);
+    const int32_t k = t.kWin - (int32_t)s + (int32_t)lane;
+    if (k >= 0 && k < a.volMk) stg<NT>(out + (rowStart + (uint32_t)k), tile[(uint32_t)(k - t.kLo) * t.pitch + r]);
   }
 }
 
@@ -488,7 +466,7 @@ bool divisorOk(const cuttHipDivisor& dv, uint32_t d) {
 
 // Number of workgroups of a tiled launch; checks the ordering parameters.
 bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk, uint32_t superM,
-              uint32_t superK, const cuttHipTileDigits& dg, const cuttHipMbar& mbar, uint64_t& blocks) {
+              uint32_t superK, const cuttHipTileDigits& dg, const cuttHipMbar& mbar, uint64_t& blocks, uint64_t threads = kTileThreads) {
   uint64_t logical = (uint64_t)tilesM * tilesK * (uint64_t)volMbar;
   if (order == 7) {
     if (dg.n < 1 || dg.n > CUTT_MAX_TILE_DIGITS) return false;
@@ -533,7 +511,7 @@ bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk,
     if ((uint64_t)xcdChunk * kNumXcd < logical) return false;
     blocks = (uint64_t)xcdChunk * kNumXcd;
   }
-  return blocks > 0 && blocks <= 0x7fffffffull && blocks * kTileThreads <= CUTT_HIP_MAX_GRID_LANES;
+  return blocks > 0 && blocks <= 0x7fffffffull && blocks * threads <= CUTT_HIP_MAX_GRID_LANES;
 }
 
 // The rows of a tile axis over fused ranks: the extents must multiply to the axis' length.
@@ -641,9 +619,14 @@ hipError_t launchKernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t 
 
 }  // namespace
 
+// Lanes of a workgroup of these arguments.
+static uint32_t tiledThreads(const cuttHipTiledArgs& a) {
+  return a.alignedStores ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.tileWidth) : (uint32_t)kTileThreads;
+}
+
 extern "C" long long cuttHipTiledGrid(const cuttHipTiledArgs* a) {
   uint64_t blocks = 0;
-  if (!a || !tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
+  if (!a || !tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return 0;
   return (long long)blocks;
 }
@@ -658,38 +641,67 @@ extern "C" long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* a) {
 extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;
   if ((a->elemSize != 4 && a->elemSize != 8) || a->volMm < 1 || a->volMk < 1 || a->volMbar < 1 ||
-      a->tilesM != (a->volMm + kTile - 1) / kTile || (a->alignedStores != 0 && a->alignedStores != 1) ||
-      a->tilesK != (a->volMk + (a->alignedStores ? 128 / a->elemSize - 1 : 0) + kTile - 1) / kTile ||
+      (a->alignedStores != 0 && a->alignedStores != 1))
+    return (int)hipErrorInvalidValue;
+  const int width = a->alignedStores ? a->tileWidth : kTile, fringe = a->alignedStores ? 128 / a->elemSize - 1 : 0;
+  if (width < 1 || (a->alignedStores && (width > cuttHipLinesMaxWidth(a->elemSize) || !divisorOk(a->widthDiv, (uint32_t)width) ||
+                                         a->volMk > 0x7fffffff - 2 * kTile || a->volMm > 0x7fffffff - 2 * kTile)) ||
+      a->tilesM != (a->volMm + width - 1) / width || a->tilesK != (a->volMk + fringe + kTile - 1) / kTile ||
       a->order < 0 || a->order > 7 || !mbarOk(a->mbar) || (a->grouped != 0 && a->grouped != 1) ||
-      (a->alignedStores && a->grouped) || !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm) ||
-      (a->alignedStores && (a->rowsK.n > 0 || a->rowsM.n > 0)))
+      !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm))
     return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
+  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
-  if (a->cachePolicy != 0 && a->cachePolicy != 1 && a->cachePolicy != 3) return (int)hipErrorInvalidValue;
+  if (a->cachePolicy < 0 || a->cachePolicy > 3) return (int)hipErrorInvalidValue;
   return 0;
+}
+
+// Line-aligned stores: 8-byte elements and wide tiles of 4-byte ones take 512 lanes.
+static int launchLines(const cuttHipTiledArgs& a, const void* in, void* out, uint32_t blocks, hipStream_t s) {
+  const uint32_t threads = tiledThreads(a);
+  const dim3 grid(blocks), block(threads);
+  const size_t lds = cuttHipLinesLdsBytes(a.elemSize, a.tileWidth);
+  const bool fused = a.rowsK.n > 0 || a.rowsM.n > 0;
+#define CUTT_LAUNCH_LINES(T, TH, NT)                                                                              \
+  return (int)(fused ? launchKernel(tiledLinesKernel<T, TH, NT, true>, grid, block, lds, s, a, (const T*)in, (T*)out) \
+                     : launchKernel(tiledLinesKernel<T, TH, NT, false>, grid, block, lds, s, a, (const T*)in, (T*)out))
+#define CUTT_LAUNCH_LINES_NT(T, TH)           \
+  switch (a.cachePolicy) {                    \
+    case 0: CUTT_LAUNCH_LINES(T, TH, 0);      \
+    case 1: CUTT_LAUNCH_LINES(T, TH, 1);      \
+    case 2: CUTT_LAUNCH_LINES(T, TH, 2);      \
+    default: CUTT_LAUNCH_LINES(T, TH, 3);     \
+  }
+  if (a.elemSize == 8) {
+    CUTT_LAUNCH_LINES_NT(uint64_t, 512)
+  } else if (threads == 512) {
+    CUTT_LAUNCH_LINES_NT(uint32_t, 512)
+  } else {
+    CUTT_LAUNCH_LINES_NT(uint32_t, 256)
+  }
+#undef CUTT_LAUNCH_LINES_NT
+#undef CUTT_LAUNCH_LINES
 }
 
 extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, void* out, void* stream) {
   if (!a || !in || !out) return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
+  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
+  if (a->alignedStores) return launchLines(*a, in, out, (uint32_t)blocks, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \
   (fused ? launchKernel(tiledKernel<T, NT, G, true>, grid, block, 0, s, *a, (const T*)in, (T*)out)               \
          : launchKernel(tiledKernel<T, NT, G, false>, grid, block, 0, s, *a, (const T*)in, (T*)out))
-#define CUTT_LAUNCH_TILED(T, NT)                                                                        \
-  return (int)(a->alignedStores                                                                         \
-                   ? launchKernel(tiledAlignedKernel<T, NT>, grid, block, 0, s, *a, (const T*)in, (T*)out) \
-                   : (a->grouped ? CUTT_LAUNCH_TILED_F(T, NT, true) : CUTT_LAUNCH_TILED_F(T, NT, false)))
+#define CUTT_LAUNCH_TILED(T, NT) return (int)(a->grouped ? CUTT_LAUNCH_TILED_F(T, NT, true) : CUTT_LAUNCH_TILED_F(T, NT, false))
 #define CUTT_LAUNCH_TILED_NT(T)                                \
   switch (a->cachePolicy) {                                    \
     case 0: CUTT_LAUNCH_TILED(T, 0);                           \
     case 1: CUTT_LAUNCH_TILED(T, 1);                           \
+    case 2: CUTT_LAUNCH_TILED(T, 2);                           \
     default: CUTT_LAUNCH_TILED(T, 3);                          \
   }
   if (a->elemSize == 4) {
@@ -711,7 +723,7 @@ extern "C" int cuttHipValidateTiledCopy(const cuttHipTiledCopyArgs* a) {
   uint64_t blocks = 0;
   if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
     return (int)hipErrorInvalidConfiguration;
-  if (a->cachePolicy != 0 && a->cachePolicy != 1 && a->cachePolicy != 3) return (int)hipErrorInvalidValue;
+  if (a->cachePolicy < 0 || a->cachePolicy > 3) return (int)hipErrorInvalidValue;
   if (a->rowGather && !rowsOk(a->rows, a->elemSize)) return (int)hipErrorInvalidValue;
   return 0;
 }
@@ -753,6 +765,7 @@ extern "C" int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* a, const void*
   switch (a->cachePolicy) {                                    \
     case 0: CUTT_LAUNCH_TCOPY(T, 0);                           \
     case 1: CUTT_LAUNCH_TCOPY(T, 1);                           \
+    case 2: CUTT_LAUNCH_TCOPY(T, 2);                           \
     default: CUTT_LAUNCH_TCOPY(T, 3);                          \
   }
   if (a->elemSize == 4) {
@@ -768,7 +781,7 @@ extern "C" int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* a, const void*
 // runtime's device-to-device copy.
 extern "C" int cuttHipLaunchCopy(const void* in, void* out, size_t bytes, int cachePolicy, void* stream) {
   if (!in || !out || bytes == 0 || bytes % 4 != 0) return (int)hipErrorInvalidValue;
-  if (cachePolicy != 0 && cachePolicy != 1 && cachePolicy != 3) return (int)hipErrorInvalidValue;
+  if (cachePolicy < 0 || cachePolicy > 3) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
   if ((((uintptr_t)in | (uintptr_t)out) & 15) != 0)
     return (int)hipMemcpyAsync(out, in, bytes, hipMemcpyDeviceToDevice, s);
@@ -780,6 +793,7 @@ extern "C" int cuttHipLaunchCopy(const void* in, void* out, size_t bytes, int ca
   switch (cachePolicy) {
     case 0: return (int)launchKernel(copyKernel<0>, grid, block, 0, s, (const Vec16*)in, (Vec16*)out, n16, tailWords);
     case 1: return (int)launchKernel(copyKernel<1>, grid, block, 0, s, (const Vec16*)in, (Vec16*)out, n16, tailWords);
+    case 2: return (int)launchKernel(copyKernel<2>, grid, block, 0, s, (const Vec16*)in, (Vec16*)out, n16, tailWords);
     default: return (int)launchKernel(copyKernel<3>, grid, block, 0, s, (const Vec16*)in, (Vec16*)out, n16, tailWords);
   }
 }
@@ -872,9 +886,11 @@ extern "C" int cuttHipPreparePacked(void) {
 #define CUTT_ALLOW(T, E)                                                  \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 0, false>, m);         \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 1, false>, m);         \
+  if (r == 0) r = allowLargeLds(packedKernel<T, E, 2, false>, m);         \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, false>, m);         \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 0, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 1, true>, m);          \
+  if (r == 0) r = allowLargeLds(packedKernel<T, E, 2, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, true>, m)
     CUTT_ALLOW(uint32_t, 1); CUTT_ALLOW(uint32_t, 2); CUTT_ALLOW(uint32_t, 4); CUTT_ALLOW(uint32_t, 8);
     CUTT_ALLOW(uint32_t, 16);
@@ -905,7 +921,7 @@ extern "C" int cuttHipValidatePacked(const cuttHipPackedArgs* a) {
       a->itemOrder < 0 || a->itemOrder > 2 ||
       (a->elemsPerThread != 1 && a->elemsPerThread != 2 && a->elemsPerThread != 4 &&
        a->elemsPerThread != 8 && !(a->elemsPerThread == 16 && a->elemSize == 4)) ||
-      (a->cachePolicy != 0 && a->cachePolicy != 1 && a->cachePolicy != 3) ||
+      a->cachePolicy < 0 || a->cachePolicy > 3 ||
       a->padShift > 31 || a->ldsElems < 1 || a->ldsElems > 65536 || !mbarOk(a->mbar) || a->volume < 1 ||
       a->volume > 0xffffffffll ||
       // 32-bit byte offsets reach 4 GB
@@ -947,6 +963,7 @@ extern "C" int cuttHipLaunchPacked(const cuttHipPackedArgs* a, const void* in, v
   switch (a->cachePolicy) {                                    \
     case 0: CUTT_LAUNCH_PACKED(T, E, 0);                       \
     case 1: CUTT_LAUNCH_PACKED(T, E, 1);                       \
+    case 2: CUTT_LAUNCH_PACKED(T, E, 2);                       \
     default: CUTT_LAUNCH_PACKED(T, E, 3);                      \
   }
 #define CUTT_LAUNCH_PACKED_E(T)                                \

@@ -147,3 +147,12 @@ extern "C" int cuttHipPackedRegsPerLane(int elemSize, int elemsPerThread, int wi
   if (row == 5 || (elemSize != 4 && elemSize != 8)) return 0;
   return elemSize == 4 ? (wideOffsets ? wide4 : narrow4)[row] : (wideOffsets ? wide8 : narrow8)[row];
 }
+
+extern "C" int cuttHipLinesMaxWidth(int elemSize) { return elemSize == 8 ? CUTT_LINE_WIDTH : 2 * CUTT_LINE_WIDTH; }
+
+// 8-byte elements and wide tiles of 4-byte ones take 512 lanes.
+extern "C" int cuttHipLinesThreads(int elemSize, int tileWidth) { return elemSize == 8 || tileWidth > CUTT_LINE_WIDTH ? 512 : 256; }
+
+extern "C" size_t cuttHipLinesLdsBytes(int elemSize, int tileWidth) {
+  return (size_t)(64 + 128 / elemSize - 1) * (size_t)(tileWidth | 1) * (size_t)elemSize;
+}

@@ -215,6 +215,70 @@ Counts tiledSample(const Plan& p, bool copy, uint32_t m, std::minstd_rand0& rng,
   return total;
 }
 
+// One tile of a Tiled launch with line-aligned stores (line_windows.h) into a line-aligned buffer.
+Counts lineTileCost(const cuttHipTiledArgs& a, int64_t offIn, int64_t offOut, int tm, int tk) {
+  const int es = a.elemSize;
+  const int64_t LE = kLineBytes / es, m0 = (int64_t)tm * a.tileWidth, w = std::min<int64_t>(a.tileWidth, a.volMm - m0);
+  int64_t bits = LE;
+  if (a.rowsM.n > 0)
+    for (int k = 0; k < a.rowsM.n; k++) bits |= a.rowsM.stride[k];
+  else
+    bits |= a.strideOutM;
+  const int64_t g = bits & -bits, sMin = offOut & (g - 1), sMax = sMin + LE - g, kWin = (int64_t)tk * kTile;
+  const int64_t lo = std::max<int64_t>(kWin - sMax, 0), hi = std::min<int64_t>(kWin - sMin + kTile, a.volMk);
+  Counts c;
+  if (hi <= lo) return c;
+  std::vector<int64_t> lines, sectors;
+  for (int64_t p0 = 0, n = (hi - lo) * w; p0 < n; p0 += 64) {
+    lines.clear();
+    sectors.clear();
+    for (int64_t p = p0, end = std::min(n, p0 + 64); p < end;) {
+      const int64_t r = p / w, col = p - r * w, len = std::min(end - p, w - col);
+      const int64_t pos = offIn + m0 + rowOffset(a.rowsK, a.strideInK, lo + r) + col;
+      for (int64_t l = pos * es / kLineBytes; l <= ((pos + len) * es - 1) / kLineBytes; l++) lines.push_back(l);
+      for (int64_t l = pos * es / kSectorBytes; l <= ((pos + len) * es - 1) / kSectorBytes; l++) sectors.push_back(l);
+      p += len;
+    }
+    std::sort(lines.begin(), lines.end());
+    c.rdLines += (double)(std::unique(lines.begin(), lines.end()) - lines.begin());
+    std::sort(sectors.begin(), sectors.end());
+    c.rdSectors += (double)(std::unique(sectors.begin(), sectors.end()) - sectors.begin());
+    c.rdInstr += 1;
+  }
+  for (int64_t m = m0; m < m0 + w; m++) {
+    const int64_t start = offOut + rowOffset(a.rowsM, a.strideOutM, m), s = start & (LE - 1);
+    const int64_t k0 = std::max<int64_t>(kWin - s, 0), k1 = std::min<int64_t>(kWin - s + kTile, a.volMk);
+    if (k1 <= k0) continue;
+    runCost(start + k0, k1 - k0, es, c.wrLines, c.wrSectors, c.wrPartial);
+    c.wrInstr += 1;
+  }
+  c.ldsCycles += (c.rdInstr + c.wrInstr) * (es == 8 ? 4 : 2);
+  return c;
+}
+
+// The tiles of one Mbar position: a few of every kind (narrower last column, first and last windows) stand for the others.
+Counts lineSample(const cuttHipTiledArgs& a, uint32_t m, std::minstd_rand0& rng, bool everyTile) {
+  int64_t offIn, offOut;
+  mbarOffsets(a.mbar, m, offIn, offOut);
+  Counts total;
+  auto sample = [&](int tmLo, int tmHi, int tkLo, int tkHi) {
+    const int64_t count = (int64_t)std::max(0, tmHi - tmLo) * std::max(0, tkHi - tkLo);
+    const int64_t n = everyTile ? count : std::min<int64_t>(count, 6);
+    for (int64_t i = 0; i < n; i++) {
+      const int64_t q = n == count ? i : (int64_t)(rng() % (uint64_t)count);
+      total.add(lineTileCost(a, offIn, offOut, tmLo + (int)(q % (tmHi - tmLo)), tkLo + (int)(q / (tmHi - tmLo))), (double)count / n);
+    }
+  };
+  const int fullM = a.volMm / a.tileWidth, edge = std::max(1, a.tilesK - 2);
+  for (int last = 0; last < 2; last++) {
+    const int tmLo = last ? fullM : 0, tmHi = last ? a.tilesM : fullM;
+    sample(tmLo, tmHi, 0, 1);
+    sample(tmLo, tmHi, 1, edge);
+    sample(tmLo, tmHi, edge, a.tilesK);
+  }
+  return total;
+}
+
 // One block of a row-gathering launch (cuttHipRowArgs) into a line-aligned buffer: a wavefront's request is 64
 // consecutive output elements.
 Counts rowBlockCost(const cuttHipRowArgs& a, int64_t block) {
@@ -347,7 +411,8 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     std::uniform_int_distribution<uint32_t> pick(0, volMbar - 1);
     for (int i = 0; i < ns; i++) {
       const uint32_t m = ((uint32_t)ns == volMbar) ? (uint32_t)i : pick(rng);
-      total.add(tiledSample(plan, copy, m, rng, numSamples == 0), (double)volMbar / ns);
+      if (!copy && plan.tiled.alignedStores) total.add(lineSample(plan.tiled, m, rng, numSamples == 0), (double)volMbar / ns);
+      else total.add(tiledSample(plan, copy, m, rng, numSamples == 0), (double)volMbar / ns);
     }
   } else {
     if (!plan.buildTables()) return false;

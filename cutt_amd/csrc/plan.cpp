@@ -784,6 +784,8 @@ struct TiledShape {
   bool beyondCache = false;        // more than 0.75 memory-side cache sizes per buffer
   bool neighbourRunsInMm = false;  // a fused Mm axis of which one rank follows Mk in the output
   bool oneRankMk = false;          // a single rank along Mk
+  bool lineWindows = false;        // stores in line-aligned windows ...
+  int tileWidth = kTile;           // ... and tiles this wide along Mm
 };
 
 int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrdering& o, cuttHipTileDigits& dg) {
@@ -916,6 +918,26 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
   sk = ceilDiv(tilesK, ceilDiv(tilesK, sk));
   o.superM = (uint32_t)sm;
   o.superK = (uint32_t)sk;
+  // Line-aligned stores share no written line between tiles; what is shared are input lines, along Mm.  Measured on
+  // 25 matrices, reversals and fused plans of 7e7-2.4e8 elements of both widths, off the line grid:
+  //  - an axis of up to 16 tiles is walked whole, so that the input is read in long pieces (201 x 700299 of 4-byte
+  //    elements: 222 us against 254 with the tiles along Mk fastest; 777 x 311 x 605 reversed, 8 bytes: 486 / 520);
+  //  - so is one of up to 32, and strips of 32 otherwise, when Mk is at least twice as long (5001 x 20001, 4 bytes:
+  //    160 us against 167 and 170 with strips of 16; 2795 x 40272: 175 / 190 / 172);
+  //  - else the output is written front to back (23425 x 8538, 8 bytes: 604 us against 639 in strips of 16 and 653 in
+  //    strips of 8; 120001 x 1201, 4 bytes: 230 / 244 / 241);
+  //  - input rows a multiple of 4 KB apart are read 4 KB at a time (8192 x 11930, 4 bytes: 148 us against 195 front
+  //    to back; 8192 x 9001, 8 bytes: 221 / 274).
+  if (shape.lineWindows && opt.superAuto && opt.tiledOrder < 0 && !neighbourRunsInMm) {
+    const bool channelRows = rowBytesIn % 4096 == 0;
+    const bool strips = channelRows || tilesM <= 16 || rowBytesOut >= 2 * rowBytesIn;
+    o.order = !strips || tilesM == 1 ? 2 : (volMbar > 1 ? 5 : 3);
+    sm = std::min<int64_t>(channelRows ? 4096 / (shape.tileWidth * elemSize) : 32, tilesM);
+    sm = ceilDiv(tilesM, ceilDiv(tilesM, sm));
+    sk = tilesK;
+    o.superM = (uint32_t)sm;
+    o.superK = (uint32_t)sk;
+  }
   int64_t logical = tilesM * tilesK * volMbar;
   if (o.order >= 3) logical = ceilDiv(tilesM, sm) * ceilDiv(tilesK, sk) * sm * sk * volMbar;
   o.xcdChunk = 0;
@@ -1097,10 +1119,27 @@ bool setupRows(const Problem& pb, const PlannerOptions& opt, cuttHipRowArgs& a) 
   return true;
 }
 
+// Width of a tile along Mm for line-aligned stores.  An axis that fits a tile is one tile; a longer one is cut into
+// tiles of 64 where that fills them to within 15 %, otherwise into equal ones, whole lines wide where the rows are
+// (rows of 132 4-byte elements: 306 us as 64 + 64 + 4, 301 as 66 + 66, 294 in one piece; 75 8-byte ones: 269 us as
+// 64 + 11, 223 as 38 + 37).  Long rows of 4-byte elements are read 512 bytes at a time: eight matrices and reversals
+// of 1e8-2.4e8 elements with 1201 ... 120001 columns ran 1-7 % faster 128 wide than 64 wide,
+// none slower; rows a multiple of 4 KB apart did not (139.7 us 64 wide, 141.6 us 128 wide on 16384 x 5642).
+int lineTileWidth(int64_t volMm, int elemSize) {
+  const int64_t most = elemSize == 4 && volMm <= cuttHipLinesMaxWidth(4) ? cuttHipLinesMaxWidth(4) : CUTT_LINE_WIDTH;
+  if (volMm <= most) return (int)volMm;
+  if (elemSize == 4 && volMm >= 640 && volMm % 1024 != 0) return 2 * kTile;
+  if (ceilDiv(volMm, kTile) * kTile * 20 <= volMm * 23) return kTile;
+  const int64_t lineElems = 128 / elemSize, w = ceilDiv(volMm, ceilDiv(volMm, most));
+  return (int)(volMm % lineElems == 0 ? std::min(ceilDiv(w, lineElems) * lineElems, (int64_t)kTile) : w);
+}
+
 bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt) {
   const Split& sp = plan.split;
   const Problem& pb = plan.pb;
-  const int64_t tilesM = ceilDiv(sp.volMm, kTile);
+  const bool lines = sp.method == kTiled && opt.tiledAligned > 0;
+  const int width = lines ? lineTileWidth(sp.volMm, pb.elemSize) : kTile;
+  const int64_t tilesM = ceilDiv(sp.volMm, width);
   if (sp.method == kTiled) {
     cuttHipTiledArgs& a = plan.tiled;
     std::memset(&a, 0, sizeof(a));
@@ -1130,7 +1169,11 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       }
     }
     a.tilesM = (int)tilesM;
-    a.alignedStores = opt.tiledAligned > 0 && sp.numMm == 1 && sp.numMk == 1 ? 1 : 0;
+    a.alignedStores = lines ? 1 : 0;
+    if (lines) {
+      a.tileWidth = width;
+      a.widthDiv = cuttHipMakeDivisor((uint32_t)width);
+    }
     a.tilesK = (int)ceilDiv(sp.volMk + (a.alignedStores ? 128 / pb.elemSize - 1 : 0), kTile);
     a.volMbar = (int)sp.volMbar;
     TileOrdering o;
@@ -1160,7 +1203,9 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       shape.tilesM = a.tilesM;
       shape.tilesK = a.tilesK;
       shape.volMbar = sp.volMbar;
-      shape.volMmLastTile = sp.volMm - (tilesM - 1) * kTile;
+      shape.volMmLastTile = sp.volMm - (tilesM - 1) * width;
+      shape.lineWindows = lines;
+      shape.tileWidth = width;
       shape.rowBytesIn = sp.volMm * pb.elemSize;
       shape.rowBytesOut = sp.volMk * pb.elemSize;
       shape.elemSize = pb.elemSize;
@@ -1180,8 +1225,8 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     const int64_t tileBytes = std::min<int64_t>(sp.volMm, kTile) * std::min<int64_t>(sp.volMk, kTile) * pb.elemSize;
     if (a.order == 7 && (opt.digitLanes > 0 || (opt.digitLanes < 0 && tileBytes <= 8192))) cuttHipFinishTileDigits(&a.digits, &a.mbar);
     a.cachePolicy = opt.cachePolicy;
-    a.grouped = opt.tiledGrouped > 0 && !a.alignedStores ? 1 : 0;  // -1: decided from the model's estimate later
-    plan.ldsBytes = (size_t)(kTile + (a.alignedStores ? 128 / pb.elemSize - 1 : 0)) * (kTile + 1) * pb.elemSize;
+    a.grouped = opt.tiledGrouped > 0 ? 1 : 0;  // -1: decided from the model's estimate later
+    plan.ldsBytes = lines ? cuttHipLinesLdsBytes(pb.elemSize, width) : (size_t)kTile * (kTile + 1) * pb.elemSize;
   } else {
     cuttHipTiledCopyArgs& a = plan.tcopy;
     std::memset(&a, 0, sizeof(a));
@@ -1209,9 +1254,9 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     if (a.order == 7 && opt.digitLanes > 0) cuttHipFinishTileDigits(&a.digits, &a.mbar);
     plan.ldsBytes = 0;
   }
-  plan.numThreads = 256;
+  plan.numThreads = lines ? cuttHipLinesThreads(pb.elemSize, width) : 256;
   // one tile per workgroup: a tensor with tens of millions of tiny tiles has no Tiled candidate
-  return plan.numBlocks <= 0x7fffffffll && (uint64_t)plan.numBlocks * 256u <= CUTT_HIP_MAX_GRID_LANES;
+  return plan.numBlocks <= 0x7fffffffll && (uint64_t)plan.numBlocks * (uint64_t)plan.numThreads <= CUTT_HIP_MAX_GRID_LANES;
 }
 
 bool sameCandidate(const Split& a, const Split& b) {

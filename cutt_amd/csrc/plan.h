@@ -169,7 +169,7 @@ struct PlannerOptions {
                              // workgroups of an XCD take the items of their chunk round by round
   int padShift = 0;          // Packed/PackedSplit: LDS slot(p) = p + (p >> padShift); 0 = the default (5), 31 = no padding
   int maxItemsPerBlock = 0;  // Packed/PackedSplit: work items one workgroup handles at most; 0 = by item size
-  int cachePolicy = 1;      // 0 default, 1 non-temporal loads, 3 non-temporal loads and stores
+  int cachePolicy = 1;      // bit 0 non-temporal loads, bit 1 non-temporal stores
   int mbarOrder = 2;        // order of the Mbar ranks: 0 = input order, 1 = output order,
                             // 2 = first input rank outside Mmk, then output order
   bool wideOffsets = false; // Packed/PackedSplit: 64-bit address arithmetic also below 4 GB (tests)
