@@ -768,10 +768,12 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     p.deviceID = deviceID;
     if (p.activate() != 0 || !timeRuns(p, 1, t)) return false;
     if (t > 2.0 * bestUs) return true;
-    const int runs = t < 100.0 ? 4 : 1;
-    double first = 0;
-    if (!timeRuns(p, runs, first) || !timeRuns(p, runs, t)) return false;
-    t = std::min(t, first);
+    const int runs = t < 30.0 ? 4 : (t < 100.0 ? 2 : 1);
+    if (!timeRuns(p, runs, t)) return false;
+    if (t > 1.1 * bestUs) return true;  // a second timing moves by a few per cent
+    double second = 0;
+    if (!timeRuns(p, runs, second)) return false;
+    t = std::min(t, second);
     return true;
   };
 
