@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kTileThreads) void countTiledKernel(const cuttHipTi
 // Mirrors tiledLinesKernel writing to a line-aligned buffer (line_windows.h: lineTile, lineElem, lineRowIn, lineRowOut).
 // The bank-conflict degree is that of the column reads.
 template <typename T, int TH>
-__global__ __launch_bounds__(TH) void countLinesKernel(const cuttHipTiledArgs a, unsigned long long* total) {
+__global__ __launch_bounds__(TH) void countLinesKernel(const cuttHipTiledArgs a, const cuttHipDivisor widthDiv, unsigned long long* total) {
   constexpr uint32_t ES = sizeof(T);
   uint32_t tm, tk, offIn, offOut;
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(TH) void countLinesKernel(const cuttHipTiledArgs a,
   const uint32_t n = t.rows * t.width;
   for (uint32_t p0 = 0; p0 < n; p0 += TH) {
     uint32_t r, col;
-    lineElem(a, t, min(p0 + tid, n - 1), r, col);
+    lineElem(a, widthDiv, t, min(p0 + tid, n - 1), r, col);
     countAccess(c, false, p0 + (tid & ~63u) >= n, offIn + t.m0 + col + lineRowIn<true>(a, (uint32_t)t.kLo + r), ES);
   }
   for (uint32_t r = tid >> 6; r < t.width; r += TH / 64) {
@@ -290,12 +290,13 @@ extern "C" int cuttHipCountTiled(const cuttHipTiledArgs* a, cuttHipStreamCounts*
   if (int v = cuttHipValidateTiled(a); v != 0) return v;
   const long long blocks = cuttHipTiledGrid(a);
   if (blocks < 1) return (int)hipErrorInvalidConfiguration;
-  if (a->alignedStores)
+  if (a->lineWidth)
     return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
-      const int threads = cuttHipLinesThreads(a->elemSize, a->tileWidth);
-      if (a->elemSize == 8) return launchCount(countLinesKernel<uint64_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, d);
-      return threads == 512 ? launchCount(countLinesKernel<uint32_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, d)
-                            : launchCount(countLinesKernel<uint32_t, 256>, dim3((uint32_t)blocks), dim3(256), s, *a, d);
+      const int threads = cuttHipLinesThreads(a->elemSize, a->lineWidth);
+      const cuttHipDivisor widthDiv = cuttHipMakeDivisor((uint32_t)a->lineWidth);
+      if (a->elemSize == 8) return launchCount(countLinesKernel<uint64_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, widthDiv, d);
+      return threads == 512 ? launchCount(countLinesKernel<uint32_t, 512>, dim3((uint32_t)blocks), dim3(512), s, *a, widthDiv, d)
+                            : launchCount(countLinesKernel<uint32_t, 256>, dim3((uint32_t)blocks), dim3(256), s, *a, widthDiv, d);
     });
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
   return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {

@@ -220,7 +220,7 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.cachePolicy = cachePolicyOf(p);
   o.elemsPerThread = p.packed.elemsPerThread;
   o.tiledGrouped = p.method == kTiled ? p.tiled.grouped : 0;
-  o.tiledAligned = p.method == kTiled ? p.tiled.alignedStores : 0;
+  o.tiledAligned = p.method == kTiled && p.tiled.lineWidth > 0 ? 1 : 0;
   o.rowGather = p.method == kTiledCopy ? p.tcopy.rowGather : 0;
   o.itemOrder = (p.method == kPacked || p.method == kPackedSplit) ? p.packed.itemOrder : 0;
   o.numPieces = 1;
@@ -272,7 +272,7 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
     setCachePolicy(p, 0);
     return;
   }
-  if (p.method == kTiled && p.tiled.alignedStores) {
+  if (p.method == kTiled && p.tiled.lineWidth > 0) {
     setCachePolicy(p, 2);
     return;
   }
@@ -331,7 +331,7 @@ bool parallelFor(int n, F&& f) {
 // 0.3-0.5 GB; outside these limits the same switch costs up to 14 % (aligned or cache-sized
 // tensors, 8-byte elements).  (Not applied when CUTT_TILED_GROUPED pins the switch.)
 void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
-  if (p.method != kTiled || std::getenv("CUTT_TILED_GROUPED") || p.tiled.alignedStores) return;
+  if (p.method != kTiled || std::getenv("CUTT_TILED_GROUPED") || p.tiled.lineWidth > 0) return;
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
   const double lines = bytes / 128.0;
   const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
@@ -350,7 +350,7 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
 // with tiles of less than 256 bytes along Mm the fringe rows, read twice, cost more than the stores gain ((7,4,99,4,...),
 // 28 columns: 247 -> 298 us).  Tensors inside the cache: 24 MB +20 % time, 120 MB -1 %, left to the ordinary tiles.
 bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
-  if (p.method != kTiled || p.tiled.alignedStores) return false;
+  if (p.method != kTiled || p.tiled.lineWidth > 0) return false;
   const Problem& pb = p.pb;
   const int64_t runBytes = p.split.volMk * pb.elemSize;
   const double bytes = (double)pb.volume * pb.elemSize;
@@ -821,7 +821,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     }
     if (plans[best].method == kTiled) {
       cur.tiledGrouped = plans[best].tiled.grouped;
-      cur.tiledAligned = plans[best].tiled.alignedStores;
+      cur.tiledAligned = plans[best].tiled.lineWidth > 0 ? 1 : 0;
     }
     const PlannerOptions start = cur;
 

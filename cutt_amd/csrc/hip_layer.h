@@ -159,7 +159,7 @@ typedef struct cuttHipTiledArgs {
   int volMm, volMk;
   uint32_t strideInK;
   uint32_t strideOutM;
-  int tilesM, tilesK; /* ceil(volMm/64), ceil(volMk/64); see alignedStores for the other geometry */
+  int tilesM, tilesK; /* ceil(volMm/64), ceil(volMk/64); see lineWidth for the other geometry */
   int volMbar;
   int order;          /* logical numbering of the workgroups: 0 = Mbar fastest, 1 = tiles along Mm
                          fastest, 2 = tiles along Mk fastest, 3 / 4 = superM x superK super-tiles with the
@@ -174,16 +174,17 @@ typedef struct cuttHipTiledArgs {
   int cachePolicy;    /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
   int grouped;        /* 0: a lane has all 16 rows of its tile in flight at once; 1: four at a time
                          (each group of 16 tile rows is waited for before the next is requested) */
-  int alignedStores;  /* 1: every tile row stores its own 64-element window of the output run, shifted
-                         so that it starts on a 128-byte line; tilesK is then
-                         ceil((volMk + 128/elemSize - 1) / 64), a tile is tileWidth elements wide along Mm
-                         (tilesM = ceil(volMm/tileWidth)), and grouped has no effect */
+  int lineWidth;      /* 0: 64x64 tiles.  1 ... cuttHipLinesMaxWidth(elemSize): line-aligned stores, every tile row
+                         stores its own 64-element window of the output run, shifted so that it starts on a
+                         128-byte line; tilesK is then ceil((volMk + 128/elemSize - 1) / 64), a tile is lineWidth
+                         elements wide along Mm (tilesM = ceil(volMm/lineWidth)), and grouped has no effect */
   cuttHipRowRadix rowsK; /* Mk index -> input offset (n == 0: index * strideInK) */
   cuttHipRowRadix rowsM; /* Mm index -> output offset (n == 0: index * strideOutM) */
   cuttHipTileDigits digits; /* order 7 only */
-  cuttHipMbar mbar;
-  int tileWidth;           /* alignedStores only: 1 ... cuttHipLinesMaxWidth(elemSize) */
-  cuttHipDivisor widthDiv; /* division by tileWidth (cuttHipMakeDivisor) */
+  cuttHipMbar mbar;         /* last: the data pointers follow it in the kernel's arguments and are then read with the line
+                               that holds its last entries.  With 16 bytes more in between, which move them into a line of
+                               their own, launches of 5-13 us took 1-8 % longer: (5,18,12758,2)/(2,3,0,1), 8 bytes, 10.3 us
+                               instead of 9.5, 867 x 3788 11.9 / 11.2, 433 x 12223, 4 bytes, 9.6 / 9.3 */
 } cuttHipTiledArgs;
 
 /*

@@ -176,13 +176,13 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
 // 512 lanes for 8-byte elements keep 11 loads per lane in flight, 256 for
 // narrow tiles of 4-byte ones 26; twice the lanes with half the loads each are 1-2 % slower, four times 10-60 %.
 //
-// A tile is tileWidth columns wide along Mm (plan.cpp: lineTileWidth): its elements are read in order of rows and
+// A tile is lineWidth columns wide along Mm (plan.cpp: lineTileWidth): its elements are read in order of rows and
 // columns, so that a width of 33 or 66 leaves no lane of a request idle.
 template <typename T, int TH>
 constexpr int kLineLoads = sizeof(T) == 8 ? 11 : 26;  // per lane: rows * width / TH, rounded up
 
 template <typename T, int TH, int NT, bool FUSED>
-__global__ __launch_bounds__(TH) void tiledLinesKernel(const cuttHipTiledArgs a, const T* __restrict__ in, T* __restrict__ out) {
+__global__ __launch_bounds__(TH) void tiledLinesKernel(const cuttHipTiledArgs a, const cuttHipDivisor widthDiv, const T* __restrict__ in, T* __restrict__ out) {
   constexpr uint32_t LE = kLineElems<T>;
   constexpr int LOADS = kLineLoads<T, TH>;
   static_assert(kLineRows<T> * (TH == 256 ? CUTT_LINE_WIDTH : kLineMaxWidth<T>) <= LOADS * TH, "the loads reach every element of a tile");
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(TH) void tiledLinesKernel(const cuttHipTiledArgs a,
     for (int j = 0; j < LOADS; j++) {
       if ((uint32_t)(j * TH) < n) {  // uniform over the workgroup
         uint32_t r, c;
-        lineElem(a, t, min(tid + j * TH, n - 1), r, c);
+        lineElem(a, widthDiv, t, min(tid + j * TH, n - 1), r, c);
         slot[j] = r * t.pitch + c;
         v[j] = ldg<NT>(in + (base + (FUSED ? rowIn[r] : r * a.strideInK) + c));
       }
@@ -621,7 +621,7 @@ hipError_t launchKernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t 
 
 // Lanes of a workgroup of these arguments.
 static uint32_t tiledThreads(const cuttHipTiledArgs& a) {
-  return a.alignedStores ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.tileWidth) : (uint32_t)kTileThreads;
+  return a.lineWidth ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.lineWidth) : (uint32_t)kTileThreads;
 }
 
 extern "C" long long cuttHipTiledGrid(const cuttHipTiledArgs* a) {
@@ -640,12 +640,11 @@ extern "C" long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* a) {
 
 extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;
-  if ((a->elemSize != 4 && a->elemSize != 8) || a->volMm < 1 || a->volMk < 1 || a->volMbar < 1 ||
-      (a->alignedStores != 0 && a->alignedStores != 1))
+  if ((a->elemSize != 4 && a->elemSize != 8) || a->volMm < 1 || a->volMk < 1 || a->volMbar < 1)
     return (int)hipErrorInvalidValue;
-  const int width = a->alignedStores ? a->tileWidth : kTile, fringe = a->alignedStores ? 128 / a->elemSize - 1 : 0;
-  if (width < 1 || (a->alignedStores && (width > cuttHipLinesMaxWidth(a->elemSize) || !divisorOk(a->widthDiv, (uint32_t)width) ||
-                                         a->volMk > 0x7fffffff - 2 * kTile || a->volMm > 0x7fffffff - 2 * kTile)) ||
+  const int width = a->lineWidth ? a->lineWidth : kTile, fringe = a->lineWidth ? 128 / a->elemSize - 1 : 0;
+  if (width < 1 || (a->lineWidth && (width > cuttHipLinesMaxWidth(a->elemSize) || a->volMk > 0x7fffffff - 2 * kTile ||
+                                     a->volMm > 0x7fffffff - 2 * kTile)) ||
       a->tilesM != (a->volMm + width - 1) / width || a->tilesK != (a->volMk + fringe + kTile - 1) / kTile ||
       a->order < 0 || a->order > 7 || !mbarOk(a->mbar) || (a->grouped != 0 && a->grouped != 1) ||
       !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm))
@@ -661,11 +660,12 @@ extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
 static int launchLines(const cuttHipTiledArgs& a, const void* in, void* out, uint32_t blocks, hipStream_t s) {
   const uint32_t threads = tiledThreads(a);
   const dim3 grid(blocks), block(threads);
-  const size_t lds = cuttHipLinesLdsBytes(a.elemSize, a.tileWidth);
+  const size_t lds = cuttHipLinesLdsBytes(a.elemSize, a.lineWidth);
+  const cuttHipDivisor widthDiv = cuttHipMakeDivisor((uint32_t)a.lineWidth);
   const bool fused = a.rowsK.n > 0 || a.rowsM.n > 0;
 #define CUTT_LAUNCH_LINES(T, TH, NT)                                                                              \
-  return (int)(fused ? launchKernel(tiledLinesKernel<T, TH, NT, true>, grid, block, lds, s, a, (const T*)in, (T*)out) \
-                     : launchKernel(tiledLinesKernel<T, TH, NT, false>, grid, block, lds, s, a, (const T*)in, (T*)out))
+  return (int)(fused ? launchKernel(tiledLinesKernel<T, TH, NT, true>, grid, block, lds, s, a, widthDiv, (const T*)in, (T*)out) \
+                     : launchKernel(tiledLinesKernel<T, TH, NT, false>, grid, block, lds, s, a, widthDiv, (const T*)in, (T*)out))
 #define CUTT_LAUNCH_LINES_NT(T, TH)           \
   switch (a.cachePolicy) {                    \
     case 0: CUTT_LAUNCH_LINES(T, TH, 0);      \
@@ -690,7 +690,7 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
   if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
-  if (a->alignedStores) return launchLines(*a, in, out, (uint32_t)blocks, s);
+  if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \

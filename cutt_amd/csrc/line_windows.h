@@ -35,9 +35,9 @@ template <typename T>
 __device__ __forceinline__ LineTile lineTile(const cuttHipTiledArgs& a, uint32_t tm, uint32_t tk, uint32_t outWord) {
   constexpr uint32_t LE = kLineElems<T>;
   LineTile t;
-  t.m0 = tm * (uint32_t)a.tileWidth;
-  t.width = min((uint32_t)a.tileWidth, (uint32_t)a.volMm - t.m0);
-  t.pitch = (uint32_t)a.tileWidth | 1u;
+  t.m0 = tm * (uint32_t)a.lineWidth;
+  t.width = min((uint32_t)a.lineWidth, (uint32_t)a.volMm - t.m0);
+  t.pitch = (uint32_t)a.lineWidth | 1u;
   t.kWin = (int32_t)(tk * kWindow);
   // The rows start s = s0 + j g (mod LE) elements past a line, g = the largest power of two that divides every
   // stride of the Mm axis: the windows together cover [kWin - sMax, kWin - sMin + 64).
@@ -64,10 +64,11 @@ __device__ __forceinline__ uint32_t lineRowOut(const cuttHipTiledArgs& a, uint32
   return FUSED && a.rowsM.n > 0 ? rowOffset(a.rowsM, m) : m * a.strideOutM;
 }
 
-// The tile's input elements are read in order of rows and columns: element p (< rows * width) is column c of row r.
-__device__ __forceinline__ void lineElem(const cuttHipTiledArgs& a, const LineTile& t, uint32_t p, uint32_t& r, uint32_t& c) {
+// The tile's input elements are read in order of rows and columns: element p (< rows * width) is column c of row r;
+// `widthDiv` divides by the width of a whole tile.
+__device__ __forceinline__ void lineElem(const cuttHipTiledArgs& a, const cuttHipDivisor& widthDiv, const LineTile& t, uint32_t p, uint32_t& r, uint32_t& c) {
   // (the last tile along Mm may be narrower than the constants' divisor)
-  r = t.width == (uint32_t)a.tileWidth ? fastDivide(p, a.widthDiv.mul, a.widthDiv.shift, a.widthDiv.add) : p / t.width;
+  r = t.width == (uint32_t)a.lineWidth ? fastDivide(p, widthDiv.mul, widthDiv.shift, widthDiv.add) : p / t.width;
   c = p - r * t.width;
 }
 

@@ -218,7 +218,7 @@ Counts tiledSample(const Plan& p, bool copy, uint32_t m, std::minstd_rand0& rng,
 // One tile of a Tiled launch with line-aligned stores (line_windows.h) into a line-aligned buffer.
 Counts lineTileCost(const cuttHipTiledArgs& a, int64_t offIn, int64_t offOut, int tm, int tk) {
   const int es = a.elemSize;
-  const int64_t LE = kLineBytes / es, m0 = (int64_t)tm * a.tileWidth, w = std::min<int64_t>(a.tileWidth, a.volMm - m0);
+  const int64_t LE = kLineBytes / es, m0 = (int64_t)tm * a.lineWidth, w = std::min<int64_t>(a.lineWidth, a.volMm - m0);
   int64_t bits = LE;
   if (a.rowsM.n > 0)
     for (int k = 0; k < a.rowsM.n; k++) bits |= a.rowsM.stride[k];
@@ -269,7 +269,7 @@ Counts lineSample(const cuttHipTiledArgs& a, uint32_t m, std::minstd_rand0& rng,
       total.add(lineTileCost(a, offIn, offOut, tmLo + (int)(q % (tmHi - tmLo)), tkLo + (int)(q / (tmHi - tmLo))), (double)count / n);
     }
   };
-  const int fullM = a.volMm / a.tileWidth, edge = std::max(1, a.tilesK - 2);
+  const int fullM = a.volMm / a.lineWidth, edge = std::max(1, a.tilesK - 2);
   for (int last = 0; last < 2; last++) {
     const int tmLo = last ? fullM : 0, tmHi = last ? a.tilesM : fullM;
     sample(tmLo, tmHi, 0, 1);
@@ -411,7 +411,7 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     std::uniform_int_distribution<uint32_t> pick(0, volMbar - 1);
     for (int i = 0; i < ns; i++) {
       const uint32_t m = ((uint32_t)ns == volMbar) ? (uint32_t)i : pick(rng);
-      if (!copy && plan.tiled.alignedStores) total.add(lineSample(plan.tiled, m, rng, numSamples == 0), (double)volMbar / ns);
+      if (!copy && plan.tiled.lineWidth > 0) total.add(lineSample(plan.tiled, m, rng, numSamples == 0), (double)volMbar / ns);
       else total.add(tiledSample(plan, copy, m, rng, numSamples == 0), (double)volMbar / ns);
     }
   } else {

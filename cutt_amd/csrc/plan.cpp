@@ -1169,12 +1169,8 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       }
     }
     a.tilesM = (int)tilesM;
-    a.alignedStores = lines ? 1 : 0;
-    if (lines) {
-      a.tileWidth = width;
-      a.widthDiv = cuttHipMakeDivisor((uint32_t)width);
-    }
-    a.tilesK = (int)ceilDiv(sp.volMk + (a.alignedStores ? 128 / pb.elemSize - 1 : 0), kTile);
+    a.lineWidth = lines ? width : 0;
+    a.tilesK = (int)ceilDiv(sp.volMk + (lines ? 128 / pb.elemSize - 1 : 0), kTile);
     a.volMbar = (int)sp.volMbar;
     TileOrdering o;
     // an Mbar rank that follows Mm in the input and Mk in the output: consecutive Mbar positions are
@@ -1186,7 +1182,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     const bool beyondCache = (double)pb.volume * pb.elemSize > 0.75 * cacheBytes;
     if (!fillMbar(pb, sp.inMmk, opt.mbarOrder, a.mbar)) return false;
     int64_t byAddressBits = 0;
-    if (opt.superAuto && opt.addressBits && opt.tiledOrder < 0 && opt.tileDigits.empty() && between && !a.alignedStores && sp.volMbar > 1 &&
+    if (opt.superAuto && opt.addressBits && opt.tiledOrder < 0 && opt.tileDigits.empty() && between && !lines && sp.volMbar > 1 &&
         beyondCache)
       byAddressBits = addressBitOrder(pb, sp, a.mbar, a.tilesM, a.tilesK, a.digits);
     if (byAddressBits > 0) {
