@@ -168,7 +168,7 @@ __global__ __launch_bounds__(TH) void countLinesKernel(const cuttHipTiledArgs a,
 }
 
 // Mirrors tiledCopyKernel (its whole address arithmetic is the three lines below).
-__global__ __launch_bounds__(kTileThreads) void countTiledCopyKernel(const cuttHipTiledCopyArgs a, unsigned long long* total) {
+__global__ __launch_bounds__(kTileThreads) void countTiledCopyKernel(const cuttHipCopyTiles a, unsigned long long* total) {
   uint32_t tm, tk, offIn, offOut;
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   const uint32_t es = (uint32_t)a.elemSize;
@@ -314,7 +314,7 @@ extern "C" int cuttHipCountTiledCopy(const cuttHipTiledCopyArgs* a, cuttHipStrea
   const long long blocks = cuttHipTiledCopyGrid(a);
   if (blocks < 1) return (int)hipErrorInvalidConfiguration;
   return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
-    return launchCount(countTiledCopyKernel, dim3((uint32_t)blocks), dim3(kTileThreads), s, *a, d);
+    return launchCount(countTiledCopyKernel, dim3((uint32_t)blocks), dim3(kTileThreads), s, a->tiles, d);
   });
 }
 

@@ -178,7 +178,7 @@ bool currentDevice(int& deviceID, cuttHipDeviceProps& props) {
 
 int cachePolicyOf(const Plan& p) {
   if (p.method == kTiled) return p.tiled.cachePolicy;
-  if (p.method == kTiledCopy) return p.tcopy.rowGather ? p.tcopy.rows.cachePolicy : p.tcopy.cachePolicy;
+  if (p.method == kTiledCopy) return p.tcopy.rowGather ? p.tcopy.rows.cachePolicy : p.tcopy.tiles.cachePolicy;
   return p.packed.cachePolicy;
 }
 
@@ -205,7 +205,7 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.numBlocks = p.numBlocks;
   o.numThreads = p.numThreads;
   o.itemsPerBlock = p.packed.itemsPerBlock;
-  o.tiledOrder = p.method == kTiled ? p.tiled.order : p.tcopy.order;
+  o.tiledOrder = p.method == kTiled ? p.tiled.order : p.tcopy.tiles.order;
   o.ldsBytes = p.ldsBytes;
   o.usPredicted = p.model.usPredicted;
   o.rdLines = p.model.rdLines;
@@ -226,13 +226,13 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.numPieces = 1;
   o.numShapes = 1;
   o.wideOffsets = (p.method == kPacked || p.method == kPackedSplit) ? p.packed.wideOffsets : 0;
-  o.superM = p.method == kTiled ? (int)p.tiled.superM : (p.method == kTiledCopy ? (int)p.tcopy.superM : 0);
-  o.superK = p.method == kTiled ? (int)p.tiled.superK : (p.method == kTiledCopy ? (int)p.tcopy.superK : 0);
+  o.superM = p.method == kTiled ? (int)p.tiled.superM : (p.method == kTiledCopy ? (int)p.tcopy.tiles.superM : 0);
+  o.superK = p.method == kTiled ? (int)p.tiled.superK : (p.method == kTiledCopy ? (int)p.tcopy.tiles.superK : 0);
   o.rdEdgeDist = p.model.rdEdgeDist;
   o.wrEdgeDist = p.model.wrEdgeDist;
   std::memset(o.tileDigits, 0, sizeof(o.tileDigits));
   if ((p.method == kTiled || p.method == kTiledCopy) && o.tiledOrder == 7) {
-    const std::string t = formatTileDigits(p.method == kTiled ? p.tiled.digits : p.tcopy.digits);
+    const std::string t = formatTileDigits(p.method == kTiled ? p.tiled.digits : p.tcopy.tiles.digits);
     std::strncpy(o.tileDigits, t.c_str(), sizeof(o.tileDigits) - 1);
   } else if ((p.method == kPacked || p.method == kPackedSplit) && p.itemDigits.n > 0) {
     const std::string t = formatTileDigits(p.itemDigits);
@@ -243,7 +243,7 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
 void setCachePolicy(Plan& p, int policy) {
   if (p.method == kTiledCopy && p.tcopy.rowGather) return;  // chosen with the row gathering (plan.cpp: setupRows)
   p.tiled.cachePolicy = policy;
-  p.tcopy.cachePolicy = policy;
+  p.tcopy.tiles.cachePolicy = policy;
   p.packed.cachePolicy = policy;
 }
 
@@ -804,12 +804,12 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     if (!rowGather) cur.cachePolicy = cachePolicyOf(plans[best]);
     if (tiled) {
       const bool t = plans[best].method == kTiled;
-      cur.tiledOrder = t ? plans[best].tiled.order : plans[best].tcopy.order;
-      cur.superM = (int)(t ? plans[best].tiled.superM : plans[best].tcopy.superM);
-      cur.superK = (int)(t ? plans[best].tiled.superK : plans[best].tcopy.superK);
+      cur.tiledOrder = t ? plans[best].tiled.order : plans[best].tcopy.tiles.order;
+      cur.superM = (int)(t ? plans[best].tiled.superM : plans[best].tcopy.tiles.superM);
+      cur.superK = (int)(t ? plans[best].tiled.superK : plans[best].tcopy.tiles.superK);
       cur.superAuto = false;
       if (cur.tiledOrder == 7) {  // a free numbering is reproduced from its digits
-        cur.tileDigits = formatTileDigits(t ? plans[best].tiled.digits : plans[best].tcopy.digits);
+        cur.tileDigits = formatTileDigits(t ? plans[best].tiled.digits : plans[best].tcopy.tiles.digits);
         cur.tiledOrder = -1;
       }
     } else if (!rowGather) {
@@ -1303,7 +1303,7 @@ extern "C" long long cuttCandidatesData(void* list, int index, int what, int cls
     const bool packed = p.method == kPacked || p.method == kPackedSplit;
     switch (what) {
       case 0: {
-        const cuttHipMbar& mb = packed ? p.packed.mbar : (p.method == kTiled ? p.tiled.mbar : p.tcopy.mbar);
+        const cuttHipMbar& mb = packed ? p.packed.mbar : (p.method == kTiled ? p.tiled.mbar : p.tcopy.tiles.mbar);
         if (p.method == kTrivial) break;
         for (int k = 0; k < mb.n; k++) {
           v.push_back(mb.d[k].extent);
@@ -1316,8 +1316,8 @@ extern "C" long long cuttCandidatesData(void* list, int index, int what, int cls
           v = {p.tiled.volMm, p.tiled.volMk, p.tiled.strideInK, p.tiled.strideOutM, p.tiled.tilesM,
                p.tiled.tilesK, p.tiled.volMbar, p.tiled.order, p.tiled.xcdChunk, p.tiled.superM, p.tiled.superK};
         else if (p.method == kTiledCopy)
-          v = {p.tcopy.volMm, p.tcopy.volMk, p.tcopy.strideInK, p.tcopy.strideOutK, p.tcopy.tilesM,
-               p.tcopy.tilesK, p.tcopy.volMbar, p.tcopy.order, p.tcopy.xcdChunk, p.tcopy.superM, p.tcopy.superK};
+          v = {p.tcopy.tiles.volMm, p.tcopy.tiles.volMk, p.tcopy.tiles.strideInK, p.tcopy.tiles.strideOutK, p.tcopy.tiles.tilesM,
+               p.tcopy.tiles.tilesK, p.tcopy.tiles.volMbar, p.tcopy.tiles.order, p.tcopy.tiles.xcdChunk, p.tcopy.tiles.superM, p.tcopy.tiles.superK};
         else
           return -1;
         break;
@@ -1360,7 +1360,7 @@ extern "C" long long cuttCandidatesData(void* list, int index, int what, int cls
       case 8:  // tile order 7 / work-item order 3: (coordinate, radix, weight) of the digits, fastest first
         if (p.method != kTiled && p.method != kTiledCopy && !packed) return -1;
         {
-          const cuttHipTileDigits& dg = packed ? p.itemDigits : (p.method == kTiled ? p.tiled.digits : p.tcopy.digits);
+          const cuttHipTileDigits& dg = packed ? p.itemDigits : (p.method == kTiled ? p.tiled.digits : p.tcopy.tiles.digits);
           for (int k = 0; k < dg.n; k++) {
             v.push_back(dg.d[k].which);
             v.push_back(dg.d[k].radix);
@@ -1372,7 +1372,7 @@ extern "C" long long cuttCandidatesData(void* list, int index, int what, int cls
                // then per digit radix, stepM, stepK, strideIn, strideOut
         if (p.method != kTiled && p.method != kTiledCopy) return -1;
         {
-          const cuttHipTileDigits& dg = p.method == kTiled ? p.tiled.digits : p.tcopy.digits;
+          const cuttHipTileDigits& dg = p.method == kTiled ? p.tiled.digits : p.tcopy.tiles.digits;
           v.push_back(dg.lanes);
           v.push_back(dg.total);
           for (int k = 0; k < dg.n && dg.lanes; k++)

@@ -220,7 +220,7 @@ uint64_t cuttHipRowGrid(const cuttHipRowArgs* a);
  * volMm) are copied; the second output rank (extent volMk, input stride
  * strideInK, output stride strideOutK) is the other tile axis.  No LDS.
  */
-typedef struct cuttHipTiledCopyArgs {
+typedef struct cuttHipCopyTiles {
   int elemSize;
   int volMm, volMk;
   uint32_t strideInK;
@@ -231,10 +231,15 @@ typedef struct cuttHipTiledCopyArgs {
   uint32_t xcdChunk;
   uint32_t superM, superK;
   int cachePolicy;
-  int rowGather;            /* 1: the launch takes `rows` (dense tensors with rows of 64 bytes and more); 0: 64x64 tiles */
-  cuttHipRowArgs rows;
   cuttHipTileDigits digits; /* order 7 only */
   cuttHipMbar mbar;
+} cuttHipCopyTiles;
+
+/* A launch hands its kernel one of the two blocks. */
+typedef struct cuttHipTiledCopyArgs {
+  cuttHipCopyTiles tiles;
+  int rowGather;  /* 1: the launch takes `rows` (dense tensors with rows of 64 bytes and more); 0: 64x64 tiles */
+  cuttHipRowArgs rows;
 } cuttHipTiledCopyArgs;
 
 /*

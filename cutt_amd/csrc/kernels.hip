@@ -234,7 +234,7 @@ __global__ __launch_bounds__(TH) void tiledLinesKernel(const cuttHipTiledArgs a,
 // TiledCopy: rank 0 stays in front; rows are copied through registers.
 // ---------------------------------------------------------------------------
 template <typename T, int NT>
-__global__ __launch_bounds__(kTileThreads) void tiledCopyKernel(const cuttHipTiledCopyArgs a,
+__global__ __launch_bounds__(kTileThreads) void tiledCopyKernel(const cuttHipCopyTiles a,
                                                                 const T* __restrict__ in,
                                                                 T* __restrict__ out) {
   uint32_t tm, tk, offIn, offOut;
@@ -619,6 +619,10 @@ hipError_t launchKernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t 
 
 }  // namespace
 
+static bool copyTileGrid(const cuttHipCopyTiles& t, uint64_t& blocks) {
+  return tileGrid(t.order, t.tilesM, t.tilesK, t.volMbar, t.xcdChunk, t.superM, t.superK, t.digits, t.mbar, blocks);
+}
+
 // Lanes of a workgroup of these arguments.
 static uint32_t tiledThreads(const cuttHipTiledArgs& a) {
   return a.lineWidth ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.lineWidth) : (uint32_t)kTileThreads;
@@ -633,8 +637,7 @@ extern "C" long long cuttHipTiledGrid(const cuttHipTiledArgs* a) {
 
 extern "C" long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* a) {
   uint64_t blocks = 0;
-  if (!a || !tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
-    return 0;
+  if (!a || !copyTileGrid(a->tiles, blocks)) return 0;
   return (long long)blocks;
 }
 
@@ -716,15 +719,14 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
 
 extern "C" int cuttHipValidateTiledCopy(const cuttHipTiledCopyArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;
-  if ((a->elemSize != 4 && a->elemSize != 8) || a->volMm < 1 || a->volMk < 1 || a->volMbar < 1 ||
-      a->tilesM != (a->volMm + kTile - 1) / kTile || a->tilesK != (a->volMk + kTile - 1) / kTile ||
-      a->order < 0 || a->order > 7 || !mbarOk(a->mbar))
+  const cuttHipCopyTiles& t = a->tiles;
+  if ((t.elemSize != 4 && t.elemSize != 8) || t.volMm < 1 || t.volMk < 1 || t.volMbar < 1 || t.tilesM != (t.volMm + kTile - 1) / kTile ||
+      t.tilesK != (t.volMk + kTile - 1) / kTile || t.order < 0 || t.order > 7 || !mbarOk(t.mbar))
     return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
-    return (int)hipErrorInvalidConfiguration;
-  if (a->cachePolicy < 0 || a->cachePolicy > 3) return (int)hipErrorInvalidValue;
-  if (a->rowGather && !rowsOk(a->rows, a->elemSize)) return (int)hipErrorInvalidValue;
+  if (!copyTileGrid(t, blocks)) return (int)hipErrorInvalidConfiguration;
+  if (t.cachePolicy < 0 || t.cachePolicy > 3) return (int)hipErrorInvalidValue;
+  if (a->rowGather && !rowsOk(a->rows, t.elemSize)) return (int)hipErrorInvalidValue;
   return 0;
 }
 
@@ -755,20 +757,19 @@ extern "C" int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* a, const void*
   if (!a || !in || !out) return (int)hipErrorInvalidValue;
   if (a->rowGather) return launchRows(a->rows, in, out, (hipStream_t)stream);
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks))
-    return (int)hipErrorInvalidConfiguration;
+  if (!copyTileGrid(a->tiles, blocks)) return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
 #define CUTT_LAUNCH_TCOPY(T, NT) \
-  return (int)launchKernel(tiledCopyKernel<T, NT>, grid, block, 0, s, *a, (const T*)in, (T*)out)
+  return (int)launchKernel(tiledCopyKernel<T, NT>, grid, block, 0, s, a->tiles, (const T*)in, (T*)out)
 #define CUTT_LAUNCH_TCOPY_NT(T)                                \
-  switch (a->cachePolicy) {                                    \
+  switch (a->tiles.cachePolicy) {                              \
     case 0: CUTT_LAUNCH_TCOPY(T, 0);                           \
     case 1: CUTT_LAUNCH_TCOPY(T, 1);                           \
     case 2: CUTT_LAUNCH_TCOPY(T, 2);                           \
     default: CUTT_LAUNCH_TCOPY(T, 3);                          \
   }
-  if (a->elemSize == 4) {
+  if (a->tiles.elemSize == 4) {
     CUTT_LAUNCH_TCOPY_NT(uint32_t)
   } else {
     CUTT_LAUNCH_TCOPY_NT(uint64_t)

@@ -161,15 +161,15 @@ Counts tileCost(bool copy, int es, int64_t offIn, int64_t offOut, int64_t m0, in
 
 Counts tiledSample(const Plan& p, bool copy, uint32_t m, std::minstd_rand0& rng, bool everyTile) {
   const int es = p.pb.elemSize;
-  const int volMm = copy ? p.tcopy.volMm : p.tiled.volMm;
-  const int volMk = copy ? p.tcopy.volMk : p.tiled.volMk;
-  const int64_t sIn = copy ? p.tcopy.strideInK : p.tiled.strideInK;
-  const int64_t sOut = copy ? p.tcopy.strideOutK : p.tiled.strideOutM;
+  const int volMm = copy ? p.tcopy.tiles.volMm : p.tiled.volMm;
+  const int volMk = copy ? p.tcopy.tiles.volMk : p.tiled.volMk;
+  const int64_t sIn = copy ? p.tcopy.tiles.strideInK : p.tiled.strideInK;
+  const int64_t sOut = copy ? p.tcopy.tiles.strideOutK : p.tiled.strideOutM;
   static const cuttHipRowRadix kSingle = {};
   const cuttHipRowRadix& rowsK = copy ? kSingle : p.tiled.rowsK;
   const cuttHipRowRadix& rowsM = copy ? kSingle : p.tiled.rowsM;
   int64_t offIn, offOut;
-  mbarOffsets(copy ? p.tcopy.mbar : p.tiled.mbar, m, offIn, offOut);
+  mbarOffsets(copy ? p.tcopy.tiles.mbar : p.tiled.mbar, m, offIn, offOut);
   const int fullM = volMm / kTile, fullK = volMk / kTile;
   const int remM = volMm % kTile, remK = volMk % kTile;
   Counts total;
@@ -497,12 +497,12 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     // tile: the next workgroup along Mm, superM workgroups on along Mk (strip order).  A rank that
     // fits one tile ends its runs at the rank's end: the next run belongs to another Mbar position.
     const bool copy = plan.method == kTiledCopy;
-    const cuttHipMbar& mb = copy ? plan.tcopy.mbar : plan.tiled.mbar;
-    const double tilesM = copy ? plan.tcopy.tilesM : plan.tiled.tilesM;
-    const double tilesK = copy ? plan.tcopy.tilesK : plan.tiled.tilesK;
-    const double superM = copy ? plan.tcopy.superM : plan.tiled.superM;
+    const cuttHipMbar& mb = copy ? plan.tcopy.tiles.mbar : plan.tiled.mbar;
+    const double tilesM = copy ? plan.tcopy.tiles.tilesM : plan.tiled.tilesM;
+    const double tilesK = copy ? plan.tcopy.tiles.tilesK : plan.tiled.tilesK;
+    const double superM = copy ? plan.tcopy.tiles.superM : plan.tiled.superM;
     const Problem& pb = plan.pb;
-    const int order = copy ? plan.tcopy.order : plan.tiled.order;
+    const int order = copy ? plan.tcopy.tiles.order : plan.tiled.order;
     auto mbarDist = [&](int rank, bool input) -> double {
       // order 5 walks the Mbar positions strip by strip, the others tensor slice by tensor slice
       double d = order >= 5 ? std::min(superM, tilesM) * tilesK : tilesM * tilesK;
@@ -583,13 +583,13 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     factor = (es == 4 ? 0.90 : 0.86) + 0.10 * kLineBytes / rowBytes + (rowBytes < 96.0 ? 0.15 : 0.0);
   } else if (plan.method == kTiled || plan.method == kTiledCopy) {
     const bool copy = plan.method == kTiledCopy;
-    const double tilesM = copy ? plan.tcopy.tilesM : plan.tiled.tilesM;
-    const double tilesK = copy ? plan.tcopy.tilesK : plan.tiled.tilesK;
+    const double tilesM = copy ? plan.tcopy.tiles.tilesM : plan.tiled.tilesM;
+    const double tilesK = copy ? plan.tcopy.tiles.tilesK : plan.tiled.tilesK;
     // Issued lane-slots over useful ones: a request is 64 lanes wide whatever the tile's width, and
     // an edge tile issues its rows in groups of 16 (loads run over Mk rows; the stores of a Tiled
     // plan run over Mm rows, those of a TiledCopy plan over Mk rows again).
-    const double volMm = copy ? plan.tcopy.volMm : plan.tiled.volMm;
-    const double volMk = copy ? plan.tcopy.volMk : plan.tiled.volMk;
+    const double volMm = copy ? plan.tcopy.tiles.volMm : plan.tiled.volMm;
+    const double volMk = copy ? plan.tcopy.tiles.volMk : plan.tiled.volMk;
     auto rows16 = [](double n) { return std::ceil(n / 16.0) * 16.0; };
     const double rdSlots = tilesM * kTile * rows16(volMk);
     const double wrSlots = copy ? rdSlots : rows16(volMm) * tilesK * kTile;

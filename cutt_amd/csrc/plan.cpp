@@ -1224,8 +1224,8 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     a.grouped = opt.tiledGrouped > 0 ? 1 : 0;  // -1: decided from the model's estimate later
     plan.ldsBytes = lines ? cuttHipLinesLdsBytes(pb.elemSize, width) : (size_t)kTile * (kTile + 1) * pb.elemSize;
   } else {
-    cuttHipTiledCopyArgs& a = plan.tcopy;
-    std::memset(&a, 0, sizeof(a));
+    std::memset(&plan.tcopy, 0, sizeof(plan.tcopy));
+    cuttHipCopyTiles& a = plan.tcopy.tiles;
     const int rk = pb.perm[sp.numMk - 1];
     a.elemSize = pb.elemSize;
     a.volMm = (int)sp.volMm;

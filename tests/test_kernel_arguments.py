@@ -12,6 +12,7 @@ PROGRAM = """
 #include "hip_layer.h"
 int main() {
   std::printf("%zu %zu\\n", offsetof(cuttHipTiledArgs, mbar) + sizeof(cuttHipMbar), sizeof(cuttHipTiledArgs));
+  std::printf("%zu %zu\\n", offsetof(cuttHipCopyTiles, mbar) + sizeof(cuttHipMbar), sizeof(cuttHipCopyTiles));
 }
 """
 
@@ -25,3 +26,12 @@ def test_data_pointers_share_the_line_of_the_last_mbar_entries(tmp_path):
     for line in subprocess.check_output([exe], text=True).splitlines():
         mbar_end, pointers = map(int, line.split())
         assert (mbar_end - 1) // 128 == pointers // 128, line
+
+
+def test_copy_tiles_carry_no_row_table(tmp_path):
+    # scalars, the digit list of a free tile order and the Mbar table: 1736 bytes; the 552 bytes of cuttHipRowArgs go to the
+    # kernel that reads them
+    src = tmp_path / "copy.cpp"
+    src.write_text('#include "hip_layer.h"\nstatic_assert(sizeof(cuttHipCopyTiles) == 13 * 4 + sizeof(cuttHipTileDigits) + sizeof(cuttHipMbar), "");\n')
+    subprocess.check_call(["g++", "-std=c++17", "-fsyntax-only", "-I" + os.path.join(ROOT, "cutt_amd", "csrc"),
+                           "-I" + os.path.join(ROOT, "include"), str(src)])
