@@ -581,6 +581,19 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     // for 150-250 bytes, about 1 at 80-100 bytes, up to 1.3 below that.
     const double rowBytes = (double)plan.tcopy.rows.rowLen * es;
     factor = (es == 4 ? 0.90 : 0.86) + 0.10 * kLineBytes / rowBytes + (rowBytes < 96.0 ? 0.15 : 0.0);
+    // Rows off the line grid share lines with the next row of the input.  Where that row is written a group of blocks
+    // or more later (another XCD, another L2) those lines are fetched again.  820 tensors of 4-400 MB per buffer with
+    // rows of 64-1500 bytes, timed on freshly written inputs, with buffers in rotation and with the same ones, against
+    // the plan taken without this kernel: with the next row at hand 0.7-1.0 of its time whatever the row length; far
+    // from it up to 16 MB the same; beyond that 0.95-1.1 at 1.4-2.3 requested lines per line of data and 1.1-1.4 above
+    // ((10,102,6062)/(0,2,1), 8 bytes: 33.5 against 23.7 us, estimated 22.3 against 23.2).  With this term 36 instead of
+    // 124 of the 820 lose more than 3 %; of 420 others, up to 1.2 GB, timed after it was chosen, 12 instead of 59 do.
+    const cuttHipRowArgs& a = plan.tcopy.rows;
+    const double cacheBytes = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
+    double nextRow = (double)a.rowLen;  // output elements between two neighbouring rows of the input
+    for (int k = 0; k < a.n && a.rank[k].stride != a.rowLen; k++) nextRow *= a.rank[k].extent;
+    const double group = (double)CUTT_ROW_BLOCK * (a.xcdGroup ? 1 << (a.xcdGroup - 1) : 1);
+    if (bytes > 0.06 * cacheBytes && nextRow >= group) factor *= 1.0 + 0.4 * std::max(0.0, rdAmp - 1.4);
   } else if (plan.method == kTiled || plan.method == kTiledCopy) {
     const bool copy = plan.method == kTiledCopy;
     const double tilesM = copy ? plan.tcopy.tiles.tilesM : plan.tiled.tilesM;
