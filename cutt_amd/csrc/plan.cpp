@@ -1092,7 +1092,7 @@ int64_t addressBitOrder(const Problem& pb, const Split& sp, const cuttHipMbar& m
 
 // Arguments of the row-gathering kernel for a problem whose leading rank stays; false where the 64x64 copy tiles
 // have to do: pieces of a larger tensor (their output has gaps) and rows of less than 64 bytes.
-bool setupRows(const Problem& pb, const PlannerOptions& opt, cuttHipRowArgs& a) {
+bool setupRows(const Problem& pb, const cuttHipDeviceProps& props, const PlannerOptions& opt, cuttHipRowArgs& a) {
   std::memset(&a, 0, sizeof(a));
   if (!pb.dense || pb.rank < 2 || pb.perm[0] != 0 || (int64_t)pb.dim[0] * pb.elemSize < 64 || pb.volume > 0xffffffffll) return false;
   a.elemSize = pb.elemSize;
@@ -1105,12 +1105,18 @@ bool setupRows(const Problem& pb, const PlannerOptions& opt, cuttHipRowArgs& a) 
     const cuttHipDivisor dv = cuttHipMakeDivisor((uint32_t)pb.dim[r]);
     a.rank[a.n++] = cuttHipRowRank{(uint32_t)pb.dim[r], (uint32_t)pb.strideIn[r], dv.mul, dv.shift | dv.add << 8};
   }
-  // Non-temporal stores always (the lines are written whole).  Non-temporal loads only for long rows of 8-byte
-  // elements beyond the caches: 4-21 % faster there ((533853,15,5)/(0,2,1) 105 -> 94 us, (159,140130,2)/(0,2,1)
-  // 117 -> 107 us), but rows share the lines at their ends, and those are read again: rows of 216-720 bytes ran
-  // 6-20 % slower, cache-sized tensors 15-30 %, 4-byte elements 0-4 %.
-  const int64_t rowBytes = (int64_t)a.rowLen * pb.elemSize, bytes = pb.volume * pb.elemSize;
-  a.cachePolicy = opt.rowPolicy >= 0 ? opt.rowPolicy : (pb.elemSize == 8 && rowBytes >= 800 && bytes >= ((int64_t)96 << 20) ? 3 : 2);
+  // Non-temporal stores always (the lines are written whole).  Against ordinary ones, with buffers in rotation / the
+  // same ones again / on an input just written: 0.87 / 0.98 / 1.00 of the time on 58 tensors of 4-byte elements that fit
+  // the memory-side cache twice, 0.93 / 0.95 / 0.99 on 56 of 8-byte ones, 0.93-0.97 / 0.84-0.95 / 0.96-1.00 on 100 larger.
+  // Non-temporal loads only for long rows of 8-byte elements of which the cache holds little: in rotation / on an input
+  // just written 0.86-1.00 / 0.85-1.05 (one cache size per buffer and more, (533853,15,5)/(0,2,1) 105 -> 94 us in
+  // rotation), but 0.88 / 1.2-1.4 at 0.4-0.75 cache sizes, and 1.15-1.25 for writing it, transposing and reading the
+  // result in turn.  Rows share the lines at their ends, and those are read again: rows below 800 bytes ran 0.95-1.07 /
+  // 0.98-1.2, 4-byte elements 1.03-1.16 / 1.1-1.4.
+  const int64_t rowBytes = (int64_t)a.rowLen * pb.elemSize;
+  const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
+  const bool streamLoads = pb.elemSize == 8 && rowBytes >= 800 && (double)pb.volume * pb.elemSize >= 0.75 * cache;
+  a.cachePolicy = opt.rowPolicy >= 0 ? opt.rowPolicy : (streamLoads ? 3 : 2);
   // Every XCD takes groups of 64 neighbouring blocks, so that the row two blocks share is read into one L2: 0-2 %
   // faster than single blocks dealt out in turn on 40 random tensors, 15-20 % where rows are 64-150 bytes long.
   // Below 8192 blocks (32 MB of 4-byte elements) the last round of groups would leave XCDs idle.
@@ -1306,7 +1312,7 @@ void addTiled(const Problem& red, const cuttHipDeviceProps& props, const Planner
     // ... or gather the rows in output order, which needs no second tile axis (unless the options pin a tile order)
     if (opt.rowGather && opt.tiledOrder < 0 && opt.tileDigits.empty()) {
       Plan q = p.clone();
-      q.tcopy.rowGather = setupRows(red, opt, q.tcopy.rows) ? 1 : 0;
+      q.tcopy.rowGather = setupRows(red, props, opt, q.tcopy.rows) ? 1 : 0;
       if (q.tcopy.rowGather) plans.push_back(std::move(q));
     }
     plans.push_back(std::move(p));
@@ -1515,7 +1521,7 @@ bool rebuildPlan(const Plan& src, const cuttHipDeviceProps& props, const Planner
     case kTiled:
     case kTiledCopy:
       if (!setupTiled(out, props, opt)) return false;
-      if (src.method == kTiledCopy && src.tcopy.rowGather) out.tcopy.rowGather = setupRows(out.pb, opt, out.tcopy.rows) ? 1 : 0;
+      if (src.method == kTiledCopy && src.tcopy.rowGather) out.tcopy.rowGather = setupRows(out.pb, props, opt, out.tcopy.rows) ? 1 : 0;
       return true;
     case kPacked:
     case kPackedSplit:

@@ -22,3 +22,17 @@ TIMED = [  # dim, perm, element bytes, row gathering, the plan without it
 def test_the_faster_of_the_two_is_chosen(cutt, dim, perm, es, gather_us, other_us):
     with cutt.Candidates(list(dim), list(perm), es) as c:
         assert c.info(c.best).rowGather == int(gather_us < other_us)
+
+
+@pytest.mark.parametrize("dim,es,policy", [
+    ((1000, 20, 30), 8, 2),       # 5 MB
+    ((1000, 130, 140), 8, 2),     # 146 MB: 0.54 cache sizes
+    ((1000, 155, 160), 8, 2),     # 0.74
+    ((1000, 160, 160), 8, 3),     # 0.76
+    ((1000, 300, 300), 8, 3),
+    ((99, 500, 900), 8, 2),       # rows of 792 bytes
+    ((2000, 300, 300), 4, 2),
+])
+def test_loads_go_past_the_caches_only_where_these_hold_little(cutt, dim, es, policy):
+    with cutt.Candidates(list(dim), [0, 2, 1], es) as c:
+        assert [c.info(i).cachePolicy for i in range(len(c)) if c.info(i).rowGather] == [policy]
