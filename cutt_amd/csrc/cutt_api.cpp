@@ -747,11 +747,15 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   void* const evStop = events.stop;
   double bestUs = 1e300;
   bool failed = false;
-  // Time of one run among runs of plan p, which is what a program that keeps the plan sees: a first run, timed only
-  // to drop hopeless plans, leaves the caches as such a program leaves them, the next ones count.  (Filling the output
-  // before every timed run instead leaves the memory-side cache full of lines that the run then overwrites in place:
-  // (40,14881,4,6,14)/(3,2,0,1,4) with 4-byte elements got plans of 299 or 320 us that way, now 294 us.)  False on a
-  // HIP error.
+  // Time of one run among runs of plan p, which is what a program that keeps the plan sees.  A first run leaves the
+  // caches as such a program leaves them; it may have to load the kernel's code (hundreds of microseconds) and drops a
+  // plan only where that cannot be the reason.  The second run, alone between the events like every plan's, drops those
+  // that take twice as long as the fastest second run; what counts comes after it, averaged over a few runs where they
+  // are short.  (Filling the output before every timed run instead leaves the memory-side cache full of lines that the
+  // run then overwrites in place: (40,14881,4,6,14)/(3,2,0,1,4) with 4-byte elements got plans of 299 or 320 us that
+  // way, 297 without.)  False on a HIP error.
+  constexpr double kFirstRunUs = 1000.0;
+  double bestSecondUs = 1e300;
   auto timeRuns = [&](Plan& p, int runs, double& t) -> bool {
     float ms = 0;
     if (cuttHipEventRecord(evStart, (void*)stream) != 0) return false;
@@ -767,10 +771,13 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     p.stream = (void*)stream;
     p.deviceID = deviceID;
     if (p.activate() != 0 || !timeRuns(p, 1, t)) return false;
-    if (t > 2.0 * bestUs) return true;
+    if (t > 2.0 * bestUs + kFirstRunUs) return true;
+    if (!timeRuns(p, 1, t)) return false;
+    if (t > 2.0 * bestSecondUs) return true;
+    bestSecondUs = std::min(bestSecondUs, t);
     const int runs = t < 30.0 ? 4 : (t < 100.0 ? 2 : 1);
-    if (!timeRuns(p, runs, t)) return false;
-    if (t > 1.1 * bestUs) return true;  // a second timing moves by a few per cent
+    if (runs > 1 && !timeRuns(p, runs, t)) return false;
+    if (t > 1.1 * bestUs) return true;  // another timing moves by a few per cent
     double second = 0;
     if (!timeRuns(p, runs, second)) return false;
     t = std::min(t, second);

@@ -1,0 +1,88 @@
+// cuttPlanMeasure on a device whose clock is simulated (no GPU): launches take the time a scenario says, events read
+// that clock, everything else is fake_hip_layer.cpp.  Prints the plan that came out.
+//   cold      - the first launch of every kernel instance takes 400 us longer (its code has to be loaded); afterwards a
+//               Packed plan takes 6 us, all others 10 us
+#define cuttHipEventCreate fakeEventCreate
+#define cuttHipEventDestroy fakeEventDestroy
+#define cuttHipEventRecord fakeEventRecord
+#define cuttHipEventElapsedMs fakeEventElapsedMs
+#define cuttHipLaunchTiled fakeLaunchTiled
+#define cuttHipLaunchTiledCopy fakeLaunchTiledCopy
+#define cuttHipLaunchPacked fakeLaunchPacked
+#include "fake_hip_layer.cpp"
+#undef cuttHipEventCreate
+#undef cuttHipEventDestroy
+#undef cuttHipEventRecord
+#undef cuttHipEventElapsedMs
+#undef cuttHipLaunchTiled
+#undef cuttHipLaunchTiledCopy
+#undef cuttHipLaunchPacked
+
+#include <cstdio>
+#include <functional>
+#include <set>
+#include <string>
+
+#include "cutt.h"
+#include "cutt_ext.h"
+
+static double gNow = 0;  // us
+static long gLaunches = 0;
+
+// What a launch takes, from its arguments; `instance` names the kernel instance.
+static std::function<double(const cuttHipTiledArgs&)> gTiledUs;
+static std::function<double(const cuttHipTiledCopyArgs&)> gCopyUs;
+static std::function<double(const cuttHipPackedArgs&)> gPackedUs;
+static double gColdUs = 0;
+static std::set<std::string> gUsed;
+
+static int launched(const std::string& instance, double us) {
+  gLaunches++;
+  gNow += us + (gUsed.insert(instance).second ? gColdUs : 0.0);
+  return 0;
+}
+
+extern "C" {
+int cuttHipEventCreate(void** event) { *event = new double(0); return 0; }
+int cuttHipEventDestroy(void* event) { delete (double*)event; return 0; }
+int cuttHipEventRecord(void* event, void*) { *(double*)event = gNow; return 0; }
+int cuttHipEventElapsedMs(void* start, void* stop, float* ms) { *ms = (float)((*(double*)stop - *(double*)start) * 1e-3); return 0; }
+int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void*, void*, void*) {
+  return launched("tiled " + std::to_string(a->elemSize) + (a->lineWidth ? " lines" : "") + (a->grouped ? " grouped" : "") +
+                  (a->rowsK.n > 0 || a->rowsM.n > 0 ? " fused" : "") + " policy " + std::to_string(a->cachePolicy), gTiledUs(*a));
+}
+int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* a, const void*, void*, void*) {
+  return launched((a->rowGather ? "rows " : "copy ") + std::to_string(a->rowGather ? a->rows.cachePolicy : a->tiles.cachePolicy), gCopyUs(*a));
+}
+int cuttHipLaunchPacked(const cuttHipPackedArgs* a, const void*, void*, void*) {
+  return launched("packed " + std::to_string(a->elemSize) + " " + std::to_string(a->elemsPerThread) + " policy " + std::to_string(a->cachePolicy), gPackedUs(*a));
+}
+}
+
+static bool oneSlab(const cuttHipPackedArgs& a) { return a.split[0].numSplit == 1 && a.split[1].numSplit == 1; }
+
+static int measure(std::vector<int> dim, std::vector<int> perm, int es) {
+  char in, out;
+  cuttHandle h;
+  const cuttResult rc = cuttPlanMeasure(&h, (int)dim.size(), dim.data(), perm.data(), es, 0, &in, &out);
+  if (rc != CUTT_SUCCESS) { std::printf("failed %d\n", (int)rc); return 1; }
+  cuttPlanInfo i;
+  if (cuttGetPlanInfo(h, &i) != CUTT_SUCCESS) return 1;
+  std::printf("method %d measured %.2f policy %d order %d super %dx%d lines %d grouped %d launches %ld\n", i.method, i.usMeasured, i.cachePolicy,
+              i.tiledOrder, i.superM, i.superK, i.tiledAligned, i.tiledGrouped, gLaunches);
+  return cuttDestroy(h) == CUTT_SUCCESS ? 0 : 1;
+}
+
+static int cold() {
+  gColdUs = 400;
+  gTiledUs = [](const cuttHipTiledArgs&) { return 10.0; };
+  gCopyUs = [](const cuttHipTiledCopyArgs&) { return 10.0; };
+  gPackedUs = [](const cuttHipPackedArgs& a) { return oneSlab(a) ? 6.0 : 10.0; };
+  return measure({100, 20, 40, 30}, {2, 1, 3, 0}, 8);
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "cold") return cold();
+  return 2;
+}

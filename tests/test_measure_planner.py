@@ -1,0 +1,38 @@
+"""What cuttPlanMeasure picks from timings that are known beforehand: on the CPU, with a simulated device clock
+(measure_planner.cpp)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+CSRC = os.path.join(ROOT, "cutt_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("measure") / "measure_planner")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
+                           os.path.join(HERE, "measure_planner.cpp")] +
+                          [os.path.join(CSRC, n) for n in ("cutt_api.cpp", "plan.cpp", "model.cpp", "layer_math.cpp", "slab.cpp")] +
+                          ["-o", exe])
+    return exe
+
+
+def measured(program, scenario):
+    out = subprocess.check_output([program, scenario], text=True, timeout=120)
+    m = re.search(r"method (\d+) measured ([\d.]+) policy (\d+) order (\d+) super (\d+)x(\d+) lines (\d+) grouped (\d+) launches (\d+)", out)
+    assert m, out
+    print(out)
+    return dict(zip(("method", "us", "policy", "order", "superM", "superK", "lines", "grouped", "launches"),
+                    (float(m.group(2)) if k == 2 else int(m.group(k)) for k in range(1, 10))))
+
+
+METHOD_PACKED = 2
+
+
+def test_first_launch_of_a_kernel_instance_does_not_decide(program):
+    p = measured(program, "cold")
+    assert p["method"] == METHOD_PACKED and p["us"] == 6.0
