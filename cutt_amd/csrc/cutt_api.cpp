@@ -373,7 +373,7 @@ void finishPlan(Plan& p, const cuttHipDeviceProps& props) {
   if (lineWindowsPay(p, props)) {
     PlannerOptions opt = plannerOptions(0);
     opt.tiledAligned = 1;
-    opt.tiledGrouped = p.tiled.grouped;
+    opt.tiledGrouped = 0;
     Plan q;
     if (rebuildPlan(p, props, opt, q)) {
       q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
@@ -887,7 +887,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         if (tryVariant(v, false)) cur = v;
       }
       // sixteen or four rows per lane in flight
-      if (!failed && plans[best].method == kTiled && !std::getenv("CUTT_TILED_GROUPED")) {
+      if (!failed && plans[best].method == kTiled && !cur.tiledAligned && !std::getenv("CUTT_TILED_GROUPED")) {
         PlannerOptions v = cur;
         v.tiledGrouped = 1 - cur.tiledGrouped;
         if (tryVariant(v, false)) cur = v;
@@ -898,6 +898,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
            (int64_t)plans[best].tiled.strideOutM * plans[best].pb.elemSize % 128 != 0)) {
         PlannerOptions v = cur;
         v.tiledAligned = 1 - cur.tiledAligned;
+        if (v.tiledAligned) v.tiledGrouped = 0;
         if (tryVariant(v, false)) cur = v;
       }
     } else {

@@ -2,6 +2,7 @@
 // that clock, everything else is fake_hip_layer.cpp.  Prints the plan that came out.
 //   cold      - the first launch of every kernel instance takes 400 us longer (its code has to be loaded); afterwards a
 //               Packed plan takes 6 us, all others 10 us
+//   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
 #define cuttHipEventRecord fakeEventRecord
@@ -81,8 +82,15 @@ static int cold() {
   return measure({100, 20, 40, 30}, {2, 1, 3, 0}, 8);
 }
 
+static int drift() {
+  gTiledUs = [](const cuttHipTiledArgs& a) { return (a.lineWidth ? 100.0 : 200.0) * (1.0 - 1e-5 * gLaunches); };
+  gPackedUs = [](const cuttHipPackedArgs&) { return 200.0; };
+  return measure({1201, 30011}, {1, 0}, 8);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "cold") return cold();
+  if (what == "drift") return drift();
   return 2;
 }

@@ -36,3 +36,9 @@ METHOD_PACKED = 2
 def test_first_launch_of_a_kernel_instance_does_not_decide(program):
     p = measured(program, "cold")
     assert p["method"] == METHOD_PACKED and p["us"] == 6.0
+
+
+def test_line_aligned_plans_are_not_timed_again_with_rows_in_groups(program):
+    # the switch changes nothing about them: whichever launch came later would win
+    p = measured(program, "drift")
+    assert p["lines"] == 1 and p["grouped"] == 0
