@@ -342,6 +342,14 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (grouped) p.model.usPredicted *= 0.96;
 }
 
+// Whether output rows of a Tiled plan start off the 128-byte grid.
+bool rowsOffLineGrid(const Plan& p) {
+  const Problem& pb = p.pb;
+  for (int r = 0; r < pb.rank; r++)
+    if (pb.inv[r] >= p.split.numMk && pb.dim[r] > 1 && pb.strideOut[r] * pb.elemSize % 128 != 0) return true;
+  return false;
+}
+
 // Whether a Tiled plan stores its rows in line-aligned windows (kernels.hip: tiledLinesKernel): output rows that start
 // off the line grid, long enough that the lines cut at the run's ends do not count, of a tensor beyond the memory-side
 // cache.  Against ordinary tiles on 60 such tensors of 0.14-1.7 GB per buffer, both widths: 3-18 % faster (23425 x 8538,
@@ -356,32 +364,32 @@ bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
   const double bytes = (double)pb.volume * pb.elemSize;
   const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
   // batches of separate matrices: the Mbar ranks are slowest on both sides
-  bool offGrid = false, batch = p.split.volMbar > 1;
+  bool batch = p.split.volMbar > 1;
   for (int r = 0; r < pb.rank; r++) {
     if (pb.inv[r] < p.split.numMk) continue;
-    offGrid = offGrid || (pb.dim[r] > 1 && pb.strideOut[r] * pb.elemSize % 128 != 0);
     if (!p.split.inMmk[r]) batch = batch && pb.strideIn[r] >= p.split.volMm * p.split.volMk && pb.strideOut[r] >= p.split.volMm * p.split.volMk;
   }
   if (2.0 * bytes <= cache || p.split.volMm * pb.elemSize < 256 || runBytes < (batch ? 4096 : 2048)) return false;
-  if (!offGrid) return false;
+  if (!rowsOffLineGrid(p)) return false;
   const PlannerOptions opt = plannerOptions(0);  // options that pin the plain kernel's variants leave the plan as it is
   return opt.tiledOrder < 0 && opt.superAuto && opt.tileDigits.empty() && opt.tiledGrouped < 0 && opt.tiledAligned < 0 && opt.digitLanes < 0;
 }
 
+// Tiled plan p with line-aligned stores (`lines`) or with 64x64 tiles, its tile order left to the options.
+bool tiledForm(const Plan& p, const cuttHipDeviceProps& props, PlannerOptions opt, bool lines, Plan& q) {
+  opt.tiledAligned = lines ? 1 : 0;
+  opt.tiledGrouped = lines ? 0 : opt.tiledGrouped;
+  if (!rebuildPlan(p, props, opt, q)) return false;
+  q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
+  return estimatePlan(q, props, 10);
+}
+
 // What is left to decide about a plan that is going to be used: line-aligned stores and the cache policy.
 void finishPlan(Plan& p, const cuttHipDeviceProps& props) {
-  if (lineWindowsPay(p, props)) {
-    PlannerOptions opt = plannerOptions(0);
-    opt.tiledAligned = 1;
-    opt.tiledGrouped = 0;
-    Plan q;
-    if (rebuildPlan(p, props, opt, q)) {
-      q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
-      if (estimatePlan(q, props, 10)) {
-        q.model.usPredicted = p.model.usPredicted;
-        p = std::move(q);
-      }
-    }
+  Plan q;
+  if (lineWindowsPay(p, props) && tiledForm(p, props, plannerOptions(0), true, q)) {
+    q.model.usPredicted = p.model.usPredicted;
+    p = std::move(q);
   }
   chooseCachePolicy(p, props);
 }
@@ -800,6 +808,29 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       p.release();
     }
   }
+  // The fastest Tiled candidate with its stores the other way - line-aligned or not (lineWindowsPay) -, in the tile order
+  // and with the cache policy the planner gives that form.
+  int bestTiled = -1;
+  for (int i = 0; i < (int)plans.size(); i++)
+    if (plans[i].method == kTiled && us[i] > 0 && (bestTiled < 0 || us[i] < us[bestTiled])) bestTiled = i;
+  if (!failed && bestTiled >= 0 && !std::getenv("CUTT_TILED_ALIGNED") && rowsOffLineGrid(plans[bestTiled])) {
+    const bool lines = plans[bestTiled].tiled.lineWidth == 0;
+    Plan q;
+    if (tiledForm(plans[bestTiled], props, plannerOptions(force), lines, q)) {
+      chooseTiledGrouping(q, props);
+      chooseCachePolicy(q, props);
+      double t;
+      if (!timePlan(q, t)) {
+        failed = true;
+      } else if (t < bestUs) {
+        bestUs = t;
+        us.push_back(t);
+        plans[best].release();
+        plans.push_back(std::move(q));
+        best = (int)plans.size() - 1;
+      }
+    }
+  }
   // Second stage: the winner's launch geometry is tuned one knob at a time (tile order, work items
   // per workgroup, order of the Mbar ranks, cache policy); a setting that measures faster is kept
   // for the knobs that follow.
@@ -890,15 +921,6 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       if (!failed && plans[best].method == kTiled && !cur.tiledAligned && !std::getenv("CUTT_TILED_GROUPED")) {
         PlannerOptions v = cur;
         v.tiledGrouped = 1 - cur.tiledGrouped;
-        if (tryVariant(v, false)) cur = v;
-      }
-      // line-aligned stores the other way (lineWindowsPay)
-      if (!failed && plans[best].method == kTiled && !std::getenv("CUTT_TILED_ALIGNED") &&
-          ((int64_t)plans[best].tiled.volMk * plans[best].pb.elemSize % 128 != 0 ||
-           (int64_t)plans[best].tiled.strideOutM * plans[best].pb.elemSize % 128 != 0)) {
-        PlannerOptions v = cur;
-        v.tiledAligned = 1 - cur.tiledAligned;
-        if (v.tiledAligned) v.tiledGrouped = 0;
         if (tryVariant(v, false)) cur = v;
       }
     } else {

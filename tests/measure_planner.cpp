@@ -2,6 +2,10 @@
 // that clock, everything else is fake_hip_layer.cpp.  Prints the plan that came out.
 //   cold      - the first launch of every kernel instance takes 400 us longer (its code has to be loaded); afterwards a
 //               Packed plan takes 6 us, all others 10 us
+//   plain     - a tensor that the rules give line-aligned stores: 64x64 tiles take 60 us in the planner's own tile order
+//               and with its cache policy, 130 us in any other form; line-aligned ones 100 us, Packed plans 90 us
+//   lines     - a tensor that the rules give 64x64 tiles: line-aligned stores take 60 us in their own order and with
+//               their own cache policy, 130 us in any other form; 64x64 tiles 100 us, Packed plans 90 us
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
@@ -82,6 +86,30 @@ static int cold() {
   return measure({100, 20, 40, 30}, {2, 1, 3, 0}, 8);
 }
 
+// What the planner makes of a Tiled plan with line-aligned stores, or without.
+static cuttPlanInfo ownForm(std::vector<int> dim, std::vector<int> perm, int es, bool lines) {
+  cuttHandle h;
+  cuttPlanInfo i = {};
+  setenv("CUTT_TILED_ALIGNED", lines ? "1" : "0", 1);
+  cuttSetMethodOverride(CUTT_METHOD_TILED);
+  if (cuttPlan(&h, (int)dim.size(), dim.data(), perm.data(), es, 0) != CUTT_SUCCESS || cuttGetPlanInfo(h, &i) != CUTT_SUCCESS) std::exit(1);
+  cuttDestroy(h);
+  cuttSetMethodOverride(0);
+  unsetenv("CUTT_TILED_ALIGNED");
+  std::printf("own form: order %d super %dx%d policy %d lines %d\n", i.tiledOrder, i.superM, i.superK, i.cachePolicy, i.tiledAligned);
+  return i;
+}
+
+static int otherForm(std::vector<int> dim, std::vector<int> perm, int es, bool lines) {
+  const cuttPlanInfo own = ownForm(dim, perm, es, lines);
+  gTiledUs = [=](const cuttHipTiledArgs& a) {
+    if ((a.lineWidth > 0) != lines) return 100.0;
+    return a.order == own.tiledOrder && (int)a.superM == own.superM && (int)a.superK == own.superK && a.cachePolicy == own.cachePolicy ? 60.0 : 130.0;
+  };
+  gPackedUs = [](const cuttHipPackedArgs&) { return 90.0; };
+  return measure(dim, perm, es);
+}
+
 static int drift() {
   gTiledUs = [](const cuttHipTiledArgs& a) { return (a.lineWidth ? 100.0 : 200.0) * (1.0 - 1e-5 * gLaunches); };
   gPackedUs = [](const cuttHipPackedArgs&) { return 200.0; };
@@ -91,6 +119,8 @@ static int drift() {
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "cold") return cold();
+  if (what == "plain") return otherForm({1201, 30011}, {1, 0}, 8, false);
+  if (what == "lines") return otherForm({96001, 407}, {1, 0}, 4, true);
   if (what == "drift") return drift();
   return 2;
 }

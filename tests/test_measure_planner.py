@@ -30,7 +30,7 @@ def measured(program, scenario):
                     (float(m.group(2)) if k == 2 else int(m.group(k)) for k in range(1, 10))))
 
 
-METHOD_PACKED = 2
+METHOD_PACKED, METHOD_TILED = 2, 4
 
 
 def test_first_launch_of_a_kernel_instance_does_not_decide(program):
@@ -42,3 +42,10 @@ def test_line_aligned_plans_are_not_timed_again_with_rows_in_groups(program):
     # the switch changes nothing about them: whichever launch came later would win
     p = measured(program, "drift")
     assert p["lines"] == 1 and p["grouped"] == 0
+
+
+@pytest.mark.parametrize("scenario,lines", [("plain", 0), ("lines", 1)])
+def test_both_forms_of_a_tiled_plan_are_timed_as_the_planner_builds_them(program, scenario, lines):
+    # ... also where a Packed plan is ahead of the form that the rules prefer
+    p = measured(program, scenario)
+    assert p["method"] == METHOD_TILED and p["lines"] == lines and p["us"] == 60.0
