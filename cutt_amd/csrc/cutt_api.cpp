@@ -419,8 +419,8 @@ void refineMbarOrder(std::vector<Plan>& plans, const cuttHipDeviceProps& props, 
   if (std::getenv("CUTT_MBAR_ORDER")) return;
   const PlannerOptions base = plannerOptions(force);
   std::vector<int> idx;
-  for (int i = 0; i < (int)plans.size(); i++)
-    if (plans[i].method != kTrivial) idx.push_back(i);
+  for (int i = 0; i < (int)plans.size(); i++)  // (gathered rows have no Mbar ranks)
+    if (plans[i].method != kTrivial && !(plans[i].method == kTiledCopy && plans[i].tcopy.rowGather)) idx.push_back(i);
   std::sort(idx.begin(), idx.end(),
             [&](int a, int b) { return plans[a].model.usPredicted < plans[b].model.usPredicted; });
   struct Trial {

@@ -6,6 +6,7 @@
 //               and with its cache policy, 130 us in any other form; line-aligned ones 100 us, Packed plans 90 us
 //   lines     - a tensor that the rules give 64x64 tiles: line-aligned stores take 60 us in their own order and with
 //               their own cache policy, 130 us in any other form; 64x64 tiles 100 us, Packed plans 90 us
+//   predicted - no timing: prints what cuttPlan expects of its plan for one tensor, with and without row gathering
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
@@ -116,11 +117,25 @@ static int drift() {
   return measure({1201, 30011}, {1, 0}, 8);
 }
 
+static int predicted() {
+  int dim[7] = {18, 39, 13, 100, 2, 3, 25}, perm[7] = {0, 3, 1, 6, 5, 2, 4};
+  for (const char* gather : {"1", "0"}) {
+    setenv("CUTT_ROW_GATHER", gather, 1);
+    cuttHandle h;
+    cuttPlanInfo i = {};
+    if (cuttPlan(&h, 7, dim, perm, 4, 0) != CUTT_SUCCESS || cuttGetPlanInfo(h, &i) != CUTT_SUCCESS) return 1;
+    std::printf("predicted %.4f gathered %d\n", i.usPredicted, i.rowGather);
+    cuttDestroy(h);
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "cold") return cold();
   if (what == "plain") return otherForm({1201, 30011}, {1, 0}, 8, false);
   if (what == "lines") return otherForm({96001, 407}, {1, 0}, 4, true);
+  if (what == "predicted") return predicted();
   if (what == "drift") return drift();
   return 2;
 }

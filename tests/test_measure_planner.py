@@ -49,3 +49,10 @@ def test_both_forms_of_a_tiled_plan_are_timed_as_the_planner_builds_them(program
     # ... also where a Packed plan is ahead of the form that the rules prefer
     p = measured(program, scenario)
     assert p["method"] == METHOD_TILED and p["lines"] == lines and p["us"] == 60.0
+
+
+def test_row_gathering_takes_no_other_candidate_its_refinement(program):
+    # the order of the Mbar ranks is refined for the three best candidates that have any
+    out = subprocess.check_output([program, "predicted"], text=True, timeout=120)
+    (with_us, gathered), (without_us, _) = [(float(a), int(b)) for a, b in re.findall(r"predicted ([\d.]+) gathered (\d)", out)]
+    assert gathered == 0 and with_us == without_us, out
