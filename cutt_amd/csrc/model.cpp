@@ -606,7 +606,9 @@ bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
     auto rows16 = [](double n) { return std::ceil(n / 16.0) * 16.0; };
     const double rdSlots = tilesM * kTile * rows16(volMk);
     const double wrSlots = copy ? rdSlots : rows16(volMm) * tilesK * kTile;
-    const double waste = 0.5 * (rdSlots + wrSlots) / (volMm * volMk) - 1.0;
+    double waste = 0.5 * (rdSlots + wrSlots) / (volMm * volMk) - 1.0;
+    // (line-aligned stores: tiles of another width, read in order of rows and columns, with a fringe)
+    if (!copy && plan.tiled.lineWidth > 0) waste = 0.5 * 64.0 * (r.rdInstr + r.wrInstr) * es / bytes - 1.0;
     // Slots of a tile that hold no element cost 4-byte elements half of what they cost 8-byte ones
     // (280 forced plans with a single tile along Mm or Mk: with 0.25 the 4-byte ones ran 0.91 /
     // 0.96 / 1.00 times the prediction at extents 17-32 / 33-48 / 49-64, the 8-byte ones 0.93-0.97
