@@ -354,6 +354,12 @@ const char* cuttHipErrorString(int err);
 int cuttHipValidateTiled(const cuttHipTiledArgs* args);
 int cuttHipValidateTiledCopy(const cuttHipTiledCopyArgs* args);
 int cuttHipValidatePacked(const cuttHipPackedArgs* args);
+/* Columns of a tile with line-aligned stores at most (twice as many with 4-byte elements and 512 lanes).  The loads a
+ * lane keeps in flight (11 of 8 bytes, 26 of 4) reach 71 and 70 columns; 68 of them leave a multiple of 4.  A leading
+ * axis of 65-68 columns runs as one tile at 5.3-5.4 TB/s, as ordinary tiles of 64 and the rest at 4.1-4.3 (8 bytes) and
+ * 3.5-3.7 (4 bytes); beyond, equal tiles take over without a step: 69-80 columns 5.0-5.4 TB/s (two tiles of 8-byte
+ * elements; 71 columns 4.2 either way), 4 bytes 4.7-4.9 as one wide tile, 5.2-5.3 at 110-136 columns, 4.8-5.2 at 137-150
+ * as three (0.9 GB per buffer, buffers in rotation). */
 #define CUTT_LINE_WIDTH 68
 /* Tiled with line-aligned stores: the widest tile along Mm, lanes per workgroup and bytes of LDS for a tile width. */
 int cuttHipLinesMaxWidth(int elemSize);

@@ -927,7 +927,9 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
   //  - else the output is written front to back (23425 x 8538, 8 bytes: 604 us against 639 in strips of 16 and 653 in
   //    strips of 8; 120001 x 1201, 4 bytes: 230 / 244 / 241);
   //  - input rows a multiple of 4 KB apart are read 4 KB at a time (8192 x 11930, 4 bytes: 148 us against 195 front
-  //    to back; 8192 x 9001, 8 bytes: 221 / 274).
+  //    to back; 8192 x 9001, 8 bytes: 221 / 274).  That is for rows next to each other: where a rank in between makes
+  //    them that far apart, (a,b,c)/(2,1,0) with a*b but not a a multiple of 4 KB, 20 tensors of 0.6-1.6 GB ran
+  //    between 6 % faster and 10 % slower in this order than in the others, 2 % slower in the mean.
   if (shape.lineWindows && opt.superAuto && opt.tiledOrder < 0 && !neighbourRunsInMm) {
     const bool channelRows = rowBytesIn % 4096 == 0;
     const bool strips = channelRows || tilesM <= 16 || rowBytesOut >= 2 * rowBytesIn;
@@ -1128,13 +1130,14 @@ bool setupRows(const Problem& pb, const cuttHipDeviceProps& props, const Planner
 // Width of a tile along Mm for line-aligned stores.  An axis that fits a tile is one tile; a longer one is cut into
 // tiles of 64 where that fills them to within 15 %, otherwise into equal ones, whole lines wide where the rows are
 // (rows of 132 4-byte elements: 306 us as 64 + 64 + 4, 301 as 66 + 66, 294 in one piece; 75 8-byte ones: 269 us as
-// 64 + 11, 223 as 38 + 37).  Long rows of 4-byte elements are read 512 bytes at a time: eight matrices and reversals
-// of 1e8-2.4e8 elements with 1201 ... 120001 columns ran 1-7 % faster 128 wide than 64 wide,
-// none slower; rows a multiple of 4 KB apart did not (139.7 us 64 wide, 141.6 us 128 wide on 16384 x 5642).
+// 64 + 11, 223 as 38 + 37).  Rows of 1000 4-byte elements and more are read 512 bytes at a time: 128 columns against 64
+// on 60 matrices, reversals and batches of 0.2-0.9 GB are 4-6 % faster with 5001 columns, even (-8 ... +3 %, 0.3 % in the
+// mean) with 1000-3001, 0.7 % slower with 700-950 and 4 % slower with 641-650, whose last tile is nearly empty; rows a
+// multiple of 4 KB apart did not gain (139.7 us 64 wide, 141.6 us 128 wide on 16384 x 5642).
 int lineTileWidth(int64_t volMm, int elemSize) {
   const int64_t most = elemSize == 4 && volMm <= cuttHipLinesMaxWidth(4) ? cuttHipLinesMaxWidth(4) : CUTT_LINE_WIDTH;
   if (volMm <= most) return (int)volMm;
-  if (elemSize == 4 && volMm >= 640 && volMm % 1024 != 0) return 2 * kTile;
+  if (elemSize == 4 && volMm >= 1000 && volMm % 1024 != 0) return 2 * kTile;
   if (ceilDiv(volMm, kTile) * kTile * 20 <= volMm * 23) return kTile;
   const int64_t lineElems = 128 / elemSize, w = ceilDiv(volMm, ceilDiv(volMm, most));
   return (int)(volMm % lineElems == 0 ? std::min(ceilDiv(w, lineElems) * lineElems, (int64_t)kTile) : w);
