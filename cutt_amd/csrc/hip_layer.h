@@ -337,8 +337,6 @@ void cuttHipCallCounts(unsigned long long* mallocs, unsigned long long* uploads)
 /* Host to device copy that has completed when the call returns. */
 int cuttHipMemcpyHtoD(void* dst, const void* src, size_t bytes);
 int cuttHipMemcpyDtoDAsync(void* dst, const void* src, size_t bytes, void* stream);
-int cuttHipMemsetAsync(void* dst, int value, size_t bytes, void* stream);
-int cuttHipDeviceSynchronize(void);
 int cuttHipEventCreate(void** event);
 int cuttHipEventDestroy(void* event);
 int cuttHipEventRecord(void* event, void* stream);

@@ -61,12 +61,6 @@ extern "C" int cuttHipMemcpyDtoDAsync(void* dst, const void* src, size_t bytes, 
   return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream);
 }
 
-extern "C" int cuttHipMemsetAsync(void* dst, int value, size_t bytes, void* stream) {
-  return (int)hipMemsetAsync(dst, value, bytes, (hipStream_t)stream);
-}
-
-extern "C" int cuttHipDeviceSynchronize(void) { return (int)hipDeviceSynchronize(); }
-
 extern "C" int cuttHipEventCreate(void** event) {
   hipEvent_t e;
   hipError_t r = hipEventCreate(&e);
