@@ -378,7 +378,7 @@ bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
 // Tiled plan p with line-aligned stores (`lines`) or with 64x64 tiles, its tile order left to the options.
 bool tiledForm(const Plan& p, const cuttHipDeviceProps& props, PlannerOptions opt, bool lines, Plan& q) {
   opt.tiledAligned = lines ? 1 : 0;
-  opt.tiledGrouped = lines ? 0 : opt.tiledGrouped;
+  if (lines) opt.tiledGrouped = p.tiled.grouped;  // (no effect with such stores: what is reported is the plan without them)
   if (!rebuildPlan(p, props, opt, q)) return false;
   q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
   return estimatePlan(q, props, 10);
