@@ -264,6 +264,14 @@ PlannerOptions plannerOptions(int forceMethod);
 //  - up to one cache size per buffer non-temporal loads leave the cache to the output: 10-28 % faster when the same
 //    buffers are used again, 0-7 % slower when they are not - unless the plan requests each line of data more than
 //    1.7 times (1.5 for the 256-byte rows of 4-byte tiles), when the re-reads must hit.
+// Timed alone, right after a kernel that writes the input, plans with ordinary stores look better than that: up to a
+// cache's worth of their output is written back during whatever runs next.  On 200 tensors of 0.13-1.6 GB such a pass
+// takes 2-13 % longer between one and three cache sizes than with non-temporal loads and ordinary stores, but it and
+// the kernel before it together 1-7 % less, with a kernel that reads the result behind it 2-7 % less; transposing and
+// reading the result, over and over, -5 ... +3 %.  (96,75,96,75)/(2,1,3,0), 8 bytes: alone 167 -> 176 us, with the
+// kernel that writes the input 320 -> 318, with the reading one too 476 -> 475, in rotation 170 -> 163;
+// (5,7,11,13,17,1093)/(4,2,0,5,1,3), 4 bytes: 159 -> 171, 304 -> 294, 443 -> 438, 164 -> 155.  One square power of two
+// loses: 8192 x 8192, 4 bytes, 97 -> 79, 204 -> 219, 312 -> 319, 112 -> 113.
 void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
   if (std::getenv("CUTT_CACHE_POLICY")) return;
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
@@ -353,8 +361,8 @@ bool rowsOffLineGrid(const Plan& p) {
 // Whether a Tiled plan stores its rows in line-aligned windows (kernels.hip: tiledLinesKernel): output rows that start
 // off the line grid, long enough that the lines cut at the run's ends do not count, of a tensor beyond the memory-side
 // cache.  Against ordinary tiles on 60 such tensors of 0.14-1.7 GB per buffer, both widths: 3-18 % faster (23425 x 8538,
-// 8 bytes: 674 -> 603 us; (50,7,13,43610)/(3,1,2,0) 656 -> 617; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 361 ->
-// 316 us).  Runs of 1.4 KB lose 5 %, so do batches of separate matrices with runs of 2 KB (those break even at 4 KB);
+// 8 bytes: 675 -> 605 us; (50,7,13,43610)/(3,1,2,0) 659 -> 616; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 358 ->
+// 323 us).  Runs of 1.4 KB lose 5 %, so do batches of separate matrices with runs of 2 KB (those break even at 4 KB);
 // with tiles of less than 256 bytes along Mm the fringe rows, read twice, cost more than the stores gain ((7,4,99,4,...),
 // 28 columns: 247 -> 298 us).  Tensors inside the cache: 24 MB +20 % time, 120 MB -1 %, left to the ordinary tiles.
 bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
@@ -970,8 +978,8 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   }
   if (failed || best < 0) return CUTT_INTERNAL_ERROR;
 
-  // Play-off against the plan cuttPlan would return.  The winner is the best of up to a hundred timings of two
-  // runs each, so its own time is an optimistic one; the heuristic plan (the model's pick with its Mbar order
+  // Play-off against the plan cuttPlan would return.  The winner is the best of up to a hundred timings,
+  // so its own time is an optimistic one; the heuristic plan (the model's pick with its Mbar order
   // and cache policy refined) is not among the candidates as such.  Both are timed again in turn and the
   // faster one is kept, so that the measuring planner does not end behind the heuristic one by more than the
   // noise of these last runs.

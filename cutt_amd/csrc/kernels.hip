@@ -170,11 +170,13 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
 // up to one line, so the workgroup reads up to 64 + (elements per line - 1) rows along Mk into a taller LDS tile;
 // the rows in the fringe are also read by the tile next door, from the L2, which is why the loads are temporal.
 //
-// 23425 x 8538, 8 bytes: 674 us with ordinary tiles (4.75 TB/s) -> 603 us (5.3 TB/s); 16411 x 9377, 4 bytes: 285 ->
-// 242 us; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 357 -> 316 us.  The same windows with ordinary stores gain
-// half of that, ordinary tiles with non-temporal stores lose 20-40 % (their partial lines go to memory twice).
-// 512 lanes for 8-byte elements keep 11 loads per lane in flight, 256 for
-// narrow tiles of 4-byte ones 26; twice the lanes with half the loads each are 1-2 % slower, four times 10-60 %.
+// 23425 x 8538, 8 bytes: 675 us with ordinary tiles (4.75 TB/s) -> 605 us (5.3 TB/s); 16411 x 9377, 4 bytes: 282 ->
+// 241 us; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 358 -> 323 us (buffers in rotation).  Read from beyond the
+// L2: 1.21 times the tensor's bytes on the first (ordinary tiles 1.03), 1.00 times on the third and on
+// (200000,2,500)/(2,1,0), where every fringe row hits the L2; written 1.000-1.002 times (1.007-1.054).  The same windows
+// with ordinary stores gain half of that, ordinary tiles with non-temporal stores lose 20-40 % (their partial lines go
+// to memory twice).  512 lanes for 8-byte elements keep 11 loads per lane in flight, 256 for narrow tiles of 4-byte
+// ones 26; twice the lanes with half the loads each are 1-2 % slower, four times 10-60 %.
 //
 // A tile is lineWidth columns wide along Mm (plan.cpp: lineTileWidth): its elements are read in order of rows and
 // columns, so that a width of 33 or 66 leaves no lane of a request idle.
@@ -282,9 +284,9 @@ __global__ __launch_bounds__(kTileThreads) void tiledCopyKernel(const cuttHipCop
 // two parts.  Here the unit of work is a piece of the output instead - CUTT_ROW_BLOCK elements from one line
 // boundary to another, whatever rows they belong to -, every store of a wave is whole lines, which can then go
 // past the caches (non-temporal), and only the loads start anywhere.  (1305,599,88)/(0,2,1) of 4-byte elements,
-// 550 MB moved: 120 us (packed kernel, 4.6 TB/s) -> 94 us (5.85 TB/s; a linear copy takes 84); 8-byte elements
-// 226 -> 185 us; (115340,289,6)/(0,2,1), 4 bytes: 338 -> 255 us; rows of 42 x 2 4-byte elements, 236 MB moved:
-// 51.6 -> 43 us.  Four elements per lane: two are 30 % slower for 4-byte elements, eight 1-3 % slower.
+// 550 MB moved: 120 us (packed kernel, 4.6 TB/s) -> 97 us (5.7 TB/s; a linear copy takes 84); 8-byte elements
+// 226 -> 187 us; (115340,289,6)/(0,2,1), 4 bytes: 336 -> 265 us; (84,700,500)/(0,2,1), 4 bytes: 56 -> 48 us (buffers
+// in rotation).  Four elements per lane: two are 30 % slower for 4-byte elements, eight 1-3 % slower.
 template <typename T, int NT>
 __global__ __launch_bounds__(kRowThreads) void rowGatherKernel(const cuttHipRowArgs a, const T* __restrict__ in,
                                                                T* __restrict__ out) {

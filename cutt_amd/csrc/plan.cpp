@@ -1111,7 +1111,7 @@ bool setupRows(const Problem& pb, const cuttHipDeviceProps& props, const Planner
   // same ones again / on an input just written: 0.87 / 0.98 / 1.00 of the time on 58 tensors of 4-byte elements that fit
   // the memory-side cache twice, 0.93 / 0.95 / 0.99 on 56 of 8-byte ones, 0.93-0.97 / 0.84-0.95 / 0.96-1.00 on 100 larger.
   // Non-temporal loads only for long rows of 8-byte elements of which the cache holds little: in rotation / on an input
-  // just written 0.86-1.00 / 0.85-1.05 (one cache size per buffer and more, (533853,15,5)/(0,2,1) 105 -> 94 us in
+  // just written 0.86-1.00 / 0.85-1.05 (one cache size per buffer and more, (533853,15,5)/(0,2,1) 105 -> 97 us in
   // rotation), but 0.88 / 1.2-1.4 at 0.4-0.75 cache sizes, and 1.15-1.25 for writing it, transposing and reading the
   // result in turn.  Rows share the lines at their ends, and those are read again: rows below 800 bytes ran 0.95-1.07 /
   // 0.98-1.2, 4-byte elements 1.03-1.16 / 1.1-1.4.
