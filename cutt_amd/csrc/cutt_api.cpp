@@ -334,8 +334,8 @@ bool parallelFor(int n, F&& f) {
 // A Tiled plan on 4-byte elements whose tile rows start off the 128-byte grid (the model counts
 // 1.2-1.6 requested lines per line of data on both sides) and whose tensor is larger than the
 // memory-side cache (from 1.1 cache sizes per buffer on) keeps four instead of sixteen rows per
-// lane in flight.  Measured on such plans of the reference's random-tensor suites: +5 % in the
-// median at 0.8 GB per buffer (164 plans, worst -3.5 %, best +17 %), single tensors +20...+34 % at
+// lane in flight.  Measured on such plans of the reference's random-tensor suites, with
+// non-temporal loads (chooseAccesses): +5 % in the median at 0.8 GB per buffer (164 plans, worst -3.5 %, best +17 %), single tensors +20...+34 % at
 // 0.3-0.5 GB; outside these limits the same switch costs up to 14 % (aligned or cache-sized
 // tensors, 8-byte elements).  (Not applied when CUTT_TILED_GROUPED pins the switch.)
 void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
@@ -348,6 +348,15 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
                        wrAmp < 1.6;
   p.tiled.grouped = grouped ? 1 : 0;
   if (grouped) p.model.usPredicted *= 0.96;
+}
+
+// Cache policy of a plan that is going to be used, and rows in groups only with non-temporal loads: four rows in flight
+// find the lines again that such loads give up.  45 plans of the rule above, 0.3-0.9 GB per buffer, buffers in rotation:
+// with non-temporal loads 3.2 % faster than sixteen rows; with ordinary ones, which such tensors get now, 2.8 % slower (2.2 %
+// on inputs just written), and sixteen rows with those are 4.5 % faster than rows in groups with non-temporal loads.
+void chooseAccesses(Plan& p, const cuttHipDeviceProps& props) {
+  chooseCachePolicy(p, props);
+  if (p.method == kTiled && p.tiled.lineWidth == 0 && !(p.tiled.cachePolicy & 1) && !std::getenv("CUTT_TILED_GROUPED")) p.tiled.grouped = 0;
 }
 
 // Whether output rows of a Tiled plan start off the 128-byte grid.
@@ -386,7 +395,7 @@ bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
 // Tiled plan p with line-aligned stores (`lines`) or with 64x64 tiles, its tile order left to the options.
 bool tiledForm(const Plan& p, const cuttHipDeviceProps& props, PlannerOptions opt, bool lines, Plan& q) {
   opt.tiledAligned = lines ? 1 : 0;
-  if (lines) opt.tiledGrouped = p.tiled.grouped;  // (no effect with such stores: what is reported is the plan without them)
+  if (lines) opt.tiledGrouped = p.tiled.grouped;  // (no effect with such stores, only reported)
   if (!rebuildPlan(p, props, opt, q)) return false;
   q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
   return estimatePlan(q, props, 10);
@@ -399,7 +408,7 @@ void finishPlan(Plan& p, const cuttHipDeviceProps& props) {
     q.model.usPredicted = p.model.usPredicted;
     p = std::move(q);
   }
-  chooseCachePolicy(p, props);
+  chooseAccesses(p, props);
 }
 
 // The model's estimate of a candidate and the launch details that follow from it.
@@ -826,7 +835,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     Plan q;
     if (tiledForm(plans[bestTiled], props, plannerOptions(force), lines, q)) {
       chooseTiledGrouping(q, props);
-      chooseCachePolicy(q, props);
+      chooseAccesses(q, props);
       double t;
       if (!timePlan(q, t)) {
         failed = true;

@@ -55,7 +55,7 @@ typedef struct cuttPlanInfo {
    * runs, on the read and on the write side (0 = no such neighbour) */
   double rdEdgeDist, wrEdgeDist;
   int tiledGrouped;     /* Tiled: 1 if a lane keeps 4 instead of 16 tile rows in flight (with tiledAligned, whose tiles are read
-                           in one go: 1 if it would without) */
+                           in one go: what the estimate of the plan without assumed) */
   int superM, superK;   /* Tiled/TiledCopy: shape of the super-tiles the workgroups walk (tiled orders 3-6) */
   int tiledAligned;     /* Tiled: 1 if every tile row stores its own line-aligned window of its output run */
   int itemOrder;        /* Packed/PackedSplit: 0 = a workgroup walks neighbouring slabs, 1 = it keeps its slabs

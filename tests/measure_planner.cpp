@@ -6,6 +6,8 @@
 //               and with its cache policy, 130 us in any other form; line-aligned ones 100 us, Packed plans 90 us
 //   lines     - a tensor that the rules give 64x64 tiles: line-aligned stores take 60 us in their own order and with
 //               their own cache policy, 130 us in any other form; 64x64 tiles 100 us, Packed plans 90 us
+//   accesses  - no timing: the plan cuttPlan makes for two tensors of 4-byte elements off the line grid with short output
+//               rows, once as it is and once with the cache policy pinned to non-temporal loads
 //   predicted - no timing: prints what cuttPlan expects of its plan for one tensor, with and without row gathering
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
@@ -130,11 +132,28 @@ static int predicted() {
   return 0;
 }
 
+static int accesses() {
+  for (const char* policy : {"", "1"}) {
+    if (*policy) setenv("CUTT_CACHE_POLICY", policy, 1);
+    for (std::vector<int> dim : {std::vector<int>{772, 586, 304}, std::vector<int>{643, 703, 331}}) {
+      int perm[3] = {2, 1, 0};
+      cuttHandle h;
+      cuttPlanInfo i = {};
+      setenv("CUTT_TILED_ALIGNED", "0", 1);
+      if (cuttPlan(&h, 3, dim.data(), perm, 4, 0) != CUTT_SUCCESS || cuttGetPlanInfo(h, &i) != CUTT_SUCCESS) return 1;
+      std::printf("accesses method %d policy %d grouped %d\n", i.method, i.cachePolicy, i.tiledGrouped);
+      cuttDestroy(h);
+    }
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "cold") return cold();
   if (what == "plain") return otherForm({1201, 30011}, {1, 0}, 8, false);
   if (what == "lines") return otherForm({96001, 407}, {1, 0}, 4, true);
+  if (what == "accesses") return accesses();
   if (what == "predicted") return predicted();
   if (what == "drift") return drift();
   return 2;

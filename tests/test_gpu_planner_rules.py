@@ -206,8 +206,10 @@ def test_strips_sixteen_wide_for_rows_32_kb_apart():
 
 def test_rows_in_groups_for_unaligned_four_byte_rows(monkeypatch):
     # 4-byte three-rank reversals off the line grid, 1.1-3.5 cache sizes per buffer (found: +5 % median on 164 plans);
-    # without line-aligned stores, which read a tile in one go and would be compared with ordinary tiles instead
+    # without line-aligned stores, which read a tile in one go and would be compared with ordinary tiles instead, and with
+    # the cache policy that goes with rows in groups
     monkeypatch.setenv("CUTT_TILED_ALIGNED", "0")
+    monkeypatch.setenv("CUTT_CACHE_POLICY", "1")
     rng = np.random.default_rng(31)
     cases = []
     while len(cases) < 8:

@@ -56,3 +56,9 @@ def test_row_gathering_takes_no_other_candidate_its_refinement(program):
     out = subprocess.check_output([program, "predicted"], text=True, timeout=120)
     (with_us, gathered), (without_us, _) = [(float(a), int(b)) for a, b in re.findall(r"predicted ([\d.]+) gathered (\d)", out)]
     assert gathered == 0 and with_us == without_us, out
+
+
+def test_rows_in_groups_go_with_loads_past_the_caches(program):
+    out = subprocess.check_output([program, "accesses"], text=True, timeout=120)
+    plans = [tuple(map(int, m)) for m in re.findall(r"accesses method (\d) policy (\d) grouped (\d)", out)]
+    assert plans == [(METHOD_TILED, 0, 0)] * 2 + [(METHOD_TILED, 1, 1)] * 2, out
