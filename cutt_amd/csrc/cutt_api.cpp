@@ -335,9 +335,9 @@ bool parallelFor(int n, F&& f) {
 // 1.2-1.6 requested lines per line of data on both sides) and whose tensor is larger than the
 // memory-side cache (from 1.1 cache sizes per buffer on) keeps four instead of sixteen rows per
 // lane in flight.  Measured on such plans of the reference's random-tensor suites, with
-// non-temporal loads (chooseAccesses): +5 % in the median at 0.8 GB per buffer (164 plans, worst -3.5 %, best +17 %), single tensors +20...+34 % at
-// 0.3-0.5 GB; outside these limits the same switch costs up to 14 % (aligned or cache-sized
-// tensors, 8-byte elements).  (Not applied when CUTT_TILED_GROUPED pins the switch.)
+// non-temporal loads (chooseAccesses): +5 % in the median at 0.8 GB per buffer (164 plans, worst
+// -3.5 %, best +17 %), single tensors +20...+34 % at 0.3-0.5 GB; outside these limits the same
+// switch costs up to 14 % (aligned or cache-sized tensors, 8-byte elements).  (Not applied when CUTT_TILED_GROUPED pins the switch.)
 void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (p.method != kTiled || std::getenv("CUTT_TILED_GROUPED") || p.tiled.lineWidth > 0) return;
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
@@ -772,17 +772,17 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   void* const evStop = events.stop;
   double bestUs = 1e300;
   bool failed = false;
-  // Time of one run among runs of plan p, which is what a program that keeps the plan sees.  A first run leaves the
-  // caches as such a program leaves them; it may have to load the kernel's code (hundreds of microseconds) and drops a
-  // plan only where that cannot be the reason.  The second run, alone between the events like every plan's, drops those
-  // that take twice as long as the fastest second run; what counts comes after it, averaged over a few runs where they
-  // are short.  (Filling the output before every timed run instead leaves the memory-side cache full of lines that the
-  // run then overwrites in place: (40,14881,4,6,14)/(3,2,0,1,4) with 4-byte elements got plans of 299 or 320 us that
-  // way, 297 without.)  False on a HIP error.
-  constexpr double kFirstRunUs = 1000.0;
+  // Time of one run among runs of plan p, which is what a program that keeps the plan sees.  A first run, untimed, loads
+  // the kernel's code (hundreds of microseconds) and leaves the caches as such a program leaves them.  The second one
+  // drops plans that take a quarter longer than the fastest second run; what counts comes after it, averaged over a few runs
+  // where they are short.  (Filling the output before every timed run instead leaves the memory-side cache full of lines
+  // that the run then overwrites in place: (40,14881,4,6,14)/(3,2,0,1,4) with 4-byte elements got plans of 299 or 320 us
+  // that way, 297 without.)  False on a HIP error.
   double bestSecondUs = 1e300;
-  auto timeRuns = [&](Plan& p, int runs, double& t) -> bool {
+  auto timeRuns = [&](Plan& p, int before, int runs, double& t) -> bool {
     float ms = 0;
+    for (int i = 0; i < before; i++)
+      if (p.launch(idata, odata) != 0) return false;
     if (cuttHipEventRecord(evStart, (void*)stream) != 0) return false;
     for (int i = 0; i < runs; i++)
       if (p.launch(idata, odata) != 0) return false;
@@ -795,16 +795,14 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   auto timePlan = [&](Plan& p, double& t) -> bool {
     p.stream = (void*)stream;
     p.deviceID = deviceID;
-    if (p.activate() != 0 || !timeRuns(p, 1, t)) return false;
-    if (t > 2.0 * bestUs + kFirstRunUs) return true;
-    if (!timeRuns(p, 1, t)) return false;
-    if (t > 2.0 * bestSecondUs) return true;
+    if (p.activate() != 0 || !timeRuns(p, 1, 1, t)) return false;
+    if (t > 1.25 * bestSecondUs) return true;
     bestSecondUs = std::min(bestSecondUs, t);
     const int runs = t < 30.0 ? 4 : (t < 100.0 ? 2 : 1);
-    if (runs > 1 && !timeRuns(p, runs, t)) return false;
+    if (runs > 1 && !timeRuns(p, 0, runs, t)) return false;
     if (t > 1.1 * bestUs) return true;  // another timing moves by a few per cent
     double second = 0;
-    if (!timeRuns(p, runs, second)) return false;
+    if (!timeRuns(p, 0, runs, second)) return false;
     t = std::min(t, second);
     return true;
   };
