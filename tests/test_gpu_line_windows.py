@@ -1,5 +1,5 @@
 """Line-aligned stores of the Tiled kernel (CUTT_TILED_ALIGNED): every row of a tile stores the window of its output
-run that starts on a 128-byte line.  Bit-exact against the oracle at the edges of the tile widths, with axes over
+run that starts on a 128-byte line.  Bit-exact against a permute on the device at the edges of the tile widths, with axes over
 fused ranks, runs around one window long, buffers off the line grid, and on tensors where the planner takes it."""
 import numpy as np
 import pytest
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 def transpose_on_device(x, dim, perm):
-    # (the oracle takes seconds for 1e8 elements; tests/test_oracle.py compares the two)
+    # (the oracle takes seconds for 1e8 elements; tests/test_oracle.py compares it with numpy's transpose)
     r = len(dim)
     return x.view(tuple(reversed(dim))).permute([r - 1 - perm[r - 1 - k] for k in range(r)]).contiguous().view(-1)
 
