@@ -249,8 +249,9 @@ def test_patches_for_eight_byte_rows_on_the_line_grid():
              0.985, 0.91, 5)
 
 
-def test_one_strip_for_a_rank_of_nine_to_fourteen_tiles():
+def test_one_strip_for_a_rank_of_nine_to_fourteen_tiles(monkeypatch):
     # a leading rank of 9-14 tiles off the line grid is walked as one strip (found: +2.8 % in the mean over 13 tensors)
+    monkeypatch.setenv("CUTT_TILED_ALIGNED", "0")  # (line-aligned stores have an order of their own)
     rng = np.random.default_rng(404)
     cases = []
     while len(cases) < 18:
@@ -267,8 +268,9 @@ def test_one_strip_for_a_rank_of_nine_to_fourteen_tiles():
              0.995, 0.88, 8)
 
 
-def test_thin_second_tile_lets_the_tiles_along_mk_run_fastest():
+def test_thin_second_tile_lets_the_tiles_along_mk_run_fastest(monkeypatch):
     # two tiles along Mm of which the second is thin, at most 64 tiles along Mk (found: 10-25 % faster in order 2)
+    monkeypatch.setenv("CUTT_TILED_ALIGNED", "0")  # (line-aligned stores have an order of their own)
     rng = np.random.default_rng(12)
     cases = []
     while len(cases) < 8:
@@ -361,8 +363,8 @@ def test_work_items_per_workgroup_and_their_order():
 
 
 def test_cache_policy_of_the_global_accesses():
-    # the policy the planner derives from size and address stream against each of the three pinned, on tensors
-    # from inside the memory-side cache to four times its size: not more than 3 % behind the best of the three in
+    # the policy the planner derives from size and address stream against each of the four pinned, on tensors
+    # from inside the memory-side cache to four times its size: not more than 3 % behind the best of the four in
     # the mean
     import baseline_configs as bc
     import torch
@@ -382,13 +384,13 @@ def test_cache_policy_of_the_global_accesses():
             perm = perm[::-1]
         cfg = dict(dim=tuple(dim), perm=tuple(perm), es=es)
         rates = {}
-        for pol in ("0", "1", "3"):
+        for pol in ("0", "1", "2", "3"):
             on, off, i_on, i_off = timed_pair(cfg, {"CUTT_CACHE_POLICY": pol})
             rates[pol] = off
             rates["planner"] = max(rates.get("planner", 0.0), on)
-        best = max(rates[p] for p in ("0", "1", "3"))
-        say("cache policy dim=%s perm=%s es=%d (%.0f MB per buffer): planner (policy %d) %.0f GB/s; pinned 0 / 1 / 3: %.0f / %.0f / %.0f" %
-            (cfg["dim"], cfg["perm"], es, np.prod(dim) * es / 1e6, i_on.cachePolicy, rates["planner"], rates["0"], rates["1"], rates["3"]))
+        best = max(rates[p] for p in ("0", "1", "2", "3"))
+        say("cache policy dim=%s perm=%s es=%d (%.0f MB per buffer): planner (policy %d) %.0f GB/s; pinned 0 / 1 / 2 / 3: %.0f / %.0f / %.0f / %.0f" %
+            (cfg["dim"], cfg["perm"], es, np.prod(dim) * es / 1e6, i_on.cachePolicy, rates["planner"], *(rates[p] for p in ("0", "1", "2", "3"))))
         behind.append(rates["planner"] / best)
     behind = np.array(behind)
     say("cache policy: planner / best pinned: mean %.3f min %.3f" % (behind.mean(), behind.min()))
@@ -414,9 +416,10 @@ def test_order_of_the_mbar_ranks():
              0.97, 0.90, 3)   # (13 changed plans of 150 random tensors: +1.9 % in the mean, -1 ... +9 %)
 
 
-def test_strips_per_mbar_position_for_fused_mm_sets():
+def test_strips_per_mbar_position_for_fused_mm_sets(monkeypatch):
     # a tile axis over fused ranks of which one follows Mk in the output: all strips along Mm pass before the Mbar
     # position moves on (found: 772-862 us against 1015-1257 us on six tensors of the reference's suites)
+    monkeypatch.setenv("CUTT_TILED_ALIGNED", "0")  # (line-aligned stores have an order of their own)
     import cutt_amd as cutt
     import baseline_configs as bc
     rng = np.random.default_rng(31337)
