@@ -120,14 +120,14 @@ __global__ __launch_bounds__(kTileThreads) void countTiledKernel(const cuttHipTi
   for (int j = 0; j < kTileRows; j++) {
     if ((uint32_t)(j / kGroupRows) >= t.groupsK) continue;
     const uint32_t row = wave + kWaves * j, r = min(row, t.wK);
-    countAccess(c, false, row > t.wK, tileReadElem<FUSED>(t, a, wave, j), es);
+    countAccess(c, false, row > t.wK, tileReadElem<FUSED>(t, a, wave, j, t.wK), es);
     if (row <= t.wK) c.maxDegree = max(c.maxDegree, waveMaxMultiplicity(((r * (kTile + 1) + t.cx) * words) & 63, __ballot(lane <= t.wM)));
   }
   // writes: lanes along the output-contiguous axis, rows along Mm
   for (int j = 0; j < kTileRows; j++) {
     if ((uint32_t)(j / kGroupRows) >= t.groupsM) continue;
     const uint32_t row = wave + kWaves * j, r = min(row, t.wM);
-    const uint32_t elem = tileWriteElem<FUSED>(t, a, wave, j);
+    const uint32_t elem = tileWriteElem<FUSED>(t, a, wave, j, t.wM);
     countAccess(c, true, row > t.wM, elem, es);
     if (row <= t.wM) c.maxDegree = max(c.maxDegree, waveMaxMultiplicity(((t.ck * (kTile + 1) + r) * words) & 63, __ballot(lane <= t.wK)));
     // lane 0 holds the first element of the row's run inside this tile

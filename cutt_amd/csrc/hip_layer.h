@@ -147,6 +147,48 @@ typedef struct cuttHipRowRadix {
 } cuttHipRowRadix;
 
 /*
+ * The numbering of a Tiled launch in the form its kernels decode without a branch, a load that waits for another load
+ * or a division by a variable (cuttHipFinishTileWalk).  It covers what the planner picks for nearly every tensor:
+ * strips of superM tiles along Mm that run through all of Mk (tile orders 3 and 5), the tiles along Mm fastest (order 1:
+ * one strip) or along Mk fastest (order 2: strips one tile wide), with at most CUTT_WALK_RANKS Mbar ranks.  The tiles come
+ * in the sequence of those orders; the last strip is as narrow as it is, so that no workgroup is left without a tile (but
+ * for the last XCD's, at most seven).  Divisions of n < 2^31 by d: mulhi32(2 n, mul) >> shift with shift = ceil(log2 d) and mul =
+ * ceil(2^(31 + shift) / d) (the error of mul is below 1, so that of the product is below n / 2^(31 + shift) < 1 / d); mul = 0 gives 0.
+ */
+#define CUTT_WALK_RANKS 8
+typedef struct cuttHipWalkRank {
+  uint32_t mul, shift, extent, strideIn, strideOut;  /* the slowest rank: mul = 0 (its index is what is left) */
+} cuttHipWalkRank;
+
+/* Offsets of the rows of a tile axis (cuttHipRowRadix): axes of a single rank have n = 1, the slowest rank's mul is 0. */
+typedef struct cuttHipWalkRows {
+  uint32_t n;
+  uint32_t mul[3], shift[3], extent[3], stride[4];
+} cuttHipWalkRows;
+
+typedef struct cuttHipWalkMbar {
+  uint32_t volMbar;
+  uint32_t stripMbar;       /* Mbar positions a strip is visited for before the next strip: volMbar (order 5) or 1 */
+  uint32_t outerMul;        /* division by tilesM * tilesK (0 in order 5) */
+  uint32_t innerMul[2];     /* division by the tiles of a strip, full width and last one (0 in the other orders) */
+  uint32_t shifts;          /* outer | inner[0] << 5 | inner[1] << 10 */
+  uint32_t n;
+  cuttHipWalkRank rank[CUTT_WALK_RANKS];
+} cuttHipWalkMbar;
+
+typedef struct cuttHipTileWalk {
+  int kind;                 /* 0: not of this form, 1: a single Mbar position, 2: with Mbar positions */
+  uint32_t blocks;          /* workgroups of the launch */
+  uint32_t chunk;           /* workgroup b is position (b % 8) * chunk + b / 8, or b itself (see shifts) */
+  uint32_t superM;
+  uint32_t stripMul;        /* division by the tiles of a strip (order 5: times the Mbar positions) */
+  uint32_t fullMul, lastMul;  /* division by the width of a full strip, of the last one */
+  uint32_t shifts;          /* strip | full << 5 | last << 10 | (3: chunks per XCD, 0: none) << 15 */
+  cuttHipWalkMbar mbar;
+  cuttHipWalkRows rowsK, rowsM;
+} cuttHipTileWalk;
+
+/*
  * Tiled method: a batch of 2-D transposes between the ranks that lead the input (Mm: fused extent
  * volMm, contiguous in the input) and the ranks that lead the output (Mk: fused extent volMk,
  * contiguous in the output), staged through a padded 64x64 LDS tile.  One workgroup per (tile, Mbar
@@ -181,11 +223,15 @@ typedef struct cuttHipTiledArgs {
   cuttHipRowRadix rowsK; /* Mk index -> input offset (n == 0: index * strideInK) */
   cuttHipRowRadix rowsM; /* Mm index -> output offset (n == 0: index * strideOutM) */
   cuttHipTileDigits digits; /* order 7 only */
+  cuttHipTileWalk walk;     /* the numbering as the usual kernels decode it, derived from the rest (cuttHipFinishTileWalk) */
   cuttHipMbar mbar;         /* last: the data pointers follow it in the kernel's arguments and are then read with the line
                                that holds its last entries.  With 16 bytes more in between, which move them into a line of
                                their own, launches of 5-13 us took 1-8 % longer: (5,18,12758,2)/(2,3,0,1), 8 bytes, 10.3 us
                                instead of 9.5, 867 x 3788 11.9 / 11.2, 433 x 12223, 4 bytes, 9.6 / 9.3 */
 } cuttHipTiledArgs;
+
+/* Derive a->walk from the other arguments (kind 0 if their numbering is not of its form). */
+void cuttHipFinishTileWalk(cuttHipTiledArgs* a);
 
 /*
  * Rows gathered into a dense output (TiledCopy method, the usual kernel): rank 0 keeps its place, so the

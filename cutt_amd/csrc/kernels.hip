@@ -74,7 +74,7 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // ---------------------------------------------------------------------------
 // GROUPED: the four row groups of a lane go one after the other - request 4 rows, wait, stage them,
 // request the next 4; store 4 rows, wait, store the next 4 - instead of all 16 rows at once.  That
-// quarters what a workgroup has in flight.  When tile rows start off the 128-byte grid (4-byte
+// quarters what a wave has in flight.  When tile rows start off the 128-byte grid (4-byte
 // elements, large tensors) it is 3-11 % faster: the neighbouring tiles' requests for a shared line
 // then arrive while the line is still in the L2.  On aligned or cache-resident tensors it is up to
 // 10 % slower, so the planner decides (cuttHipTiledArgs.grouped).
@@ -83,80 +83,82 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // ranks that lead the output on the Mk side), so the rows of a tile are not equally far apart.  Lane l
 // derives the offset of row l of either axis with a short mixed-radix decode (tileRowOffsets) and the
 // wave picks a row's offset out of that lane; the elements of a row are contiguous as before.
+template <typename T, int NT, bool GROUPED, bool FUSED, typename Args>
+__device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
+  __shared__ T tile[kTile][kTile + 1];
+  const uint32_t wave = threadIdx.x >> 6;
+
+  // One straight piece of code per number of row groups (4 for a whole tile, fewer at an edge): with one group behind
+  // the other and a test in between the compiler waits for a group's loads before the next one's go out, since the rows'
+  // registers meet again behind the test.  WHOLE: all 64 rows are there, no index needs clamping.
+  auto read = [&](auto groups, auto whole) __attribute__((always_inline)) {  // lanes run along the input-contiguous axis (Mm), rows along Mk
+    constexpr int kRows = decltype(groups)::value * kGroupRows, kStep = GROUPED ? kGroupRows : kRows;
+    const uint32_t lastRow = decltype(whole)::value ? kTile - 1u : t.wK;
+#pragma unroll
+    for (int g = 0; g < kRows; g += kStep) {
+      T v[kStep];
+#pragma unroll
+      for (int j = 0; j < kStep; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, g + j, lastRow));
+      if constexpr (GROUPED) waitForGlobalAccesses();
+#pragma unroll
+      for (int j = 0; j < kStep; j++) tile[min(wave + kWaves * (g + j), lastRow)][t.cx] = v[j];
+    }
+  };
+  auto write = [&](auto groups, auto whole) __attribute__((always_inline)) {  // lanes run along the output-contiguous axis (Mk), rows along Mm
+    constexpr int kRows = decltype(groups)::value * kGroupRows, kStep = GROUPED ? kGroupRows : kRows;
+    const uint32_t lastRow = decltype(whole)::value ? kTile - 1u : t.wM;
+#pragma unroll
+    for (int g = 0; g < kRows; g += kStep) {
+      T v[kStep];
+#pragma unroll
+      for (int j = 0; j < kStep; j++) v[j] = tile[t.ck][min(wave + kWaves * (g + j), lastRow)];
+#pragma unroll
+      for (int j = 0; j < kStep; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, g + j, lastRow), v[j]);
+      if constexpr (GROUPED) waitForGlobalAccesses();
+    }
+  };
+  auto byGroups = [](uint32_t lastRow, auto&& f) __attribute__((always_inline)) {
+    if (lastRow == kTile - 1) f(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (lastRow >= 48) f(std::integral_constant<int, 4>{}, std::false_type{});
+    else if (lastRow >= 32) f(std::integral_constant<int, 3>{}, std::false_type{});
+    else if (lastRow >= 16) f(std::integral_constant<int, 2>{}, std::false_type{});
+    else f(std::integral_constant<int, 1>{}, std::false_type{});
+  };
+  static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
+  byGroups(t.wK, read);
+  __syncthreads();
+  byGroups(t.wM, write);
+}
+
+// Any numbering of the workgroups (tile_order.h: locateTile).
 template <typename T, int NT, bool GROUPED, bool FUSED>
 __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledArgs a,
                                                             const T* __restrict__ in,
                                                             T* __restrict__ out) {
-  __shared__ T tile[kTile][kTile + 1];
-
   uint32_t tm, tk, offIn, offOut;
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
-
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = threadIdx.x >> 6;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
-  const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, lane, wave);
+  const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
+  moveTile<T, NT, GROUPED, FUSED>(t, a, in, out);
+}
 
-  // Read: lanes run along the input-contiguous axis (Mm), rows along Mk.
-  {
-    T v[kTileRows];
-#pragma unroll
-    for (int g = 0; g < kRowGroups; g++) {
-      if ((uint32_t)g < t.groupsK) {
-#pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j));
-        if constexpr (GROUPED) {
-          waitForGlobalAccesses();
-#pragma unroll
-          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) {
-            const uint32_t r = min(wave + kWaves * j, t.wK);
-            tile[r][t.cx] = v[j];
-          }
-        }
-      }
-    }
-    if constexpr (!GROUPED) {
-#pragma unroll
-      for (int g = 0; g < kRowGroups; g++) {
-        if ((uint32_t)g < t.groupsK) {
-#pragma unroll
-          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) {
-            const uint32_t r = min(wave + kWaves * j, t.wK);
-            tile[r][t.cx] = v[j];
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();
-  // Write: lanes run along the output-contiguous axis (Mk), rows along Mm.
-  {
-    T v[kTileRows];
-#pragma unroll
-    for (int g = 0; g < kRowGroups; g++) {
-      if ((uint32_t)g < t.groupsM) {
-#pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) {
-          const uint32_t r = min(wave + kWaves * j, t.wM);
-          v[j] = tile[t.ck][r];
-        }
-        if constexpr (GROUPED) {
-#pragma unroll
-          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j), v[j]);
-          waitForGlobalAccesses();
-        }
-      }
-    }
-    if constexpr (!GROUPED) {
-#pragma unroll
-      for (int g = 0; g < kRowGroups; g++) {
-        if ((uint32_t)g < t.groupsM) {
-#pragma unroll
-          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j), v[j]);
-        }
-      }
-    }
-  }
+// The numberings of cuttHipTileWalk.  The arguments up to `shifts`, 14 words, are in scalar registers when a wave starts
+// (the Makefile's kernarg-preload-count), so that a plain matrix transpose waits for nothing before its first load;
+// MB and ROWS hold what launches with Mbar positions and with fused axes need besides.
+// Bound by latency up to some 20 MB, by memory beyond.  Against the kernel above as it was before (its loads in groups of
+// four that waited for each other): 2011 x 1163, 4 bytes, 5.94 -> 4.38 us; (24,32,36,43)/(3,1,2,0), 8 bytes, 5.99 -> 4.86;
+// 4297 x 1731, 8 bytes, 28.2 -> 25.5; (7,149,21,189)/(3,2,1,0), 4 bytes, 9.5 -> 7.8; (96,75,96,75)/(2,1,3,0), 8 bytes, 161.7 -> 159.0.
+template <typename T, int NT, typename MB, typename ROWS>
+__global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restrict__ in, T* __restrict__ out, uint32_t volMm, uint32_t volMk,
+                                                                uint32_t strideInK, uint32_t strideOutM, uint32_t chunk, uint32_t superM,
+                                                                uint32_t stripMul, uint32_t fullMul, uint32_t lastMul, uint32_t shifts,
+                                                                const MB mb, const ROWS rows) {
+  constexpr bool kFused = std::is_same_v<ROWS, WalkAxes>;
+  uint32_t tm, tk, offIn, offOut;
+  if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
+  const WalkShape<ROWS> shape{volMm, volMk, strideInK, strideOutM, rows};
+  const TileLanes t = tileLanes<kFused>(shape, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
+  moveTile<T, NT, false, kFused>(t, shape, in, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -658,6 +660,11 @@ extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
   if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
   if (a->cachePolicy < 0 || a->cachePolicy > 3) return (int)hipErrorInvalidValue;
+  if (a->walk.kind != 0) {  // the walk must be the one that follows from the other arguments
+    cuttHipTiledArgs want = *a;
+    cuttHipFinishTileWalk(&want);
+    if (std::memcmp(&want.walk, &a->walk, sizeof(want.walk)) != 0) return (int)hipErrorInvalidValue;
+  }
   return 0;
 }
 
@@ -689,6 +696,36 @@ static int launchLines(const cuttHipTiledArgs& a, const void* in, void* out, uin
 #undef CUTT_LAUNCH_LINES
 }
 
+// Tiles in the sequence of a walk.
+template <typename T, int NT, typename MB, typename ROWS>
+static int launchWalkOf(const cuttHipTiledArgs& a, const MB& mb, const ROWS& rows, const void* in, void* out, hipStream_t s) {
+  const cuttHipTileWalk& w = a.walk;
+  return (int)launchKernel(tiledWalkKernel<T, NT, MB, ROWS>, dim3(w.blocks), dim3(kTileThreads), 0, s, (const T*)in, (T*)out, (uint32_t)a.volMm,
+                           (uint32_t)a.volMk, a.strideInK, a.strideOutM, w.chunk, w.superM, w.stripMul, w.fullMul, w.lastMul, w.shifts, mb, rows);
+}
+
+template <typename T, int NT>
+static int launchWalkNt(const cuttHipTiledArgs& a, const void* in, void* out, hipStream_t s) {
+  const bool fused = a.rowsK.n > 0 || a.rowsM.n > 0;
+  const WalkAxes axes{a.walk.rowsK, a.walk.rowsM};
+  if (a.walk.kind == 1) return fused ? launchWalkOf<T, NT>(a, NoMbar{}, axes, in, out, s) : launchWalkOf<T, NT>(a, NoMbar{}, NoAxes{}, in, out, s);
+  return fused ? launchWalkOf<T, NT>(a, a.walk.mbar, axes, in, out, s) : launchWalkOf<T, NT>(a, a.walk.mbar, NoAxes{}, in, out, s);
+}
+
+template <typename T>
+static int launchWalkOfWidth(const cuttHipTiledArgs& a, const void* in, void* out, hipStream_t s) {
+  switch (a.cachePolicy) {
+    case 0: return launchWalkNt<T, 0>(a, in, out, s);
+    case 1: return launchWalkNt<T, 1>(a, in, out, s);
+    case 2: return launchWalkNt<T, 2>(a, in, out, s);
+    default: return launchWalkNt<T, 3>(a, in, out, s);
+  }
+}
+
+static int launchWalk(const cuttHipTiledArgs& a, const void* in, void* out, hipStream_t s) {
+  return a.elemSize == 4 ? launchWalkOfWidth<uint32_t>(a, in, out, s) : launchWalkOfWidth<uint64_t>(a, in, out, s);
+}
+
 extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, void* out, void* stream) {
   if (!a || !in || !out) return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
@@ -696,6 +733,7 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
+  if (a->walk.kind && !a->grouped) return launchWalk(*a, in, out, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \

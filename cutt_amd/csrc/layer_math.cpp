@@ -6,6 +6,8 @@
  */
 #include "hip_layer.h"
 
+#include <cstring>
+
 extern "C" cuttHipDivisor cuttHipMakeDivisor(uint32_t d) {
   cuttHipDivisor dv = {0u, 0u, 1u};  // d <= 1: n / 1
   if (d >= 2) {
@@ -103,6 +105,75 @@ static int finishTileDigits(cuttHipTileDigits* dg, const cuttHipMbar* mb) {
   dg->total = (uint32_t)below;
   dg->lanes = 1;
   return 0;
+}
+
+namespace {
+// mulhi32(2 n, mul) >> shift == n / d for n < 2^31 (d >= 1).
+void walkDivisor(uint64_t d, uint32_t& mul, uint32_t& shift) {
+  shift = 0;
+  while ((1ull << shift) < d) shift++;
+  mul = (uint32_t)(((1ull << (31 + shift)) + d - 1) / d);
+}
+
+void walkRows(const cuttHipRowRadix& rr, uint32_t stride, cuttHipWalkRows& w) {
+  w.n = rr.n > 0 ? (uint32_t)rr.n : 1u;
+  w.stride[0] = stride;
+  for (int k = 0; k < rr.n; k++) {
+    w.stride[k] = rr.stride[k];
+    if (k + 1 == rr.n) break;
+    w.extent[k] = rr.extent[k];
+    walkDivisor(rr.extent[k], w.mul[k], w.shift[k]);
+  }
+}
+}  // namespace
+
+extern "C" void cuttHipFinishTileWalk(cuttHipTiledArgs* a) {
+  cuttHipTileWalk& w = a->walk;
+  std::memset(&w, 0, sizeof(w));
+  const uint64_t tilesM = (uint64_t)a->tilesM, tilesK = (uint64_t)a->tilesK, volMbar = (uint64_t)a->volMbar;
+  const bool strips = (a->order == 3 || a->order == 5) && a->superK >= tilesK;
+  if (a->tilesM < 1 || a->tilesK < 1 || a->volMbar < 1 || (!strips && a->order != 1 && a->order != 2)) return;
+  if (a->mbar.n < 0 || a->mbar.n > CUTT_WALK_RANKS || a->rowsK.n < 0 || a->rowsK.n > CUTT_MAX_TILE_SET || a->rowsM.n < 0 || a->rowsM.n > CUTT_MAX_TILE_SET) return;
+  // (every division is of a number below 2^31; two of the factors are)
+  const uint64_t tiles = tilesM * tilesK;
+  if (tiles > 0x7fffffffull || tiles * volMbar > 0x7fffffffull) return;
+  const uint64_t total = tiles * volMbar;
+  w.superM = a->order == 1 ? (uint32_t)tilesM : (a->order == 2 ? 1u : (a->superM < tilesM ? a->superM : (uint32_t)tilesM));
+  if (w.superM < 1) return;
+  const uint64_t stripMbar = a->order == 5 ? volMbar : 1, last = tilesM % w.superM;
+  uint32_t strip = 0, full = 0, lastShift = 0;
+  walkDivisor(w.superM * tilesK * stripMbar, w.stripMul, strip);
+  walkDivisor(w.superM, w.fullMul, full);
+  walkDivisor(last ? last : 1, w.lastMul, lastShift);
+  const bool perXcd = a->xcdChunk != 0;
+  w.chunk = perXcd ? (uint32_t)((total + 7) / 8) : 0u;
+  w.blocks = perXcd ? 8 * w.chunk : (uint32_t)total;
+  w.shifts = strip | full << 5 | lastShift << 10 | (perXcd ? 3u : 0u) << 15;
+  w.kind = volMbar > 1 ? 2 : 1;
+  if (w.kind == 2) {
+    cuttHipWalkMbar& b = w.mbar;
+    b.volMbar = (uint32_t)volMbar;
+    b.stripMbar = (uint32_t)stripMbar;
+    uint32_t outer = 0, inner[2] = {0, 0};
+    if (a->order == 5) {
+      walkDivisor(w.superM * tilesK, b.innerMul[0], inner[0]);
+      walkDivisor((last ? last : 1) * tilesK, b.innerMul[1], inner[1]);
+    } else {
+      walkDivisor(tiles, b.outerMul, outer);
+    }
+    b.shifts = outer | inner[0] << 5 | inner[1] << 10;
+    b.n = (uint32_t)a->mbar.n;
+    for (int k = 0; k < a->mbar.n; k++) {
+      cuttHipWalkRank& r = b.rank[k];
+      r.strideIn = a->mbar.d[k].strideIn;
+      r.strideOut = a->mbar.d[k].strideOut;
+      if (k + 1 == a->mbar.n) break;
+      r.extent = a->mbar.d[k].extent;
+      walkDivisor(r.extent, r.mul, r.shift);
+    }
+  }
+  walkRows(a->rowsK, a->strideInK, w.rowsK);
+  walkRows(a->rowsM, a->strideOutM, w.rowsM);
 }
 
 extern "C" long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* a) {

@@ -1688,7 +1688,11 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
 }
 
 int Plan::activate() {
-  if (method == kTiled) return launchable ? 0 : ((launchable = cuttHipValidateTiled(&tiled) == 0) ? 0 : -1);
+  if (method == kTiled) {
+    if (launchable) return 0;
+    cuttHipFinishTileWalk(&tiled);
+    return (launchable = cuttHipValidateTiled(&tiled) == 0) ? 0 : -1;
+  }
   if (method == kTiledCopy) {
     if (tcopy.rowGather) numBlocks = (int64_t)cuttHipRowGrid(&tcopy.rows);
     return launchable ? 0 : ((launchable = cuttHipValidateTiledCopy(&tcopy) == 0) ? 0 : -1);

@@ -8,6 +8,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "hip_layer.h"
 #include "mbar_decode.h"
 
@@ -146,6 +148,80 @@ __device__ __forceinline__ bool locateTile(const Args& a, uint32_t& tm, uint32_t
   return true;
 }
 
+// n / d for n < 2^31 (constants of cuttHipTileWalk).
+__device__ __forceinline__ uint32_t walkDivide(uint32_t n, uint32_t mul, uint32_t shift) { return __umulhi(2 * n, mul) >> shift; }
+
+// What every workgroup of a walk (cuttHipTileWalk) decodes its index with.
+struct WalkHead {
+  uint32_t chunk, superM, stripMul, fullMul, lastMul, shifts;
+};
+
+// The Mbar part of a walk for launches without one.
+struct NoMbar {};
+
+// locateTile for a numbering in walk form: multiply-high divisions on the scalar unit, whose constants are all there from
+// the start (in registers, or in memory at addresses that are), and no branch but the test for the end - where locateTile
+// waits for the order's number, its parameters, two to seven divisions by variables and the Mbar table one after the other.
+template <typename MB>
+__device__ __forceinline__ bool walkTile(const WalkHead& h, const MB& mb, uint32_t tilesM, uint32_t tilesK, uint32_t& tm, uint32_t& tk, uint32_t& offIn, uint32_t& offOut) {
+  constexpr bool kMbar = !std::is_same_v<MB, NoMbar>;
+  const uint32_t xs = h.shifts >> 15;  // 3: XCD b % 8 walks its own chunk
+  uint32_t l = (blockIdx.x & ((1u << xs) - 1)) * h.chunk + (blockIdx.x >> xs), m = 0, perStrip = tilesK;
+  const uint32_t tiles = tilesM * tilesK;
+  offIn = offOut = 0;
+  if constexpr (kMbar) {
+    if (l >= tiles * mb.volMbar) return false;
+    m = walkDivide(l, mb.outerMul, mb.shifts & 31);
+    l -= m * tiles;
+    perStrip *= mb.stripMbar;
+  } else {
+    if (l >= tiles) return false;
+  }
+  const uint32_t first = walkDivide(l, h.stripMul, h.shifts & 31) * h.superM;  // the strip's first tile along Mm
+  const uint32_t width = min(h.superM, tilesM - first);
+  const bool full = width == h.superM;
+  l -= first * perStrip;  // (all strips before are full ones)
+  if constexpr (kMbar) {
+    const uint32_t mi = walkDivide(l, full ? mb.innerMul[0] : mb.innerMul[1], (full ? mb.shifts >> 5 : mb.shifts >> 10) & 31);
+    l -= mi * (width * tilesK);
+    m += mi;
+  }
+  tk = walkDivide(l, full ? h.fullMul : h.lastMul, (full ? h.shifts >> 5 : h.shifts >> 10) & 31);
+  tm = first + (l - tk * width);
+  if constexpr (kMbar) {
+    auto ranks = [&](int from) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = from; k < from + 4; k++) {  // (unused ranks have zeros everywhere)
+        const uint32_t q = walkDivide(m, mb.rank[k].mul, mb.rank[k].shift);
+        const uint32_t i = m - q * mb.rank[k].extent;
+        offIn += i * mb.rank[k].strideIn;
+        offOut += i * mb.rank[k].strideOut;
+        m = q;
+      }
+    };
+    ranks(0);
+    static_assert(CUTT_WALK_RANKS == 8, "two steps of four ranks");
+    if (mb.n > 4) ranks(4);
+  }
+  return true;
+}
+
+// Offset of row `i` of a tile axis, per lane.
+__device__ __forceinline__ uint32_t walkRowOffset(const cuttHipWalkRows& r, uint32_t i) {
+  uint32_t q = walkDivide(i, r.mul[0], r.shift[0]);
+  uint32_t off = (i - q * r.extent[0]) * r.stride[0];
+  if (r.n > 2) {
+#pragma unroll
+    for (int k = 1; k < 3; k++) {
+      const uint32_t q2 = walkDivide(q, r.mul[k], r.shift[k]);
+      off += (q - q2 * r.extent[k]) * r.stride[k];
+      q = q2;
+    }
+    return off + q * r.stride[3];
+  }
+  return off + q * r.stride[1];
+}
+
 // Offset of row `i` of a tile axis that runs over the fused ranks of `rr` (rr.n >= 1), per lane.
 __device__ __forceinline__ uint32_t rowOffset(const cuttHipRowRadix& rr, uint32_t i) {
   uint32_t off = 0;
@@ -176,8 +252,29 @@ struct TileLanes {
   uint32_t rowK, rowM, waveU; // FUSED: row offsets held one per lane, and the wave index as a scalar
 };
 
-template <bool FUSED>
-__device__ __forceinline__ TileLanes tileLanes(const cuttHipTiledArgs& a, uint32_t tm, uint32_t tk, uint32_t offIn,
+// The row offsets of a tile's two axes, one row per lane, from a launch's arguments.
+__device__ __forceinline__ void tileAxes(const cuttHipTiledArgs& a, uint32_t k0, uint32_t m0, uint32_t lane, uint32_t& rowK, uint32_t& rowM) {
+  rowK = tileRowOffsets(a.rowsK, a.strideInK, k0, (uint32_t)a.volMk, lane);
+  rowM = tileRowOffsets(a.rowsM, a.strideOutM, m0, (uint32_t)a.volMm, lane);
+}
+
+// The tile geometry of a launch whose numbering is a walk; ROWS = cuttHipWalkAxes for fused axes.
+struct WalkAxes {
+  cuttHipWalkRows k, m;
+};
+struct NoAxes {};
+template <typename ROWS>
+struct WalkShape {
+  uint32_t volMm, volMk, strideInK, strideOutM;
+  const ROWS& rows;
+};
+__device__ __forceinline__ void tileAxes(const WalkShape<WalkAxes>& a, uint32_t k0, uint32_t m0, uint32_t lane, uint32_t& rowK, uint32_t& rowM) {
+  rowK = walkRowOffset(a.rows.k, min(k0 + lane, a.volMk - 1));
+  rowM = walkRowOffset(a.rows.m, min(m0 + lane, a.volMm - 1));
+}
+
+template <bool FUSED, typename Args>
+__device__ __forceinline__ TileLanes tileLanes(const Args& a, uint32_t tm, uint32_t tk, uint32_t offIn,
                                                uint32_t offOut, uint32_t lane, uint32_t wave) {
   TileLanes t;
   t.m0 = tm * kTile;
@@ -201,32 +298,31 @@ __device__ __forceinline__ TileLanes tileLanes(const cuttHipTiledArgs& a, uint32
   if constexpr (FUSED) {
     // lane l holds the input offset of row k0 + l along Mk and the output offset of row m0 + l along
     // Mm; the row a wave asks for is wave-uniform
-    t.rowK = tileRowOffsets(a.rowsK, a.strideInK, t.k0, (uint32_t)a.volMk, lane);
-    t.rowM = tileRowOffsets(a.rowsM, a.strideOutM, t.m0, (uint32_t)a.volMm, lane);
+    tileAxes(a, t.k0, t.m0, lane, t.rowK, t.rowM);
     t.waveU = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
   }
   return t;
 }
 
 // Element offset of the lane's j-th load (row wave + 4 j of the tile, clamped) / store.
-template <bool FUSED>
-__device__ __forceinline__ uint32_t tileReadElem(const TileLanes& t, const cuttHipTiledArgs& a, uint32_t wave, int j) {
+template <bool FUSED, typename Args>
+__device__ __forceinline__ uint32_t tileReadElem(const TileLanes& t, const Args& a, uint32_t wave, int j, uint32_t lastRow) {
   if constexpr (FUSED) {
-    const uint32_t r = min(t.waveU + kWaves * j, t.wK);
+    const uint32_t r = min(t.waveU + kWaves * j, lastRow);
     return t.rdBase + (uint32_t)__builtin_amdgcn_readlane((int)t.rowK, (int)r);
   } else {
-    const uint32_t r = min(wave + kWaves * j, t.wK);
+    const uint32_t r = min(wave + kWaves * j, lastRow);
     return t.rdBase + (t.k0 + r) * a.strideInK;
   }
 }
 
-template <bool FUSED>
-__device__ __forceinline__ uint32_t tileWriteElem(const TileLanes& t, const cuttHipTiledArgs& a, uint32_t wave, int j) {
+template <bool FUSED, typename Args>
+__device__ __forceinline__ uint32_t tileWriteElem(const TileLanes& t, const Args& a, uint32_t wave, int j, uint32_t lastRow) {
   if constexpr (FUSED) {
-    const uint32_t r = min(t.waveU + kWaves * j, t.wM);
+    const uint32_t r = min(t.waveU + kWaves * j, lastRow);
     return t.wrBase + (uint32_t)__builtin_amdgcn_readlane((int)t.rowM, (int)r);
   } else {
-    const uint32_t r = min(wave + kWaves * j, t.wM);
+    const uint32_t r = min(wave + kWaves * j, lastRow);
     return t.wrBase + (t.m0 + r) * a.strideOutM;
   }
 }
