@@ -320,10 +320,8 @@ extern "C" int cuttHipCountTiledCopy(const cuttHipTiledCopyArgs* a, cuttHipStrea
 
 extern "C" int cuttHipCountPacked(const cuttHipPackedArgs* a, cuttHipStreamCounts* out, void* stream) {
   if (int v = cuttHipValidatePacked(a); v != 0) return v;
-  const long long numbers = cuttHipPackedItemNumbers(a);
-  if (numbers < 1) return (int)hipErrorInvalidConfiguration;
-  uint64_t blocks = ((uint64_t)numbers + a->itemsPerBlock - 1) / a->itemsPerBlock;
-  if (a->xcdChunk) blocks = (uint64_t)a->xcdChunk * kNumXcd;
+  const long long blocks = cuttHipPackedGrid(a);
+  if (blocks < 1) return (int)hipErrorInvalidConfiguration;
   return runCount(out, stream, [&](unsigned long long* d, hipStream_t s) {
     return launchCount(countPackedKernel, dim3((uint32_t)blocks), dim3(a->numThreads), s, *a, d);
   });

@@ -84,7 +84,7 @@ std::string planKey(int deviceID, int force, int rank, const int* dim, const int
   put(deviceID); put(force); put((long long)sizeofType); put(rank);
   for (int i = 0; i < rank; i++) put(dim[i]);
   for (int i = 0; i < rank; i++) put(perm[i]);
-  for (const char* name : {"CUTT_TILED_ORDER", "CUTT_XCD_AWARE", "CUTT_ELEMS_PER_THREAD", "CUTT_PACKED_ROUNDS",
+  for (const char* name : {"CUTT_TILED_ORDER", "CUTT_XCD_AWARE", "CUTT_XCD_GROUP", "CUTT_ELEMS_PER_THREAD", "CUTT_PACKED_ROUNDS",
                            "CUTT_MAX_ITEMS", "CUTT_ITEM_ORDER", "CUTT_PAD_SHIFT", "CUTT_CACHE_POLICY", "CUTT_WIDE_OFFSETS", "CUTT_MBAR_ORDER",
                            "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
     const char* e = std::getenv(name);
@@ -350,12 +350,42 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (grouped) p.model.usPredicted *= 0.96;
 }
 
+// XCD b % 8 takes groups of 2^(g-1) neighbouring workgroups in turn instead of one chunk of the whole sequence (0).  Plans
+// whose workgroups are not dealt out to the XCDs, or whose XCDs each get a part of their own by address bits (order 7), stay.
+void setXcdGroup(Plan& p, int g) {
+  const bool packed = p.method == kPacked || p.method == kPackedSplit;
+  if (g < 0 || g > 20 || (!packed && p.method != kTiled)) return;
+  const uint32_t chunk = packed ? p.packed.xcdChunk : p.tiled.xcdChunk;
+  if (chunk == 0 || (packed ? p.itemDigits.n > 0 : p.tiled.order == 7)) return;
+  const int64_t unit = g > 0 ? (int64_t)kNumXcd << (g - 1) : 1, blocks = ((int64_t)chunk * kNumXcd + unit - 1) / unit * unit;
+  if (blocks > 0x7fffffffll || (uint64_t)blocks * (uint64_t)p.numThreads > CUTT_HIP_MAX_GRID_LANES) return;
+  if (packed) p.packed.xcdGroup = g;
+  else p.tiled.xcdGroup = (int16_t)g;
+  p.numBlocks = blocks;
+}
+
+// What the XCDs have in flight at one time lies together in memory when they share the sequence in groups of 16 workgroups,
+// at eight places a chunk apart otherwise, which costs the memory 2-10 %: 23425 x 8538, 8 bytes, 607 -> 565 us; (96,75,96,75)/
+// (2,1,3,0) 159 -> 157; 8192 x 8192, 4 bytes, 108 -> 102; (40,14881,4,6,14)/(3,2,0,1,4) 304 -> 293; (64,64,64,64,4)/(3,2,1,0,4)
+// 134 -> 99; 35 random Tiled plans +4 % in the mean, -3.5 % at worst.  (Groups of 4 and 32 are as good, 64 and more
+// lose part of it, single workgroups lose what neighbours share in an L2.)  That holds where every line is written whole
+// and past the caches.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 such plans
+// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.
+void chooseXcdGroup(Plan& p) {
+  if (const char* e = std::getenv("CUTT_XCD_GROUP")) {
+    setXcdGroup(p, std::atoi(e));
+    return;
+  }
+  setXcdGroup(p, (cachePolicyOf(p) & 2) && p.numBlocks >= 2048 ? 5 : 0);
+}
+
 // Cache policy of a plan that is going to be used, and rows in groups only with non-temporal loads: four rows in flight
 // find the lines again that such loads give up.  45 plans of the rule above, 0.3-0.9 GB per buffer, buffers in rotation:
 // with non-temporal loads 3.2 % faster than sixteen rows; with ordinary ones, which such tensors get now, 2.8 % slower (2.2 %
 // on inputs just written), and sixteen rows with those are 4.5 % faster than rows in groups with non-temporal loads.
 void chooseAccesses(Plan& p, const cuttHipDeviceProps& props) {
   chooseCachePolicy(p, props);
+  chooseXcdGroup(p);
   if (p.method == kTiled && p.tiled.lineWidth == 0 && !(p.tiled.cachePolicy & 1) && !std::getenv("CUTT_TILED_GROUPED")) p.tiled.grouped = 0;
 }
 
@@ -872,6 +902,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       // left to the planner again, which re-derives the numbering for the variant's geometry)
       if (plans[best].itemDigits.n > 0) cur.itemOrder = -1;
     }
+    cur.xcdGroup = tiled ? plans[best].tiled.xcdGroup : plans[best].packed.xcdGroup;
     if (plans[best].method == kTiled) {
       cur.tiledGrouped = plans[best].tiled.grouped;
       cur.tiledAligned = plans[best].tiled.lineWidth > 0 ? 1 : 0;
@@ -882,6 +913,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     auto tryVariant = [&](const PlannerOptions& v, bool sameGridIsSamePlan) -> bool {
       Plan q;
       if (!rebuildPlan(plans[best], props, v, q)) return false;
+      setXcdGroup(q, v.xcdGroup);
       if (sameGridIsSamePlan && q.numBlocks == plans[best].numBlocks) return false;
       setCachePolicy(q, v.cachePolicy);
       if (!estimatePlan(q, props, 10)) return false;
@@ -972,6 +1004,14 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     if (!failed && !rowGather && !std::getenv("CUTT_XCD_AWARE") && cur.xcdAware) {
       PlannerOptions v = cur;
       v.xcdAware = false;
+      if (tryVariant(v, false)) cur = v;
+    }
+    // ... or one chunk each, or groups of workgroups in turn
+    for (int g : {0, 3, 5}) {
+      if (failed || rowGather || std::getenv("CUTT_XCD_GROUP") || !cur.xcdAware) break;
+      if (g == start.xcdGroup) continue;
+      PlannerOptions v = cur;
+      v.xcdGroup = g;
       if (tryVariant(v, false)) cur = v;
     }
     // ... and the other cache policies of the global accesses

@@ -179,11 +179,13 @@ typedef struct cuttHipWalkMbar {
 typedef struct cuttHipTileWalk {
   int kind;                 /* 0: not of this form, 1: a single Mbar position, 2: with Mbar positions */
   uint32_t blocks;          /* workgroups of the launch */
-  uint32_t chunk;           /* workgroup b is position (b % 8) * chunk + b / 8, or b itself (see shifts) */
+  uint32_t chunk;           /* workgroup b is position (b % 8) * chunk + b / 8, in groups (b % 8) * chunk + (b / 8) % chunk +
+                               8 chunk ((b / 8) / chunk), or b itself (see shifts) */
   uint32_t superM;
   uint32_t stripMul;        /* division by the tiles of a strip (order 5: times the Mbar positions) */
   uint32_t fullMul, lastMul;  /* division by the width of a full strip, of the last one */
-  uint32_t shifts;          /* strip | full << 5 | last << 10 | (3: chunks per XCD, 0: none) << 15 */
+  uint32_t shifts;          /* strip | full << 5 | last << 10 | (3: XCD b % 8 has positions of its own, 0: not) << 15 |
+                               xcdGroup << 17 */
   cuttHipWalkMbar mbar;
   cuttHipWalkRows rowsK, rowsM;
 } cuttHipTileWalk;
@@ -214,8 +216,10 @@ typedef struct cuttHipTiledArgs {
                          grid has 8*xcdChunk workgroups */
   uint32_t superM, superK;
   int cachePolicy;    /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
-  int grouped;        /* 0: a lane has all 16 rows of its tile in flight at once; 1: four at a time
+  int16_t grouped;    /* 0: a lane has all 16 rows of its tile in flight at once; 1: four at a time
                          (each group of 16 tile rows is waited for before the next is requested) */
+  int16_t xcdGroup;   /* 0: the XCDs share the workgroups as xcdChunk says; g >= 1: XCD b % 8 takes groups of 2^(g-1)
+                         logical positions in turn, and the grid is a multiple of 8 groups */
   int lineWidth;      /* 0: 64x64 tiles.  1 ... cuttHipLinesMaxWidth(elemSize): line-aligned stores, every tile row
                          stores its own 64-element window of the output run, shifted so that it starts on a
                          128-byte line; tilesK is then ceil((volMk + 128/elemSize - 1) / 64), a tile is lineWidth
@@ -352,6 +356,7 @@ typedef struct cuttHipPackedArgs {
                           and the grid has 8*xcdChunk workgroups */
   int cachePolicy;     /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
   long long volume;    /* elements from the first to the last one of the tensor, on its wider side (bounds every offset) */
+  int xcdGroup;        /* as in cuttHipTiledArgs, for logical blocks */
   int wideOffsets;     /* 0: the tensor is below 4 GB and the kernel keeps 32-bit byte offsets;
                           1: element offsets with 64-bit address arithmetic (required from 4 GB on) */
   cuttHipPackedClass cls[4];
@@ -412,6 +417,7 @@ size_t cuttHipLinesLdsBytes(int elemSize, int tileWidth);
 /* Workgroups of a tiled launch with these arguments (padding workgroups included), 0 if they have no valid grid. */
 long long cuttHipTiledGrid(const cuttHipTiledArgs* args);
 long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* args);
+long long cuttHipPackedGrid(const cuttHipPackedArgs* args);
 int cuttHipLaunchTiled(const cuttHipTiledArgs* args, const void* in, void* out, void* stream);
 int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* args, const void* in, void* out, void* stream);
 int cuttHipLaunchPacked(const cuttHipPackedArgs* args, const void* in, void* out, void* stream);

@@ -469,7 +469,7 @@ bool divisorOk(const cuttHipDivisor& dv, uint32_t d) {
 }
 
 // Number of workgroups of a tiled launch; checks the ordering parameters.
-bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk, uint32_t superM,
+bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk, int xcdGroup, uint32_t superM,
               uint32_t superK, const cuttHipTileDigits& dg, const cuttHipMbar& mbar, uint64_t& blocks, uint64_t threads = kTileThreads) {
   uint64_t logical = (uint64_t)tilesM * tilesK * (uint64_t)volMbar;
   if (order == 7) {
@@ -511,7 +511,11 @@ bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk,
               (uint64_t)volMbar;
   }
   blocks = logical;
-  if (xcdChunk) {
+  if (xcdGroup < 0 || xcdGroup > 20) return false;
+  if (xcdGroup) {
+    const uint64_t unit = (uint64_t)kNumXcd << (xcdGroup - 1);
+    blocks = (logical + unit - 1) / unit * unit;
+  } else if (xcdChunk) {
     if ((uint64_t)xcdChunk * kNumXcd < logical) return false;
     blocks = (uint64_t)xcdChunk * kNumXcd;
   }
@@ -624,7 +628,7 @@ hipError_t launchKernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t 
 }  // namespace
 
 static bool copyTileGrid(const cuttHipCopyTiles& t, uint64_t& blocks) {
-  return tileGrid(t.order, t.tilesM, t.tilesK, t.volMbar, t.xcdChunk, t.superM, t.superK, t.digits, t.mbar, blocks);
+  return tileGrid(t.order, t.tilesM, t.tilesK, t.volMbar, t.xcdChunk, 0, t.superM, t.superK, t.digits, t.mbar, blocks);
 }
 
 // Lanes of a workgroup of these arguments.
@@ -634,7 +638,7 @@ static uint32_t tiledThreads(const cuttHipTiledArgs& a) {
 
 extern "C" long long cuttHipTiledGrid(const cuttHipTiledArgs* a) {
   uint64_t blocks = 0;
-  if (!a || !tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
+  if (!a || !tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->xcdGroup, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return 0;
   return (long long)blocks;
 }
@@ -657,7 +661,7 @@ extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
       !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm))
     return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
+  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->xcdGroup, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
   if (a->cachePolicy < 0 || a->cachePolicy > 3) return (int)hipErrorInvalidValue;
   if (a->walk.kind != 0) {  // the walk must be the one that follows from the other arguments
@@ -729,7 +733,7 @@ static int launchWalk(const cuttHipTiledArgs& a, const void* in, void* out, hipS
 extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, void* out, void* stream) {
   if (!a || !in || !out) return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
-  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
+  if (!tileGrid(a->order, a->tilesM, a->tilesK, a->volMbar, a->xcdChunk, a->xcdGroup, a->superM, a->superK, a->digits, a->mbar, blocks, tiledThreads(*a)))
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
@@ -948,12 +952,18 @@ static uint64_t packedGrid(const cuttHipPackedArgs* a) {
   const long long items = cuttHipPackedItemNumbers(a);
   if (items < 1) return 0;
   uint64_t blocks = ((uint64_t)items + a->itemsPerBlock - 1) / a->itemsPerBlock;
-  if (a->xcdChunk) {
+  if (a->xcdGroup < 0 || a->xcdGroup > 20) return 0;
+  if (a->xcdGroup) {
+    const uint64_t unit = (uint64_t)kNumXcd << (a->xcdGroup - 1);
+    blocks = (blocks + unit - 1) / unit * unit;
+  } else if (a->xcdChunk) {
     if ((uint64_t)a->xcdChunk * kNumXcd < blocks) return 0;
     blocks = (uint64_t)a->xcdChunk * kNumXcd;
   }
   return blocks <= 0x7fffffffull && blocks * (uint64_t)a->numThreads <= CUTT_HIP_MAX_GRID_LANES ? blocks : 0;
 }
+
+extern "C" long long cuttHipPackedGrid(const cuttHipPackedArgs* a) { return a ? (long long)packedGrid(a) : 0; }
 
 extern "C" int cuttHipValidatePacked(const cuttHipPackedArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;

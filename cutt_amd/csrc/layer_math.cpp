@@ -145,10 +145,18 @@ extern "C" void cuttHipFinishTileWalk(cuttHipTiledArgs* a) {
   walkDivisor(w.superM * tilesK * stripMbar, w.stripMul, strip);
   walkDivisor(w.superM, w.fullMul, full);
   walkDivisor(last ? last : 1, w.lastMul, lastShift);
-  const bool perXcd = a->xcdChunk != 0;
-  w.chunk = perXcd ? (uint32_t)((total + 7) / 8) : 0u;
-  w.blocks = perXcd ? 8 * w.chunk : (uint32_t)total;
-  w.shifts = strip | full << 5 | lastShift << 10 | (perXcd ? 3u : 0u) << 15;
+  const bool perXcd = a->xcdChunk != 0 || a->xcdGroup > 0;
+  if (a->xcdGroup < 0 || a->xcdGroup > 20) return;
+  if (a->xcdGroup > 0) {
+    w.chunk = 1u << (a->xcdGroup - 1);
+    const uint64_t unit = 8ull * w.chunk, blocks = (total + unit - 1) / unit * unit;
+    if (blocks > 0x7fffffffull) return;
+    w.blocks = (uint32_t)blocks;
+  } else {
+    w.chunk = perXcd ? (uint32_t)((total + 7) / 8) : 0u;
+    w.blocks = perXcd ? 8 * w.chunk : (uint32_t)total;
+  }
+  w.shifts = strip | full << 5 | lastShift << 10 | (perXcd ? 3u : 0u) << 15 | (uint32_t)a->xcdGroup << 17;
   w.kind = volMbar > 1 ? 2 : 1;
   if (w.kind == 2) {
     cuttHipWalkMbar& b = w.mbar;

@@ -30,8 +30,7 @@ __device__ __forceinline__ PackedItems packedItems(const cuttHipPackedArgs& a) {
                                         : (uint32_t)a.volMbar * ns0 * ns1;
   // XCD-aware numbering: XCD x (= blockIdx.x % 8) walks its own contiguous chunk of the work
   // items, so that neighbouring slabs and Mbar positions share an L2.
-  it.lb = blockIdx.x;
-  if (a.xcdChunk) it.lb = (blockIdx.x % kNumXcd) * (uint32_t)a.xcdChunk + blockIdx.x / kNumXcd;
+  it.lb = xcdPosition(blockIdx.x, a.xcdChunk, (uint32_t)a.xcdGroup);
   // Orders 0 and 1: ipb consecutive numbers.  Order 2: the workgroups of one XCD take the numbers
   // of their chunk in turn, so that the items in flight at one time are neighbours and a
   // workgroup's next item lies a whole round ahead.
@@ -39,7 +38,7 @@ __device__ __forceinline__ PackedItems packedItems(const cuttHipPackedArgs& a) {
   it.wStride = 1;
   it.count = it.wBase < totalItems ? min(ipb, totalItems - it.wBase) : 0;
   if (a.itemOrder == 2) {
-    const uint32_t chunkBlocks = a.xcdChunk ? (uint32_t)a.xcdChunk : gridDim.x;
+    const uint32_t chunkBlocks = a.xcdChunk && !a.xcdGroup ? (uint32_t)a.xcdChunk : gridDim.x;
     const uint32_t x = it.lb / chunkBlocks;
     const uint32_t chunkStart = x * chunkBlocks * ipb;
     const uint32_t chunkEnd = min(chunkStart + chunkBlocks * ipb, totalItems);

@@ -21,7 +21,6 @@ namespace {
 constexpr int kTile = 64;
 constexpr int kPadShift = 5;            // one LDS pad slot per 32 elements
 constexpr int64_t kMaxLdsSlots = 65536; // the gather index is 16 bits wide
-constexpr int64_t kNumXcd = 8;          // XCDs (private L2s); workgroup b runs on XCD b % 8
 
 inline int64_t ceilDiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int roundUp64(int64_t v) { return (int)(ceilDiv(v, 64) * 64); }

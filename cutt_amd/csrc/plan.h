@@ -147,6 +147,8 @@ struct Plan {
   std::string describe() const;
 };
 
+constexpr int64_t kNumXcd = 8;  // XCDs (private L2s); workgroup b runs on XCD b % 8
+
 struct PlannerOptions {
   int forceMethod = 0;      // 0 = all methods, else only this Method (Trivial always allowed)
   int tiledOrder = -1;      // -1 = planner's choice (super-tiles)
@@ -175,7 +177,8 @@ struct PlannerOptions {
   bool wideOffsets = false; // Packed/PackedSplit: 64-bit address arithmetic also below 4 GB (tests)
   bool rowGather = true;    // TiledCopy: gather the rows of dense tensors in output order instead of copying tiles
   int rowPolicy = -1, rowGroup = -1;  // ... its cache policy and XCD grouping, -1 = planner's choice
-  bool xcdAware = true;     // give every XCD (private L2) a contiguous chunk of the workgroup sequence
+  bool xcdAware = true;     // give every XCD (private L2) a contiguous chunk of the workgroup sequence ...
+  int xcdGroup = 0;         // ... or, g >= 1, groups of 2^(g-1) workgroups in turn (variants of the measuring planner)
 };
 
 // Build every candidate for the original and the fused problem

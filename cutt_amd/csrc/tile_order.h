@@ -43,16 +43,29 @@ constexpr int kWaves = kTileThreads / 64;
 // coordinates (cuttHipTileDigits): any nesting of patches, strips and Mbar runs can be written that way.
 constexpr uint32_t kNumXcd = 8;
 
+// Workgroup index -> logical position (cuttHipTiledArgs.xcdChunk, xcdGroup).
+__device__ __forceinline__ uint32_t xcdPosition(uint32_t bid, uint32_t chunk, uint32_t group) {
+  const uint32_t q = bid / kNumXcd, x = bid % kNumXcd;
+  if (group) {
+    const uint32_t g = group - 1;
+    return ((((q >> g) * kNumXcd) + x) << g) + (q & ((1u << g) - 1));
+  }
+  return chunk ? x * chunk + q : bid;
+}
+
+__device__ __forceinline__ uint32_t xcdGroupOf(const cuttHipTiledArgs& a) { return (uint32_t)a.xcdGroup; }
+__device__ __forceinline__ uint32_t xcdGroupOf(const cuttHipCopyTiles&) { return 0; }
+
 struct TileOrder {
   int order;
-  uint32_t xcdChunk, superM, superK;
+  uint32_t xcdChunk, xcdGroup, superM, superK;
   const cuttHipTileDigits* digits;  // order 7 (points into the kernel arguments)
 };
 
 __device__ __forceinline__ bool decodeTile(uint32_t bid, const TileOrder o, uint32_t tilesM,
                                            uint32_t tilesK, uint32_t volMbar, uint32_t& tm,
                                            uint32_t& tk, uint32_t& m) {
-  const uint32_t l = o.xcdChunk ? (bid % kNumXcd) * o.xcdChunk + bid / kNumXcd : bid;
+  const uint32_t l = xcdPosition(bid, o.xcdChunk, o.xcdGroup);
   if (o.order == 0) {
     const uint32_t t = l / volMbar;
     m = l - t * volMbar;
@@ -125,7 +138,7 @@ __device__ __forceinline__ bool decodeTile(uint32_t bid, const TileOrder o, uint
 template <bool SKIP = false, typename Args>
 __device__ __forceinline__ bool locateTile(const Args& a, uint32_t& tm, uint32_t& tk, uint32_t& offIn, uint32_t& offOut) {
   if (a.order == 7 && a.digits.lanes) {
-    const uint32_t l = a.xcdChunk ? (blockIdx.x % kNumXcd) * a.xcdChunk + blockIdx.x / kNumXcd : blockIdx.x;
+    const uint32_t l = xcdPosition(blockIdx.x, a.xcdChunk, xcdGroupOf(a));
     if (l >= a.digits.total) return false;
     static_assert(CUTT_MAX_TILE_DIGITS == 16, "one DPP row of 16 lanes holds the digits");
     const cuttHipDigitLane d = a.digits.lane[threadIdx.x & 15];  // (entries beyond the list contribute 0)
@@ -139,7 +152,7 @@ __device__ __forceinline__ bool locateTile(const Args& a, uint32_t& tm, uint32_t
     return tm < (uint32_t)a.tilesM && tk < (uint32_t)a.tilesK;
   }
   uint32_t m;
-  if (!decodeTile(blockIdx.x, TileOrder{a.order, a.xcdChunk, a.superM, a.superK, &a.digits}, a.tilesM, a.tilesK, a.volMbar, tm, tk, m)) return false;
+  if (!decodeTile(blockIdx.x, TileOrder{a.order, a.xcdChunk, xcdGroupOf(a), a.superM, a.superK, &a.digits}, a.tilesM, a.tilesK, a.volMbar, tm, tk, m)) return false;
   if constexpr (SKIP) {
     offIn = offOut = 0;
     if (a.volMbar == 1) return true;
@@ -165,8 +178,9 @@ struct NoMbar {};
 template <typename MB>
 __device__ __forceinline__ bool walkTile(const WalkHead& h, const MB& mb, uint32_t tilesM, uint32_t tilesK, uint32_t& tm, uint32_t& tk, uint32_t& offIn, uint32_t& offOut) {
   constexpr bool kMbar = !std::is_same_v<MB, NoMbar>;
-  const uint32_t xs = h.shifts >> 15;  // 3: XCD b % 8 walks its own chunk
-  uint32_t l = (blockIdx.x & ((1u << xs) - 1)) * h.chunk + (blockIdx.x >> xs), m = 0, perStrip = tilesK;
+  const uint32_t xs = (h.shifts >> 15) & 3, g = ((h.shifts >> 17) - 1) & 31;  // 3: XCD b % 8 has positions of its own; in groups of 2^g (31: no groups)
+  const uint32_t q = blockIdx.x >> xs;
+  uint32_t l = (blockIdx.x & ((1u << xs) - 1)) * h.chunk + (q & ((1u << g) - 1)) + (((q >> g) << g) << 3), m = 0, perStrip = tilesK;
   const uint32_t tiles = tilesM * tilesK;
   offIn = offOut = 0;
   if constexpr (kMbar) {

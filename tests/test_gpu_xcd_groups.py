@@ -1,0 +1,46 @@
+"""Workgroups handed to the XCDs in groups, bit-exact against the oracle: every Tiled numbering, line-aligned stores and the packed
+kernel's three item orders, group sizes from one workgroup to more than there are."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def method(monkeypatch):
+    import torch  # noqa: F401  (before the library is loaded: both must share one HIP runtime)
+    import cutt_amd as cutt
+    yield lambda m: cutt.set_method_override(m)
+    cutt.set_method_override(0)
+
+
+@pytest.mark.parametrize("es", [4, 8])
+@pytest.mark.parametrize("group", [1, 3, 5, 12])
+def test_tiled(method, monkeypatch, es, group):
+    import cutt_amd as cutt
+    from gpu_util import check_case
+    method(cutt.METHOD_TILED)
+    monkeypatch.setenv("CUTT_XCD_GROUP", str(group))
+    for order in ("0", "1", "2", "3", "5", "6", "-1"):
+        for aligned in ("0", "1"):
+            monkeypatch.setenv("CUTT_TILED_ALIGNED", aligned)
+            monkeypatch.setenv("CUTT_TILED_ORDER", order)
+            for dim, perm in [((600, 1130), (1, 0)), ((577, 130, 9), (2, 1, 0)), ((65, 4, 33, 70), (3, 2, 1, 0))]:
+                info = check_case(dim, perm, es)
+                assert info.method_name == "Tiled" and info.numBlocks % (8 << (group - 1)) == 0
+
+
+@pytest.mark.parametrize("es", [4, 8])
+@pytest.mark.parametrize("group", [1, 5, 12])
+def test_packed(method, monkeypatch, es, group):
+    import cutt_amd as cutt
+    from gpu_util import check_case
+    monkeypatch.setenv("CUTT_XCD_GROUP", str(group))
+    for how in (cutt.METHOD_PACKED, cutt.METHOD_PACKEDSPLIT):
+        method(how)
+        for order in "012":
+            monkeypatch.setenv("CUTT_ITEM_ORDER", order)
+            grouped = 0
+            for dim, perm in [((5, 7, 11, 13, 17, 19), (4, 2, 0, 5, 1, 3)), ((9, 1700, 5, 26), (2, 1, 0, 3)), ((3, 40, 61, 129), (1, 3, 2, 0))]:
+                info = check_case(dim, perm, es)
+                grouped += info.numBlocks % (8 << (group - 1)) == 0
+            assert grouped >= 2
