@@ -288,6 +288,17 @@ int runCount(cuttHipStreamCounts* out, void* stream, F&& launch) {
 
 extern "C" int cuttHipCountTiled(const cuttHipTiledArgs* a, cuttHipStreamCounts* out, void* stream) {
   if (int v = cuttHipValidateTiled(a); v != 0) return v;
+  cuttHipTiledArgs plain;
+  if (a->wide) {  // a wide tile makes the requests of four 64x64 ones, which the kernels below count in any order
+    plain = *a;
+    plain.wide = 0;
+    plain.tilesM = a->volMm / kTile;
+    plain.tilesK = a->volMk / kTile;
+    plain.order = 1;
+    plain.xcdChunk = 0;
+    plain.xcdGroup = 0;
+    a = &plain;
+  }
   const long long blocks = cuttHipTiledGrid(a);
   if (blocks < 1) return (int)hipErrorInvalidConfiguration;
   if (a->lineWidth)

@@ -86,7 +86,7 @@ std::string planKey(int deviceID, int force, int rank, const int* dim, const int
   for (int i = 0; i < rank; i++) put(perm[i]);
   for (const char* name : {"CUTT_TILED_ORDER", "CUTT_XCD_AWARE", "CUTT_XCD_GROUP", "CUTT_ELEMS_PER_THREAD", "CUTT_PACKED_ROUNDS",
                            "CUTT_MAX_ITEMS", "CUTT_ITEM_ORDER", "CUTT_PAD_SHIFT", "CUTT_CACHE_POLICY", "CUTT_WIDE_OFFSETS", "CUTT_MBAR_ORDER",
-                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
+                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILED_WIDE", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
     const char* e = std::getenv(name);
     k += e ? e : "-";
     k += ';';
@@ -431,9 +431,28 @@ bool tiledForm(const Plan& p, const cuttHipDeviceProps& props, PlannerOptions op
   return estimatePlan(q, props, 10);
 }
 
-// What is left to decide about a plan that is going to be used: line-aligned stores and the cache policy.
+// Tiled plan p with 128x128 tiles of 4-byte elements where they fit it and it lies beyond the memory-side cache; its
+// numbering must have a walk.  A tile reads and writes 512 bytes of a row instead of 256, what 8-byte elements have
+// with 64x64 tiles.  Against those, both in XCD groups, on 32 matrices and batches of 0.27-0.8 GB per buffer: 5 % faster in the mean
+// (8192 x 8192 101 -> 95 us, 16384 x 8192 214 -> 176, 8192 x 16384 213 -> 185, 1024 x 1024 x 64 103 -> 87, 10240 x 10240 163 -> 147;
+// (1280,50,1024)/(2,1,0) 103 -> 105 the worst).  Tensors inside the cache: +10 ... -7 %, left to the small tiles.
+bool wideForm(const Plan& p, const cuttHipDeviceProps& props, Plan& q) {
+  if (!wideTilesFit(p.split, p.pb) || p.tiled.lineWidth > 0 || p.tiled.order == 7 || p.tiled.grouped) return false;
+  PlannerOptions opt = plannerOptions(0);
+  if (opt.tiledWide < 0 && 2.0 * (double)p.pb.volume * p.pb.elemSize <= (double)props.infinityCacheBytes) return false;
+  const bool pinned = opt.tiledOrder >= 0 || !opt.superAuto || !opt.tileDigits.empty() || opt.tiledGrouped >= 0 || opt.tiledAligned > 0 || opt.digitLanes >= 0;
+  if (opt.tiledWide == 0 || (pinned && opt.tiledWide < 0)) return false;
+  opt.tiledWide = 1;
+  if (!rebuildPlan(p, props, opt, q) || !q.tiled.wide) return false;
+  q.tiled.mbar = p.tiled.mbar;  // (the order of the Mbar ranks may have been refined)
+  q.model = p.model;            // (a wide tile makes the requests of four others)
+  return true;
+}
+
+// What is left to decide about a plan that is going to be used: line-aligned stores, wide tiles and the cache policy.
 void finishPlan(Plan& p, const cuttHipDeviceProps& props) {
   Plan q;
+  if (wideForm(p, props, q)) p = std::move(q);
   if (lineWindowsPay(p, props) && tiledForm(p, props, plannerOptions(0), true, q)) {
     q.model.usPredicted = p.model.usPredicted;
     p = std::move(q);
@@ -527,6 +546,7 @@ PlannerOptions plannerOptions(int forceMethod) {
   if (const char* e = std::getenv("CUTT_SUPER_M")) { opt.superM = std::max(1, std::atoi(e)); opt.superAuto = false; }
   if (const char* e = std::getenv("CUTT_SUPER_K")) { opt.superK = std::max(1, std::atoi(e)); opt.superAuto = false; }
   if (const char* e = std::getenv("CUTT_TILED_GROUPED")) opt.tiledGrouped = std::atoi(e) != 0 ? 1 : 0;
+  if (const char* e = std::getenv("CUTT_TILED_WIDE")) opt.tiledWide = std::atoi(e) != 0 ? 1 : 0;
   if (const char* e = std::getenv("CUTT_TILED_ALIGNED")) opt.tiledAligned = std::atoi(e) != 0 ? 1 : 0;
   if (const char* e = std::getenv("CUTT_TILE_DIGITS")) opt.tileDigits = e;
   if (const char* e = std::getenv("CUTT_ITEM_DIGITS")) opt.itemDigits = e;
@@ -906,6 +926,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     if (plans[best].method == kTiled) {
       cur.tiledGrouped = plans[best].tiled.grouped;
       cur.tiledAligned = plans[best].tiled.lineWidth > 0 ? 1 : 0;
+      cur.tiledWide = plans[best].tiled.wide;
     }
     const PlannerOptions start = cur;
 
@@ -962,6 +983,13 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         PlannerOptions v = cur;
         v.tiledOrder = k.order; v.superM = k.superM; v.superK = k.superK;
         v.tileDigits.clear();
+        if (tryVariant(v, false)) cur = v;
+      }
+      // 64x64 instead of wide tiles
+      if (!failed && cur.tiledWide > 0) {
+        PlannerOptions v = cur;
+        v.tiledWide = 0;
+        v.superM *= 2;
         if (tryVariant(v, false)) cur = v;
       }
       // sixteen or four rows per lane in flight

@@ -220,7 +220,9 @@ typedef struct cuttHipTiledArgs {
                          (each group of 16 tile rows is waited for before the next is requested) */
   int16_t xcdGroup;   /* 0: the XCDs share the workgroups as xcdChunk says; g >= 1: XCD b % 8 takes groups of 2^(g-1)
                          logical positions in turn, and the grid is a multiple of 8 groups */
-  int lineWidth;      /* 0: 64x64 tiles.  1 ... cuttHipLinesMaxWidth(elemSize): line-aligned stores, every tile row
+  int16_t wide;       /* 1: tiles of 128x128 4-byte elements (CUTT_WIDE_TILE), for single-rank axes that are multiples of it and
+                         numberings with a walk; tilesM, tilesK, superM and superK count those tiles */
+  int16_t lineWidth;  /* 0: 64x64 tiles.  1 ... cuttHipLinesMaxWidth(elemSize): line-aligned stores, every tile row
                          stores its own 64-element window of the output run, shifted so that it starts on a
                          128-byte line; tilesK is then ceil((volMk + 128/elemSize - 1) / 64), a tile is lineWidth
                          elements wide along Mm (tilesM = ceil(volMm/lineWidth)), and grouped has no effect */
@@ -410,6 +412,9 @@ int cuttHipValidatePacked(const cuttHipPackedArgs* args);
  * elements; 71 columns 4.2 either way), 4 bytes 4.7-4.9 as one wide tile, 5.2-5.3 at 110-136 columns, 4.8-5.2 at 137-150
  * as three (0.9 GB per buffer, buffers in rotation). */
 #define CUTT_LINE_WIDTH 68
+/* Edge and lanes of the wide tiles. */
+#define CUTT_WIDE_TILE 128
+#define CUTT_WIDE_THREADS 1024
 /* Tiled with line-aligned stores: the widest tile along Mm, lanes per workgroup and bytes of LDS for a tile width. */
 int cuttHipLinesMaxWidth(int elemSize);
 int cuttHipLinesThreads(int elemSize, int tileWidth);

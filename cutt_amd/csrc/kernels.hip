@@ -161,6 +161,29 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
   moveTile<T, NT, false, kFused>(t, shape, in, out);
 }
 
+// Tiles of 128x128 4-byte elements.
+template <int NT, typename MB>
+__global__ __launch_bounds__(CUTT_WIDE_THREADS, 8) void wideTileKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t volMm, uint32_t volMk,
+                                                                   uint32_t strideInK, uint32_t strideOutM, uint32_t chunk, uint32_t superM,
+                                                                   uint32_t stripMul, uint32_t fullMul, uint32_t lastMul, uint32_t shifts,
+                                                                   const MB mb) {
+  constexpr uint32_t kEdge = CUTT_WIDE_TILE, kStep = CUTT_WIDE_THREADS / kEdge;
+  constexpr int kRows = kEdge / kStep;
+  __shared__ uint32_t tile[kEdge][kEdge + 1];
+  uint32_t tm, tk, offIn, offOut;
+  if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, volMm / kEdge, volMk / kEdge, tm, tk, offIn, offOut)) return;
+  const uint32_t c = threadIdx.x % kEdge, r = threadIdx.x / kEdge;
+  const uint32_t rd = offIn + tm * kEdge + c + (tk * kEdge + r) * strideInK, wr = offOut + tk * kEdge + c + (tm * kEdge + r) * strideOutM;
+  uint32_t v[kRows];
+#pragma unroll
+  for (int j = 0; j < kRows; j++) v[j] = ldg<NT>(in + (rd + j * kStep * strideInK));
+#pragma unroll
+  for (int j = 0; j < kRows; j++) tile[r + j * kStep][c] = v[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRows; j++) stg<NT>(out + (wr + j * kStep * strideOutM), tile[c][r + j * kStep]);
+}
+
 // ---------------------------------------------------------------------------
 // Tiled with line-aligned stores.
 // ---------------------------------------------------------------------------
@@ -633,7 +656,7 @@ static bool copyTileGrid(const cuttHipCopyTiles& t, uint64_t& blocks) {
 
 // Lanes of a workgroup of these arguments.
 static uint32_t tiledThreads(const cuttHipTiledArgs& a) {
-  return a.lineWidth ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.lineWidth) : (uint32_t)kTileThreads;
+  return a.lineWidth ? (uint32_t)cuttHipLinesThreads(a.elemSize, a.lineWidth) : (a.wide ? CUTT_WIDE_THREADS : (uint32_t)kTileThreads);
 }
 
 extern "C" long long cuttHipTiledGrid(const cuttHipTiledArgs* a) {
@@ -653,10 +676,14 @@ extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;
   if ((a->elemSize != 4 && a->elemSize != 8) || a->volMm < 1 || a->volMk < 1 || a->volMbar < 1)
     return (int)hipErrorInvalidValue;
-  const int width = a->lineWidth ? a->lineWidth : kTile, fringe = a->lineWidth ? 128 / a->elemSize - 1 : 0;
+  if ((a->wide != 0 && a->wide != 1) || (a->wide && (a->elemSize != 4 || a->lineWidth || a->grouped || a->rowsK.n > 0 || a->rowsM.n > 0 ||
+                                                     a->volMm % CUTT_WIDE_TILE || a->volMk % CUTT_WIDE_TILE || a->walk.kind == 0)))
+    return (int)hipErrorInvalidValue;
+  const int edge = a->wide ? CUTT_WIDE_TILE : kTile;
+  const int width = a->lineWidth ? a->lineWidth : edge, fringe = a->lineWidth ? 128 / a->elemSize - 1 : 0;
   if (width < 1 || (a->lineWidth && (width > cuttHipLinesMaxWidth(a->elemSize) || a->volMk > 0x7fffffff - 2 * kTile ||
                                      a->volMm > 0x7fffffff - 2 * kTile)) ||
-      a->tilesM != (a->volMm + width - 1) / width || a->tilesK != (a->volMk + fringe + kTile - 1) / kTile ||
+      a->tilesM != (a->volMm + width - 1) / width || a->tilesK != (a->volMk + fringe + edge - 1) / edge ||
       a->order < 0 || a->order > 7 || !mbarOk(a->mbar) || (a->grouped != 0 && a->grouped != 1) ||
       !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm))
     return (int)hipErrorInvalidValue;
@@ -726,6 +753,23 @@ static int launchWalkOfWidth(const cuttHipTiledArgs& a, const void* in, void* ou
   }
 }
 
+template <int NT, typename MB>
+static int launchWideOf(const cuttHipTiledArgs& a, const MB& mb, const void* in, void* out, hipStream_t s) {
+  const cuttHipTileWalk& w = a.walk;
+  return (int)launchKernel(wideTileKernel<NT, MB>, dim3(w.blocks), dim3(CUTT_WIDE_THREADS), 0, s, (const uint32_t*)in, (uint32_t*)out, (uint32_t)a.volMm,
+                           (uint32_t)a.volMk, a.strideInK, a.strideOutM, w.chunk, w.superM, w.stripMul, w.fullMul, w.lastMul, w.shifts, mb);
+}
+
+static int launchWide(const cuttHipTiledArgs& a, const void* in, void* out, hipStream_t s) {
+  const bool single = a.walk.kind == 1;
+  switch (a.cachePolicy) {
+    case 0: return single ? launchWideOf<0>(a, NoMbar{}, in, out, s) : launchWideOf<0>(a, a.walk.mbar, in, out, s);
+    case 1: return single ? launchWideOf<1>(a, NoMbar{}, in, out, s) : launchWideOf<1>(a, a.walk.mbar, in, out, s);
+    case 2: return single ? launchWideOf<2>(a, NoMbar{}, in, out, s) : launchWideOf<2>(a, a.walk.mbar, in, out, s);
+    default: return single ? launchWideOf<3>(a, NoMbar{}, in, out, s) : launchWideOf<3>(a, a.walk.mbar, in, out, s);
+  }
+}
+
 static int launchWalk(const cuttHipTiledArgs& a, const void* in, void* out, hipStream_t s) {
   return a.elemSize == 4 ? launchWalkOfWidth<uint32_t>(a, in, out, s) : launchWalkOfWidth<uint64_t>(a, in, out, s);
 }
@@ -737,6 +781,7 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
+  if (a->wide) return launchWide(*a, in, out, s);
   if (a->walk.kind && !a->grouped) return launchWalk(*a, in, out, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;

@@ -785,6 +785,7 @@ struct TiledShape {
   bool oneRankMk = false;          // a single rank along Mk
   bool lineWindows = false;        // stores in line-aligned windows ...
   int tileWidth = kTile;           // ... and tiles this wide along Mm
+  bool wide = false;               // 128x128 tiles
 };
 
 int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrdering& o, cuttHipTileDigits& dg) {
@@ -896,8 +897,12 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
     // rank between; 12, 24, 32 and 64 wide and patches of 16 x 16 ... 32 x 32 all gained less), on two boxes.
     // Rows that are multiples of 4, 8 or 16 KB only: -0.3 % (-3 ... +3 %), left alone.  Tensors inside the
     // memory-side cache lose 1-5 % (8192 x 354 ... 3911); from 0.75 cache sizes per buffer on it pays.
+    // Wide tiles read 512 bytes of a row each: strips of 8 of them, of 2 where the output rows are 32 KB apart as well (19 matrices,
+    // us in strips of 2 / 4 / 8 / 16: 8192 x 16384 185 / 190 / 206 / 221, 8192 x 24576 281 / 299 / 304 / 326, 24576 x 8192 265 /
+    // 264 / 273 / 275; 32768 x 4096 187 / 187 / 179 / 189, 16384 x 12800 308 / 315 / 300 / 309), of 16 for batches
+    // (8192 x 512 x 16: 97 / 96 / 99 / 92).
     gridRule = true;
-    superM = 16;
+    superM = !shape.wide || volMbar > 1 ? 16 : (rowBytesOut % 32768 == 0 ? 2 : 8);
   }
   if (opt.superAuto && !gridRule && (o.order == 5 || o.order == 3) && tilesM > superM && tilesM <= 14 &&
       !(elemSize == 8 && rowBytesIn % 128 == 0 && rowBytesOut % 128 == 0)) {
@@ -1146,7 +1151,9 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
   const Split& sp = plan.split;
   const Problem& pb = plan.pb;
   const bool lines = sp.method == kTiled && opt.tiledAligned > 0;
-  const int width = lines ? lineTileWidth(sp.volMm, pb.elemSize) : kTile;
+  const bool wide = sp.method == kTiled && !lines && opt.tiledWide > 0 && opt.tiledGrouped <= 0 && wideTilesFit(sp, pb);
+  const int edge = wide ? CUTT_WIDE_TILE : kTile;
+  const int width = lines ? lineTileWidth(sp.volMm, pb.elemSize) : edge;
   const int64_t tilesM = ceilDiv(sp.volMm, width);
   if (sp.method == kTiled) {
     cuttHipTiledArgs& a = plan.tiled;
@@ -1177,8 +1184,9 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       }
     }
     a.tilesM = (int)tilesM;
-    a.lineWidth = lines ? width : 0;
-    a.tilesK = (int)ceilDiv(sp.volMk + (lines ? 128 / pb.elemSize - 1 : 0), kTile);
+    a.lineWidth = (int16_t)(lines ? width : 0);
+    a.wide = wide ? 1 : 0;
+    a.tilesK = (int)ceilDiv(sp.volMk + (lines ? 128 / pb.elemSize - 1 : 0), edge);
     a.volMbar = (int)sp.volMbar;
     TileOrdering o;
     // an Mbar rank that follows Mm in the input and Mk in the output: consecutive Mbar positions are
@@ -1209,6 +1217,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       shape.volMbar = sp.volMbar;
       shape.volMmLastTile = sp.volMm - (tilesM - 1) * width;
       shape.lineWindows = lines;
+      shape.wide = wide;
       shape.tileWidth = width;
       shape.rowBytesIn = sp.volMm * pb.elemSize;
       shape.rowBytesOut = sp.volMk * pb.elemSize;
@@ -1220,6 +1229,14 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       plan.numBlocks = tiledBlocks(opt, shape, o, a.digits);
     }
     a.order = o.order; a.xcdChunk = o.xcdChunk; a.superM = o.superM; a.superK = o.superK;
+    if (wide) {  // (the wide tiles' kernel decodes walks only)
+      cuttHipFinishTileWalk(&a);
+      if (a.walk.kind == 0) {
+        PlannerOptions narrow = opt;
+        narrow.tiledWide = 0;
+        return setupTiled(plan, props, narrow);
+      }
+    }
     // How the kernels decode a free numbering.  Digit by digit costs a chain of up to 16 dependent scalar loads
     // per workgroup, which a workgroup that moves a full tile hides but one that moves a quarter of it does not
     // (a (4194304,32) transpose of 4-byte elements in the digits of its default order: 4.4 TB/s digit by digit,
@@ -1230,7 +1247,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     if (a.order == 7 && (opt.digitLanes > 0 || (opt.digitLanes < 0 && tileBytes <= 8192))) cuttHipFinishTileDigits(&a.digits, &a.mbar);
     a.cachePolicy = opt.cachePolicy;
     a.grouped = opt.tiledGrouped > 0 ? 1 : 0;  // -1: decided from the model's estimate later
-    plan.ldsBytes = lines ? cuttHipLinesLdsBytes(pb.elemSize, width) : (size_t)kTile * (kTile + 1) * pb.elemSize;
+    plan.ldsBytes = lines ? cuttHipLinesLdsBytes(pb.elemSize, width) : (size_t)edge * (edge + 1) * pb.elemSize;
   } else {
     std::memset(&plan.tcopy, 0, sizeof(plan.tcopy));
     cuttHipCopyTiles& a = plan.tcopy.tiles;
@@ -1258,7 +1275,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     if (a.order == 7 && opt.digitLanes > 0) cuttHipFinishTileDigits(&a.digits, &a.mbar);
     plan.ldsBytes = 0;
   }
-  plan.numThreads = lines ? cuttHipLinesThreads(pb.elemSize, width) : 256;
+  plan.numThreads = lines ? cuttHipLinesThreads(pb.elemSize, width) : (wide ? CUTT_WIDE_THREADS : 256);
   // one tile per workgroup: a tensor with tens of millions of tiny tiles has no Tiled candidate
   return plan.numBlocks <= 0x7fffffffll && (uint64_t)plan.numBlocks * (uint64_t)plan.numThreads <= CUTT_HIP_MAX_GRID_LANES;
 }
@@ -1503,6 +1520,10 @@ void addPackedSplit(const Problem& pb, bool fromReduced, const cuttHipDeviceProp
 }  // namespace
 
 // Text form of a digit list (what parseTileDigits reads).
+bool wideTilesFit(const Split& sp, const Problem& pb) {
+  return sp.method == kTiled && pb.elemSize == 4 && sp.numMm == 1 && sp.numMk == 1 && sp.volMm % CUTT_WIDE_TILE == 0 && sp.volMk % CUTT_WIDE_TILE == 0;
+}
+
 std::string formatTileDigits(const cuttHipTileDigits& dg) {
   std::string t;
   for (int i = 0; i < dg.n; i++) {

@@ -163,6 +163,7 @@ struct PlannerOptions {
   bool addressBits = true;  // Tiled: number the workgroups by the address bits their digits move where that rule applies (addressBitOrder)
   int tiledFuse = -1;       // Tiled over fused rank sets: -1 = planner's choice, 0 = one rank per side only
   int tiledAligned = -1;    // Tiled: line-aligned stores, -1 = planner's choice, 0 = off, 1 = on
+  int tiledWide = -1;       // Tiled: 128x128 tiles where they fit (4-byte elements), -1 = planner's choice (finishPlan), 0 = off, 1 = on
   int tiledGrouped = -1;    // Tiled: rows of a lane in flight, -1 = planner's choice, 0 = all 16, 1 = 4 at a time
   int elemsPerThread = 0;    // Packed/PackedSplit: 0 = planner's choice, else 1, 2, 4, 8 or 16
   int packedRounds = 0;      // > 0: size the grid for this many waves of resident workgroups
@@ -185,6 +186,9 @@ struct PlannerOptions {
 // (reference src/cuttplan.cpp:681-698).  Returns false on an internal error.
 bool createPlans(const Problem& orig, const Problem& red, const cuttHipDeviceProps& props,
                  const PlannerOptions& opt, std::vector<Plan>& plans);
+
+// Whether a Tiled plan's axes are whole tiles of 128x128 4-byte elements.
+bool wideTilesFit(const Split& sp, const Problem& pb);
 
 // Same index sets as `src`, launch geometry recomputed under different options (used by the
 // measuring planner to try ordering and granularity variants of its best candidate).
