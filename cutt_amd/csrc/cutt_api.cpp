@@ -350,6 +350,8 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (grouped) p.model.usPredicted *= 0.96;
 }
 
+PlannerOptions plannerOptions(int forceMethod);
+
 // XCD b % 8 takes groups of 2^(g-1) neighbouring workgroups in turn instead of one chunk of the whole sequence (0).  Plans
 // whose workgroups are not dealt out to the XCDs, or whose XCDs each get a part of their own by address bits (order 7), stay.
 void setXcdGroup(Plan& p, int g) {
@@ -370,13 +372,37 @@ void setXcdGroup(Plan& p, int g) {
 // 134 -> 99; 35 random Tiled plans +4 % in the mean, -3.5 % at worst.  (Groups of 4 and 32 are as good, 64 and more
 // lose part of it, single workgroups lose what neighbours share in an L2.)  That holds where every line is written whole
 // and past the caches.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 such plans
-// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.
-void chooseXcdGroup(Plan& p) {
+// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.  Nor where 64x64 tiles write long rows a
+// multiple of 32 KB apart, which fall into few memory channels unless the XCDs work far from each other: 8224 x 8192, 4 bytes,
+// 98 -> 137 us, 8192 x 8192, 8 bytes, 196 -> 205 (16384 x 4096 175 -> 174 the best of six); rows of 48 KB gain, 6144 x 6144 115 -> 105.
+void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
   if (const char* e = std::getenv("CUTT_XCD_GROUP")) {
     setXcdGroup(p, std::atoi(e));
     return;
   }
-  setXcdGroup(p, (cachePolicyOf(p) & 2) && p.numBlocks >= 2048 ? 5 : 0);
+  cuttHipTiledArgs& a = p.tiled;
+  const bool sameChannels = p.method == kTiled && !a.wide && a.lineWidth == 0 && a.rowsM.n == 0 && (int64_t)a.strideOutM * a.elemSize % 32768 == 0 &&
+                            (int64_t)a.volMk * a.elemSize >= 8192;
+  // 8-byte input rows a multiple of 64 KB apart beside long output rows: 8192 x 12352 294 -> 304 us.
+  const bool longRows = p.method == kTiled && a.lineWidth == 0 && a.elemSize == 8 && a.tilesK > 160 && (int64_t)a.volMm * a.elemSize % 65536 == 0;
+  // (a packed workgroup moves several blocks: 1024 of them are 16 MB and more)
+  if (!(cachePolicyOf(p) & 2) || sameChannels || longRows || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
+    setXcdGroup(p, 0);
+    return;
+  }
+  // the orders that belong to groups (plan.cpp: tiledBlocks), unless options pin one
+  PlannerOptions opt = plannerOptions(0);
+  Plan q;
+  opt.groupOrders = true;
+  if (p.method == kTiled && !a.wide && a.lineWidth == 0 && a.order != 7 && opt.tiledOrder < 0 && opt.superAuto && opt.tileDigits.empty() &&
+      rebuildPlan(p, props, opt, q) && q.tiled.order != 7) {
+    a.order = q.tiled.order;
+    a.superM = q.tiled.superM;
+    a.superK = q.tiled.superK;
+    a.xcdChunk = q.tiled.xcdChunk;
+    p.numBlocks = q.numBlocks;
+  }
+  setXcdGroup(p, 5);
 }
 
 // Cache policy of a plan that is going to be used, and rows in groups only with non-temporal loads: four rows in flight
@@ -385,7 +411,7 @@ void chooseXcdGroup(Plan& p) {
 // on inputs just written), and sixteen rows with those are 4.5 % faster than rows in groups with non-temporal loads.
 void chooseAccesses(Plan& p, const cuttHipDeviceProps& props) {
   chooseCachePolicy(p, props);
-  chooseXcdGroup(p);
+  chooseXcdGroup(p, props);
   if (p.method == kTiled && p.tiled.lineWidth == 0 && !(p.tiled.cachePolicy & 1) && !std::getenv("CUTT_TILED_GROUPED")) p.tiled.grouped = 0;
 }
 

@@ -83,7 +83,11 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // ranks that lead the output on the Mk side), so the rows of a tile are not equally far apart.  Lane l
 // derives the offset of row l of either axis with a short mixed-radix decode (tileRowOffsets) and the
 // wave picks a row's offset out of that lane; the elements of a row are contiguous as before.
-template <typename T, int NT, bool GROUPED, bool FUSED, typename Args>
+//
+// TESTED (without GROUPED): one piece of code whose row groups are tested one after the other, for numberings that have no
+// walk.  Its loads wait for each other, which costs a small tensor 1 us but paces 4-byte tensors numbered by address bits, which
+// are beyond every cache: (1024,64,1024)/(2,1,0) 105.2 -> 102.5 us, (1024,16,1024,12)/(2,1,0,3) 279.9 -> 276.2; 8-byte ones lose 1-2 %.
+template <typename T, int NT, bool GROUPED, bool TESTED, bool FUSED, typename Args>
 __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
   __shared__ T tile[kTile][kTile + 1];
   const uint32_t wave = threadIdx.x >> 6;
@@ -125,9 +129,27 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
     else f(std::integral_constant<int, 1>{}, std::false_type{});
   };
   static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
-  byGroups(t.wK, read);
-  __syncthreads();
-  byGroups(t.wM, write);
+  if constexpr (TESTED && !GROUPED && sizeof(T) == 4) {
+    T v[kTileRows];
+#pragma unroll
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsK) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+#pragma unroll
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsK) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+    __syncthreads();
+    T u[kTileRows];
+#pragma unroll
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsM) u[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+#pragma unroll
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsM) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), u[j]);
+  } else {
+    byGroups(t.wK, read);
+    __syncthreads();
+    byGroups(t.wM, write);
+  }
 }
 
 // Any numbering of the workgroups (tile_order.h: locateTile).
@@ -139,7 +161,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  moveTile<T, NT, GROUPED, FUSED>(t, a, in, out);
+  moveTile<T, NT, GROUPED, true, FUSED>(t, a, in, out);
 }
 
 // The numberings of cuttHipTileWalk.  The arguments up to `shifts`, 14 words, are in scalar registers when a wave starts
@@ -158,7 +180,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
   if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
   const WalkShape<ROWS> shape{volMm, volMk, strideInK, strideOutM, rows};
   const TileLanes t = tileLanes<kFused>(shape, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  moveTile<T, NT, false, kFused>(t, shape, in, out);
+  moveTile<T, NT, false, false, kFused>(t, shape, in, out);
 }
 
 // Tiles of 128x128 4-byte elements.

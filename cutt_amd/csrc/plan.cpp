@@ -858,6 +858,16 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
       rowBytesIn > 0 && rowBytesIn % 128 == 0 && rowBytesOut % 128 == 0 && tilesM >= 16 && tilesK >= 17 && tilesK <= 700 &&
       rowBytesIn % 4096 != 0 && rowBytesIn % 16384 >= 1024 && rowBytesIn % 16384 <= 16384 - 1024)
     o.order = 2;
+  // Input rows a multiple of 4 KB apart and output rows that are not a multiple of 32 KB, when the XCDs share the sequence in groups of
+  // 16 tiles (cutt_api.cpp: chooseXcdGroup): strips of 8 then lie in few rows' channels.  4-byte elements take strips of 16 (one row of
+  // such a strip is a group), 8-byte ones the tiles along Mk fastest up to 160 of them, beyond that strips of 16 up to 32 tiles along
+  // Mm.  us with one chunk per XCD / strips of 8 in groups / this: 1024 x 1056 x 64, 4 bytes, 93.6 / 100.8 / 88.4, 2048 x 2080 x 16 92.1 /
+  // 100.5 / 89.3, 12288 x 12832 233 / 253 / 224; 8 bytes 8192 x 8208 204 / 209 / 195, 1024 x 1040 x 64 178 / 180 / 173, 2048 x 2048 x 8
+  // 89 / 91 / 89, 2048 x 40016 260 / 254 / 242.
+  const bool fewChannels = opt.groupOrders && opt.superAuto && opt.tiledOrder < 0 && (o.order == 3 || o.order == 5) && !mbarBetween && !neighbourRunsInMm &&
+                           beyondCache && rowBytesIn > 0 && rowBytesIn % 4096 == 0 && rowBytesOut % 128 == 0 && rowBytesOut % 32768 != 0 && tilesM >= 16 &&
+                           tilesK >= 16;
+  if (fewChannels && elemSize == 8 && tilesK <= 160) o.order = 2;
   // Super-tiles of up to superM x superK tiles, shrunk where a direction has fewer tiles.
   int64_t superM = opt.superM, superK = opt.superK;
   bool gridRule = false;
@@ -903,6 +913,10 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
     // (8192 x 512 x 16: 97 / 96 / 99 / 92).
     gridRule = true;
     superM = !shape.wide || volMbar > 1 ? 16 : (rowBytesOut % 32768 == 0 ? 2 : 8);
+  }
+  if (fewChannels && (elemSize == 4 || tilesM <= 32)) {
+    gridRule = true;
+    superM = 16;
   }
   if (opt.superAuto && !gridRule && (o.order == 5 || o.order == 3) && tilesM > superM && tilesM <= 14 &&
       !(elemSize == 8 && rowBytesIn % 128 == 0 && rowBytesOut % 128 == 0)) {

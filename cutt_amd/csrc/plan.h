@@ -179,6 +179,7 @@ struct PlannerOptions {
   bool rowGather = true;    // TiledCopy: gather the rows of dense tensors in output order instead of copying tiles
   int rowPolicy = -1, rowGroup = -1;  // ... its cache policy and XCD grouping, -1 = planner's choice
   bool xcdAware = true;     // give every XCD (private L2) a contiguous chunk of the workgroup sequence ...
+  bool groupOrders = false; // Tiled: the orders for workgroups that the XCDs share in groups (finishPlan)
   int xcdGroup = 0;         // ... or, g >= 1, groups of 2^(g-1) workgroups in turn (variants of the measuring planner)
 };
 
