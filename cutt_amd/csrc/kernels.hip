@@ -84,9 +84,10 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // derives the offset of row l of either axis with a short mixed-radix decode (tileRowOffsets) and the
 // wave picks a row's offset out of that lane; the elements of a row are contiguous as before.
 //
-// TESTED (without GROUPED): one piece of code whose row groups are tested one after the other, for numberings that have no
-// walk.  Its loads wait for each other, which costs a small tensor 1 us but paces 4-byte tensors numbered by address bits, which
-// are beyond every cache: (1024,64,1024)/(2,1,0) 105.2 -> 102.5 us, (1024,16,1024,12)/(2,1,0,3) 279.9 -> 276.2; 8-byte ones lose 1-2 %.
+// TESTED (without GROUPED): one piece of code whose row groups are tested one after the other, so that their loads wait for each
+// other.  That costs a small tensor 1 us but paces large ones whose neighbouring tiles must find shared lines in the L2, and 4-byte
+// ones numbered by address bits: (9,6,1739,45,42)/(2,1,0,3,4), 4 bytes, 339 -> 312 us, (850,226,354)/(1,0,2), 8 bytes, 215 -> 212,
+// (1024,64,1024)/(2,1,0), 4 bytes, 105.2 -> 102.5; 8-byte ones numbered by address bits lose 1-2 %.
 template <typename T, int NT, bool GROUPED, bool TESTED, bool FUSED, typename Args>
 __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
   __shared__ T tile[kTile][kTile + 1];
@@ -129,7 +130,7 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
     else f(std::integral_constant<int, 1>{}, std::false_type{});
   };
   static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
-  if constexpr (TESTED && !GROUPED && sizeof(T) == 4) {
+  if constexpr (TESTED && !GROUPED && (sizeof(T) == 4 || !(NT & 2))) {
     T v[kTileRows];
 #pragma unroll
     for (int j = 0; j < kTileRows; j++)
@@ -804,7 +805,9 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
   if (a->wide) return launchWide(*a, in, out, s);
-  if (a->walk.kind && !a->grouped) return launchWalk(*a, in, out, s);
+  // Tensors beyond the memory-side cache (192 MB and more per buffer) with ordinary stores take the kernel that paces its loads.
+  const bool paced = !(a->cachePolicy & 2) && (uint64_t)a->volMm * a->volMk * a->volMbar * a->elemSize > (192ull << 20);
+  if (a->walk.kind && !a->grouped && !paced) return launchWalk(*a, in, out, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \
