@@ -386,7 +386,10 @@ void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
   // 8-byte input rows a multiple of 64 KB apart beside long output rows: 8192 x 12352 294 -> 304 us.
   const bool longRows = p.method == kTiled && a.lineWidth == 0 && a.elemSize == 8 && a.tilesK > 160 && (int64_t)a.volMm * a.elemSize % 65536 == 0;
   // (a packed workgroup moves several blocks: 1024 of them are 16 MB and more)
-  if (!(cachePolicyOf(p) & 2) || sameChannels || longRows || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
+  // Line-aligned stores read a third of a 4-byte tile's rows again with the next window along Mk (an eighth of an 8-byte one's): in strips that
+  // window is a strip's width away, outside the group.  (379,6,21988)/(1,2,0) 83 -> 93 us, (94,519,944)/(2,1,0) 76 -> 79.
+  const bool fringeApart = p.method == kTiled && a.lineWidth > 0 && a.elemSize == 4 && a.order != 2 && a.superM > 1;
+  if (!(cachePolicyOf(p) & 2) || sameChannels || longRows || fringeApart || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
     setXcdGroup(p, 0);
     return;
   }
