@@ -350,8 +350,6 @@ void chooseTiledGrouping(Plan& p, const cuttHipDeviceProps& props) {
   if (grouped) p.model.usPredicted *= 0.96;
 }
 
-PlannerOptions plannerOptions(int forceMethod);
-
 // XCD b % 8 takes groups of 2^(g-1) neighbouring workgroups in turn instead of one chunk of the whole sequence (0).  Plans
 // whose workgroups are not dealt out to the XCDs, or whose XCDs each get a part of their own by address bits (order 7), stay.
 void setXcdGroup(Plan& p, int g) {
@@ -393,12 +391,12 @@ void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
     setXcdGroup(p, 0);
     return;
   }
-  // the orders that belong to groups (plan.cpp: tiledBlocks), unless options pin one
   PlannerOptions opt = plannerOptions(0);
+  if (p.method == kTiled && (opt.tiledOrder >= 0 || !opt.superAuto || !opt.tileDigits.empty())) return;  // options that pin the sequence
+  // the orders that belong to groups (plan.cpp: tiledBlocks)
   Plan q;
   opt.groupOrders = true;
-  if (p.method == kTiled && !a.wide && a.lineWidth == 0 && a.order != 7 && opt.tiledOrder < 0 && opt.superAuto && opt.tileDigits.empty() &&
-      rebuildPlan(p, props, opt, q) && q.tiled.order != 7) {
+  if (p.method == kTiled && !a.wide && a.lineWidth == 0 && a.order != 7 && rebuildPlan(p, props, opt, q) && q.tiled.order != 7) {
     a.order = q.tiled.order;
     a.superM = q.tiled.superM;
     a.superK = q.tiled.superK;

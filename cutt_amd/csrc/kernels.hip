@@ -170,7 +170,8 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
 // MB and ROWS hold what launches with Mbar positions and with fused axes need besides.
 // Bound by latency up to some 20 MB, by memory beyond.  Against the kernel above as it was before (its loads in groups of
 // four that waited for each other): 2011 x 1163, 4 bytes, 5.94 -> 4.38 us; (24,32,36,43)/(3,1,2,0), 8 bytes, 5.99 -> 4.86;
-// 4297 x 1731, 8 bytes, 28.2 -> 25.5; (7,149,21,189)/(3,2,1,0), 4 bytes, 9.5 -> 7.8; (96,75,96,75)/(2,1,3,0), 8 bytes, 161.7 -> 159.0.
+// 4297 x 1731, 8 bytes, 28.2 -> 25.5; (7,149,21,189)/(3,2,1,0), 4 bytes, 9.5 -> 7.8; (96,75,96,75)/(2,1,3,0), 8 bytes, 161.7 -> 159.0,
+// 157.7 in XCD groups.
 template <typename T, int NT, typename MB, typename ROWS>
 __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restrict__ in, T* __restrict__ out, uint32_t volMm, uint32_t volMk,
                                                                 uint32_t strideInK, uint32_t strideOutM, uint32_t chunk, uint32_t superM,
@@ -184,7 +185,11 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
   moveTile<T, NT, false, false, kFused>(t, shape, in, out);
 }
 
-// Tiles of 128x128 4-byte elements.
+// Tiles of 128x128 4-byte elements, whole ones only, numbered by a walk.
+// Bound by the memory channels: a 64x64 tile touches 256 bytes of a row at a time, and with rows a power of two apart the
+// pieces in flight crowd into few channels.  512 bytes of each row on both sides spread them: 8192 x 8192 101 (64x64) -> 95 us,
+// 16384 x 8192 214 -> 176, 8192 x 16384 213 -> 185, 10240 x 10240 163 -> 147.  1024 lanes with 16 loads each, two workgroups per CU
+// (66 KB of LDS); reading and writing the same pieces without transposing is 2 % slower with 512 lanes, 5-20 % with tiles of 256x64 or 64x256.
 template <int NT, typename MB>
 __global__ __launch_bounds__(CUTT_WIDE_THREADS, 8) void wideTileKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t volMm, uint32_t volMk,
                                                                    uint32_t strideInK, uint32_t strideOutM, uint32_t chunk, uint32_t superM,
@@ -218,8 +223,10 @@ __global__ __launch_bounds__(CUTT_WIDE_THREADS, 8) void wideTileKernel(const uin
 // up to one line, so the workgroup reads up to 64 + (elements per line - 1) rows along Mk into a taller LDS tile;
 // the rows in the fringe are also read by the tile next door, from the L2, which is why the loads are temporal.
 //
-// 23425 x 8538, 8 bytes: 675 us with ordinary tiles (4.75 TB/s) -> 605 us (5.3 TB/s); 16411 x 9377, 4 bytes: 282 ->
-// 241 us; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 358 -> 323 us (buffers in rotation).  Read from beyond the
+// 23425 x 8538, 8 bytes: 675 us with ordinary tiles (4.75 TB/s) -> 605 us, 560 (5.7 TB/s) since the XCDs share the
+// workgroups in groups; 16411 x 9377, 4 bytes: 282 -> 241, 227; (132,11,3,47,14,2,35)/(2,1,3,6,5,0,4), 4 bytes: 358 -> 323, 315
+// (buffers in rotation).  One workgroup for two to nine windows in turn, which reads no fringe row twice, is 0-10 % slower with
+// 8-byte elements and 10-50 % with 4-byte ones.  Read from beyond the
 // L2: 1.21 times the tensor's bytes on the first (ordinary tiles 1.03), 1.00 times on the third and on
 // (200000,2,500)/(2,1,0), where every fringe row hits the L2; written 1.000-1.002 times (1.007-1.054).  The same windows
 // with ordinary stores gain half of that, ordinary tiles with non-temporal stores lose 20-40 % (their partial lines go

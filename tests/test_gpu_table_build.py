@@ -1,14 +1,16 @@
 """Index tables built on the device for cuttExecuteNoAlloc, against the oracle: lists of few, of up to eight and of more ranks, with
-the Packed and the PackedSplit method."""
+the Packed method and, on a tensor that has such a plan, with PackedSplit."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
+SPLIT = (20000, 2, 50)
+
 
 @pytest.mark.parametrize("es", [4, 8])
 @pytest.mark.parametrize("dim,perm", [
-    ((63, 65, 33), (2, 1, 0)), ((5, 7, 11, 13, 3), (4, 2, 0, 3, 1)), ((3, 2, 5, 4, 3, 2, 7, 5), (7, 5, 3, 1, 6, 4, 2, 0)),
+    (SPLIT, (2, 1, 0)), ((5, 7, 11, 13, 3), (4, 2, 0, 3, 1)), ((3, 2, 5, 4, 3, 2, 7, 5), (7, 5, 3, 1, 6, 4, 2, 0)),
     ((2, 3, 2, 3, 2, 3, 2, 3, 2, 3), (9, 7, 5, 3, 1, 8, 6, 4, 2, 0)),
     ((2, 2, 3, 2, 2, 3, 2, 2, 2, 3, 2, 2), (11, 9, 7, 5, 3, 1, 10, 8, 6, 4, 2, 0)),
 ])
@@ -22,6 +24,8 @@ def test_tables_built_on_the_device(dim, perm, es):
     expect = oracle.transpose(list(dim), list(perm), data)
     try:
         for method in (cutt.METHOD_PACKED, cutt.METHOD_PACKEDSPLIT):
+            if (method == cutt.METHOD_PACKEDSPLIT) != (dim == SPLIT):
+                continue
             cutt.set_method_override(method)
             d_out = torch.full_like(d_in, -1)
             rc = cutt.cuttExecuteNoAlloc(len(dim), list(dim), list(perm), es, gpu_util.stream_handle(), d_in.data_ptr(), d_out.data_ptr())

@@ -44,3 +44,25 @@ def test_packed(method, monkeypatch, es, group):
                 info = check_case(dim, perm, es)
                 grouped += info.numBlocks % (8 << (group - 1)) == 0
             assert grouped >= 2
+
+
+@pytest.mark.parametrize("dim,perm,es,grouped", [
+    ((6000, 6080), (1, 0), 4, True),       # whole lines, past the caches
+    ((8200, 5003), (1, 0), 8, True),       # line-aligned windows
+    ((379, 131928), (1, 0), 4, False),     # ... of 4-byte elements in strips
+    ((1201, 3001), (1, 0), 8, False),      # inside the cache: neighbours share lines
+    ((3001, 2999), (1, 0), 4, False),
+])
+def test_planner_takes_groups_where_lines_are_written_whole(method, monkeypatch, dim, perm, es, grouped):
+    import torch
+    import cutt_amd as cutt
+    st = torch.cuda.current_stream().cuda_stream
+    blocks = []
+    for group in (None, "0", "5"):
+        if group:
+            monkeypatch.setenv("CUTT_XCD_GROUP", group)
+        rc, h = cutt.cuttPlan(len(dim), list(dim), list(perm), es, st)
+        assert rc == cutt.CUTT_SUCCESS
+        blocks.append(cutt.get_plan_info(h).numBlocks)
+        cutt.cuttDestroy(h)
+    assert blocks[1] != blocks[2] and (blocks[0] == blocks[2]) == grouped and blocks[2] % 128 == 0

@@ -1,9 +1,7 @@
 """Workgroups handed to the XCDs in groups: every logical position is visited exactly once, in both forms the kernels decode
-(tile_order.h: xcdPosition and walkTile), and plans take groups only where lines are written whole and past the caches (no GPU)."""
+(tile_order.h: xcdPosition and walkTile; no GPU)."""
 import os
 import subprocess
-
-import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
