@@ -131,21 +131,33 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
   };
   static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
   if constexpr (TESTED && !GROUPED && (sizeof(T) == 4 || !(NT & 2))) {
+    // (one test per group of four rows: a test per row makes the compiler branch around every single load, 1-2 % slower)
     T v[kTileRows];
 #pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsK) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+    for (int g = 0; g < kRowGroups; g++)
+      if ((uint32_t)g < t.groupsK) {
 #pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsK) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+      }
+#pragma unroll
+    for (int g = 0; g < kRowGroups; g++)
+      if ((uint32_t)g < t.groupsK) {
+#pragma unroll
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+      }
     __syncthreads();
-    T u[kTileRows];
 #pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsM) u[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+    for (int g = 0; g < kRowGroups; g++)
+      if ((uint32_t)g < t.groupsM) {
 #pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsM) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), u[j]);
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+      }
+#pragma unroll
+    for (int g = 0; g < kRowGroups; g++)
+      if ((uint32_t)g < t.groupsM) {
+#pragma unroll
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
+      }
   } else {
     byGroups(t.wK, read);
     __syncthreads();
