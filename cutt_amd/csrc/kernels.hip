@@ -84,10 +84,9 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // derives the offset of row l of either axis with a short mixed-radix decode (tileRowOffsets) and the
 // wave picks a row's offset out of that lane; the elements of a row are contiguous as before.
 //
-// TESTED (without GROUPED): one piece of code whose row groups are tested one after the other, so that their loads wait for each
-// other.  That costs a small tensor 1 us but paces large ones whose neighbouring tiles must find shared lines in the L2, and 4-byte
-// ones numbered by address bits: (9,6,1739,45,42)/(2,1,0,3,4), 4 bytes, 339 -> 312 us, (850,226,354)/(1,0,2), 8 bytes, 215 -> 212,
-// (1024,64,1024)/(2,1,0), 4 bytes, 105.2 -> 102.5; 8-byte ones numbered by address bits lose 1-2 %.
+// TESTED: one piece of code with a test for every row, whose loads the compiler makes wait for each other.  For 4-byte elements with non-temporal stores
+// in numberings that have no walk (address bits, mostly): (1024,64,1024)/(2,1,0) 105.2 -> 103.1 us, 103.5 in the form of tiledKernel,
+// (1024,16,1024,12)/(2,1,0,3) 278.2 there -> 275.4; 8-byte elements lose 1-2 %.
 template <typename T, int NT, bool GROUPED, bool TESTED, bool FUSED, typename Args>
 __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
   __shared__ T tile[kTile][kTile + 1];
@@ -130,34 +129,22 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
     else f(std::integral_constant<int, 1>{}, std::false_type{});
   };
   static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
-  if constexpr (TESTED && !GROUPED && (sizeof(T) == 4 || !(NT & 2))) {
-    // (one test per group of four rows: a test per row makes the compiler branch around every single load, 1-2 % slower)
+  if constexpr (TESTED) {
     T v[kTileRows];
 #pragma unroll
-    for (int g = 0; g < kRowGroups; g++)
-      if ((uint32_t)g < t.groupsK) {
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsK) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
 #pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
-      }
-#pragma unroll
-    for (int g = 0; g < kRowGroups; g++)
-      if ((uint32_t)g < t.groupsK) {
-#pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
-      }
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsK) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
     __syncthreads();
+    T u[kTileRows];
 #pragma unroll
-    for (int g = 0; g < kRowGroups; g++)
-      if ((uint32_t)g < t.groupsM) {
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsM) u[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
 #pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
-      }
-#pragma unroll
-    for (int g = 0; g < kRowGroups; g++)
-      if ((uint32_t)g < t.groupsM) {
-#pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
-      }
+    for (int j = 0; j < kTileRows; j++)
+      if ((uint32_t)(j / kGroupRows) < t.groupsM) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), u[j]);
   } else {
     byGroups(t.wK, read);
     __syncthreads();
@@ -174,7 +161,51 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  moveTile<T, NT, GROUPED, true, FUSED>(t, a, in, out);
+  if constexpr (!GROUPED && !(NT & 2)) {
+    // Ordinary stores, a large tensor (cuttHipLaunchTiled): one piece of code whose row groups are tested one after the other.  A group's
+    // loads go out while the next one's addresses are computed, and no load is waited for before all are out.  All sixteen at once
+    // (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no longer find shared lines in the L2.
+    // Written out here: as a function of its own, forced inline, the compiler keeps a lane's rows in one register tuple and merges it behind every
+    // test with copies that wait for the loads: (777,111,1000)/(1,0,2), 8 bytes, 246.7 us here, 252.5 that way, (633,147,1602)/(1,0,2) 442.5 / 453.4,
+    // (9,7,23,7,46,11,5,3)/(4,7,0,6,3,1,5,2), 4 bytes, 157.1 / 160.3; 24 such tensors 0.9 % in the mean, -1.5 ... +2.4 %.
+    const uint32_t wave = threadIdx.x >> 6;
+    __shared__ T tile[kTile][kTile + 1];
+    {
+      T v[kTileRows];
+#pragma unroll
+      for (int g = 0; g < kRowGroups; g++) {
+        if ((uint32_t)g < t.groupsK) {
+#pragma unroll
+          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < kRowGroups; g++) {
+        if ((uint32_t)g < t.groupsK) {
+#pragma unroll
+          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+        }
+      }
+    }
+    __syncthreads();
+    T v[kTileRows];
+#pragma unroll
+    for (int g = 0; g < kRowGroups; g++) {
+      if ((uint32_t)g < t.groupsM) {
+#pragma unroll
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < kRowGroups; g++) {
+      if ((uint32_t)g < t.groupsM) {
+#pragma unroll
+        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
+      }
+    }
+  } else {
+    moveTile<T, NT, GROUPED, !GROUPED && sizeof(T) == 4, FUSED>(t, a, in, out);
+  }
 }
 
 // The numberings of cuttHipTileWalk.  The arguments up to `shifts`, 14 words, are in scalar registers when a wave starts

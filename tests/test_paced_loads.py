@@ -1,6 +1,6 @@
-"""The instance of the Tiled kernel that paces its loads, in the machine code of the library built here: the four row groups wait
-for each other, the four loads of a group go out back to back.  A test per row instead of one per group leaves a branch before every
-load (large 8-byte tensors with ordinary stores took 1-2.5 % longer)."""
+"""The Tiled kernel for large tensors with ordinary stores, in the machine code of the library built here: a lane's sixteen loads go out in
+four groups, and nothing waits for a load before the last one is out.  (Where the compiler keeps the rows in one register tuple, the tests between
+the groups merge it with copies that wait for the loads: 1-2.5 % on such tensors.)"""
 import os
 import re
 import struct
@@ -22,7 +22,7 @@ def code_objects(path):
         at = data.find(b"\x7fELF", at + 1)
 
 
-def test_loads_of_a_row_group_go_out_back_to_back(tmp_path):
+def test_no_load_is_waited_for_before_all_are_out(tmp_path):
     checked = 0
     for i, obj in enumerate(code_objects(cutt_amd.lib_path())):
         path = os.path.join(str(tmp_path), "%d.co" % i)
@@ -32,8 +32,7 @@ def test_loads_of_a_row_group_go_out_back_to_back(tmp_path):
         # 8-byte elements, ordinary stores, rows not in groups, a single rank per axis
         for name in sorted(set(re.findall(r"FUNC .* (\S+11tiledKernelImLi[01]ELb0ELb0EE\w+)\n", names))):
             code = subprocess.check_output([LLVM + "llvm-objdump", "-d", "--disassemble-symbols=" + name, path], text=True)
-            straight = re.split(r"\n\s+s_c?branch\S*", code)
-            loads = [len(re.findall(r"global_load_dwordx2", piece)) for piece in straight]
-            assert [n for n in loads if n] == [4, 4, 4, 4], (name, loads)
+            at = [m.start() for m in re.finditer("global_load_dwordx2", code)]
+            assert len(at) == 16 and "vmcnt" not in code[at[0]:at[-1]], name
             checked += 1
     assert checked == 2
