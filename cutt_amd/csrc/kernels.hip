@@ -87,7 +87,7 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // TESTED: one piece of code with a test for every row, whose loads the compiler makes wait for each other.  For 4-byte elements with non-temporal stores
 // in numberings that have no walk (address bits, mostly): (1024,64,1024)/(2,1,0) 105.2 -> 103.1 us, 103.5 in the form of tiledKernel,
 // (1024,16,1024,12)/(2,1,0,3) 278.2 there -> 275.4; 8-byte elements lose 1-2 %.
-template <typename T, int NT, bool GROUPED, bool TESTED, bool FUSED, typename Args>
+template <typename T, int NT, bool TESTED, bool FUSED, typename Args>
 __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
   __shared__ T tile[kTile][kTile + 1];
   const uint32_t wave = threadIdx.x >> 6;
@@ -96,30 +96,22 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
   // the other and a test in between the compiler waits for a group's loads before the next one's go out, since the rows'
   // registers meet again behind the test.  WHOLE: all 64 rows are there, no index needs clamping.
   auto read = [&](auto groups, auto whole) __attribute__((always_inline)) {  // lanes run along the input-contiguous axis (Mm), rows along Mk
-    constexpr int kRows = decltype(groups)::value * kGroupRows, kStep = GROUPED ? kGroupRows : kRows;
+    constexpr int kRows = decltype(groups)::value * kGroupRows;
     const uint32_t lastRow = decltype(whole)::value ? kTile - 1u : t.wK;
+    T v[kRows];
 #pragma unroll
-    for (int g = 0; g < kRows; g += kStep) {
-      T v[kStep];
+    for (int j = 0; j < kRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, lastRow));
 #pragma unroll
-      for (int j = 0; j < kStep; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, g + j, lastRow));
-      if constexpr (GROUPED) waitForGlobalAccesses();
-#pragma unroll
-      for (int j = 0; j < kStep; j++) tile[min(wave + kWaves * (g + j), lastRow)][t.cx] = v[j];
-    }
+    for (int j = 0; j < kRows; j++) tile[min(wave + kWaves * j, lastRow)][t.cx] = v[j];
   };
   auto write = [&](auto groups, auto whole) __attribute__((always_inline)) {  // lanes run along the output-contiguous axis (Mk), rows along Mm
-    constexpr int kRows = decltype(groups)::value * kGroupRows, kStep = GROUPED ? kGroupRows : kRows;
+    constexpr int kRows = decltype(groups)::value * kGroupRows;
     const uint32_t lastRow = decltype(whole)::value ? kTile - 1u : t.wM;
+    T v[kRows];
 #pragma unroll
-    for (int g = 0; g < kRows; g += kStep) {
-      T v[kStep];
+    for (int j = 0; j < kRows; j++) v[j] = tile[t.ck][min(wave + kWaves * j, lastRow)];
 #pragma unroll
-      for (int j = 0; j < kStep; j++) v[j] = tile[t.ck][min(wave + kWaves * (g + j), lastRow)];
-#pragma unroll
-      for (int j = 0; j < kStep; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, g + j, lastRow), v[j]);
-      if constexpr (GROUPED) waitForGlobalAccesses();
-    }
+    for (int j = 0; j < kRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, lastRow), v[j]);
   };
   auto byGroups = [](uint32_t lastRow, auto&& f) __attribute__((always_inline)) {
     if (lastRow == kTile - 1) f(std::integral_constant<int, 4>{}, std::true_type{});
@@ -161,13 +153,15 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  if constexpr (!GROUPED && !(NT & 2)) {
-    // Ordinary stores, a large tensor (cuttHipLaunchTiled): one piece of code whose row groups are tested one after the other.  A group's
-    // loads go out while the next one's addresses are computed, and no load is waited for before all are out.  All sixteen at once
-    // (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no longer find shared lines in the L2.
+  if constexpr (GROUPED || !(NT & 2)) {
+    // Rows in groups, or ordinary stores and a large tensor (cuttHipLaunchTiled): one piece of code whose row groups are tested one after the
+    // other.  Without GROUPED a group's loads go out while the next one's addresses are computed, and no load is waited for before all are
+    // out.  All sixteen at once (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no
+    // longer find shared lines in the L2.
     // Written out here: as a function of its own, forced inline, the compiler keeps a lane's rows in one register tuple and merges it behind every
     // test with copies that wait for the loads: (777,111,1000)/(1,0,2), 8 bytes, 246.7 us here, 252.5 that way, (633,147,1602)/(1,0,2) 442.5 / 453.4,
-    // (9,7,23,7,46,11,5,3)/(4,7,0,6,3,1,5,2), 4 bytes, 157.1 / 160.3; 24 such tensors 0.9 % in the mean, -1.5 ... +2.4 %.
+    // (9,7,23,7,46,11,5,3)/(4,7,0,6,3,1,5,2), 4 bytes, 157.1 / 160.3; 24 such tensors 0.9 % in the mean, -1.5 ... +2.4 %.  With rows in
+    // groups a straight piece of code per number of row groups costs 3.5-5.5 % instead: 16411 x 9377, 4 bytes, 282.4 us here, 296.3 that way.
     const uint32_t wave = threadIdx.x >> 6;
     __shared__ T tile[kTile][kTile + 1];
     {
@@ -177,13 +171,20 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
         if ((uint32_t)g < t.groupsK) {
 #pragma unroll
           for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+          if constexpr (GROUPED) {
+            waitForGlobalAccesses();
+#pragma unroll
+            for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+          }
         }
       }
+      if constexpr (!GROUPED) {
 #pragma unroll
-      for (int g = 0; g < kRowGroups; g++) {
-        if ((uint32_t)g < t.groupsK) {
+        for (int g = 0; g < kRowGroups; g++) {
+          if ((uint32_t)g < t.groupsK) {
 #pragma unroll
-          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+            for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+          }
         }
       }
     }
@@ -194,17 +195,24 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
       if ((uint32_t)g < t.groupsM) {
 #pragma unroll
         for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) v[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+        if constexpr (GROUPED) {
+#pragma unroll
+          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
+          waitForGlobalAccesses();
+        }
       }
     }
+    if constexpr (!GROUPED) {
 #pragma unroll
-    for (int g = 0; g < kRowGroups; g++) {
-      if ((uint32_t)g < t.groupsM) {
+      for (int g = 0; g < kRowGroups; g++) {
+        if ((uint32_t)g < t.groupsM) {
 #pragma unroll
-        for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
+          for (int j = g * kGroupRows; j < (g + 1) * kGroupRows; j++) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), v[j]);
+        }
       }
     }
   } else {
-    moveTile<T, NT, GROUPED, !GROUPED && sizeof(T) == 4, FUSED>(t, a, in, out);
+    moveTile<T, NT, sizeof(T) == 4, FUSED>(t, a, in, out);
   }
 }
 
@@ -225,7 +233,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
   if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
   const WalkShape<ROWS> shape{volMm, volMk, strideInK, strideOutM, rows};
   const TileLanes t = tileLanes<kFused>(shape, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  moveTile<T, NT, false, false, kFused>(t, shape, in, out);
+  moveTile<T, NT, false, kFused>(t, shape, in, out);
 }
 
 // Tiles of 128x128 4-byte elements, whole ones only, numbered by a walk.
