@@ -230,10 +230,13 @@ typedef struct cuttHipTiledArgs {
   cuttHipRowRadix rowsM; /* Mm index -> output offset (n == 0: index * strideOutM) */
   cuttHipTileDigits digits; /* order 7 only */
   cuttHipTileWalk walk;     /* the numbering as the usual kernels decode it, derived from the rest (cuttHipFinishTileWalk) */
-  cuttHipMbar mbar;         /* last: the data pointers follow it in the kernel's arguments and are then read with the line
-                               that holds its last entries.  With 16 bytes more in between, which move them into a line of
+  cuttHipMbar mbar;         /* last: the data pointers follow it in the kernel's arguments and are then read with the 128-byte
+                               line that holds its last entries.  With 16 bytes more in between, which move them into a line of
                                their own, launches of 5-13 us took 1-8 % longer: (5,18,12758,2)/(2,3,0,1), 8 bytes, 10.3 us
-                               instead of 9.5, 867 x 3788 11.9 / 11.2, 433 x 12223, 4 bytes, 9.6 / 9.3 */
+                               instead of 9.5, 867 x 3788 11.9 / 11.2, 433 x 12223, 4 bytes, 9.6 / 9.3; with only the second
+                               pointer in the next line, in tile order 0, 8.95 / 8.65, 10.4 / 10.2, 8.9 / 8.6.  (That the walk's 332
+                               bytes lie in front of them, not read by these kernels, costs nothing: 8.67, 10.17, 8.64 with them,
+                               8.64, 10.15, 8.64 without.) */
 } cuttHipTiledArgs;
 
 /* Derive a->walk from the other arguments (kind 0 if their numbering is not of its form). */

@@ -25,7 +25,9 @@ def test_data_pointers_share_the_line_of_the_last_mbar_entries(tmp_path):
                            "-I" + os.path.join(ROOT, "include"), str(src), "-o", exe])
     for line in subprocess.check_output([exe], text=True).splitlines():
         mbar_end, pointers = map(int, line.split())
-        assert (mbar_end - 1) // 128 == pointers // 128, line
+        # (both pointers: with the second one in the next line launches of 8-10 us take 2-3 % longer)
+        first = (pointers + 7) // 8 * 8
+        assert (mbar_end - 1) // 128 == first // 128 == (first + 15) // 128, line
 
 
 def test_copy_tiles_carry_no_row_table(tmp_path):
