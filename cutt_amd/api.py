@@ -55,6 +55,7 @@ class PlanInfo(ctypes.Structure):
         ("tiledAligned", ctypes.c_int), ("itemOrder", ctypes.c_int),
         ("numPieces", ctypes.c_int), ("numShapes", ctypes.c_int), ("wideOffsets", ctypes.c_int),
         ("tileDigits", ctypes.c_char * 192), ("rowGather", ctypes.c_int),
+        ("xcdGroup", ctypes.c_int), ("tiledWide", ctypes.c_int), ("tiledPaced", ctypes.c_int),
     ]
 
     @property

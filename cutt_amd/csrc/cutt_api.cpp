@@ -86,7 +86,7 @@ std::string planKey(int deviceID, int force, int rank, const int* dim, const int
   for (int i = 0; i < rank; i++) put(perm[i]);
   for (const char* name : {"CUTT_TILED_ORDER", "CUTT_XCD_AWARE", "CUTT_XCD_GROUP", "CUTT_ELEMS_PER_THREAD", "CUTT_PACKED_ROUNDS",
                            "CUTT_MAX_ITEMS", "CUTT_ITEM_ORDER", "CUTT_PAD_SHIFT", "CUTT_CACHE_POLICY", "CUTT_WIDE_OFFSETS", "CUTT_MBAR_ORDER",
-                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILED_WIDE", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
+                           "CUTT_SUPER_M", "CUTT_SUPER_K", "CUTT_TILED_GROUPED", "CUTT_TILED_ALIGNED", "CUTT_TILED_WIDE", "CUTT_TILED_PACED", "CUTT_TILE_DIGITS", "CUTT_ITEM_DIGITS", "CUTT_DIGIT_LANES", "CUTT_TILED_FUSE", "CUTT_ROW_GATHER", "CUTT_ADDRESS_BITS", "CUTT_MODEL_RUN_LENGTH"}) {
     const char* e = std::getenv(name);
     k += e ? e : "-";
     k += ';';
@@ -222,6 +222,9 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.tiledGrouped = p.method == kTiled ? p.tiled.grouped : 0;
   o.tiledAligned = p.method == kTiled && p.tiled.lineWidth > 0 ? 1 : 0;
   o.rowGather = p.method == kTiledCopy ? p.tcopy.rowGather : 0;
+  o.xcdGroup = p.method == kTiled ? p.tiled.xcdGroup : (p.method == kPacked || p.method == kPackedSplit ? p.packed.xcdGroup : 0);
+  o.tiledWide = p.method == kTiled ? p.tiled.wide : 0;
+  o.tiledPaced = p.method == kTiled ? p.tiled.paced : 0;
   o.itemOrder = (p.method == kPacked || p.method == kPackedSplit) ? p.packed.itemOrder : 0;
   o.numPieces = 1;
   o.numShapes = 1;
@@ -240,14 +243,15 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   }
 }
 
-void setCachePolicy(Plan& p, int policy) {
+PlannerOptions plannerOptions(int forceMethod);
+
+void setCachePolicy(Plan& p, int policy, const cuttHipDeviceProps& props) {
   if (p.method == kTiledCopy && p.tcopy.rowGather) return;  // chosen with the row gathering (plan.cpp: setupRows)
   p.tiled.cachePolicy = policy;
   p.tcopy.tiles.cachePolicy = policy;
   p.packed.cachePolicy = policy;
+  choosePacing(p, props, plannerOptions(0));
 }
-
-PlannerOptions plannerOptions(int forceMethod);
 
 // Cache policy of a plan's global accesses, from its size and the model's sampled address stream.  (Not applied when
 // CUTT_CACHE_POLICY pins the policy.)  Timed on 120 random tensors of 0.14-1.6 GB per buffer, buffers in rotation and
@@ -277,24 +281,24 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
   const double cache = (double)props.infinityCacheBytes;
   if (cache > 0 && 2.0 * bytes <= cache) {
-    setCachePolicy(p, 0);
+    setCachePolicy(p, 0, props);
     return;
   }
   if (p.method == kTiled && p.tiled.lineWidth > 0) {
-    setCachePolicy(p, 2);
+    setCachePolicy(p, 2, props);
     return;
   }
   const double lines = bytes / 128.0;
   if (p.method == kTrivial) {
-    setCachePolicy(p, bytes <= 3.5 * cache ? 1 : 3);
+    setCachePolicy(p, bytes <= 3.5 * cache ? 1 : 3, props);
     return;
   }
   if (p.model.wrPartialLines <= 0.01 * lines) {
-    setCachePolicy(p, bytes > cache && p.model.rdLines <= 1.02 * lines ? 3 : 2);
+    setCachePolicy(p, bytes > cache && p.model.rdLines <= 1.02 * lines ? 3 : 2, props);
     return;
   }
   const bool narrowTiles = (p.method == kTiled || p.method == kTiledCopy) && p.pb.elemSize == 4;
-  setCachePolicy(p, bytes <= cache && p.model.rdLines < (narrowTiles ? 1.5 : 1.7) * lines ? 1 : 0);
+  setCachePolicy(p, bytes <= cache && p.model.rdLines < (narrowTiles ? 1.5 : 1.7) * lines ? 1 : 0, props);
 }
 
 // Runs f(0) .. f(n-1) on up to eight host threads (CUTT_PLAN_THREADS caps the number; 1 = the
@@ -574,6 +578,7 @@ PlannerOptions plannerOptions(int forceMethod) {
   if (const char* e = std::getenv("CUTT_SUPER_K")) { opt.superK = std::max(1, std::atoi(e)); opt.superAuto = false; }
   if (const char* e = std::getenv("CUTT_TILED_GROUPED")) opt.tiledGrouped = std::atoi(e) != 0 ? 1 : 0;
   if (const char* e = std::getenv("CUTT_TILED_WIDE")) opt.tiledWide = std::atoi(e) != 0 ? 1 : 0;
+  if (const char* e = std::getenv("CUTT_TILED_PACED")) opt.tiledPaced = std::atoi(e) != 0 ? 1 : 0;
   if (const char* e = std::getenv("CUTT_TILED_ALIGNED")) opt.tiledAligned = std::atoi(e) != 0 ? 1 : 0;
   if (const char* e = std::getenv("CUTT_TILE_DIGITS")) opt.tileDigits = e;
   if (const char* e = std::getenv("CUTT_ITEM_DIGITS")) opt.itemDigits = e;
@@ -963,7 +968,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       if (!rebuildPlan(plans[best], props, v, q)) return false;
       setXcdGroup(q, v.xcdGroup);
       if (sameGridIsSamePlan && q.numBlocks == plans[best].numBlocks) return false;
-      setCachePolicy(q, v.cachePolicy);
+      setCachePolicy(q, v.cachePolicy, props);
       if (!estimatePlan(q, props, 10)) return false;
       double t;
       if (!timePlan(q, t)) { failed = true; return false; }

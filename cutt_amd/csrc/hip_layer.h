@@ -226,6 +226,8 @@ typedef struct cuttHipTiledArgs {
                          stores its own 64-element window of the output run, shifted so that it starts on a
                          128-byte line; tilesK is then ceil((volMk + 128/elemSize - 1) / 64), a tile is lineWidth
                          elements wide along Mm (tilesM = ceil(volMm/lineWidth)), and grouped has no effect */
+  int paced;          /* 1: 64x64 tiles go through the general kernel, whose loads leave row group by row group, also
+                         where their numbering has a walk (plan.cpp: choosePacing) */
   cuttHipRowRadix rowsK; /* Mk index -> input offset (n == 0: index * strideInK) */
   cuttHipRowRadix rowsM; /* Mm index -> output offset (n == 0: index * strideOutM) */
   cuttHipTileDigits digits; /* order 7 only */

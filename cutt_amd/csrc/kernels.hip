@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
   if constexpr (GROUPED || !(NT & 2)) {
-    // Rows in groups, or ordinary stores and a large tensor (cuttHipLaunchTiled): one piece of code whose row groups are tested one after the
+    // Rows in groups, or ordinary stores and a large tensor (cuttHipTiledArgs.paced): one piece of code whose row groups are tested one after the
     // other.  Without GROUPED a group's loads go out while the next one's addresses are computed, and no load is waited for before all are
     // out.  All sixteen at once (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no
     // longer find shared lines in the L2.
@@ -765,7 +765,7 @@ extern "C" int cuttHipValidateTiled(const cuttHipTiledArgs* a) {
   if (width < 1 || (a->lineWidth && (width > cuttHipLinesMaxWidth(a->elemSize) || a->volMk > 0x7fffffff - 2 * kTile ||
                                      a->volMm > 0x7fffffff - 2 * kTile)) ||
       a->tilesM != (a->volMm + width - 1) / width || a->tilesK != (a->volMk + fringe + edge - 1) / edge ||
-      a->order < 0 || a->order > 7 || !mbarOk(a->mbar) || (a->grouped != 0 && a->grouped != 1) ||
+      a->order < 0 || a->order > 7 || !mbarOk(a->mbar) || (a->grouped != 0 && a->grouped != 1) || (a->paced != 0 && a->paced != 1) ||
       !rowRadixOk(a->rowsK, a->volMk) || !rowRadixOk(a->rowsM, a->volMm))
     return (int)hipErrorInvalidValue;
   uint64_t blocks = 0;
@@ -863,9 +863,7 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
   if (a->wide) return launchWide(*a, in, out, s);
-  // Tensors beyond the memory-side cache (192 MB and more per buffer) with ordinary stores take the kernel that paces its loads.
-  const bool paced = !(a->cachePolicy & 2) && (uint64_t)a->volMm * a->volMk * a->volMbar * a->elemSize > (192ull << 20);
-  if (a->walk.kind && !a->grouped && !paced) return launchWalk(*a, in, out, s);
+  if (a->walk.kind && !a->grouped && !a->paced) return launchWalk(*a, in, out, s);
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \

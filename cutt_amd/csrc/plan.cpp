@@ -1261,6 +1261,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     if (a.order == 7 && (opt.digitLanes > 0 || (opt.digitLanes < 0 && tileBytes <= 8192))) cuttHipFinishTileDigits(&a.digits, &a.mbar);
     a.cachePolicy = opt.cachePolicy;
     a.grouped = opt.tiledGrouped > 0 ? 1 : 0;  // -1: decided from the model's estimate later
+    choosePacing(plan, props, opt);
     plan.ldsBytes = lines ? cuttHipLinesLdsBytes(pb.elemSize, width) : (size_t)edge * (edge + 1) * pb.elemSize;
   } else {
     std::memset(&plan.tcopy, 0, sizeof(plan.tcopy));
@@ -1533,11 +1534,22 @@ void addPackedSplit(const Problem& pb, bool fromReduced, const cuttHipDeviceProp
 
 }  // namespace
 
-// Text form of a digit list (what parseTileDigits reads).
+// 64x64 tiles with ordinary stores and more than 0.75 memory-side cache sizes per buffer (192 MB): the general kernel, whose loads go out
+// row group by row group (kernels.hip: tiledKernel), instead of the walk's.  56 random tensors with ordinary stores, time by the walk's kernel over time by
+// the general one, mean and range: 24-64 MB per buffer 0.91 (0.82-0.96), 64-160 MB 0.98 (0.94-1.07), 160-192 MB 1.00, 192-900 MB 1.006 (0.97-1.05).
+void choosePacing(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt) {
+  if (plan.method != kTiled) return;
+  cuttHipTiledArgs& a = plan.tiled;
+  const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
+  const bool pays = !(a.cachePolicy & 2) && (double)plan.pb.volume * plan.pb.elemSize > 0.75 * cache;
+  a.paced = !a.wide && a.lineWidth == 0 && (opt.tiledPaced < 0 ? pays : opt.tiledPaced > 0) ? 1 : 0;
+}
+
 bool wideTilesFit(const Split& sp, const Problem& pb) {
   return sp.method == kTiled && pb.elemSize == 4 && sp.numMm == 1 && sp.numMk == 1 && sp.volMm % CUTT_WIDE_TILE == 0 && sp.volMk % CUTT_WIDE_TILE == 0;
 }
 
+// Text form of a digit list (what parseTileDigits reads).
 std::string formatTileDigits(const cuttHipTileDigits& dg) {
   std::string t;
   for (int i = 0; i < dg.n; i++) {

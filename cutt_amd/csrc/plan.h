@@ -164,6 +164,7 @@ struct PlannerOptions {
   int tiledFuse = -1;       // Tiled over fused rank sets: -1 = planner's choice, 0 = one rank per side only
   int tiledAligned = -1;    // Tiled: line-aligned stores, -1 = planner's choice, 0 = off, 1 = on
   int tiledWide = -1;       // Tiled: 128x128 tiles where they fit (4-byte elements), -1 = planner's choice (finishPlan), 0 = off, 1 = on
+  int tiledPaced = -1;      // Tiled: the general kernel also for numberings with a walk, -1 = planner's choice (choosePacing), 0 = off, 1 = on
   int tiledGrouped = -1;    // Tiled: rows of a lane in flight, -1 = planner's choice, 0 = all 16, 1 = 4 at a time
   int elemsPerThread = 0;    // Packed/PackedSplit: 0 = planner's choice, else 1, 2, 4, 8 or 16
   int packedRounds = 0;      // > 0: size the grid for this many waves of resident workgroups
@@ -190,6 +191,9 @@ bool createPlans(const Problem& orig, const Problem& red, const cuttHipDevicePro
 
 // Whether a Tiled plan's axes are whole tiles of 128x128 4-byte elements.
 bool wideTilesFit(const Split& sp, const Problem& pb);
+
+// Decides tiled.paced of a Tiled plan from its size and cache policy.
+void choosePacing(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt);
 
 // Same index sets as `src`, launch geometry recomputed under different options (used by the
 // measuring planner to try ordering and granularity variants of its best candidate).

@@ -72,6 +72,9 @@ typedef struct cuttPlanInfo {
                            first, second cut rank; b = Mbar position): those digits; else empty */
   int rowGather;        /* TiledCopy: 1 if the rows are gathered in output order (dense tensors), 0 if 64x64 tiles are
                            copied */
+  int xcdGroup;         /* Tiled, Packed/PackedSplit: 0 = an XCD takes one chunk of the workgroups, g = groups of 2^(g-1) in turn */
+  int tiledWide;        /* Tiled: 1 = tiles of 128x128 4-byte elements */
+  int tiledPaced;       /* Tiled: 1 = the kernel whose loads leave row group by row group, for large tensors with ordinary stores */
 } cuttPlanInfo;
 
 /* Describe an existing plan. */

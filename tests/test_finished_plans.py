@@ -1,0 +1,25 @@
+"""What cuttPlan decides about a plan after the cost model has chosen it, without a GPU."""
+import pytest
+
+import fake_planner
+
+TILED = 4
+
+
+@pytest.fixture(scope="module")
+def planner(tmp_path_factory):
+    return fake_planner.build(tmp_path_factory.mktemp("planner"))
+
+
+def test_pacing_is_part_of_the_plan(planner):
+    # 8-byte batches off the line grid with output rows of 888 bytes: ordinary stores, below and above 0.75 cache sizes per buffer
+    large, small = ((777, 111, 1000), (1, 0, 2), 8), ((777, 111, 200), (1, 0, 2), 8)
+    assert [planner.plan(*large).tiledPaced, planner.plan(*small).tiledPaced] == [1, 0]
+    assert planner.plan(*large).cachePolicy == 0
+    # the option reaches plans of both sizes, also where the same tensor has been planned without it
+    assert [planner.plan(*t, CUTT_TILED_PACED=0).tiledPaced for t in (large, small)] == [0, 0]
+    assert [planner.plan(*t, CUTT_TILED_PACED=1).tiledPaced for t in (large, small)] == [1, 1]
+    # past the caches, wide tiles, line-aligned stores: other kernels
+    for dim, es in (((6000, 6080), 4), ((8192, 8192), 4), ((8200, 5003), 8)):
+        assert planner.plan(dim, (1, 0), es).tiledPaced == 0
+    assert planner.plan(*large, CUTT_CACHE_POLICY=3).tiledPaced == 0 and planner.plan(*large, CUTT_CACHE_POLICY=1).tiledPaced == 1

@@ -1,6 +1,6 @@
 """The Tiled kernel at the edges of its 64x64 tiles and strips, bit-exact against the oracle: every number of rows and columns in
-the last tile that takes another piece of code, strips with a narrower last one, one to nine Mbar ranks, axes over fused ranks, and every
-tile order and cache policy."""
+the last tile that takes another piece of code, strips with a narrower last one, one to nine Mbar ranks, axes over fused ranks, and tile
+orders 0 to 6 with every cache policy, through the kernel of the walk and through the general one."""
 import math
 
 import pytest
@@ -39,3 +39,19 @@ def test_strips_and_mbar_ranks(tiled, es, order):
         for c in range(min(4, check_case(dim, perm, es).numCandidates)):
             info = check_case(dim, perm, es, how="candidate", candidate=c)
             assert info.method_name == "Tiled" and math.prod(dim) == info.volMmk * info.volMbar
+
+
+@pytest.mark.parametrize("es", [4, 8])
+@pytest.mark.parametrize("order", range(7))
+def test_edges_in_every_order_policy_and_kernel(tiled, es, order):
+    from gpu_util import check_case
+    tiled.setenv("CUTT_TILED_ORDER", str(order))
+    for i, m in enumerate(EDGES):
+        for j, k in enumerate(EDGES):
+            policy, paced = (i + 2 * j) % 4, (i // 4 + j) % 2
+            tiled.setenv("CUTT_CACHE_POLICY", str(policy))
+            tiled.setenv("CUTT_TILED_PACED", str(paced))
+            tiled.setenv("CUTT_TILED_GROUPED", str(int(i == j)))
+            dim, perm = [((m, k), (1, 0)), ((m, 3, k), (2, 1, 0)), ((m, 2, k, 3), (3, 2, 0, 1))][(i + j) % 3]
+            info = check_case(dim, perm, es)
+            assert info.method_name == "Tiled" and (info.tiledOrder, info.cachePolicy, info.tiledPaced) == (order, policy, paced)
