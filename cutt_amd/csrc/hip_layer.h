@@ -151,8 +151,8 @@ typedef struct cuttHipRowRadix {
  * or a division by a variable (cuttHipFinishTileWalk).  It covers what the planner picks for nearly every tensor:
  * strips of superM tiles along Mm that run through all of Mk (tile orders 3 and 5), the tiles along Mm fastest (order 1:
  * one strip) or along Mk fastest (order 2: strips one tile wide), with at most CUTT_WALK_RANKS Mbar ranks.  The tiles come
- * in the sequence of those orders; the last strip is as narrow as it is, so that no workgroup is left without a tile (but
- * for the last XCD's, at most seven).  Divisions of n < 2^31 by d: mulhi32(2 n, mul) >> shift with shift = ceil(log2 d) and mul =
+ * in the sequence of those orders; the last strip is as narrow as it is, so that no workgroup is left without a tile but the
+ * last ones, at most seven where each XCD has a chunk and one less than 8 groups where it takes groups.  Divisions of n < 2^31 by d: mulhi32(2 n, mul) >> shift with shift = ceil(log2 d) and mul =
  * ceil(2^(31 + shift) / d) (the error of mul is below 1, so that of the product is below n / 2^(31 + shift) < 1 / d); mul = 0 gives 0.
  */
 #define CUTT_WALK_RANKS 8
@@ -243,6 +243,8 @@ typedef struct cuttHipTiledArgs {
 
 /* Derive a->walk from the other arguments (kind 0 if their numbering is not of its form). */
 void cuttHipFinishTileWalk(cuttHipTiledArgs* a);
+/* Whether a launch with these arguments decodes the walk: it then has walk.blocks workgroups, cuttHipTiledGrid otherwise. */
+int cuttHipTiledTakesWalk(const cuttHipTiledArgs* a);
 
 /*
  * Rows gathered into a dense output (TiledCopy method, the usual kernel): rank 0 keeps its place, so the
@@ -424,7 +426,8 @@ int cuttHipValidatePacked(const cuttHipPackedArgs* args);
 int cuttHipLinesMaxWidth(int elemSize);
 int cuttHipLinesThreads(int elemSize, int tileWidth);
 size_t cuttHipLinesLdsBytes(int elemSize, int tileWidth);
-/* Workgroups of a tiled launch with these arguments (padding workgroups included), 0 if they have no valid grid. */
+/* Workgroups of a tiled launch with these arguments by the kernels that decode the order itself (padding workgroups included),
+ * 0 if they have no valid grid. */
 long long cuttHipTiledGrid(const cuttHipTiledArgs* args);
 long long cuttHipTiledCopyGrid(const cuttHipTiledCopyArgs* args);
 long long cuttHipPackedGrid(const cuttHipPackedArgs* args);

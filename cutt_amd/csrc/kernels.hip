@@ -862,8 +862,8 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
     return (int)hipErrorInvalidConfiguration;
   hipStream_t s = (hipStream_t)stream;
   if (a->lineWidth) return launchLines(*a, in, out, (uint32_t)blocks, s);
-  if (a->wide) return launchWide(*a, in, out, s);
-  if (a->walk.kind && !a->grouped && !a->paced) return launchWalk(*a, in, out, s);
+  if (cuttHipTiledTakesWalk(a)) return a->wide ? launchWide(*a, in, out, s) : launchWalk(*a, in, out, s);
+  if (a->wide) return (int)hipErrorInvalidValue;  // (no other kernel knows such tiles)
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
 #define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \

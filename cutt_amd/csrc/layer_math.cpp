@@ -184,6 +184,10 @@ extern "C" void cuttHipFinishTileWalk(cuttHipTiledArgs* a) {
   walkRows(a->rowsM, a->strideOutM, w.rowsM);
 }
 
+extern "C" int cuttHipTiledTakesWalk(const cuttHipTiledArgs* a) {
+  return a->walk.kind != 0 && a->lineWidth == 0 && (a->wide || (!a->grouped && !a->paced)) ? 1 : 0;
+}
+
 extern "C" long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* a) {
   const unsigned long long slabs = (unsigned long long)a->split[0].numSplit * (unsigned long long)a->split[1].numSplit;
   unsigned long long n = (unsigned long long)a->volMbar * slabs;

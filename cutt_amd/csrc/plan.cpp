@@ -1737,6 +1737,7 @@ int Plan::activate() {
   if (method == kTiled) {
     if (launchable) return 0;
     cuttHipFinishTileWalk(&tiled);
+    if (cuttHipTiledTakesWalk(&tiled)) numBlocks = (int64_t)tiled.walk.blocks;
     return (launchable = cuttHipValidateTiled(&tiled) == 0) ? 0 : -1;
   }
   if (method == kTiledCopy) {

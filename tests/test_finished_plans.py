@@ -23,3 +23,14 @@ def test_pacing_is_part_of_the_plan(planner):
     for dim, es in (((6000, 6080), 4), ((8192, 8192), 4), ((8200, 5003), 8)):
         assert planner.plan(dim, (1, 0), es).tiledPaced == 0
     assert planner.plan(*large, CUTT_CACHE_POLICY=3).tiledPaced == 0 and planner.plan(*large, CUTT_CACHE_POLICY=1).tiledPaced == 1
+
+
+def test_blocks_are_those_of_the_launch(planner):
+    # strips of tiles (8224 x 8192: 129 x 128 in strips of 8, the last one a tile wide): the kernels that decode a walk launch no padding
+    # workgroups but the last XCD's, the general one all of the padded strips
+    tiles = 129 * 128
+    assert planner.plan((8224, 8192), (1, 0), 4, CUTT_XCD_GROUP=0).numBlocks == (tiles + 7) // 8 * 8
+    assert planner.plan((8224, 8192), (1, 0), 4, CUTT_XCD_GROUP=5).numBlocks == (tiles + 127) // 128 * 128
+    assert planner.plan((8224, 8192), (1, 0), 4, CUTT_XCD_GROUP=0, CUTT_TILED_PACED=1).numBlocks == 17 * 8 * 128
+    # wide tiles: 65 x 64 in strips of 16
+    assert planner.plan((8320, 8192), (1, 0), 4, CUTT_XCD_GROUP=0, CUTT_SUPER_M=16, CUTT_TILED_WIDE=1).numBlocks == (65 * 64 + 7) // 8 * 8

@@ -56,13 +56,20 @@ def test_packed(method, monkeypatch, es, group):
 def test_planner_takes_groups_where_lines_are_written_whole(method, monkeypatch, dim, perm, es, grouped):
     import torch
     import cutt_amd as cutt
+    import sweep_runner
     st = torch.cuda.current_stream().cuda_stream
-    blocks = []
+    src = sweep_runner.index_pattern(dim[0] * dim[1], es)
+    want = sweep_runner.expected_on_device(src, list(dim), list(perm))
+    groups = []
     for group in (None, "0", "5"):
         if group:
             monkeypatch.setenv("CUTT_XCD_GROUP", group)
         rc, h = cutt.cuttPlan(len(dim), list(dim), list(perm), es, st)
         assert rc == cutt.CUTT_SUCCESS
-        blocks.append(cutt.get_plan_info(h).numBlocks)
+        groups.append(cutt.get_plan_info(h).xcdGroup)
+        dst = torch.full_like(src, -1)
+        assert cutt.cuttExecute(h, src.data_ptr(), dst.data_ptr()) == cutt.CUTT_SUCCESS
+        torch.cuda.synchronize()
+        assert torch.equal(dst, want), (dim, es, group)
         cutt.cuttDestroy(h)
-    assert blocks[1] != blocks[2] and (blocks[0] == blocks[2]) == grouped and blocks[2] % 128 == 0
+    assert groups == [5 if grouped else 0, 0, 5]
