@@ -396,8 +396,7 @@ void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
     return;
   }
   PlannerOptions opt = plannerOptions(0);
-  if (p.method == kTiled && (opt.tiledOrder >= 0 || !opt.superAuto || !opt.tileDigits.empty())) return;  // options that pin the sequence
-  // the orders that belong to groups (plan.cpp: tiledBlocks)
+  // the orders that belong to groups (plan.cpp: tiledBlocks), which options that pin the order override there
   Plan q;
   opt.groupOrders = true;
   if (p.method == kTiled && !a.wide && a.lineWidth == 0 && a.order != 7 && rebuildPlan(p, props, opt, q) && q.tiled.order != 7) {

@@ -828,7 +828,9 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
   // two sets (extents with and without powers of two, both widths, with and without Mbar ranks) ran +3.2 % in the
   // mean against the strips, -1.8 % at worst; the tiles along Mk fastest +2 % (-6 ... +14 %), order 5 -0.5 %.
   // (All of those with a single rank along Mk; of two plans with a fused Mk axis one lost 10 %: left to the strips.)
-  if (opt.superAuto && opt.tiledOrder < 0 && neighbourRunsInMm && oneRankMk && beyondCache && rowBytesIn > 0 &&
+  // Not where the XCDs share the sequence in groups of 16 tiles: there the strips are 0.8 % faster in the mean over 26 such plans, -4 ...
+  // +8 % ((6,320,8,4704)/(3,1,2,0), 8 bytes, 219 -> 203 us, (12,128,7,8192)/(3,1,2,0) 277 -> 263; (24,44,3,30624)/(3,1,2,0), 4 bytes, 144 -> 150).
+  if (opt.superAuto && opt.tiledOrder < 0 && neighbourRunsInMm && oneRankMk && beyondCache && rowBytesIn > 0 && !opt.groupOrders &&
       rowBytesIn % 128 == 0 && rowBytesOut % 128 == 0)
     o.order = 1;
   // One measured exception (forced-Tiled sweep over random shapes, all orders timed): with two

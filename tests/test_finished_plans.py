@@ -34,3 +34,21 @@ def test_blocks_are_those_of_the_launch(planner):
     assert planner.plan((8224, 8192), (1, 0), 4, CUTT_XCD_GROUP=0, CUTT_TILED_PACED=1).numBlocks == 17 * 8 * 128
     # wide tiles: 65 x 64 in strips of 16
     assert planner.plan((8320, 8192), (1, 0), 4, CUTT_XCD_GROUP=0, CUTT_SUPER_M=16, CUTT_TILED_WIDE=1).numBlocks == (65 * 64 + 7) // 8 * 8
+
+
+def test_groups_do_not_depend_on_who_chose_the_order(planner):
+    # a pinned order is walked in the same groups as the planner's own
+    for dim, perm, es in (((6000, 6080), (1, 0), 4), ((96, 75, 96, 75), (2, 1, 3, 0), 8), ((8200, 5003), (1, 0), 8)):
+        own = planner.plan(dim, perm, es)
+        assert own.xcdGroup == 5
+        for env in (dict(CUTT_TILED_ORDER=own.tiledOrder), dict(CUTT_SUPER_M=8), dict(CUTT_SUPER_M=8, CUTT_SUPER_K=4096)):
+            pinned = planner.plan(dim, perm, es, TILED, CUTT_TILED_ALIGNED=own.tiledAligned, **env)
+            assert pinned.xcdGroup == 5, (dim, perm, es, env)
+
+
+def test_whole_mm_axis_at_a_stretch_in_chunks_only(planner):
+    # a fused Mm axis on the line grid: strips where the XCDs take groups
+    dim, perm = (6, 320, 8, 4704), (3, 1, 2, 0)
+    groups, chunks = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_XCD_GROUP=0)
+    assert (groups.xcdGroup, groups.tiledOrder, groups.superM) == (5, 3, 8)
+    assert (chunks.xcdGroup, chunks.tiledOrder) == (0, 1)
