@@ -779,7 +779,8 @@ struct TiledShape {
   int64_t volMmLastTile = kTile;            // elements along Mm in the last tile
   int64_t rowBytesIn = 0, rowBytesOut = 0;  // bytes of one row of the Mm / Mk axis (0: not known, TiledCopy)
   int elemSize = 4;
-  bool mbarBetween = false;        // an Mbar rank follows Mm in the input and Mk in the output
+  bool mbarBetween = false;        // an Mbar rank follows Mm in the input and Mk in the output ...
+  bool batchOfFew = false;         // ... of at most 14 positions, and another one is slower than Mm and Mk on both sides
   bool beyondCache = false;        // more than 0.75 memory-side cache sizes per buffer
   bool neighbourRunsInMm = false;  // a fused Mm axis of which one rank follows Mk in the output
   bool oneRankMk = false;          // a single rank along Mk
@@ -890,8 +891,12 @@ int64_t tiledBlocks(const PlannerOptions& opt, const TiledShape& shape, TileOrde
     // over 27 (-7 ... +9 %; +4 % over ten batched transposes whose extents are multiples of 256), for
     // batches of separate matrices - the Mbar rank slowest on both sides, which used to get 8 x 8
     // patches - -1.3 % over 20 (-7 ... +3 %): those walk strips again.
+    // Where the XCDs share the sequence in groups of 16 tiles, batches of such tensors with 3-14 rows between walk strips as well: 20 seeded
+    // plans of 1.3 GB per buffer, all of them 0.2 ... 10 % faster, 5.0 % in the mean ((1792,4,1664,13)/(2,1,0,3) 464 us in patches, 431 in
+    // strips, 440 in patches with a chunk per XCD).  With 16-60 rows between strips lose 0.9 % in the mean over 13, without a batch
+    // 1.7 % over 20 with 42-217 rows and -16 ... +18 % over 20 with 3-14.
     const bool onGrid = rowBytesIn % 128 == 0 && rowBytesOut % 128 == 0;
-    gridRule = onGrid && elemSize == 8 && tilesK >= 16 && tilesM >= 3 && mbarBetween;
+    gridRule = onGrid && elemSize == 8 && tilesK >= 16 && tilesM >= 3 && mbarBetween && !(opt.groupOrders && shape.batchOfFew);
     if (gridRule) {
       superK = 8;
       // (Not two wide for input rows a multiple of 32 KB apart: ten such tensors ran 3.4 % faster 8 wide,
@@ -1207,9 +1212,16 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
     TileOrdering o;
     // an Mbar rank that follows Mm in the input and Mk in the output: consecutive Mbar positions are
     // neighbouring rows on both sides
-    bool between = false;
-    for (int r = 0; r < pb.rank; r++)
-      if (!sp.inMmk[r] && pb.strideIn[r] == sp.volMm && pb.strideOut[r] == sp.volMk) between = true;
+    bool between = false, slowerOnBoth = false;
+    int64_t betweenExtent = 0;
+    for (int r = 0; r < pb.rank; r++) {
+      if (sp.inMmk[r]) continue;
+      if (pb.strideIn[r] == sp.volMm && pb.strideOut[r] == sp.volMk) {
+        between = true;
+        betweenExtent = pb.dim[r];
+      }
+      slowerOnBoth = slowerOnBoth || (pb.strideIn[r] >= sp.volMm * sp.volMk && pb.strideOut[r] >= sp.volMm * sp.volMk);
+    }
     const double cacheBytes = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
     const bool beyondCache = (double)pb.volume * pb.elemSize > 0.75 * cacheBytes;
     if (!fillMbar(pb, sp.inMmk, opt.mbarOrder, a.mbar)) return false;
@@ -1239,6 +1251,7 @@ bool setupTiled(Plan& plan, const cuttHipDeviceProps& props, const PlannerOption
       shape.rowBytesOut = sp.volMk * pb.elemSize;
       shape.elemSize = pb.elemSize;
       shape.mbarBetween = between;
+      shape.batchOfFew = between && betweenExtent <= 14 && slowerOnBoth;
       shape.beyondCache = beyondCache;
       shape.neighbourRunsInMm = sp.numMm > 1 && sp.numMk < pb.rank && pb.perm[sp.numMk] > 0 && pb.perm[sp.numMk] < sp.numMm;
       shape.oneRankMk = sp.numMk == 1;

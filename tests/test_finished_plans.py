@@ -52,3 +52,12 @@ def test_whole_mm_axis_at_a_stretch_in_chunks_only(planner):
     groups, chunks = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_XCD_GROUP=0)
     assert (groups.xcdGroup, groups.tiledOrder, groups.superM) == (5, 3, 8)
     assert (chunks.xcdGroup, chunks.tiledOrder) == (0, 1)
+
+
+def test_batches_with_few_rows_between_walk_strips_in_groups(planner):
+    # (few rows between, many, no batch): patches 8 tiles along Mk everywhere but for the first in groups
+    for dim, perm, strips in (((640, 11, 1344, 16), (2, 1, 0, 3), True), ((1088, 40, 1280, 3), (2, 1, 0, 3), False), ((1856, 67, 1280), (2, 1, 0), False)):
+        tiles = (dim[2] + 63) // 64
+        groups, chunks = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_XCD_GROUP=0)
+        assert (groups.xcdGroup, chunks.xcdGroup) == (5, 0)
+        assert chunks.superK < tiles and (groups.superK == tiles) == strips, (dim, groups.superK, chunks.superK)
