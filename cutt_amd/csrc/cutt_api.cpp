@@ -368,33 +368,61 @@ void setXcdGroup(Plan& p, int g) {
   p.numBlocks = blocks;
 }
 
+// Whether the Mbar ranks of a Tiled plan are slowest on both sides: separate matrices, one after the other.
+bool separateMatrices(const Plan& p) {
+  bool batch = p.split.volMbar > 1;
+  const int64_t matrix = p.split.volMm * p.split.volMk;
+  for (int r = 0; r < p.pb.rank; r++)
+    if (!p.split.inMmk[r]) batch = batch && p.pb.strideIn[r] >= matrix && p.pb.strideOut[r] >= matrix;
+  return batch;
+}
+
+// Plans that do not gain in groups of 16 workgroups, each class on tensors the condition was not found on (times of one
+// chunk per XCD over times in groups: mean, range, number of tensors of 0.24-1.5 GB per buffer).
+bool groupsLose(const Plan& p) {
+  if (p.method != kTiled) return false;
+  const cuttHipTiledArgs& a = p.tiled;
+  const int64_t rowBytesIn = p.split.volMm * a.elemSize, rowBytesOut = p.split.volMk * a.elemSize;
+  const bool strips = a.order != 1 && a.order != 2 && (int64_t)a.superM < a.tilesM;
+  if (a.lineWidth == 0) {
+    // 64x64 tiles that write rows of 8 KB and more a multiple of 32 KB apart: 1.03 in the mean, but 0.71 at worst and 10 of 59 below 0.98: 8224 x 8192, 4
+    // bytes, 97 -> 137 us, (5040,2,8192)/(2,1,0), 8 bytes, 227 -> 244; 6176 x 16384, 4 bytes, 145 -> 138, which this gives up.
+    if (!a.wide && a.rowsM.n == 0 && (int64_t)a.strideOutM * a.elemSize % 32768 == 0 && rowBytesOut >= 8192) return true;
+    // 8-byte input rows 64 KB long beside more than 160 tiles along Mk, in strips of 8: 0.98, 0.95-1.01 (8); rows of 128 KB and more 1.04,
+    // 1.03-1.06 (7).
+    if (a.elemSize == 8 && a.tilesK > 160 && rowBytesIn == 65536) return true;
+    // Separate matrices with input rows off the line grid, cut into strips that are each visited for all matrices: 0.985, 0.92-1.04 (33).  In
+    // one strip, which reads whole rows, 1.04, 1.01-1.07 (8).
+    return a.order == 5 && strips && rowBytesIn % 128 != 0 && separateMatrices(p);
+  }
+  // Line-aligned stores read rows at a window's fringe again with the next window along Mk (31 of 95 rows of 4-byte elements, 15 of
+  // 79 of 8-byte ones), which in strips lies a strip's width away.  4-byte strips: 1.02, but 0.81 at worst and 7 of 40 below 0.98:
+  // (502,25,10574)/(2,1,0) 222 -> 271 us, (94,519,944)/(2,1,0) 76 -> 79; 201 x 700299 222 -> 212, which this gives up.
+  if (a.elemSize == 4) return a.order != 2 && a.superM > 1;
+  // 8-byte elements: 1.04, 0.92-1.20 (147), but with both axes over fused ranks and no Mbar rank 1.01, 0.83-1.12 and 6 of 43 below 0.98:
+  // (60,36,2764,3)/(3,2,1,0) 60 -> 67 us, (22,18,23118,5)/(3,2,1,0) 146 -> 166; (49,27,11187,3)/(3,2,1,0) 157 -> 141 (with Mbar ranks 1.05,
+  // 1.01-1.09 (15)).
+  return p.split.numMm > 1 && p.split.numMk > 1 && p.split.volMbar == 1;
+}
+
 // What the XCDs have in flight at one time lies together in memory when they share the sequence in groups of 16 workgroups,
 // at eight places a chunk apart otherwise, which costs the memory 2-10 %: 23425 x 8538, 8 bytes, 607 -> 565 us; (96,75,96,75)/
 // (2,1,3,0) 159 -> 157; 8192 x 8192, 4 bytes, 108 -> 102; (40,14881,4,6,14)/(3,2,0,1,4) 304 -> 293; (64,64,64,64,4)/(3,2,1,0,4)
-// 134 -> 99; 35 random Tiled plans +4 % in the mean, -3.5 % at worst.  (Groups of 4 and 32 are as good, 64 and more
-// lose part of it, single workgroups lose what neighbours share in an L2.)  That holds where every line is written whole
-// and past the caches.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 such plans
-// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.  Nor where 64x64 tiles write long rows a
-// multiple of 32 KB apart, which fall into few memory channels unless the XCDs work far from each other: 8224 x 8192, 4 bytes,
-// 98 -> 137 us, 8192 x 8192, 8 bytes, 196 -> 205 (16384 x 4096 175 -> 174 the best of six); rows of 48 KB gain, 6144 x 6144 115 -> 105.
+// 134 -> 99; 295 random Tiled plans of 0.16-1.3 GB per buffer outside the classes above 1.04 times as fast in the mean, 0.88 ... 1.22, 17 of them
+// below 0.98 ((4,30,783,592)/(2,3,0,1), 8 bytes, 168 -> 192 us); nothing found in their strides tells those from the others.  (Groups of 8 and 32 are as good; single workgroups lose what neighbours share in an L2.)  That holds where every line is
+// written whole and past the caches.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 such plans
+// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.
 void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
   if (const char* e = std::getenv("CUTT_XCD_GROUP")) {
     setXcdGroup(p, std::atoi(e));
     return;
   }
-  cuttHipTiledArgs& a = p.tiled;
-  const bool sameChannels = p.method == kTiled && !a.wide && a.lineWidth == 0 && a.rowsM.n == 0 && (int64_t)a.strideOutM * a.elemSize % 32768 == 0 &&
-                            (int64_t)a.volMk * a.elemSize >= 8192;
-  // 8-byte input rows a multiple of 64 KB apart beside long output rows: 8192 x 12352 294 -> 304 us.
-  const bool longRows = p.method == kTiled && a.lineWidth == 0 && a.elemSize == 8 && a.tilesK > 160 && (int64_t)a.volMm * a.elemSize % 65536 == 0;
-  // (a packed workgroup moves several blocks: 1024 of them are 16 MB and more)
-  // Line-aligned stores read a third of a 4-byte tile's rows again with the next window along Mk (an eighth of an 8-byte one's): in strips that
-  // window is a strip's width away, outside the group.  (379,6,21988)/(1,2,0) 83 -> 93 us, (94,519,944)/(2,1,0) 76 -> 79.
-  const bool fringeApart = p.method == kTiled && a.lineWidth > 0 && a.elemSize == 4 && a.order != 2 && a.superM > 1;
-  if (!(cachePolicyOf(p) & 2) || sameChannels || longRows || fringeApart || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
+  // (a packed workgroup moves several blocks: 512 of them are 8 MB and more)
+  if (!(cachePolicyOf(p) & 2) || groupsLose(p) || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
     setXcdGroup(p, 0);
     return;
   }
+  cuttHipTiledArgs& a = p.tiled;
   PlannerOptions opt = plannerOptions(0);
   // the orders that belong to groups (plan.cpp: tiledBlocks), which options that pin the order override there
   Plan q;
@@ -440,12 +468,7 @@ bool lineWindowsPay(const Plan& p, const cuttHipDeviceProps& props) {
   const int64_t runBytes = p.split.volMk * pb.elemSize;
   const double bytes = (double)pb.volume * pb.elemSize;
   const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
-  // batches of separate matrices: the Mbar ranks are slowest on both sides
-  bool batch = p.split.volMbar > 1;
-  for (int r = 0; r < pb.rank; r++) {
-    if (pb.inv[r] < p.split.numMk) continue;
-    if (!p.split.inMmk[r]) batch = batch && pb.strideIn[r] >= p.split.volMm * p.split.volMk && pb.strideOut[r] >= p.split.volMm * p.split.volMk;
-  }
+  const bool batch = separateMatrices(p);
   if (2.0 * bytes <= cache || p.split.volMm * pb.elemSize < 256 || runBytes < (batch ? 4096 : 2048)) return false;
   if (!rowsOffLineGrid(p)) return false;
   const PlannerOptions opt = plannerOptions(0);  // options that pin the plain kernel's variants leave the plan as it is

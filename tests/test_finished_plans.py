@@ -61,3 +61,20 @@ def test_batches_with_few_rows_between_walk_strips_in_groups(planner):
         groups, chunks = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_XCD_GROUP=0)
         assert (groups.xcdGroup, chunks.xcdGroup) == (5, 0)
         assert chunks.superK < tiles and (groups.superK == tiles) == strips, (dim, groups.superK, chunks.superK)
+
+
+@pytest.mark.parametrize("dim,perm,es,group", [
+    # output rows a multiple of 32 KB apart under 64x64 tiles; others; wide tiles
+    ((8224, 8192), (1, 0), 4, 0), ((5040, 2, 8192), (2, 1, 0), 8, 0), ((8224, 8160), (1, 0), 4, 5), ((8192, 8192), (1, 0), 4, 5),
+    # 8-byte rows of 64 KB beside 160 tiles along Mk and more, of 128 KB
+    ((8192, 12352), (1, 0), 8, 0), ((16384, 10832), (1, 0), 8, 5), ((8192, 9200), (1, 0), 8, 5),
+    # separate matrices off the line grid in strips, in one strip, on the grid; without a batch
+    ((1768, 64, 773), (1, 0, 2), 8, 0), ((979, 320, 558), (1, 0, 2), 4, 0), ((717, 448, 272), (1, 0, 2), 8, 5), ((512, 256, 667), (1, 0, 2), 8, 5),
+    ((1768, 40976), (1, 0), 8, 5),
+    # line-aligned stores: 4-byte strips, front to back; both axes over fused ranks without an Mbar rank, with one, one axis
+    ((379, 131928), (1, 0), 4, 0), ((28309, 1348), (1, 0), 4, 5), ((60, 36, 2764, 3), (3, 2, 1, 0), 8, 0),
+    ((14, 103, 1509, 9, 5), (3, 2, 1, 4, 0), 8, 5), ((62, 12, 42642), (2, 1, 0), 8, 5),
+])
+def test_plans_that_do_not_gain_in_groups(planner, dim, perm, es, group):
+    info = planner.plan(dim, perm, es)
+    assert info.method == TILED and info.xcdGroup == group
