@@ -368,22 +368,12 @@ void setXcdGroup(Plan& p, int g) {
   p.numBlocks = blocks;
 }
 
-// Whether the Mbar ranks of a Tiled plan are slowest on both sides: separate matrices, one after the other.
-bool separateMatrices(const Plan& p) {
-  bool batch = p.split.volMbar > 1;
-  const int64_t matrix = p.split.volMm * p.split.volMk;
-  for (int r = 0; r < p.pb.rank; r++)
-    if (!p.split.inMmk[r]) batch = batch && p.pb.strideIn[r] >= matrix && p.pb.strideOut[r] >= matrix;
-  return batch;
-}
-
 // Plans that do not gain in groups of 16 workgroups, each class on tensors the condition was not found on (times of one
 // chunk per XCD over times in groups: mean, range, number of tensors of 0.24-1.5 GB per buffer).
-bool groupsLose(const Plan& p) {
+bool groupsLose(const Plan& p, const cuttHipDeviceProps& props) {
   if (p.method != kTiled) return false;
   const cuttHipTiledArgs& a = p.tiled;
   const int64_t rowBytesIn = p.split.volMm * a.elemSize, rowBytesOut = p.split.volMk * a.elemSize;
-  const bool strips = a.order != 1 && a.order != 2 && (int64_t)a.superM < a.tilesM;
   if (a.lineWidth == 0) {
     // 64x64 tiles that write rows of 8 KB and more a multiple of 32 KB apart: 1.03 in the mean, but 0.71 at worst and 10 of 59 below 0.98: 8224 x 8192, 4
     // bytes, 97 -> 137 us, (5040,2,8192)/(2,1,0), 8 bytes, 227 -> 244; 6176 x 16384, 4 bytes, 145 -> 138, which this gives up.
@@ -391,9 +381,8 @@ bool groupsLose(const Plan& p) {
     // 8-byte input rows 64 KB long beside more than 160 tiles along Mk, in strips of 8: 0.98, 0.95-1.01 (8); rows of 128 KB and more 1.04,
     // 1.03-1.06 (7).
     if (a.elemSize == 8 && a.tilesK > 160 && rowBytesIn == 65536) return true;
-    // Separate matrices with input rows off the line grid, cut into strips that are each visited for all matrices: 0.985, 0.92-1.04 (33).  In
-    // one strip, which reads whole rows, 1.04, 1.01-1.07 (8).
-    return a.order == 5 && strips && rowBytesIn % 128 != 0 && separateMatrices(p);
+    // Separate matrices off the line grid in several strips: 0.985, 0.92-1.04 (33).  In one strip, which reads whole rows, 1.04, 1.01-1.07 (8).
+    return stripsOfMatrices(p, props);
   }
   // Line-aligned stores read rows at a window's fringe again with the next window along Mk (31 of 95 rows of 4-byte elements, 15 of
   // 79 of 8-byte ones), which in strips lies a strip's width away.  4-byte strips: 1.02, but 0.81 at worst and 7 of 40 below 0.98:
@@ -418,7 +407,7 @@ void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
     return;
   }
   // (a packed workgroup moves several blocks: 512 of them are 8 MB and more)
-  if (!(cachePolicyOf(p) & 2) || groupsLose(p) || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
+  if (!(cachePolicyOf(p) & 2) || groupsLose(p, props) || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
     setXcdGroup(p, 0);
     return;
   }

@@ -144,8 +144,11 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
   }
 }
 
+// How tiledKernel's loads leave: as in moveTile, row group by row group without waiting, row group by row group waiting for each.
+enum { kLoadsAtOnce, kLoadsPaced, kLoadsGrouped };
+
 // Any numbering of the workgroups (tile_order.h: locateTile).
-template <typename T, int NT, bool GROUPED, bool FUSED>
+template <typename T, int NT, int LOADS, bool FUSED>
 __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledArgs a,
                                                             const T* __restrict__ in,
                                                             T* __restrict__ out) {
@@ -153,8 +156,8 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  if constexpr (GROUPED || !(NT & 2)) {
-    // Rows in groups, or ordinary stores and a large tensor (cuttHipTiledArgs.paced): one piece of code whose row groups are tested one after the
+  if constexpr (LOADS != kLoadsAtOnce) {
+    // Rows in groups, or paced loads (cuttHipTiledArgs.paced): one piece of code whose row groups are tested one after the
     // other.  Without GROUPED a group's loads go out while the next one's addresses are computed, and no load is waited for before all are
     // out.  All sixteen at once (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no
     // longer find shared lines in the L2.
@@ -162,6 +165,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
     // test with copies that wait for the loads: (777,111,1000)/(1,0,2), 8 bytes, 246.7 us here, 252.5 that way, (633,147,1602)/(1,0,2) 442.5 / 453.4,
     // (9,7,23,7,46,11,5,3)/(4,7,0,6,3,1,5,2), 4 bytes, 157.1 / 160.3; 24 such tensors 0.9 % in the mean, -1.5 ... +2.4 %.  With rows in
     // groups a straight piece of code per number of row groups costs 3.5-5.5 % instead: 16411 x 9377, 4 bytes, 282.4 us here, 296.3 that way.
+    constexpr bool GROUPED = LOADS == kLoadsGrouped;
     const uint32_t wave = threadIdx.x >> 6;
     __shared__ T tile[kTile][kTile + 1];
     {
@@ -866,10 +870,14 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
   if (a->wide) return (int)hipErrorInvalidValue;  // (no other kernel knows such tiles)
   const dim3 grid((uint32_t)blocks), block(kTileThreads);
   const bool fused = a->rowsK.n > 0 || a->rowsM.n > 0;
-#define CUTT_LAUNCH_TILED_F(T, NT, G)                                                                            \
-  (fused ? launchKernel(tiledKernel<T, NT, G, true>, grid, block, 0, s, *a, (const T*)in, (T*)out)               \
-         : launchKernel(tiledKernel<T, NT, G, false>, grid, block, 0, s, *a, (const T*)in, (T*)out))
-#define CUTT_LAUNCH_TILED(T, NT) return (int)(a->grouped ? CUTT_LAUNCH_TILED_F(T, NT, true) : CUTT_LAUNCH_TILED_F(T, NT, false))
+#define CUTT_LAUNCH_TILED_F(T, NT, LOADS)                                                                        \
+  (fused ? launchKernel(tiledKernel<T, NT, LOADS, true>, grid, block, 0, s, *a, (const T*)in, (T*)out)           \
+         : launchKernel(tiledKernel<T, NT, LOADS, false>, grid, block, 0, s, *a, (const T*)in, (T*)out))
+  // (with ordinary stores nothing takes the loads at once through this kernel)
+#define CUTT_LAUNCH_TILED(T, NT)                                                                                 \
+  return (int)(a->grouped                        ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsGrouped)                     \
+               : a->paced || !(a->cachePolicy & 2) ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsPaced)                     \
+                                                   : CUTT_LAUNCH_TILED_F(T, NT | 2, kLoadsAtOnce))
 #define CUTT_LAUNCH_TILED_NT(T)                                \
   switch (a->cachePolicy) {                                    \
     case 0: CUTT_LAUNCH_TILED(T, 0);                           \

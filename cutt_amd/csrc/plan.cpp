@@ -1549,14 +1549,33 @@ void addPackedSplit(const Problem& pb, bool fromReduced, const cuttHipDeviceProp
 
 }  // namespace
 
-// 64x64 tiles with ordinary stores and more than 0.75 memory-side cache sizes per buffer (192 MB): the general kernel, whose loads go out
-// row group by row group (kernels.hip: tiledKernel), instead of the walk's.  56 random tensors with ordinary stores, time by the walk's kernel over time by
-// the general one, mean and range: 24-64 MB per buffer 0.91 (0.82-0.96), 64-160 MB 0.98 (0.94-1.07), 160-192 MB 1.00, 192-900 MB 1.006 (0.97-1.05).
+bool separateMatrices(const Plan& plan) {
+  const Split& sp = plan.split;
+  const Problem& pb = plan.pb;
+  bool batch = sp.volMbar > 1;
+  for (int r = 0; r < pb.rank; r++)
+    if (!sp.inMmk[r]) batch = batch && pb.strideIn[r] >= sp.volMm * sp.volMk && pb.strideOut[r] >= sp.volMm * sp.volMk;
+  return batch;
+}
+
+bool stripsOfMatrices(const Plan& plan, const cuttHipDeviceProps& props) {
+  const cuttHipTiledArgs& a = plan.tiled;
+  const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
+  return plan.method == kTiled && !a.wide && a.lineWidth == 0 && a.order == 5 && (int64_t)a.superM < a.tilesM && plan.split.volMm * a.elemSize % 128 != 0 &&
+         (double)plan.pb.volume * a.elemSize > cache && separateMatrices(plan);
+}
+
+// The general kernel, whose loads go out row group by row group (kernels.hip: tiledKernel), instead of the walk's:
+//  - 64x64 tiles with ordinary stores and more than 0.75 memory-side cache sizes per buffer (192 MB).  56 random tensors with such stores, time by
+//    the walk's kernel over time by this one, mean and range: 24-64 MB per buffer 0.91 (0.82-0.96), 64-160 MB 0.98 (0.94-1.07), 160-192 MB 1.00,
+//    192-900 MB 1.006 (0.97-1.05);
+//  - separate matrices off the line grid in strips, whatever their stores.  8 bytes, 31 of 0.27-1.3 GB: 1.026 (0.98-1.11), (1822,320,150)/(1,0,2)
+//    254 -> 236 us, (3750,96,166)/(1,0,2) 179 -> 161; 4 bytes, 18: 1.007 (0.95-1.08).  Up to one cache size per buffer 0.99 (7).
 void choosePacing(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt) {
   if (plan.method != kTiled) return;
   cuttHipTiledArgs& a = plan.tiled;
   const double cache = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
-  const bool pays = !(a.cachePolicy & 2) && (double)plan.pb.volume * plan.pb.elemSize > 0.75 * cache;
+  const bool pays = (!(a.cachePolicy & 2) && (double)plan.pb.volume * plan.pb.elemSize > 0.75 * cache) || stripsOfMatrices(plan, props);
   a.paced = !a.wide && a.lineWidth == 0 && (opt.tiledPaced < 0 ? pays : opt.tiledPaced > 0) ? 1 : 0;
 }
 

@@ -192,7 +192,12 @@ bool createPlans(const Problem& orig, const Problem& red, const cuttHipDevicePro
 // Whether a Tiled plan's axes are whole tiles of 128x128 4-byte elements.
 bool wideTilesFit(const Split& sp, const Problem& pb);
 
-// Decides tiled.paced of a Tiled plan from its size and cache policy.
+// Whether the Mbar ranks are slowest on both sides: separate matrices, one after the other.
+bool separateMatrices(const Plan& plan);
+// Whether a Tiled plan moves separate matrices whose input rows lie off the line grid, a strip of each after the other, beyond the memory-side cache.
+bool stripsOfMatrices(const Plan& plan, const cuttHipDeviceProps& props);
+
+// Decides tiled.paced of a Tiled plan from its size, cache policy and numbering.
 void choosePacing(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptions& opt);
 
 // Same index sets as `src`, launch geometry recomputed under different options (used by the

@@ -68,8 +68,8 @@ def test_batches_with_few_rows_between_walk_strips_in_groups(planner):
     ((8224, 8192), (1, 0), 4, 0), ((5040, 2, 8192), (2, 1, 0), 8, 0), ((8224, 8160), (1, 0), 4, 5), ((8192, 8192), (1, 0), 4, 5),
     # 8-byte rows of 64 KB beside 160 tiles along Mk and more, of 128 KB
     ((8192, 12352), (1, 0), 8, 0), ((16384, 10832), (1, 0), 8, 5), ((8192, 9200), (1, 0), 8, 5),
-    # separate matrices off the line grid in strips, in one strip, on the grid; without a batch
-    ((1768, 64, 773), (1, 0, 2), 8, 0), ((979, 320, 558), (1, 0, 2), 4, 0), ((717, 448, 272), (1, 0, 2), 8, 5), ((512, 256, 667), (1, 0, 2), 8, 5),
+    # separate matrices off the line grid in strips, inside one cache size, in one strip, on the grid; without a batch
+    ((2463, 128, 72), (1, 0, 2), 8, 5), ((1768, 64, 773), (1, 0, 2), 8, 0), ((979, 320, 558), (1, 0, 2), 4, 0), ((717, 448, 272), (1, 0, 2), 8, 5), ((512, 256, 667), (1, 0, 2), 8, 5),
     ((1768, 40976), (1, 0), 8, 5),
     # line-aligned stores: 4-byte strips, front to back; both axes over fused ranks without an Mbar rank, with one, one axis
     ((379, 131928), (1, 0), 4, 0), ((28309, 1348), (1, 0), 4, 5), ((60, 36, 2764, 3), (3, 2, 1, 0), 8, 0),
@@ -78,3 +78,11 @@ def test_batches_with_few_rows_between_walk_strips_in_groups(planner):
 def test_plans_that_do_not_gain_in_groups(planner, dim, perm, es, group):
     info = planner.plan(dim, perm, es)
     assert info.method == TILED and info.xcdGroup == group
+
+
+def test_matrices_in_strips_off_the_line_grid_are_paced(planner):
+    # beyond one cache size per buffer, whatever their stores; not in one strip, not on the grid, not inside the cache
+    for dim, es, paced in (((1822, 320, 150), 8, 1), ((981, 448, 398), 4, 1), ((717, 448, 272), 8, 0), ((512, 256, 667), 8, 0), ((2463, 128, 72), 8, 0)):
+        info = planner.plan(dim, (1, 0, 2), es)
+        assert (info.method, info.tiledPaced, info.cachePolicy & 2) == (TILED, paced, 2), dim
+    assert planner.plan((1822, 320, 150), (1, 0, 2), 8, CUTT_TILED_PACED=0).tiledPaced == 0
