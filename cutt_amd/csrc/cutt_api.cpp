@@ -182,6 +182,11 @@ int cachePolicyOf(const Plan& p) {
   return p.packed.cachePolicy;
 }
 
+int xcdGroupOf(const Plan& p) {
+  if (p.method == kTiled) return p.tiled.xcdGroup;
+  return p.method == kPacked || p.method == kPackedSplit ? p.packed.xcdGroup : 0;
+}
+
 void fillInfo(const Plan& p, cuttPlanInfo& o) {
   std::memset(&o, 0, sizeof(o));
   o.method = p.method;
@@ -222,7 +227,7 @@ void fillInfo(const Plan& p, cuttPlanInfo& o) {
   o.tiledGrouped = p.method == kTiled ? p.tiled.grouped : 0;
   o.tiledAligned = p.method == kTiled && p.tiled.lineWidth > 0 ? 1 : 0;
   o.rowGather = p.method == kTiledCopy ? p.tcopy.rowGather : 0;
-  o.xcdGroup = p.method == kTiled ? p.tiled.xcdGroup : (p.method == kPacked || p.method == kPackedSplit ? p.packed.xcdGroup : 0);
+  o.xcdGroup = xcdGroupOf(p);
   o.tiledWide = p.method == kTiled ? p.tiled.wide : 0;
   o.tiledPaced = p.method == kTiled ? p.tiled.paced : 0;
   o.itemOrder = (p.method == kPacked || p.method == kPackedSplit) ? p.packed.itemOrder : 0;
@@ -965,7 +970,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       // left to the planner again, which re-derives the numbering for the variant's geometry)
       if (plans[best].itemDigits.n > 0) cur.itemOrder = -1;
     }
-    cur.xcdGroup = tiled ? plans[best].tiled.xcdGroup : plans[best].packed.xcdGroup;
+    cur.xcdGroup = xcdGroupOf(plans[best]);
     if (plans[best].method == kTiled) {
       cur.tiledGrouped = plans[best].tiled.grouped;
       cur.tiledAligned = plans[best].tiled.lineWidth > 0 ? 1 : 0;
@@ -1028,7 +1033,8 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
         v.tileDigits.clear();
         if (tryVariant(v, false)) cur = v;
       }
-      // 64x64 instead of wide tiles
+      // 64x64 instead of wide tiles (which a kept variant may have left: orders without a walk have none)
+      cur.tiledWide = plans[best].method == kTiled && plans[best].tiled.wide ? 1 : std::min(0, cur.tiledWide);
       if (!failed && cur.tiledWide > 0) {
         PlannerOptions v = cur;
         v.tiledWide = 0;
@@ -1083,7 +1089,10 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
       if (g == start.xcdGroup) continue;
       PlannerOptions v = cur;
       v.xcdGroup = g;
-      if (tryVariant(v, false)) cur = v;
+      Plan probe;  // (plans whose workgroups are not dealt out that way stay as they are)
+      if (!rebuildPlan(plans[best], props, v, probe)) continue;
+      setXcdGroup(probe, g);
+      if (xcdGroupOf(probe) == g && xcdGroupOf(plans[best]) != g && tryVariant(v, false)) cur = v;
     }
     // ... and the other cache policies of the global accesses
     for (int pol : {0, 1, 2, 3}) {

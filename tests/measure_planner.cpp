@@ -9,6 +9,10 @@
 //   accesses  - no timing: the plan cuttPlan makes for two tensors of 4-byte elements off the line grid with short output
 //               rows, once as it is and once with the cache policy pinned to non-temporal loads
 //   predicted - no timing: prints what cuttPlan expects of its plan for one tensor, with and without row gathering
+//   groups    - Tiled plans numbered by address bits, whose XCDs each have a part of their own, 50 us, all others 100 us: prints how
+//               often the winner was launched
+//   narrow    - wide tiles 100 us, 64x64 tiles in tile order 6 40 us in patches of 2 x 2 and 41 us in others, 60 us in any other order:
+//               prints how often one plan in order 6 other than the winner was launched
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
@@ -28,6 +32,7 @@
 
 #include <cstdio>
 #include <functional>
+#include <map>
 #include <set>
 #include <string>
 
@@ -119,6 +124,40 @@ static int drift() {
   return measure({1201, 30011}, {1, 0}, 8);
 }
 
+static int groups() {
+  setenv("CUTT_MEASURE_NO_PLAYOFF", "1", 1);
+  std::map<std::string, int> launches;
+  gTiledUs = [&](const cuttHipTiledArgs& a) {
+    if (a.order == 7) launches[std::string((const char*)static_cast<const void*>(&a), sizeof(a))]++;
+    return a.order == 7 ? 50.0 : 100.0;
+  };
+  gPackedUs = [](const cuttHipPackedArgs&) { return 100.0; };
+  if (measure({1024, 64, 1024, 3}, {2, 1, 0, 3}, 8)) return 1;
+  int most = 0;
+  for (const auto& l : launches) most = std::max(most, l.second);
+  std::printf("most launches of one plan %d\n", most);
+  return 0;
+}
+
+static int narrow() {
+  setenv("CUTT_MEASURE_NO_PLAYOFF", "1", 1);
+  std::map<std::string, int> launches;
+  gTiledUs = [&](const cuttHipTiledArgs& a) {
+    if (a.wide) return 100.0;
+    if (a.order != 6) return 60.0;
+    const bool first = a.superM == 2 && a.superK == 2;
+    if (!first) launches[std::string((const char*)static_cast<const void*>(&a), sizeof(a))]++;
+    return first ? 40.0 : 41.0;
+  };
+  gPackedUs = [](const cuttHipPackedArgs&) { return 100.0; };
+  cuttSetMethodOverride(CUTT_METHOD_TILED);
+  if (measure({1024, 1024, 96}, {1, 0, 2}, 4)) return 1;
+  int most = 0;
+  for (const auto& l : launches) most = std::max(most, l.second);
+  std::printf("most launches of one plan %d\n", most);
+  return 0;
+}
+
 static int predicted() {
   int dim[7] = {18, 39, 13, 100, 2, 3, 25}, perm[7] = {0, 3, 1, 6, 5, 2, 4};
   for (const char* gather : {"1", "0"}) {
@@ -156,5 +195,7 @@ int main(int argc, char** argv) {
   if (what == "accesses") return accesses();
   if (what == "predicted") return predicted();
   if (what == "drift") return drift();
+  if (what == "groups") return groups();
+  if (what == "narrow") return narrow();
   return 2;
 }

@@ -62,3 +62,11 @@ def test_rows_in_groups_go_with_loads_past_the_caches(program):
     out = subprocess.check_output([program, "accesses"], text=True, timeout=120)
     plans = [tuple(map(int, m)) for m in re.findall(r"accesses method (\d) policy (\d) grouped (\d)", out)]
     assert plans == [(METHOD_TILED, 0, 0)] * 2 + [(METHOD_TILED, 1, 1)] * 2, out
+
+
+@pytest.mark.parametrize("scenario,launches", [("groups", 18), ("narrow", 6)])
+def test_no_plan_is_timed_again_as_a_variant_of_itself(program, scenario, launches):
+    # groups of workgroups for plans that have none: three timings of six launches, for itself and two orders of the Mbar ranks that are
+    # the same here, not five; "64x64 instead of wide" for a winner that has 64x64 tiles: one timing, not two
+    out = subprocess.check_output([program, scenario], text=True, timeout=120)
+    assert int(re.search(r"most launches of one plan (\d+)", out).group(1)) == launches, out
