@@ -384,6 +384,22 @@ Counts packedSample(const Plan& p, int cls, int64_t offIn, int64_t offOut) {
 }  // namespace
 
 bool estimatePlan(Plan& plan, const cuttHipDeviceProps& props, int numSamples) {
+  if (plan.method == kTiled && plan.tiled.wide) {  // a wide tile makes the requests of four 64x64 ones, which is what the terms below are for
+    constexpr int kEdges = CUTT_WIDE_TILE / kTile;
+    Plan narrow = plan.clone();
+    cuttHipTiledArgs& a = narrow.tiled;
+    a.wide = 0;
+    a.tilesM *= kEdges;
+    a.tilesK *= kEdges;
+    a.superM *= kEdges;
+    a.superK *= kEdges;
+    narrow.numBlocks *= kEdges * kEdges;
+    narrow.numThreads = 256;
+    narrow.ldsBytes = (size_t)kTile * (kTile + 1) * plan.pb.elemSize;
+    const bool ok = estimatePlan(narrow, props, numSamples);
+    plan.model = narrow.model;
+    return ok;
+  }
   ModelResult& r = plan.model;
   r = ModelResult();
   const int es = plan.pb.elemSize;

@@ -86,3 +86,13 @@ def test_matrices_in_strips_off_the_line_grid_are_paced(planner):
         info = planner.plan(dim, (1, 0, 2), es)
         assert (info.method, info.tiledPaced, info.cachePolicy & 2) == (TILED, paced, 2), dim
     assert planner.plan((1822, 320, 150), (1, 0, 2), 8, CUTT_TILED_PACED=0).tiledPaced == 0
+
+
+def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
+    # (counted as tiles of 64 elements they seem to issue a quarter of the requests)
+    for dim, perm in (((8192, 8192), (1, 0)), ((4096, 256, 64), (1, 0, 2)), ((256, 400, 512), (2, 1, 0))):
+        wide = planner.plan(dim, perm, 4, TILED, CUTT_TILED_WIDE=1)
+        small = planner.plan(dim, perm, 4, TILED, CUTT_TILED_WIDE=0)
+        assert (wide.tiledWide, small.tiledWide, wide.volMm, wide.volMk) == (1, 0, small.volMm, small.volMk)
+        assert abs(wide.usPredicted / small.usPredicted - 1) < 0.01, (dim, wide.usPredicted, small.usPredicted)
+        assert (wide.rdLines, wide.wrLines, wide.rdInstr, wide.wrInstr) == (small.rdLines, small.wrLines, small.rdInstr, small.wrInstr)
