@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
                                                                 const MB mb, const ROWS rows) {
   constexpr bool kFused = std::is_same_v<ROWS, WalkAxes>;
   uint32_t tm, tk, offIn, offOut;
-  if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
+  if (!walkTile(blockIdx.x, WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
   const WalkShape<ROWS> shape{volMm, volMk, strideInK, strideOutM, rows};
   const TileLanes t = tileLanes<kFused>(shape, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
   moveTile<T, NT, false, kFused>(t, shape, in, out);
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(CUTT_WIDE_THREADS, 8) void wideTileKernel(const uin
   constexpr int kRows = kEdge / kStep;
   __shared__ uint32_t tile[kEdge][kEdge + 1];
   uint32_t tm, tk, offIn, offOut;
-  if (!walkTile(WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, volMm / kEdge, volMk / kEdge, tm, tk, offIn, offOut)) return;
+  if (!walkTile(blockIdx.x, WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, volMm / kEdge, volMk / kEdge, tm, tk, offIn, offOut)) return;
   const uint32_t c = threadIdx.x % kEdge, r = threadIdx.x / kEdge;
   const uint32_t rd = offIn + tm * kEdge + c + (tk * kEdge + r) * strideInK, wr = offOut + tk * kEdge + c + (tm * kEdge + r) * strideOutM;
   uint32_t v[kRows];

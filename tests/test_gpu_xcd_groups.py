@@ -1,5 +1,7 @@
 """Workgroups handed to the XCDs in groups, bit-exact against the oracle: every Tiled numbering, line-aligned stores and the packed
 kernel's three item orders, group sizes from one workgroup to more than there are."""
+import math
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -52,13 +54,17 @@ def test_packed(method, monkeypatch, es, group):
     ((379, 131928), (1, 0), 4, False),     # ... of 4-byte elements in strips
     ((1201, 3001), (1, 0), 8, False),      # inside the cache: neighbours share lines
     ((3001, 2999), (1, 0), 4, False),
+    # ... with an order that goes with groups: rows in few channels, few rows between the two axes, a fused axis on the line grid
+    ((1024, 1056, 64), (1, 0, 2), 4, True), ((1024, 1040, 40), (1, 0, 2), 8, True), ((640, 11, 1344, 4), (2, 1, 0, 3), 8, True), ((6, 320, 8, 2400), (3, 1, 2, 0), 8, True),
+    # separate matrices in strips off the line grid, by the kernel that paces its loads
+    ((1822, 320, 60), (1, 0, 2), 8, False), ((2001, 448, 100), (1, 0, 2), 4, False),
 ])
 def test_planner_takes_groups_where_lines_are_written_whole(method, monkeypatch, dim, perm, es, grouped):
     import torch
     import cutt_amd as cutt
     import sweep_runner
     st = torch.cuda.current_stream().cuda_stream
-    src = sweep_runner.index_pattern(dim[0] * dim[1], es)
+    src = sweep_runner.index_pattern(math.prod(dim), es)
     want = sweep_runner.expected_on_device(src, list(dim), list(perm))
     groups = []
     for group in (None, "0", "5"):

@@ -1,7 +1,7 @@
 """The walk form of a Tiled launch's numbering (cuttHipTileWalk) against the tile orders it stands for.
 
-A C++ program decodes every workgroup index of random launches as the kernels do (multiply-high divisions with the constants of
-cuttHipFinishTileWalk) and compares the sequence of tiles, the Mbar offsets and the rows' offsets with the orders' own
+A C++ program decodes every workgroup index of random launches with the kernels' own code (tile_walk.h, compiled for the host, and the constants of
+cuttHipFinishTileWalk), one chunk per XCD or groups, and compares the sequence of tiles, the Mbar offsets and the rows' offsets with the orders' own
 definition, divisions and all; divisors near the limits are checked at the numerators where a wrong rounding shows first.
 """
 import os
@@ -16,9 +16,8 @@ PROGRAM = r"""
 #include <cstring>
 #include <random>
 #include <vector>
-#include "hip_layer.h"
+#include "tile_walk.h"
 typedef uint32_t u;
-static u wd(u n, u mul, u shift) { return (u)(((uint64_t)(u)(2 * n) * mul) >> 32) >> shift; }
 struct Pos { u tm, tk, in, out; bool operator!=(const Pos& o) const { return tm != o.tm || tk != o.tk || in != o.in || out != o.out; } };
 static void offsets(const cuttHipTiledArgs& a, u m, Pos& p) {
   p.in = p.out = 0;
@@ -48,30 +47,17 @@ static std::vector<Pos> byOrder(const cuttHipTiledArgs& a) {  // the orders' def
   }
   return v;
 }
-static bool decode(const cuttHipTiledArgs& a, u bid, Pos& p) {  // as tile_order.h: walkTile
-  const cuttHipTileWalk& h = a.walk; const cuttHipWalkMbar& b = h.mbar;
-  const u M = a.tilesM, K = a.tilesK, xs = h.shifts >> 15;
-  u l = (bid & ((1u << xs) - 1)) * h.chunk + (bid >> xs), m = 0, per = K;
-  if (l >= M * K * (h.kind == 2 ? b.volMbar : 1)) return false;
-  if (h.kind == 2) { m = wd(l, b.outerMul, b.shifts & 31); l -= m * M * K; per *= b.stripMbar; }
-  const u first = wd(l, h.stripMul, h.shifts & 31) * h.superM, width = std::min(h.superM, M - first);
-  const bool full = width == h.superM;
-  l -= first * per;
-  if (h.kind == 2) { const u mi = wd(l, b.innerMul[!full], b.shifts >> (full ? 5 : 10) & 31); l -= mi * width * K; m += mi; }
-  p.tk = wd(l, full ? h.fullMul : h.lastMul, h.shifts >> (full ? 5 : 10) & 31);
-  p.tm = first + l - p.tk * width; p.in = p.out = 0;
-  if (h.kind == 2)
-    for (int k = 0; k < (b.n > 4 ? 8 : 4); k++) {
-      const u q = wd(m, b.rank[k].mul, b.rank[k].shift), i = m - q * b.rank[k].extent;
-      p.in += i * b.rank[k].strideIn; p.out += i * b.rank[k].strideOut; m = q;
-    }
-  return true;
+static bool decode(const cuttHipTiledArgs& a, u bid, Pos& p) {
+  const cuttHipTileWalk& h = a.walk;
+  const cutt::WalkHead head{h.chunk, h.superM, h.stripMul, h.fullMul, h.lastMul, h.shifts};
+  return h.kind == 2 ? cutt::walkTile(bid, head, h.mbar, a.tilesM, a.tilesK, p.tm, p.tk, p.in, p.out)
+                     : cutt::walkTile(bid, head, cutt::NoMbar{}, a.tilesM, a.tilesK, p.tm, p.tk, p.in, p.out);
 }
-static u rowWalk(const cuttHipWalkRows& r, u i) {  // as tile_order.h: walkRowOffset
-  u q = wd(i, r.mul[0], r.shift[0]), off = (i - q * r.extent[0]) * r.stride[0];
-  if (r.n <= 2) return off + q * r.stride[1];
-  for (int k = 1; k < 3; k++) { const u t = wd(q, r.mul[k], r.shift[k]); off += (q - t * r.extent[k]) * r.stride[k]; q = t; }
-  return off + q * r.stride[3];
+static size_t position(const cuttHipTiledArgs& a, u bid) {  // what the fields' comments say
+  if (!a.xcdChunk) return bid;
+  if (!a.xcdGroup) return (size_t)(bid % 8) * a.walk.chunk + bid / 8;
+  const u g = 1u << (a.xcdGroup - 1), turn = bid / 8 / g;  // XCD b % 8 takes groups of g in turn
+  return (size_t)(turn * 8 + bid % 8) * g + bid / 8 % g;
 }
 static u rowPlain(const cuttHipRowRadix& rr, u stride, u i) {
   if (rr.n == 0) return i * stride;
@@ -96,6 +82,8 @@ int main() {
     }
     const uint64_t logical = (uint64_t)a.tilesM * a.tilesK * a.volMbar;
     a.xcdChunk = logical >= 64 ? (u)((logical + 7) / 8) : 0;
+    a.xcdGroup = (int16_t)(a.xcdChunk && r(0, 1) ? r(1, 9) : 0);
+    const uint64_t unit = a.xcdGroup ? 8ull << (a.xcdGroup - 1) : (a.xcdChunk ? 8 : 1);
     a.strideInK = g(); a.strideOutM = g();
     for (cuttHipRowRadix* rr : {&a.rowsK, &a.rowsM}) {
       rr->n = r(0, 4);
@@ -108,10 +96,11 @@ int main() {
     if (!a.walk.kind) continue;
     walks++;
     const std::vector<Pos> want = byOrder(a);
-    if (want.size() != logical || a.walk.blocks < logical || a.walk.blocks > logical + 7) return std::printf("%zu positions, %u workgroups\n", want.size(), a.walk.blocks), 1;
+    if (want.size() != logical || a.walk.blocks != (logical + unit - 1) / unit * unit) return std::printf("%zu positions, %u workgroups\n", want.size(), a.walk.blocks), 1;
     size_t seen = 0;
     for (u b = 0; b < a.walk.blocks; b++) {
-      const size_t l = a.xcdChunk ? (size_t)(b % 8) * a.walk.chunk + b / 8 : b;
+      const size_t l = position(a, b);
+      if (l != cutt::xcdPosition(b, a.xcdGroup ? a.xcdChunk : a.walk.chunk, a.xcdGroup)) return std::printf("workgroup %u: position\n", b), 1;
       Pos p;
       if (decode(a, b, p) != (l < logical)) return std::printf("workgroup %u: end\n", b), 1;
       if (l >= logical) continue;
@@ -124,7 +113,7 @@ int main() {
       for (int j = 0; j < a.rowsK.n; j++) k *= a.rowsK.extent[j];
       for (int j = 0; j < a.rowsM.n; j++) m *= a.rowsM.extent[j];
       k = g() % (a.rowsK.n ? k : 0x7fffffffu); m = g() % (a.rowsM.n ? m : 0x7fffffffu);
-      if (rowWalk(a.walk.rowsK, k) != rowPlain(a.rowsK, a.strideInK, k) || rowWalk(a.walk.rowsM, m) != rowPlain(a.rowsM, a.strideOutM, m)) return std::printf("row offsets\n"), 1;
+      if (cutt::walkRowOffset(a.walk.rowsK, k) != rowPlain(a.rowsK, a.strideInK, k) || cutt::walkRowOffset(a.walk.rowsM, m) != rowPlain(a.rowsM, a.strideOutM, m)) return std::printf("row offsets\n"), 1;
     }
   }
   if (walks < 1000) return std::printf("only %ld walks\n", walks), 1;
@@ -139,7 +128,7 @@ int main() {
       const uint64_t q = (g() % (0x7fffffffull / d + 1)) * d;
       for (uint64_t n : {q, q + d - 1, q > 0 ? q - 1 : 0, (uint64_t)0x7fffffff}) {
         if (n > 0x7fffffffull) continue;
-        if (rowWalk(a.walk.rowsK, (u)n) != (u)n / d) return std::printf("%llu / %u\n", (unsigned long long)n, d), 1;
+        if (cutt::walkRowOffset(a.walk.rowsK, (u)n) != (u)n / d) return std::printf("%llu / %u\n", (unsigned long long)n, d), 1;
       }
     }
   }

@@ -1,5 +1,5 @@
 """Workgroups handed to the XCDs in groups: every logical position is visited exactly once, in both forms the kernels decode
-(tile_order.h: xcdPosition and walkTile; no GPU)."""
+(tile_walk.h: xcdPosition and walkTile, the kernels' own code compiled for the host; no GPU)."""
 import os
 import subprocess
 
@@ -10,17 +10,8 @@ PROGRAM = r"""
 #include <cstdio>
 #include <cstring>
 #include <vector>
-#include "hip_layer.h"
+#include "tile_walk.h"
 typedef uint32_t u;
-static u position(u bid, u chunk, u group) {  // as tile_order.h: xcdPosition
-  const u q = bid / 8, x = bid % 8;
-  if (group) { const u g = group - 1; return ((((q >> g) * 8) + x) << g) + (q & ((1u << g) - 1)); }
-  return chunk ? x * chunk + q : bid;
-}
-static u walked(const cuttHipTileWalk& h, u bid) {  // as tile_order.h: walkTile
-  const u xs = (h.shifts >> 15) & 3, g = ((h.shifts >> 17) - 1) & 31, q = bid >> xs;
-  return (bid & ((1u << xs) - 1)) * h.chunk + (q & ((1u << g) - 1)) + (((q >> g) << g) << 3);
-}
 int main() {
   for (u tiles : {1u, 7u, 8u, 63u, 64u, 65u, 127u, 128u, 129u, 1000u, 4097u})
     for (u group = 0; group <= 10; group++) {
@@ -31,9 +22,12 @@ int main() {
       cuttHipFinishTileWalk(&a);
       if (a.walk.kind != 1 || a.walk.blocks % 8) return std::printf("walk %u %u\n", tiles, group), 1;
       std::vector<int> seen(a.walk.blocks, 0);
+      const cutt::WalkHead head{a.walk.chunk, a.walk.superM, a.walk.stripMul, a.walk.fullMul, a.walk.lastMul, a.walk.shifts};
       for (u b = 0; b < a.walk.blocks; b++) {
-        const u l = position(b, a.walk.chunk, group);
-        if (l != walked(a.walk, b)) return std::printf("two forms differ: %u %u %u\n", tiles, group, b), 1;
+        const u l = cutt::xcdPosition(b, a.walk.chunk, group);
+        u tm = 0, tk = 0, in, out;
+        const bool tile = cutt::walkTile(b, head, cutt::NoMbar{}, tiles, 1, tm, tk, in, out);
+        if (tile != (l < tiles) || (tile && (tm != l || tk != 0))) return std::printf("two forms differ: %u %u %u\n", tiles, group, b), 1;
         if (l >= a.walk.blocks || seen[l]++) return std::printf("position %u of %u\n", l, a.walk.blocks), 1;
       }
     }
