@@ -13,6 +13,7 @@
 //               often the winner was launched
 //   narrow    - wide tiles 100 us, 64x64 tiles in tile order 6 40 us in patches of 2 x 2 and 41 us in others, 60 us in any other order:
 //               prints how often one plan in order 6 other than the winner was launched
+//   tie98, tie99 - Packed plans: the one cuttPlan makes 100 us, all others 98 or 99.5 us; prints the policy of cuttPlan's plan
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
@@ -124,6 +125,20 @@ static int drift() {
   return measure({1201, 30011}, {1, 0}, 8);
 }
 
+static int tie(double othersUs) {
+  int dim[4] = {1544, 426, 76, 4}, perm[4] = {2, 0, 1, 3};
+  cuttHandle h;
+  cuttPlanInfo own = {};
+  if (cuttPlan(&h, 4, dim, perm, 8, 0) != CUTT_SUCCESS || cuttGetPlanInfo(h, &own) != CUTT_SUCCESS) return 1;
+  cuttDestroy(h);
+  std::printf("own policy %d\n", own.cachePolicy);
+  gTiledUs = [](const cuttHipTiledArgs&) { return 200.0; };
+  gPackedUs = [=](const cuttHipPackedArgs& a) {
+    return a.split[0].numSplit == own.numSplit && a.cachePolicy == own.cachePolicy ? 100.0 : othersUs;
+  };
+  return measure({1544, 426, 76, 4}, {2, 0, 1, 3}, 8);
+}
+
 static int groups() {
   setenv("CUTT_MEASURE_NO_PLAYOFF", "1", 1);
   std::map<std::string, int> launches;
@@ -195,6 +210,8 @@ int main(int argc, char** argv) {
   if (what == "accesses") return accesses();
   if (what == "predicted") return predicted();
   if (what == "drift") return drift();
+  if (what == "tie98") return tie(98.0);
+  if (what == "tie99") return tie(99.5);
   if (what == "groups") return groups();
   if (what == "narrow") return narrow();
   return 2;

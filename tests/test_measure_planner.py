@@ -70,3 +70,9 @@ def test_no_plan_is_timed_again_as_a_variant_of_itself(program, scenario, launch
     # the same here, not five; "64x64 instead of wide" for a winner that has 64x64 tiles: one timing, not two
     out = subprocess.check_output([program, scenario], text=True, timeout=120)
     assert int(re.search(r"most launches of one plan (\d+)", out).group(1)) == launches, out
+
+
+@pytest.mark.parametrize("scenario,us", [("tie98", 98.0), ("tie99", 100.0)])
+def test_the_heuristic_plan_wins_ties(program, scenario, us):
+    # half a per cent is what two timings of one plan differ by, two per cent are not
+    assert measured(program, scenario)["us"] == us
