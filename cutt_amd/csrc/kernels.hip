@@ -83,11 +83,7 @@ __device__ __forceinline__ void waitForGlobalAccesses() { asm volatile("s_waitcn
 // ranks that lead the output on the Mk side), so the rows of a tile are not equally far apart.  Lane l
 // derives the offset of row l of either axis with a short mixed-radix decode (tileRowOffsets) and the
 // wave picks a row's offset out of that lane; the elements of a row are contiguous as before.
-//
-// TESTED: one piece of code with a test for every row, whose loads the compiler makes wait for each other.  For 4-byte elements with non-temporal stores
-// in numberings that have no walk (address bits, mostly): (1024,64,1024)/(2,1,0) 105.2 -> 103.1 us, 103.5 in the form of tiledKernel,
-// (1024,16,1024,12)/(2,1,0,3) 278.2 there -> 275.4; 8-byte elements lose 1-2 %.
-template <typename T, int NT, bool TESTED, bool FUSED, typename Args>
+template <typename T, int NT, bool FUSED, typename Args>
 __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
   __shared__ T tile[kTile][kTile + 1];
   const uint32_t wave = threadIdx.x >> 6;
@@ -121,31 +117,37 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
     else f(std::integral_constant<int, 1>{}, std::false_type{});
   };
   static_assert(kRowGroups == 4 && kGroupRows * kWaves == 16, "row groups of 16 tile rows");
-  if constexpr (TESTED) {
-    T v[kTileRows];
-#pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsK) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
-#pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsK) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
-    __syncthreads();
-    T u[kTileRows];
-#pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsM) u[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
-#pragma unroll
-    for (int j = 0; j < kTileRows; j++)
-      if ((uint32_t)(j / kGroupRows) < t.groupsM) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), u[j]);
-  } else {
-    byGroups(t.wK, read);
-    __syncthreads();
-    byGroups(t.wM, write);
-  }
+  byGroups(t.wK, read);
+  __syncthreads();
+  byGroups(t.wM, write);
 }
 
-// How tiledKernel's loads leave: as in moveTile, row group by row group without waiting, row group by row group waiting for each.
-enum { kLoadsAtOnce, kLoadsPaced, kLoadsGrouped };
+// The same with a test for every row in one piece of code, whose loads the compiler makes wait for each other.  For 4-byte elements with
+// non-temporal stores in numberings that have no walk (address bits, mostly): (1024,64,1024)/(2,1,0) 103.5 us with paced loads, 103.1 here,
+// (1024,16,1024,12)/(2,1,0,3) 278.2 / 275.4, (256,1024,512)/(2,1,0) 197.8 / 195.4; eight such tensors 0.4 % in the mean.
+template <typename T, int NT, bool FUSED, typename Args>
+__device__ __forceinline__ void moveTileTested(const TileLanes& t, const Args& a, const T* __restrict__ in, T* __restrict__ out) {
+  __shared__ T tile[kTile][kTile + 1];
+  const uint32_t wave = threadIdx.x >> 6;
+  T v[kTileRows];
+#pragma unroll
+  for (int j = 0; j < kTileRows; j++)
+    if ((uint32_t)(j / kGroupRows) < t.groupsK) v[j] = ldg<NT>(in + tileReadElem<FUSED>(t, a, wave, j, t.wK));
+#pragma unroll
+  for (int j = 0; j < kTileRows; j++)
+    if ((uint32_t)(j / kGroupRows) < t.groupsK) tile[min(wave + kWaves * j, t.wK)][t.cx] = v[j];
+  __syncthreads();
+  T u[kTileRows];
+#pragma unroll
+  for (int j = 0; j < kTileRows; j++)
+    if ((uint32_t)(j / kGroupRows) < t.groupsM) u[j] = tile[t.ck][min(wave + kWaves * j, t.wM)];
+#pragma unroll
+  for (int j = 0; j < kTileRows; j++)
+    if ((uint32_t)(j / kGroupRows) < t.groupsM) stg<NT>(out + tileWriteElem<FUSED>(t, a, wave, j, t.wM), u[j]);
+}
+
+// How tiledKernel's loads leave: row group by row group without waiting, row group by row group waiting for each, as in moveTileTested.
+enum { kLoadsPaced, kLoadsGrouped, kLoadsTested };
 
 // Any numbering of the workgroups (tile_order.h: locateTile).
 template <typename T, int NT, int LOADS, bool FUSED>
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
   if (!locateTile(a, tm, tk, offIn, offOut)) return;
   // tile geometry, clamped edges, skipped row groups: tile_order.h
   const TileLanes t = tileLanes<FUSED>(a, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  if constexpr (LOADS != kLoadsAtOnce) {
+  if constexpr (LOADS != kLoadsTested) {
     // Rows in groups, or paced loads (cuttHipTiledArgs.paced): one piece of code whose row groups are tested one after the
     // other.  Without GROUPED a group's loads go out while the next one's addresses are computed, and no load is waited for before all are
     // out.  All sixteen at once (moveTile), what a small tensor needs, cost large ones up to 10 %, since neighbouring tiles no
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
       }
     }
   } else {
-    moveTile<T, NT, sizeof(T) == 4, FUSED>(t, a, in, out);
+    moveTileTested<T, NT, FUSED>(t, a, in, out);
   }
 }
 
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(kTileThreads) void tiledWalkKernel(const T* __restr
   if (!walkTile(blockIdx.x, WalkHead{chunk, superM, stripMul, fullMul, lastMul, shifts}, mb, (volMm + kTile - 1) / kTile, (volMk + kTile - 1) / kTile, tm, tk, offIn, offOut)) return;
   const WalkShape<ROWS> shape{volMm, volMk, strideInK, strideOutM, rows};
   const TileLanes t = tileLanes<kFused>(shape, tm, tk, offIn, offOut, threadIdx.x & 63, threadIdx.x >> 6);
-  moveTile<T, NT, false, kFused>(t, shape, in, out);
+  moveTile<T, NT, kFused>(t, shape, in, out);
 }
 
 // Tiles of 128x128 4-byte elements, whole ones only, numbered by a walk.
@@ -619,7 +621,7 @@ bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk,
               (uint64_t)volMbar;
   }
   blocks = logical;
-  if (xcdGroup < 0 || xcdGroup > 20 || (xcdGroup && !xcdChunk)) return false;
+  if (xcdGroup < 0 || xcdGroup > 20 || (xcdGroup && (!xcdChunk || order == 7))) return false;
   if (xcdGroup) {
     const uint64_t unit = (uint64_t)kNumXcd << (xcdGroup - 1);
     blocks = (logical + unit - 1) / unit * unit;
@@ -873,11 +875,10 @@ extern "C" int cuttHipLaunchTiled(const cuttHipTiledArgs* a, const void* in, voi
 #define CUTT_LAUNCH_TILED_F(T, NT, LOADS)                                                                        \
   (fused ? launchKernel(tiledKernel<T, NT, LOADS, true>, grid, block, 0, s, *a, (const T*)in, (T*)out)           \
          : launchKernel(tiledKernel<T, NT, LOADS, false>, grid, block, 0, s, *a, (const T*)in, (T*)out))
-  // (with ordinary stores nothing takes the loads at once through this kernel)
 #define CUTT_LAUNCH_TILED(T, NT)                                                                                 \
-  return (int)(a->grouped                        ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsGrouped)                     \
-               : a->paced || !(a->cachePolicy & 2) ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsPaced)                     \
-                                                   : CUTT_LAUNCH_TILED_F(T, NT | 2, kLoadsAtOnce))
+  return (int)(a->grouped                                               ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsGrouped) \
+               : sizeof(T) == 8 || a->paced || !(a->cachePolicy & 2) ? CUTT_LAUNCH_TILED_F(T, NT, kLoadsPaced)   \
+                                                                     : CUTT_LAUNCH_TILED_F(uint32_t, NT | 2, kLoadsTested))
 #define CUTT_LAUNCH_TILED_NT(T)                                \
   switch (a->cachePolicy) {                                    \
     case 0: CUTT_LAUNCH_TILED(T, 0);                           \
