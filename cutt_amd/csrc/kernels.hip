@@ -88,9 +88,9 @@ __device__ __forceinline__ void moveTile(const TileLanes& t, const Args& a, cons
   __shared__ T tile[kTile][kTile + 1];
   const uint32_t wave = threadIdx.x >> 6;
 
-  // One straight piece of code per number of row groups (4 for a whole tile, fewer at an edge): with one group behind
-  // the other and a test in between the compiler waits for a group's loads before the next one's go out, since the rows'
-  // registers meet again behind the test.  WHOLE: all 64 rows are there, no index needs clamping.
+  // One straight piece of code per number of row groups (4 for a whole tile, fewer at an edge): all loads go out back to back, where tests
+  // between the groups would keep them apart or even, in a function like this one, make them wait for each other (tiledKernel).  WHOLE: all
+  // 64 rows are there, no index needs clamping.
   auto read = [&](auto groups, auto whole) __attribute__((always_inline)) {  // lanes run along the input-contiguous axis (Mm), rows along Mk
     constexpr int kRows = decltype(groups)::value * kGroupRows;
     const uint32_t lastRow = decltype(whole)::value ? kTile - 1u : t.wK;
@@ -225,8 +225,8 @@ __global__ __launch_bounds__(kTileThreads) void tiledKernel(const cuttHipTiledAr
 // The numberings of cuttHipTileWalk.  The arguments up to `shifts`, 14 words, are in scalar registers when a wave starts
 // (the Makefile's kernarg-preload-count), so that a plain matrix transpose waits for nothing before its first load;
 // MB and ROWS hold what launches with Mbar positions and with fused axes need besides.
-// Bound by latency up to some 20 MB, by memory beyond.  Against the kernel above as it was before (its loads in groups of
-// four that waited for each other): 2011 x 1163, 4 bytes, 5.94 -> 4.38 us; (24,32,36,43)/(3,1,2,0), 8 bytes, 5.99 -> 4.86;
+// Bound by latency up to some 20 MB, by memory beyond.  Against the kernel above, with
+// its loads in groups of four: 2011 x 1163, 4 bytes, 5.94 -> 4.38 us; (24,32,36,43)/(3,1,2,0), 8 bytes, 5.99 -> 4.86;
 // 4297 x 1731, 8 bytes, 28.2 -> 25.5; (7,149,21,189)/(3,2,1,0), 4 bytes, 9.5 -> 7.8; (96,75,96,75)/(2,1,3,0), 8 bytes, 161.7 -> 159.0,
 // 157.7 in XCD groups.
 template <typename T, int NT, typename MB, typename ROWS>

@@ -443,3 +443,48 @@ def test_strips_per_mbar_position_for_fused_mm_sets(monkeypatch):
     run_rule("strips per Mbar position", cases, {"CUTT_TILED_ORDER": "5"},
              lambda on, off: on.method_name == "Tiled" and off.method_name == "Tiled" and on.tiledOrder == 3 and off.tiledOrder == 5,
              1.0, 0.93, 3)
+
+
+def test_xcd_groups_against_one_chunk_per_xcd():
+    # random tensors whose plan deals the workgroups out in groups (found: Tiled plans +4 % in the mean over 295, -12 ... +22 %, packed ones
+    # with whole lines +2 ... +12 %); the plan without also has the orders that go with chunks
+    import baseline_configs as bc
+    rng = np.random.default_rng(606)
+    cases = []
+    while len(cases) < 24:
+        rank = int(rng.integers(2, 6))
+        es = 8 if len(cases) % 2 == 0 else 4
+        dim = bc.random_dims(rng, rank, target=8.0e8 / es * float(2.0 ** rng.uniform(-1, 0.5)), tol=0.2)
+        perm = [int(p) for p in rng.permutation(rank)]
+        if perm == list(range(rank)):
+            continue
+        cases.append(dict(dim=tuple(int(d) for d in dim), perm=tuple(perm), es=es))
+    run_rule("XCD groups", cases, {"CUTT_XCD_GROUP": "0"}, lambda on, off: on.xcdGroup > 0 and off.xcdGroup == 0, 1.005, 0.86, 8)
+
+
+def test_orders_for_rows_in_few_channels_in_groups():
+    # input rows a multiple of 4 KB apart on the line grid (found: +6 % against a chunk per XCD on 4-byte tensors, +9 % on 8-byte ones)
+    rng = np.random.default_rng(4096)
+    cases = []
+    while len(cases) < 10:
+        es = 4 if len(cases) % 2 == 0 else 8
+        m, k = 4096 // es * int(rng.integers(3, 24)), 128 // es * int(rng.integers(40, 300))
+        batch = max(2, round(float(rng.uniform(3e8, 9e8)) / (m * k * es)))
+        if es == 4 and k % 128 == 0 or k * es % 32768 == 0:
+            continue
+        cases.append(dict(dim=(m, k, batch), perm=(1, 0, 2), es=es))
+    run_rule("rows in few channels", cases, {"CUTT_XCD_GROUP": "0"}, lambda on, off: on.method_name == "Tiled" and on.xcdGroup > 0 and off.xcdGroup == 0,
+             1.02, 0.92, 6)
+
+
+def test_paced_loads_for_matrices_in_strips_off_the_line_grid():
+    # (found: +2.6 % in the mean over 31 8-byte batches, -2 ... +11 %, +0.7 % over 18 4-byte ones, -5 ... +8 %)
+    rng = np.random.default_rng(99)
+    cases = []
+    while len(cases) < 10:
+        es = 4 if len(cases) % 3 == 0 else 8
+        m, k = int(rng.integers(1000, 4000)), 128 // es * int(rng.integers(6, 40))
+        if m * es % 128 == 0:
+            continue
+        cases.append(dict(dim=(m, k, int(6.0e8 / es / (m * k)) + 2), perm=(1, 0, 2), es=es))
+    run_rule("paced matrices", cases, {"CUTT_TILED_PACED": "0"}, lambda on, off: on.tiledPaced == 1 and on.cachePolicy & 2 and off.tiledPaced == 0, 0.995, 0.92, 6)
