@@ -363,9 +363,9 @@ typedef struct cuttHipPackedArgs {
   int maxVol;          /* largest class volume */
   uint32_t xcdChunk;   /* 0: workgroup b is logical block b; else logical block = (b % 8)*xcdChunk + b/8
                           and the grid has 8*xcdChunk workgroups */
-  int xcdGroup;        /* as in cuttHipTiledArgs, for logical blocks; beside xcdChunk: read with it */
   int cachePolicy;     /* bit 0 = non-temporal loads, bit 1 = non-temporal stores */
   long long volume;    /* elements from the first to the last one of the tensor, on its wider side (bounds every offset) */
+  int xcdGroup;        /* as in cuttHipTiledArgs, for logical blocks */
   int wideOffsets;     /* 0: the tensor is below 4 GB and the kernel keeps 32-bit byte offsets;
                           1: element offsets with 64-bit address arithmetic (required from 4 GB on) */
   cuttHipPackedClass cls[4];

@@ -621,7 +621,7 @@ bool tileGrid(int order, int tilesM, int tilesK, int volMbar, uint32_t xcdChunk,
               (uint64_t)volMbar;
   }
   blocks = logical;
-  if (xcdGroup < 0 || xcdGroup > 20 || (xcdGroup && (!xcdChunk || order == 7))) return false;
+  if (xcdGroup < 0 || xcdGroup > 20 || (xcdGroup && order == 7)) return false;
   if (xcdGroup) {
     const uint64_t unit = (uint64_t)kNumXcd << (xcdGroup - 1);
     blocks = (logical + unit - 1) / unit * unit;
@@ -1123,7 +1123,7 @@ static uint64_t packedGrid(const cuttHipPackedArgs* a) {
   const long long items = cuttHipPackedItemNumbers(a);
   if (items < 1) return 0;
   uint64_t blocks = ((uint64_t)items + a->itemsPerBlock - 1) / a->itemsPerBlock;
-  if (a->xcdGroup < 0 || a->xcdGroup > 20 || (a->xcdGroup && !a->xcdChunk)) return 0;
+  if (a->xcdGroup < 0 || a->xcdGroup > 20) return 0;
   if (a->xcdGroup) {
     const uint64_t unit = (uint64_t)kNumXcd << (a->xcdGroup - 1);
     blocks = (blocks + unit - 1) / unit * unit;

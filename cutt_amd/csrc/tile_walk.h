@@ -22,12 +22,14 @@ namespace cutt {
 
 constexpr uint32_t kNumXcd = 8;
 
-// Workgroup index -> logical position (cuttHipTiledArgs.xcdChunk, xcdGroup; groups have a chunk as well).  Without a branch, so that both are
-// read at once: with one, packed launches of 5 us waited for one after the other and took 0.5-1 % longer.
+// Workgroup index -> logical position (cuttHipTiledArgs.xcdChunk, xcdGroup).
 CUTT_DEVICE uint32_t xcdPosition(uint32_t bid, uint32_t chunk, uint32_t group) {
-  const uint32_t q = bid / kNumXcd, x = bid % kNumXcd, g = (group - 1) & 31;  // (31: no groups)
-  const uint32_t l = x * (group ? 1u << g : chunk) + (q & ((1u << g) - 1)) + (((q >> g) << g) * kNumXcd);
-  return chunk ? l : bid;
+  const uint32_t q = bid / kNumXcd, x = bid % kNumXcd;
+  if (group) {
+    const uint32_t g = group - 1;
+    return ((((q >> g) * kNumXcd) + x) << g) + (q & ((1u << g) - 1));
+  }
+  return chunk ? x * chunk + q : bid;
 }
 
 CUTT_DEVICE uint32_t walkMulHi(uint32_t a, uint32_t b) {

@@ -37,12 +37,3 @@ def test_copy_tiles_carry_no_row_table(tmp_path):
     src.write_text('#include "hip_layer.h"\nstatic_assert(sizeof(cuttHipCopyTiles) == 13 * 4 + sizeof(cuttHipTileDigits) + sizeof(cuttHipMbar), "");\n')
     subprocess.check_call(["g++", "-std=c++17", "-fsyntax-only", "-I" + os.path.join(ROOT, "cutt_amd", "csrc"),
                            "-I" + os.path.join(ROOT, "include"), str(src)])
-
-
-def test_chunk_and_group_of_packed_launches_are_read_together(tmp_path):
-    # (waited for one after the other in different lines, launches of 5 us took 0.5-1 % longer)
-    src = tmp_path / "pair.cpp"
-    src.write_text('#include <cstddef>\n#include "hip_layer.h"\nstatic_assert(offsetof(cuttHipPackedArgs, xcdGroup) == offsetof(cuttHipPackedArgs, xcdChunk) + 4 && '
-                   'offsetof(cuttHipPackedArgs, xcdGroup) / 64 == offsetof(cuttHipPackedArgs, xcdChunk) / 64, "");\n')
-    subprocess.check_call(["g++", "-std=c++17", "-fsyntax-only", "-I" + os.path.join(ROOT, "cutt_amd", "csrc"),
-                           "-I" + os.path.join(ROOT, "include"), str(src)])
