@@ -260,8 +260,16 @@ void setCachePolicy(Plan& p, int policy, const cuttHipDeviceProps& props) {
 
 // Cache policy of a plan's global accesses, from its size and the model's sampled address stream.  (Not applied when
 // CUTT_CACHE_POLICY pins the policy.)  Timed on 120 random tensors of 0.14-1.6 GB per buffer, buffers in rotation and
-// the same ones again and again:
-//  - input and output inside the memory-side cache together: ordinary accesses (non-temporal ones go past it);
+// the same ones again and again (the smaller ones: 0.03-0.14 GB):
+//  - up to a sixth of the memory-side cache per buffer: ordinary accesses (non-temporal ones go past it);
+//  - from there to half of it, where the cache holds one or two tensors but not what else a program works on, packed plans
+//    leave it to the input (non-temporal stores), and so do Tiled ones that write whole lines.  850 tensors, times over those with
+//    ordinary accesses: three pairs of buffers in rotation / as many pairs as make 4 GB / right after a kernel that writes the input /
+//    with such a kernel before and one that reads the result behind.  Packed plans 0.71 / 0.94 / 0.92 / 0.89 at 45-75 MB per buffer,
+//    0.77 / 0.94 / 0.88 / 0.93 at 75-95, 0.92 / 0.94 / 0.90 / 0.88 at 95-135; Tiled ones 0.77 / 0.93 / 1.01 / 0.92, 0.73 / 0.95 / 1.05 / 0.96,
+//    0.89 / 0.91 / 1.03 / 0.92.  The packed plans may cover up to 16 % of their lines partly there, any number below a third
+//    of the cache, and 4 % up to a whole cache size (0.95 / 0.96 / 0.91 / 0.92).  Other Tiled plans lose by such stores (0.81-1.1 / 1.03-1.13);
+//    with non-temporal loads they gain in rotation (0.96 at 45 MB, 0.84 at 75, 1.02 at 115), but a pass on an input just written takes 3-15 % longer;
 //  - outputs written in whole lines - at most one line in a hundred left partly covered by a workgroup -:
 //    non-temporal stores, 2-10 % faster than ordinary ones ((37,59,7,16,6,30) 146 -> 132 us, (985024,28,4) 345 ->
 //    317 us); from 3 partial lines in a hundred on they lose (4-byte rows of 9 KB: 188 -> 207 us).  Where the reads
@@ -285,7 +293,8 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
   if (std::getenv("CUTT_CACHE_POLICY")) return;
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
   const double cache = (double)props.infinityCacheBytes;
-  if (cache > 0 && 2.0 * bytes <= cache) {
+  const bool copies = p.method == kTrivial || p.method == kTiledCopy;
+  if (cache > 0 && 2.0 * bytes <= (copies ? cache : cache / 3)) {
     setCachePolicy(p, 0, props);
     return;
   }
@@ -298,8 +307,15 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
     setCachePolicy(p, bytes <= 3.5 * cache ? 1 : 3, props);
     return;
   }
-  if (p.model.wrPartialLines <= 0.01 * lines) {
+  const bool packed = p.method == kPacked || p.method == kPackedSplit;
+  double partial = 0.01;
+  if (packed && bytes <= cache) partial = bytes <= cache / 3 ? 2.0 : (2.0 * bytes <= cache ? 0.16 : 0.04);
+  if (p.model.wrPartialLines <= partial * lines) {
     setCachePolicy(p, bytes > cache && p.model.rdLines <= 1.02 * lines ? 3 : 2, props);
+    return;
+  }
+  if (2.0 * bytes <= cache) {
+    setCachePolicy(p, 0, props);
     return;
   }
   const bool narrowTiles = (p.method == kTiled || p.method == kTiledCopy) && p.pb.elemSize == 4;

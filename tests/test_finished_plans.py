@@ -88,6 +88,26 @@ def test_matrices_in_strips_off_the_line_grid_are_paced(planner):
     assert planner.plan((1822, 320, 150), (1, 0, 2), 8, CUTT_TILED_PACED=0).tiledPaced == 0
 
 
+CACHE = 256 << 20  # what the stand-in device reports
+
+
+@pytest.mark.parametrize("dim,perm,es,policy", [
+    # packed plans whose lines are written whole, on either side of a sixth of the cache per buffer
+    ((16, 12, 32, 909), (2, 0, 1, 3), 8, 0), ((16, 12, 32, 912), (2, 0, 1, 3), 8, 2), ((16, 12, 32, 2600), (2, 0, 1, 3), 8, 2),
+    # with 16 % and more of them covered partly: below a third of the cache, above
+    ((26, 218, 12, 120), (1, 2, 0, 3), 8, 2), ((26, 218, 12, 228), (1, 2, 0, 3), 8, 0),
+    # Tiled plans that write whole lines, others
+    ((512, 512, 21), (1, 0, 2), 8, 0), ((512, 512, 22), (1, 0, 2), 8, 2), ((2177, 2585), (1, 0), 8, 0), ((2177, 7177), (1, 0), 8, 0),
+])
+def test_cache_policy_of_tensors_up_to_half_a_cache_size(planner, dim, perm, es, policy):
+    info = planner.plan(dim, perm, es)
+    size = es
+    for d in dim:
+        size *= d
+    assert 2 * size <= CACHE
+    assert info.cachePolicy == policy, (info.method, info.wrPartialLines / (size / 128))
+
+
 def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
     # (counted as tiles of 64 elements they seem to issue a quarter of the requests)
     for dim, perm in (((8192, 8192), (1, 0)), ((4096, 256, 64), (1, 0, 2)), ((256, 400, 512), (2, 1, 0))):
