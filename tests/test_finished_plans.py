@@ -95,7 +95,7 @@ CACHE = 256 << 20  # what the stand-in device reports
     # packed plans whose lines are written whole, on either side of a sixth of the cache per buffer
     ((16, 12, 32, 909), (2, 0, 1, 3), 8, 0), ((16, 12, 32, 912), (2, 0, 1, 3), 8, 2), ((16, 12, 32, 2600), (2, 0, 1, 3), 8, 2),
     # with 16 % and more of them covered partly: below a third of the cache, above
-    ((26, 218, 12, 120), (1, 2, 0, 3), 8, 2), ((26, 218, 12, 228), (1, 2, 0, 3), 8, 0),
+    ((26, 218, 12, 120), (1, 2, 0, 3), 8, 2), ((4, 6, 2071, 4, 10, 15), (4, 2, 0, 3, 1, 5), 4, 0),
     # Tiled plans that write whole lines, others
     ((512, 512, 21), (1, 0, 2), 8, 0), ((512, 512, 22), (1, 0, 2), 8, 2), ((2177, 2585), (1, 0), 8, 0), ((2177, 7177), (1, 0), 8, 0),
 ])
