@@ -332,6 +332,33 @@ typedef struct cuttHipSplitRank {
 } cuttHipSplitRank;
 
 /*
+ * What the packed kernel for one block per workgroup (itemsPerBlock 1) decodes its arguments from; derived from cuttHipPackedArgs
+ * by cuttHipFinishPackedOnce.  Divisions as in cuttHipTileWalk.
+ */
+#define CUTT_ONCE_RANKS 12
+typedef struct cuttHipOnceClass {
+  uint32_t last, inCont, outCont;      /* elements of the block - 1, run lengths */
+  uint32_t inMul, outMul, shifts;      /* divisions by the run lengths: in | out << 5 */
+  uint32_t rowIn, rowOut, shIdx;       /* the class's tables, in bytes from the first one */
+} cuttHipOnceClass;
+
+typedef struct cuttHipOnceSlab {
+  uint32_t rem, stepIn, stepOut, strideIn, strideOut;  /* slab s starts s * step + min(s, rem) * stride into the tensor */
+} cuttHipOnceSlab;
+
+typedef struct cuttHipPackedOnce {
+  uint32_t blocks;                     /* workgroups of the launch; 0: the arguments are not of this form */
+  uint32_t chunk, items;
+  uint32_t num[2], mul[2];             /* slabs of the cut ranks and divisions by them */
+  uint32_t shifts;                     /* division by num[0] | by num[1] << 5 | as in cuttHipTileWalk from bit 15 on */
+  uint32_t padThreads;                 /* padShift | numThreads << 8 */
+  uint32_t n;
+  cuttHipOnceSlab slab[2];
+  cuttHipWalkRank rank[CUTT_ONCE_RANKS];
+  cuttHipOnceClass cls[4];
+} cuttHipPackedOnce;
+
+/*
  * Packed and PackedSplit methods.  A staged block is the index set Mmk with up to two of its
  * ranks cut into slabs (typically the last rank of the input-contiguous set and the last rank of
  * the output-contiguous set, which makes the block a 2-D tile over fused rank sets).  Work items
@@ -369,8 +396,12 @@ typedef struct cuttHipPackedArgs {
   int wideOffsets;     /* 0: the tensor is below 4 GB and the kernel keeps 32-bit byte offsets;
                           1: element offsets with 64-bit address arithmetic (required from 4 GB on) */
   cuttHipPackedClass cls[4];
+  cuttHipPackedOnce once;
   cuttHipMbar mbar;
 } cuttHipPackedArgs;
+
+/* Derive a->once from the other arguments, the table pointers included. */
+void cuttHipFinishPackedOnce(cuttHipPackedArgs* a);
 
 /* Work-item numbers of these arguments (some of them empty in order 1), or -1 if beyond 31 bits. */
 long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* args);

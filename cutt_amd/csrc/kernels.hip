@@ -43,6 +43,7 @@
 #include "line_windows.h"
 #include "mbar_decode.h"
 #include "packed_items.h"
+#include "packed_once.h"
 #include "row_blocks.h"
 #include "tile_order.h"
 
@@ -560,6 +561,48 @@ __global__ __launch_bounds__(1024, (kPackedMinWaves<T, E, WIDE>)) void packedKer
     w++;
     offOut = offOutNext;
   }
+}
+
+// One block per workgroup.
+template <typename T, int E, int NT>
+__global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ in, T* __restrict__ out, const unsigned char* __restrict__ tables, uint32_t chunk,
+                                                         uint32_t shifts, uint32_t items, uint32_t num0, uint32_t mul0, uint32_t num1, uint32_t mul1,
+                                                         uint32_t padThreads, const cuttHipPackedOnce a) {
+  extern __shared__ __align__(16) unsigned char ldsRaw[];
+  T* const tile = reinterpret_cast<T*>(ldsRaw);
+  uint32_t c, m, offIn, offOut;
+  if (!packedOnceSlabs(blockIdx.x, chunk, shifts, items, num0, mul0, num1, mul1, a, c, m, offIn, offOut)) return;
+  const uint32_t tid = threadIdx.x, nt = padThreads >> 8, padShift = padThreads & 31;
+  const cuttHipOnceClass k = a.cls[c];
+  // Lanes beyond the block's end repeat its last element (same addresses, same value).
+  uint32_t rowIn[E], rowOut[E], sh[E];
+  T v[E];
+#pragma unroll
+  for (int j = 0; j < E; j++) {
+    const uint32_t p = min(tid + j * nt, k.last), r = walkDivide(p, k.inMul, k.shifts & 31);
+    rowIn[j] = *reinterpret_cast<const uint32_t*>(tables + (k.rowIn + r * 4u)) + (p - r * k.inCont);
+  }
+#pragma unroll
+  for (int j = 0; j < E; j++) {
+    const uint32_t p = min(tid + j * nt, k.last), r = walkDivide(p, k.outMul, k.shifts >> 5);
+    sh[j] = *reinterpret_cast<const uint16_t*>(tables + (k.shIdx + p * 2u));
+    rowOut[j] = *reinterpret_cast<const uint32_t*>(tables + (k.rowOut + r * 4u)) + (p - r * k.outCont);
+  }
+  packedOnceMbar(a, m, offIn, offOut);
+  const unsigned char* const src = reinterpret_cast<const unsigned char*>(in + offIn);  // wave-uniform base, 32-bit byte offsets
+  unsigned char* const dst = reinterpret_cast<unsigned char*>(out + offOut);
+#pragma unroll
+  for (int j = 0; j < E; j++) v[j] = ldg<NT>(reinterpret_cast<const T*>(src + rowIn[j] * (uint32_t)sizeof(T)));
+#pragma unroll
+  for (int j = 0; j < E; j++) {
+    const uint32_t p = min(tid + j * nt, k.last);
+    tile[p + (p >> padShift)] = v[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < E; j++) v[j] = tile[sh[j]];
+#pragma unroll
+  for (int j = 0; j < E; j++) stg<NT>(reinterpret_cast<T*>(dst + rowOut[j] * (uint32_t)sizeof(T)), v[j]);
 }
 
 // The table must carry the division constants cuttHipFinishMbar derives from its extents.
@@ -1107,7 +1150,11 @@ extern "C" int cuttHipPreparePacked(void) {
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 0, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 1, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 2, true>, m);          \
-  if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, true>, m)
+  if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, true>, m);          \
+  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 0>, m);            \
+  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 1>, m);            \
+  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 2>, m);            \
+  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 3>, m)
     CUTT_ALLOW(uint32_t, 1); CUTT_ALLOW(uint32_t, 2); CUTT_ALLOW(uint32_t, 4); CUTT_ALLOW(uint32_t, 8);
     CUTT_ALLOW(uint32_t, 16);
     CUTT_ALLOW(uint64_t, 1); CUTT_ALLOW(uint64_t, 2); CUTT_ALLOW(uint64_t, 4); CUTT_ALLOW(uint64_t, 8);
@@ -1167,7 +1214,19 @@ extern "C" int cuttHipValidatePacked(const cuttHipPackedArgs* a) {
     if ((int)(last + (last >> a->padShift)) >= a->ldsElems) return (int)hipErrorInvalidValue;
   }
   if (packedGrid(a) == 0) return (int)hipErrorInvalidConfiguration;
+  if (a->once.blocks != 0) {  // must be what follows from the other arguments
+    cuttHipPackedArgs want = *a;
+    cuttHipFinishPackedOnce(&want);
+    if (std::memcmp(&want.once, &a->once, sizeof(want.once)) != 0 || want.once.blocks != packedGrid(a)) return (int)hipErrorInvalidValue;
+  }
   return 0;
+}
+
+template <typename T, int E, int NT>
+static int launchPackedOnce(const cuttHipPackedArgs& a, const void* in, void* out, hipStream_t s) {
+  const cuttHipPackedOnce& o = a.once;
+  return (int)launchKernel(packedOnceKernel<T, E, NT>, dim3(o.blocks), dim3(a.numThreads), cuttHipPackedLdsBytes(&a), s, (const T*)in, (T*)out,
+                           (const unsigned char*)a.cls[0].rowIn, o.chunk, o.shifts, o.items, o.num[0], o.mul[0], o.num[1], o.mul[1], o.padThreads, o);
 }
 
 extern "C" int cuttHipLaunchPacked(const cuttHipPackedArgs* a, const void* in, void* out, void* stream) {
@@ -1179,7 +1238,8 @@ extern "C" int cuttHipLaunchPacked(const cuttHipPackedArgs* a, const void* in, v
   const dim3 grid((uint32_t)blocks), block(a->numThreads);
   const bool wide = a->wideOffsets != 0;
 #define CUTT_LAUNCH_PACKED(T, E, NT)                                                                              \
-  return (int)(wide ? launchKernel(packedKernel<T, E, NT, true>, grid, block, lds, s, *a, (const T*)in, (T*)out)  \
+  return a->once.blocks ? launchPackedOnce<T, E, NT>(*a, in, out, s)                                              \
+                        : (int)(wide ? launchKernel(packedKernel<T, E, NT, true>, grid, block, lds, s, *a, (const T*)in, (T*)out)  \
                     : launchKernel(packedKernel<T, E, NT, false>, grid, block, lds, s, *a, (const T*)in, (T*)out))
 #define CUTT_LAUNCH_PACKED_NT(T, E)                            \
   switch (a->cachePolicy) {                                    \

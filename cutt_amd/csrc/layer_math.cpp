@@ -6,6 +6,7 @@
  */
 #include "hip_layer.h"
 
+#include <cstdint>
 #include <cstring>
 
 extern "C" cuttHipDivisor cuttHipMakeDivisor(uint32_t d) {
@@ -186,6 +187,68 @@ extern "C" void cuttHipFinishTileWalk(cuttHipTiledArgs* a) {
 
 extern "C" int cuttHipTiledTakesWalk(const cuttHipTiledArgs* a) {
   return a->walk.kind != 0 && a->lineWidth == 0 && (a->wide || (!a->grouped && !a->paced)) ? 1 : 0;
+}
+
+extern "C" void cuttHipFinishPackedOnce(cuttHipPackedArgs* a) {
+  cuttHipPackedOnce& o = a->once;
+  std::memset(&o, 0, sizeof(o));
+  // (positions of the last XCD's padding must stay below 2^31, the divisions' range)
+  const long long items = cuttHipPackedItemNumbers(a);
+  if (a->itemsPerBlock != 1 || a->wideOffsets || a->mbar.n < 0 || a->mbar.n > CUTT_ONCE_RANKS || a->xcdGroup < 0 || a->xcdGroup > 20 || items < 1) return;
+  unsigned long long blocks = (unsigned long long)items;
+  if (a->xcdGroup > 0) {
+    o.chunk = 1u << (a->xcdGroup - 1);
+    blocks = (blocks + 8ull * o.chunk - 1) / (8ull * o.chunk) * (8ull * o.chunk);
+  } else if (a->xcdChunk) {
+    o.chunk = a->xcdChunk;
+    if (8ull * o.chunk < blocks) return;
+    blocks = 8ull * o.chunk;
+  }
+  if (blocks > 0x7fffffffull) return;
+  o.items = (uint32_t)items;
+  uint32_t shift[2];
+  for (int i = 0; i < 2; i++) {
+    const cuttHipSplitRank& s = a->split[i];
+    o.num[i] = (uint32_t)s.numSplit;
+    walkDivisor(o.num[i], o.mul[i], shift[i]);
+    o.slab[i] = cuttHipOnceSlab{(uint32_t)s.slabRem, (uint32_t)s.slabFloor * s.strideIn, (uint32_t)s.slabFloor * s.strideOut, s.strideIn, s.strideOut};
+  }
+  o.shifts = shift[0] | shift[1] << 5 | (a->xcdGroup > 0 || a->xcdChunk ? 3u : 0u) << 15 | (uint32_t)a->xcdGroup << 17;
+  o.padThreads = (uint32_t)a->padShift | (uint32_t)a->numThreads << 8;
+  o.n = (uint32_t)a->mbar.n;
+  for (int k = 0; k < a->mbar.n; k++) {
+    cuttHipWalkRank& r = o.rank[k];
+    r.strideIn = a->mbar.d[k].strideIn;
+    r.strideOut = a->mbar.d[k].strideOut;
+    if (k + 1 == a->mbar.n) break;
+    r.extent = a->mbar.d[k].extent;
+    walkDivisor(r.extent, r.mul, r.shift);
+  }
+  const unsigned char* const first = (const unsigned char*)a->cls[0].rowIn;
+  for (int c = 0; c < 4; c++) {
+    if (((c & 1) && a->split[0].slabRem == 0) || ((c & 2) && a->split[1].slabRem == 0)) continue;
+    const cuttHipPackedClass& k = a->cls[c];
+    const void* const table[3] = {k.rowIn, k.rowOut, k.shIdx};
+    uint32_t at[3];
+    for (int i = 0; i < 3; i++) {
+      const uintptr_t d = (uintptr_t)table[i] - (uintptr_t)first;
+      if (!table[i] || d > 0x7fffffffu) return;  // (one piece of memory, class 0 first)
+      at[i] = (uint32_t)d;
+    }
+    if (k.vol < 1 || k.inCont < 1 || k.outCont < 1) return;
+    cuttHipOnceClass& w = o.cls[c];
+    uint32_t inShift = 0, outShift = 0;
+    walkDivisor((uint64_t)k.inCont, w.inMul, inShift);
+    walkDivisor((uint64_t)k.outCont, w.outMul, outShift);
+    w.last = (uint32_t)k.vol - 1;
+    w.inCont = (uint32_t)k.inCont;
+    w.outCont = (uint32_t)k.outCont;
+    w.shifts = inShift | outShift << 5;
+    w.rowIn = at[0];
+    w.rowOut = at[1];
+    w.shIdx = at[2];
+  }
+  o.blocks = (uint32_t)blocks;
 }
 
 extern "C" long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* a) {

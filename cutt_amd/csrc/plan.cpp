@@ -268,6 +268,7 @@ Plan Plan::clone() const {
     q.packed.cls[c].rowOut = nullptr;
     q.packed.cls[c].shIdx = nullptr;
   }
+  q.packed.once.blocks = 0;
   q.ldsBytes = ldsBytes;
   q.numBlocks = numBlocks;
   q.numThreads = numThreads;
@@ -287,6 +288,7 @@ void Plan::release() {
       packed.cls[c].rowOut = nullptr;
       packed.cls[c].shIdx = nullptr;
     }
+    packed.once.blocks = 0;
   }
 }
 
@@ -1764,6 +1766,7 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
     packed.cls[c].rowOut = b.rowOut;
     packed.cls[c].shIdx = b.shIdx;
   }
+  cuttHipFinishPackedOnce(&packed);
   if (int v = cuttHipValidatePacked(&packed); v != 0) return v;
   launchable = true;
   return 0;
@@ -1812,6 +1815,7 @@ int Plan::activate() {
     packed.cls[c].rowOut = (const uint32_t*)(base + off[c][1]);
     packed.cls[c].shIdx = (const uint16_t*)(base + off[c][2]);
   }
+  cuttHipFinishPackedOnce(&packed);
   if (int v = cuttHipValidatePacked(&packed); v != 0) {
     release();
     return v;

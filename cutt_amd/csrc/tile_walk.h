@@ -43,6 +43,13 @@ CUTT_DEVICE uint32_t walkMulHi(uint32_t a, uint32_t b) {
 // n / d for n < 2^31 (constants of cuttHipTileWalk).
 CUTT_DEVICE uint32_t walkDivide(uint32_t n, uint32_t mul, uint32_t shift) { return walkMulHi(2 * n, mul) >> shift; }
 
+// Workgroup index -> position: chunk and bits 15 and up of `shifts` as in cuttHipTileWalk.
+CUTT_DEVICE uint32_t walkPosition(uint32_t bid, uint32_t chunk, uint32_t shifts) {
+  const uint32_t xs = (shifts >> 15) & 3, g = ((shifts >> 17) - 1) & 31;  // 3: XCD b % 8 has positions of its own; in groups of 2^g (31: no groups)
+  const uint32_t q = bid >> xs;
+  return (bid & ((1u << xs) - 1)) * chunk + (q & ((1u << g) - 1)) + (((q >> g) << g) << 3);
+}
+
 // What every workgroup of a walk (cuttHipTileWalk) decodes its index with.
 struct WalkHead {
   uint32_t chunk, superM, stripMul, fullMul, lastMul, shifts;
@@ -58,9 +65,7 @@ struct NoMbar {};
 template <typename MB>
 CUTT_DEVICE bool walkTile(uint32_t bid, const WalkHead& h, const MB& mb, uint32_t tilesM, uint32_t tilesK, uint32_t& tm, uint32_t& tk, uint32_t& offIn, uint32_t& offOut) {
   constexpr bool kMbar = !std::is_same_v<MB, NoMbar>;
-  const uint32_t xs = (h.shifts >> 15) & 3, g = ((h.shifts >> 17) - 1) & 31;  // 3: XCD b % 8 has positions of its own; in groups of 2^g (31: no groups)
-  const uint32_t q = bid >> xs;
-  uint32_t l = (bid & ((1u << xs) - 1)) * h.chunk + (q & ((1u << g) - 1)) + (((q >> g) << g) << 3), m = 0, perStrip = tilesK;
+  uint32_t l = walkPosition(bid, h.chunk, h.shifts), m = 0, perStrip = tilesK;
   const uint32_t tiles = tilesM * tilesK;
   offIn = offOut = 0;
   if constexpr (kMbar) {

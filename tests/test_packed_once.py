@@ -1,0 +1,108 @@
+"""The packed kernel for one block per workgroup (cuttHipPackedOnce) against the arguments it is derived from.
+
+A C++ program decodes every workgroup index of random launches with the kernel's own code (packed_once.h, compiled for the host) and compares
+slab class and offsets with the work items' definition, and the class's constants with its tables and run lengths.
+"""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include <vector>
+#include "packed_once.h"
+typedef uint32_t u;
+#define CHECK(x) do { if (!(x)) { printf("failed: %s (launch %d)\n", #x, t); return 1; } } while (0)
+int main() {
+  std::mt19937 g(7);
+  auto r = [&](int lo, int hi) { return lo + (int)(g() % (unsigned)(hi - lo + 1)); };
+  static unsigned char mem[1 << 20];
+  long items = 0, classes = 0;
+  for (int t = 0; t < 3000; t++) {
+    cuttHipPackedArgs a; std::memset(&a, 0, sizeof(a));
+    a.elemSize = r(0, 1) ? 4 : 8; a.itemsPerBlock = 1; a.itemOrder = r(0, 2); a.numThreads = 64 * r(1, 16); a.padShift = r(0, 3) ? 5 : 31;
+    a.mbar.n = r(0, CUTT_ONCE_RANKS); a.volMbar = 1;
+    for (int k = 0; k < a.mbar.n; k++) {
+      a.mbar.d[k].extent = a.volMbar > 100 ? 1 : r(1, 7);
+      a.mbar.d[k].strideIn = g(); a.mbar.d[k].strideOut = g();
+      a.volMbar *= a.mbar.d[k].extent;
+    }
+    for (int i = 0; i < 2; i++) {
+      cuttHipSplitRank& s = a.split[i];
+      s.numSplit = r(0, 1) ? 1 : r(1, 30);
+      if (s.numSplit > 1) { s.slabFloor = r(1, 9); s.slabRem = r(0, 1) ? 0 : r(0, s.numSplit - 1); s.strideIn = g(); s.strideOut = g(); }
+    }
+    const long n = (long)a.volMbar * a.split[0].numSplit * a.split[1].numSplit;
+    if (r(0, 2)) a.xcdChunk = (u)((n + 7) / 8);
+    if (a.xcdChunk && r(0, 1)) a.xcdGroup = r(1, 6);
+    size_t at = 64 * r(0, 9);
+    for (int c = 0; c < 4; c++) {
+      if (((c & 1) && !a.split[0].slabRem) || ((c & 2) && !a.split[1].slabRem)) continue;
+      cuttHipPackedClass& k = a.cls[c];
+      k.inCont = r(1, 50); k.outCont = r(1, 50); k.vol = k.inCont * k.outCont * r(1, 20);
+      k.rowIn = (const u*)(mem + at); at += 16 * r(1, 9); k.rowOut = (const u*)(mem + at); at += 16 * r(1, 9); k.shIdx = (const uint16_t*)(mem + at); at += 16 * r(1, 9);
+    }
+    cuttHipFinishPackedOnce(&a);
+    const cuttHipPackedOnce& o = a.once;
+    CHECK(o.blocks > 0 && (o.padThreads & 31) == (u)a.padShift && (o.padThreads >> 8) == (u)a.numThreads);
+    const unsigned char* base = (const unsigned char*)a.cls[0].rowIn;
+    for (int c = 0; c < 4; c++) {
+      const cuttHipPackedClass& k = a.cls[c];
+      if (!k.vol) continue;
+      const cuttHipOnceClass& w = o.cls[c];
+      CHECK(w.last + 1 == (u)k.vol && w.inCont == (u)k.inCont && w.outCont == (u)k.outCont);
+      CHECK(base + w.rowIn == (const unsigned char*)k.rowIn && base + w.rowOut == (const unsigned char*)k.rowOut && base + w.shIdx == (const unsigned char*)k.shIdx);
+      for (u p = 0; p < 65536; p += 1 + g() % 97)
+        CHECK(cutt::walkDivide(p, w.inMul, w.shifts & 31) == p / w.inCont && cutt::walkDivide(p, w.outMul, w.shifts >> 5) == p / w.outCont);
+      classes++;
+    }
+    std::vector<char> seen(n, 0);
+    for (u b = 0; b < o.blocks; b++) {
+      u c, m, in, out;
+      const bool some = cutt::packedOnceSlabs(b, o.chunk, o.shifts, o.items, o.num[0], o.mul[0], o.num[1], o.mul[1], o, c, m, in, out);
+      u l = b;  // the comments of xcdChunk and xcdGroup
+      if (a.xcdGroup) { const u q = 1u << (a.xcdGroup - 1), turn = b / 8 / q; l = (turn * 8 + b % 8) * q + b / 8 % q; }
+      else if (a.xcdChunk) l = b % 8 * a.xcdChunk + b / 8;
+      CHECK(some == (l < (u)n));
+      if (!some) continue;
+      cutt::packedOnceMbar(o, m, in, out);
+      CHECK(!seen[l]); seen[l] = 1;
+      const u s0 = l % a.split[0].numSplit, s1 = l / a.split[0].numSplit % a.split[1].numSplit;
+      u mm = l / a.split[0].numSplit / a.split[1].numSplit, wantIn = 0, wantOut = 0;
+      const u s[2] = {s0, s1};
+      for (int i = 0; i < 2; i++) {
+        const cuttHipSplitRank& sr = a.split[i];
+        const u first = s[i] * sr.slabFloor + std::min<u>(s[i], sr.slabRem);
+        wantIn += first * sr.strideIn; wantOut += first * sr.strideOut;
+      }
+      for (int k = 0; k < a.mbar.n; k++) {
+        wantIn += mm % a.mbar.d[k].extent * a.mbar.d[k].strideIn; wantOut += mm % a.mbar.d[k].extent * a.mbar.d[k].strideOut;
+        mm /= a.mbar.d[k].extent;
+      }
+      CHECK(c == (s0 < (u)a.split[0].slabRem ? 1u : 0u) + (s1 < (u)a.split[1].slabRem ? 2u : 0u) && in == wantIn && out == wantOut);
+      items++;
+    }
+    for (char x : seen) CHECK(x);
+    // forms that stay with the general kernel
+    cuttHipPackedArgs b = a; b.itemsPerBlock = 2; cuttHipFinishPackedOnce(&b); CHECK(b.once.blocks == 0);
+    b = a; b.wideOffsets = 1; cuttHipFinishPackedOnce(&b); CHECK(b.once.blocks == 0);
+    b = a; b.mbar.n = CUTT_ONCE_RANKS + 1; cuttHipFinishPackedOnce(&b); CHECK(b.once.blocks == 0);
+    b = a; b.cls[0].shIdx = nullptr; cuttHipFinishPackedOnce(&b); CHECK(b.once.blocks == 0);
+  }
+  printf("ok %ld %ld\n", items, classes);
+  return 0;
+}
+"""
+
+
+def test_items_and_tables(tmp_path):
+    src = tmp_path / "once.cpp"
+    src.write_text(PROGRAM)
+    csrc = os.path.join(ROOT, "cutt_amd", "csrc")
+    exe = str(tmp_path / "once")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-include", "algorithm", "-I" + csrc, str(src), os.path.join(csrc, "layer_math.cpp"), "-o", exe])
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.startswith("ok"), out.stdout + out.stderr
