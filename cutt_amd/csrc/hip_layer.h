@@ -332,31 +332,34 @@ typedef struct cuttHipSplitRank {
 } cuttHipSplitRank;
 
 /*
- * What the packed kernel for one block per workgroup (itemsPerBlock 1) decodes its arguments from; derived from cuttHipPackedArgs
- * by cuttHipFinishPackedOnce.  Divisions as in cuttHipTileWalk.
+ * What the usual packed kernels decode a workgroup's blocks with; derived from cuttHipPackedArgs by cuttHipFinishPackedWalk.  Divisions as
+ * in cuttHipTileWalk.  Workgroup b, whose position is l (chunk and shifts, as there), moves the blocks i = 0, 1, ... < perGroup with the
+ * numbers n = l * first + i * stepN: slabs n % num[0] and n / num[0] % num[1], Mbar position n / num[0] / num[1] * mulM + i * stepM, as
+ * long as n < items and that position is below volMbar.
  */
-#define CUTT_ONCE_RANKS 12
-typedef struct cuttHipOnceClass {
+#define CUTT_PACKED_RANKS 12
+typedef struct cuttHipPackedWalkClass {
   uint32_t last, inCont, outCont;      /* elements of the block - 1, run lengths */
   uint32_t inMul, outMul, shifts;      /* divisions by the run lengths: in | out << 5 */
   uint32_t rowIn, rowOut, shIdx;       /* the class's tables, in bytes from the first one */
-} cuttHipOnceClass;
+} cuttHipPackedWalkClass;
 
-typedef struct cuttHipOnceSlab {
+typedef struct cuttHipPackedWalkSlab {
   uint32_t rem, stepIn, stepOut, strideIn, strideOut;  /* slab s starts s * step + min(s, rem) * stride into the tensor */
-} cuttHipOnceSlab;
+} cuttHipPackedWalkSlab;
 
-typedef struct cuttHipPackedOnce {
+typedef struct cuttHipPackedWalk {
   uint32_t blocks;                     /* workgroups of the launch; 0: the arguments are not of this form */
   uint32_t chunk, items;
   uint32_t num[2], mul[2];             /* slabs of the cut ranks and divisions by them */
   uint32_t shifts;                     /* division by num[0] | by num[1] << 5 | as in cuttHipTileWalk from bit 15 on */
   uint32_t padThreads;                 /* padShift | numThreads << 8 */
   uint32_t n;
-  cuttHipOnceSlab slab[2];
-  cuttHipWalkRank rank[CUTT_ONCE_RANKS];
-  cuttHipOnceClass cls[4];
-} cuttHipPackedOnce;
+  uint32_t perGroup, first, stepN, mulM, stepM, volMbar;
+  cuttHipPackedWalkSlab slab[2];
+  cuttHipWalkRank rank[CUTT_PACKED_RANKS];
+  cuttHipPackedWalkClass cls[4];
+} cuttHipPackedWalk;
 
 /*
  * Packed and PackedSplit methods.  A staged block is the index set Mmk with up to two of its
@@ -396,12 +399,12 @@ typedef struct cuttHipPackedArgs {
   int wideOffsets;     /* 0: the tensor is below 4 GB and the kernel keeps 32-bit byte offsets;
                           1: element offsets with 64-bit address arithmetic (required from 4 GB on) */
   cuttHipPackedClass cls[4];
-  cuttHipPackedOnce once;
+  cuttHipPackedWalk walk;
   cuttHipMbar mbar;
 } cuttHipPackedArgs;
 
-/* Derive a->once from the other arguments, the table pointers included. */
-void cuttHipFinishPackedOnce(cuttHipPackedArgs* a);
+/* Derive a->walk from the other arguments, the table pointers included. */
+void cuttHipFinishPackedWalk(cuttHipPackedArgs* a);
 
 /* Work-item numbers of these arguments (some of them empty in order 1), or -1 if beyond 31 bits. */
 long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* args);

@@ -43,7 +43,7 @@
 #include "line_windows.h"
 #include "mbar_decode.h"
 #include "packed_items.h"
-#include "packed_once.h"
+#include "packed_walk.h"
 #include "row_blocks.h"
 #include "tile_order.h"
 
@@ -563,17 +563,25 @@ __global__ __launch_bounds__(1024, (kPackedMinWaves<T, E, WIDE>)) void packedKer
   }
 }
 
-// One block per workgroup.
+// The usual packed kernels (cuttHipPackedWalk): below 4 GB, up to twelve Mbar ranks.  The arguments up to `padThreads`, 14 words, are in scalar
+// registers when a wave starts (the Makefile's kernarg-preload-count), the others are read at addresses known from the start, and
+// the table reads go out before the Mbar position is decoded: the kernel above waits for some ten reads, one after the other, before its first load.
+//
+// One block per workgroup.  Bound by latency up to some 10 MB per buffer, by memory and the table reads (three of them per element, from the L2)
+// beyond.  Against the kernel above, 100 tensors of 4-90 MB per buffer: 0.91 of the time in the mean, 0.73-1.05; (4,2,40,2,14,9,14)/(2,0,3,4,5,6,1),
+// 4 bytes, 4.6 -> 3.8 us; (24,32,16,36,9)/(4,1,3,2,0), 8 bytes, 12.9 -> 11.7; (13,509,1082)/(1,0,2), 4 bytes, 16.5 -> 12.0: 56
+// registers instead of 72 leave room for a second workgroup of 13 waves.  Tables with every lane's offsets ready, read 16 bytes at a time, are 5 %
+// faster below 6 MB and 2-20 % slower beyond (10 bytes per element from the L2); run tables read by the scalar unit 20 % slower there.
 template <typename T, int E, int NT>
 __global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ in, T* __restrict__ out, const unsigned char* __restrict__ tables, uint32_t chunk,
                                                          uint32_t shifts, uint32_t items, uint32_t num0, uint32_t mul0, uint32_t num1, uint32_t mul1,
-                                                         uint32_t padThreads, const cuttHipPackedOnce a) {
+                                                         uint32_t padThreads, const cuttHipPackedWalk a) {
   extern __shared__ __align__(16) unsigned char ldsRaw[];
   T* const tile = reinterpret_cast<T*>(ldsRaw);
   uint32_t c, m, offIn, offOut;
-  if (!packedOnceSlabs(blockIdx.x, chunk, shifts, items, num0, mul0, num1, mul1, a, c, m, offIn, offOut)) return;
+  if (!packedWalkSlabs<true>(walkPosition(blockIdx.x, chunk, shifts), 0, shifts, items, num0, mul0, num1, mul1, a, c, m, offIn, offOut)) return;
   const uint32_t tid = threadIdx.x, nt = padThreads >> 8, padShift = padThreads & 31;
-  const cuttHipOnceClass k = a.cls[c];
+  const cuttHipPackedWalkClass k = a.cls[c];
   // Lanes beyond the block's end repeat its last element (same addresses, same value).
   uint32_t rowIn[E], rowOut[E], sh[E];
   T v[E];
@@ -588,7 +596,7 @@ __global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ i
     sh[j] = *reinterpret_cast<const uint16_t*>(tables + (k.shIdx + p * 2u));
     rowOut[j] = *reinterpret_cast<const uint32_t*>(tables + (k.rowOut + r * 4u)) + (p - r * k.outCont);
   }
-  packedOnceMbar(a, m, offIn, offOut);
+  packedWalkMbar(a, m, offIn, offOut);
   const unsigned char* const src = reinterpret_cast<const unsigned char*>(in + offIn);  // wave-uniform base, 32-bit byte offsets
   unsigned char* const dst = reinterpret_cast<unsigned char*>(out + offOut);
 #pragma unroll
@@ -603,6 +611,108 @@ __global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ i
   for (int j = 0; j < E; j++) v[j] = tile[sh[j]];
 #pragma unroll
   for (int j = 0; j < E; j++) stg<NT>(reinterpret_cast<T*>(dst + rowOut[j] * (uint32_t)sizeof(T)), v[j]);
+}
+
+// Where the walk lies among the arguments of the kernel below: behind three pointers and eight words.
+constexpr uint32_t kPackedWalkAt = 3 * 8 + 8 * 4;
+static_assert(alignof(cuttHipPackedWalk) == 4, "no gap in front of it");
+
+// Several blocks per workgroup (4-byte elements beyond some 60 MB, where the table reads weigh most), in a software pipeline: a block's loads are issued before the LDS gather and the stores of the one before, so
+// they overlap, and the wait for them (the memory counter counts loads and stores in issue order) does not also wait for those stores to
+// complete.  Bound by memory.  Against packedKernel, 70 tensors of 90-700 MB per buffer: 0.7 % faster in the mean, (6,18,5,14,8,24,17)/(0,5,1,6,2,3,4), 4
+// bytes, 42.3 -> 39.2 us, (15,2842,3021)/(1,0,2), 4 bytes, 193 -> 188, (2,8,...) 8 bytes +2.6 % the worst.
+// (The instances with 8 elements per lane are held to the 72 and 80 registers that let seven and six of their waves share a SIMD.  64, and eight
+// waves, cost the 4-byte one 1 % in the mean over 70 tensors, up to 7 %: what is in flight then crowds the L2, which has to hold the lines
+// that neighbouring blocks complete.)
+template <typename T, int E>
+constexpr int kLoopMinWaves = E == 8 ? (sizeof(T) == 4 ? 7 : 6) : 1;
+
+template <typename T, int E, int NT>
+__global__ __launch_bounds__(1024, (kLoopMinWaves<T, E>)) void packedLoopKernel(const T* __restrict__ in, T* __restrict__ out, const unsigned char* __restrict__ tables, uint32_t chunk,
+                                                         uint32_t shifts, uint32_t items, uint32_t num0, uint32_t mul0, uint32_t num1, uint32_t mul1,
+                                                         uint32_t padThreads, const cuttHipPackedWalk a) {
+  extern __shared__ __align__(16) unsigned char ldsRaw[];
+  T* const tile = reinterpret_cast<T*>(ldsRaw);
+  const uint32_t tid = threadIdx.x, nt = padThreads >> 8, padShift = padThreads & 31;
+  const uint32_t first = walkPosition(blockIdx.x, chunk, shifts) * a.first;
+  uint32_t c, m, offIn, offOut;
+  if (!packedWalkSlabs<false>(first, 0, shifts, items, num0, mul0, num1, mul1, a, c, m, offIn, offOut)) return;
+  // Lanes beyond the block's end repeat its last element (same addresses, same value).
+  uint32_t rd[E], wr[E];  // byte offsets
+  uint32_t sh[(E + 1) / 2];  // LDS slots, two to a register
+  uint32_t last = 0;  // last element of the class whose data is being loaded
+  auto readSide = [&](uint32_t cls) __attribute__((always_inline)) {
+    const cuttHipPackedWalkClass k = a.cls[cls];
+    last = k.last;
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+      const uint32_t p = min(tid + j * nt, k.last), r = walkDivide(p, k.inMul, k.shifts & 31);
+      rd[j] = (*reinterpret_cast<const uint32_t*>(tables + (k.rowIn + r * 4u)) + (p - r * k.inCont)) * (uint32_t)sizeof(T);
+    }
+  };
+  auto writeSide = [&](uint32_t cls) __attribute__((always_inline)) {
+    const cuttHipPackedWalkClass k = a.cls[cls];
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+      const uint32_t p = min(tid + j * nt, k.last), r = walkDivide(p, k.outMul, k.shifts >> 5);
+      const uint32_t slot = *reinterpret_cast<const uint16_t*>(tables + (k.shIdx + p * 2u));
+      sh[j / 2] = j % 2 ? sh[j / 2] | slot << 16 : slot;
+      wr[j] = (*reinterpret_cast<const uint32_t*>(tables + (k.rowOut + r * 4u)) + (p - r * k.outCont)) * (uint32_t)sizeof(T);
+    }
+  };
+  T v[E];  // data on its way in: global memory -> registers -> LDS
+  auto request = [&](uint32_t off) __attribute__((always_inline)) {
+    const unsigned char* const src = reinterpret_cast<const unsigned char*>(in + off);
+#pragma unroll
+    for (int j = 0; j < E; j++) v[j] = ldg<NT>(reinterpret_cast<const T*>(src + rd[j]));
+  };
+  // (computed for every block from a value the compiler cannot see through, so that the slots do not take E more registers)
+  auto stage = [&]() __attribute__((always_inline)) {
+    uint32_t tv = tid;
+    asm volatile("" : "+v"(tv));
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+      const uint32_t p = min(tv + j * nt, last);
+      tile[p + (p >> padShift)] = v[j];
+    }
+  };
+  auto gatherAndStore = [&](uint32_t off) __attribute__((always_inline)) {
+    unsigned char* const dst = reinterpret_cast<unsigned char*>(out + off);
+    T u[E];
+#pragma unroll
+    for (int j = 0; j < E; j++) u[j] = tile[j % 2 ? sh[j / 2] >> 16 : sh[j / 2] & 0xffffu];
+#pragma unroll
+    for (int j = 0; j < E; j++) stg<NT>(reinterpret_cast<T*>(dst + wr[j]), u[j]);
+  };
+  readSide(c);
+  packedWalkMbar(a, m, offIn, offOut);
+  request(offIn);
+  writeSide(c);  // its latency hides behind the data's
+  stage();
+  for (uint32_t i = 1;; i++) {
+    // The arguments are read again for every block, from where the launch put them (the cache of the scalar unit, that is): kept, they take
+    // all scalar registers, and some to memory.
+    typedef const __attribute__((address_space(4))) unsigned char* KernelArguments;
+    KernelArguments args = (KernelArguments)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const auto& w = *reinterpret_cast<const __attribute__((address_space(4))) cuttHipPackedWalk*>(args + kPackedWalkAt);
+    uint32_t next, offInNext, offOutNext;
+    if (i >= w.perGroup || !packedWalkSlabs<false>(first + i * w.stepN, i, shifts, items, num0, mul0, num1, mul1, w, next, m, offInNext, offOutNext)) break;
+    packedWalkMbar(w, m, offInNext, offOutNext);
+    if (next != c) readSide(next);  // (wave-uniform; at most a few times per workgroup)
+    request(offInNext);
+    __syncthreads();  // the block is complete in LDS
+    gatherAndStore(offOut);
+    if (next != c) {
+      writeSide(next);
+      c = next;
+    }
+    __syncthreads();  // every lane has taken its elements out
+    stage();
+    offOut = offOutNext;
+  }
+  __syncthreads();
+  gatherAndStore(offOut);
 }
 
 // The table must carry the division constants cuttHipFinishMbar derives from its extents.
@@ -1152,8 +1262,12 @@ extern "C" int cuttHipPreparePacked(void) {
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 2, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, true>, m);          \
   if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 0>, m);            \
+  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 0>, m);            \
   if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 1>, m);            \
+  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 1>, m);            \
   if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 2>, m);            \
+  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 2>, m);            \
+  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 3>, m);            \
   if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 3>, m)
     CUTT_ALLOW(uint32_t, 1); CUTT_ALLOW(uint32_t, 2); CUTT_ALLOW(uint32_t, 4); CUTT_ALLOW(uint32_t, 8);
     CUTT_ALLOW(uint32_t, 16);
@@ -1214,18 +1328,18 @@ extern "C" int cuttHipValidatePacked(const cuttHipPackedArgs* a) {
     if ((int)(last + (last >> a->padShift)) >= a->ldsElems) return (int)hipErrorInvalidValue;
   }
   if (packedGrid(a) == 0) return (int)hipErrorInvalidConfiguration;
-  if (a->once.blocks != 0) {  // must be what follows from the other arguments
+  if (a->walk.blocks != 0) {  // must be what follows from the other arguments
     cuttHipPackedArgs want = *a;
-    cuttHipFinishPackedOnce(&want);
-    if (std::memcmp(&want.once, &a->once, sizeof(want.once)) != 0 || want.once.blocks != packedGrid(a)) return (int)hipErrorInvalidValue;
+    cuttHipFinishPackedWalk(&want);
+    if (std::memcmp(&want.walk, &a->walk, sizeof(want.walk)) != 0 || want.walk.blocks != packedGrid(a)) return (int)hipErrorInvalidValue;
   }
   return 0;
 }
 
 template <typename T, int E, int NT>
-static int launchPackedOnce(const cuttHipPackedArgs& a, const void* in, void* out, hipStream_t s) {
-  const cuttHipPackedOnce& o = a.once;
-  return (int)launchKernel(packedOnceKernel<T, E, NT>, dim3(o.blocks), dim3(a.numThreads), cuttHipPackedLdsBytes(&a), s, (const T*)in, (T*)out,
+static int launchPackedWalk(const cuttHipPackedArgs& a, const void* in, void* out, hipStream_t s) {
+  const cuttHipPackedWalk& o = a.walk;
+  return (int)launchKernel(o.perGroup > 1 ? packedLoopKernel<T, E, NT> : packedOnceKernel<T, E, NT>, dim3(o.blocks), dim3(a.numThreads), cuttHipPackedLdsBytes(&a), s, (const T*)in, (T*)out,
                            (const unsigned char*)a.cls[0].rowIn, o.chunk, o.shifts, o.items, o.num[0], o.mul[0], o.num[1], o.mul[1], o.padThreads, o);
 }
 
@@ -1238,7 +1352,7 @@ extern "C" int cuttHipLaunchPacked(const cuttHipPackedArgs* a, const void* in, v
   const dim3 grid((uint32_t)blocks), block(a->numThreads);
   const bool wide = a->wideOffsets != 0;
 #define CUTT_LAUNCH_PACKED(T, E, NT)                                                                              \
-  return a->once.blocks ? launchPackedOnce<T, E, NT>(*a, in, out, s)                                              \
+  return a->walk.blocks ? launchPackedWalk<T, E, NT>(*a, in, out, s)                                              \
                         : (int)(wide ? launchKernel(packedKernel<T, E, NT, true>, grid, block, lds, s, *a, (const T*)in, (T*)out)  \
                     : launchKernel(packedKernel<T, E, NT, false>, grid, block, lds, s, *a, (const T*)in, (T*)out))
 #define CUTT_LAUNCH_PACKED_NT(T, E)                            \

@@ -189,13 +189,18 @@ extern "C" int cuttHipTiledTakesWalk(const cuttHipTiledArgs* a) {
   return a->walk.kind != 0 && a->lineWidth == 0 && (a->wide || (!a->grouped && !a->paced)) ? 1 : 0;
 }
 
-extern "C" void cuttHipFinishPackedOnce(cuttHipPackedArgs* a) {
-  cuttHipPackedOnce& o = a->once;
+extern "C" void cuttHipFinishPackedWalk(cuttHipPackedArgs* a) {
+  cuttHipPackedWalk& o = a->walk;
   std::memset(&o, 0, sizeof(o));
-  // (positions of the last XCD's padding must stay below 2^31, the divisions' range)
-  const long long items = cuttHipPackedItemNumbers(a);
-  if (a->itemsPerBlock != 1 || a->wideOffsets || a->mbar.n < 0 || a->mbar.n > CUTT_ONCE_RANKS || a->xcdGroup < 0 || a->xcdGroup > 20 || items < 1) return;
-  unsigned long long blocks = (unsigned long long)items;
+  const long long numbers = cuttHipPackedItemNumbers(a);
+  // (a loop over blocks of few elements per lane is slower this way: (5,4,1374779)/(1,0,2), 8 bytes, one element per lane, 212 -> 254 us)
+  if (a->itemsPerBlock > 1 && a->elemsPerThread < 4) return;
+  if (a->itemsPerBlock < 1 || a->wideOffsets || a->mbar.n < 0 || a->mbar.n > CUTT_PACKED_RANKS || a->xcdGroup < 0 || a->xcdGroup > 20 || numbers < 1) return;
+  const unsigned long long per = (unsigned long long)a->itemsPerBlock, groups = ((unsigned long long)numbers + per - 1) / per;
+  unsigned long long blocks = groups;
+  o.perGroup = (uint32_t)per;
+  o.volMbar = (uint32_t)a->volMbar;
+  o.first = o.stepN = o.mulM = 1;
   if (a->xcdGroup > 0) {
     o.chunk = 1u << (a->xcdGroup - 1);
     blocks = (blocks + 8ull * o.chunk - 1) / (8ull * o.chunk) * (8ull * o.chunk);
@@ -204,14 +209,27 @@ extern "C" void cuttHipFinishPackedOnce(cuttHipPackedArgs* a) {
     if (8ull * o.chunk < blocks) return;
     blocks = 8ull * o.chunk;
   }
-  if (blocks > 0x7fffffffull) return;
-  o.items = (uint32_t)items;
+  // (the divisions are of numbers below 2^31; those of padding workgroups only have to stay below 2^32)
+  if (blocks > 0x7fffffffull || blocks * per > 0xffffffffull) return;
+  o.items = (uint32_t)numbers;
+  if (a->itemOrder == 1) {  // the workgroup keeps its slabs
+    o.items = (uint32_t)groups;
+    o.stepN = 0;
+    o.mulM = (uint32_t)per;
+    o.stepM = 1;
+  } else if (a->itemOrder == 2) {  // the workgroups of a chunk take its blocks in turn
+    const bool chunks = a->xcdChunk && !a->xcdGroup;
+    o.stepN = chunks ? o.chunk : (uint32_t)blocks;
+    if (chunks) o.chunk *= o.perGroup;
+  } else {
+    o.first = (uint32_t)per;
+  }
   uint32_t shift[2];
   for (int i = 0; i < 2; i++) {
     const cuttHipSplitRank& s = a->split[i];
     o.num[i] = (uint32_t)s.numSplit;
     walkDivisor(o.num[i], o.mul[i], shift[i]);
-    o.slab[i] = cuttHipOnceSlab{(uint32_t)s.slabRem, (uint32_t)s.slabFloor * s.strideIn, (uint32_t)s.slabFloor * s.strideOut, s.strideIn, s.strideOut};
+    o.slab[i] = cuttHipPackedWalkSlab{(uint32_t)s.slabRem, (uint32_t)s.slabFloor * s.strideIn, (uint32_t)s.slabFloor * s.strideOut, s.strideIn, s.strideOut};
   }
   o.shifts = shift[0] | shift[1] << 5 | (a->xcdGroup > 0 || a->xcdChunk ? 3u : 0u) << 15 | (uint32_t)a->xcdGroup << 17;
   o.padThreads = (uint32_t)a->padShift | (uint32_t)a->numThreads << 8;
@@ -236,7 +254,7 @@ extern "C" void cuttHipFinishPackedOnce(cuttHipPackedArgs* a) {
       at[i] = (uint32_t)d;
     }
     if (k.vol < 1 || k.inCont < 1 || k.outCont < 1) return;
-    cuttHipOnceClass& w = o.cls[c];
+    cuttHipPackedWalkClass& w = o.cls[c];
     uint32_t inShift = 0, outShift = 0;
     walkDivisor((uint64_t)k.inCont, w.inMul, inShift);
     walkDivisor((uint64_t)k.outCont, w.outMul, outShift);

@@ -268,7 +268,7 @@ Plan Plan::clone() const {
     q.packed.cls[c].rowOut = nullptr;
     q.packed.cls[c].shIdx = nullptr;
   }
-  q.packed.once.blocks = 0;
+  q.packed.walk.blocks = 0;
   q.ldsBytes = ldsBytes;
   q.numBlocks = numBlocks;
   q.numThreads = numThreads;
@@ -288,7 +288,7 @@ void Plan::release() {
       packed.cls[c].rowOut = nullptr;
       packed.cls[c].shIdx = nullptr;
     }
-    packed.once.blocks = 0;
+    packed.walk.blocks = 0;
   }
 }
 
@@ -1766,7 +1766,7 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
     packed.cls[c].rowOut = b.rowOut;
     packed.cls[c].shIdx = b.shIdx;
   }
-  cuttHipFinishPackedOnce(&packed);
+  cuttHipFinishPackedWalk(&packed);
   if (int v = cuttHipValidatePacked(&packed); v != 0) return v;
   launchable = true;
   return 0;
@@ -1815,7 +1815,7 @@ int Plan::activate() {
     packed.cls[c].rowOut = (const uint32_t*)(base + off[c][1]);
     packed.cls[c].shIdx = (const uint16_t*)(base + off[c][2]);
   }
-  cuttHipFinishPackedOnce(&packed);
+  cuttHipFinishPackedWalk(&packed);
   if (int v = cuttHipValidatePacked(&packed); v != 0) {
     release();
     return v;
