@@ -258,6 +258,17 @@ void setCachePolicy(Plan& p, int policy, const cuttHipDeviceProps& props) {
   choosePacing(p, props, plannerOptions(0));
 }
 
+// Whether a plan (no copy, no line-aligned stores) stores past the caches, for tensors that are not kept in the memory-side cache as a whole:
+// chooseCachePolicy.
+bool storesPastCaches(const Plan& p, const cuttHipDeviceProps& props) {
+  const double bytes = (double)p.pb.volume * p.pb.elemSize, cache = (double)props.infinityCacheBytes;
+  if (cache > 0 && 2.0 * bytes <= (p.method == kTiledCopy ? cache : cache / 3)) return false;
+  const bool packed = p.method == kPacked || p.method == kPackedSplit;
+  double partial = 0.01;
+  if (packed && bytes <= cache) partial = bytes <= cache / 3 ? 2.0 : (2.0 * bytes <= cache ? 0.16 : 0.04);
+  return p.model.wrPartialLines <= partial * bytes / 128.0;
+}
+
 // Cache policy of a plan's global accesses, from its size and the model's sampled address stream.  (Not applied when
 // CUTT_CACHE_POLICY pins the policy.)  Timed on 120 random tensors of 0.14-1.6 GB per buffer, buffers in rotation and
 // the same ones again and again (the smaller ones: 0.03-0.14 GB):
@@ -293,8 +304,7 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
   if (std::getenv("CUTT_CACHE_POLICY")) return;
   const double bytes = (double)p.pb.volume * p.pb.elemSize;
   const double cache = (double)props.infinityCacheBytes;
-  const bool copies = p.method == kTrivial || p.method == kTiledCopy;
-  if (cache > 0 && 2.0 * bytes <= (copies ? cache : cache / 3)) {
+  if (cache > 0 && 2.0 * bytes <= (p.method == kTrivial ? cache : cache / 3)) {
     setCachePolicy(p, 0, props);
     return;
   }
@@ -307,10 +317,7 @@ void chooseCachePolicy(Plan& p, const cuttHipDeviceProps& props) {
     setCachePolicy(p, bytes <= 3.5 * cache ? 1 : 3, props);
     return;
   }
-  const bool packed = p.method == kPacked || p.method == kPackedSplit;
-  double partial = 0.01;
-  if (packed && bytes <= cache) partial = bytes <= cache / 3 ? 2.0 : (2.0 * bytes <= cache ? 0.16 : 0.04);
-  if (p.model.wrPartialLines <= partial * lines) {
+  if (storesPastCaches(p, props)) {
     setCachePolicy(p, bytes > cache && p.model.rdLines <= 1.02 * lines ? 3 : 2, props);
     return;
   }
@@ -552,6 +559,14 @@ bool estimateAndTune(Plan& p, const cuttHipDeviceProps& props) {
   if (!estimatePlan(p, props, 10)) return false;
   chooseTiledGrouping(p, props);
   if (lineWindowsPay(p, props)) p.model.usPredicted *= 0.92;
+  // The model's constants stem from plans whose stores all went through the caches up to half of the memory-side one.  450 tensors of 45-134 MB per buffer, forced to each method: packed plans that store past the caches ran at 0.72-0.78 of
+  // their estimates (buffers in rotation; 0.92 on new ones), Tiled plans with partly written lines at 0.93-1.0.  With 0.87, up to 100 MB, a fifth
+  // of the plans change: 7 % faster in rotation, the same on 4 GB of buffers, 1 % faster on inputs just written, 3.5 % with kernels before and behind.
+  const double bytes = (double)p.pb.volume * p.pb.elemSize, cache = (double)props.infinityCacheBytes;
+  const bool rows = p.method == kTiledCopy && p.tcopy.rowGather;  // (gathered rows store past the caches at every size: as they stood to packed plans)
+  const bool blocks = (p.method == kTiled && p.tiled.lineWidth == 0) || p.method == kPacked || p.method == kPackedSplit;
+  if (rows ? 2.0 * bytes <= cache / 3 : !blocks || lineWindowsPay(p, props) || !storesPastCaches(p, props)) return true;
+  if (bytes <= 0.375 * cache) p.model.usPredicted *= 0.87;
   return true;
 }
 
@@ -600,13 +615,24 @@ void refineMbarOrder(std::vector<Plan>& plans, const cuttHipDeviceProps& props, 
 
 // Index of the candidate with the smallest predicted time; Trivial always wins and ties go to
 // the later candidate (reference src/cuttplan.cpp:700-768).
-int chooseHeuristic(const std::vector<Plan>& plans) {
-  int best = -1;
+//
+// A packed plan gives way to the best Tiled one, beyond half a cache size, if that writes whole lines, in 64x64 tiles whose order is no
+// numbering by address bits, and is not estimated 1.18 (4 bytes) or 1.1 times as long: the model's constants stem from plans whose workgroups the
+// XCDs took in chunks, and in groups such Tiled plans run at 0.89 and 0.93 of their estimates (130 tensors), packed ones at 0.95.  2 % of 1600 tensors
+// change their plan for it, 5 % faster in the mean: (8,4,262144,24)/(2,1,3,0), 4 bytes, 302 -> 249 us; (6,17,8,156,32,9)/(2,3,0,1,4,5), 4 bytes, 52 -> 55.
+int chooseHeuristic(const std::vector<Plan>& plans, const cuttHipDeviceProps& props) {
+  int best = -1, tiled = -1;
   for (int i = 0; i < (int)plans.size(); i++) {
     if (plans[i].method == kTrivial) return i;
     if (best < 0 || plans[i].model.usPredicted <= plans[best].model.usPredicted) best = i;
+    if (plans[i].method == kTiled && (tiled < 0 || plans[i].model.usPredicted <= plans[tiled].model.usPredicted)) tiled = i;
   }
-  return best;
+  if (best < 0 || tiled < 0 || (plans[best].method != kPacked && plans[best].method != kPackedSplit)) return best;
+  const Plan& t = plans[tiled];
+  if (2.0 * (double)t.pb.volume * t.pb.elemSize <= (double)props.infinityCacheBytes || t.tiled.lineWidth > 0 || t.tiled.order == 7 ||
+      lineWindowsPay(t, props) || !storesPastCaches(t, props))
+    return best;
+  return t.model.usPredicted <= (t.pb.elemSize == 4 ? 1.18 : 1.1) * plans[best].model.usPredicted ? tiled : best;
 }
 
 PlannerOptions plannerOptions(int forceMethod) {
@@ -717,7 +743,7 @@ static cuttResult decideHeuristically(int rank, int* dim, int* permutation, size
   if (!enumerate(rank, dim, permutation, sizeofType, props, force, plans)) return CUTT_INTERNAL_ERROR;
   if (!estimateAll(plans, props)) return CUTT_INTERNAL_ERROR;
   refineMbarOrder(plans, props, force);
-  const int best = chooseHeuristic(plans);
+  const int best = chooseHeuristic(plans, props);
   if (best < 0) return CUTT_INTERNAL_ERROR;
   finishPlan(plans[best], props);
   if (useCache) planCacheInsert(key, plans[best], (int)plans.size());
@@ -775,7 +801,7 @@ static cuttResult planLarge(cuttHandle* handle, int rank, int* dim, int* permuta
       if (!createPlans(shape, shape, props, plannerOptions(force), plans) || plans.empty()) return CUTT_INTERNAL_ERROR;
       if (!estimateAll(plans, props)) return CUTT_INTERNAL_ERROR;
       refineMbarOrder(plans, props, force);
-      const int best = chooseHeuristic(plans);
+      const int best = chooseHeuristic(plans, props);
       if (best < 0) return CUTT_INTERNAL_ERROR;
       finishPlan(plans[best], props);
       if (s == 0) numCandidates = (int)plans.size();
@@ -1156,7 +1182,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
     std::vector<Plan> again;
     if (createPlans(orig, red, props, plannerOptions(force), again) && !again.empty() && estimateAll(again, props)) {
       refineMbarOrder(again, props, force);
-      const int h = chooseHeuristic(again);
+      const int h = chooseHeuristic(again, props);
       if (h >= 0 && again[h].method != kTrivial) {
         finishPlan(again[h], props);
         Plan heur = std::move(again[h]);
@@ -1420,7 +1446,7 @@ extern "C" void* cuttCandidatesCreateEx(int rank, const int* dim, const int* per
     if (ldsPerBlock) props.ldsPerBlock = props.ldsPerCU = ldsPerBlock;
     if (!enumerate(rank, dim, permutation, sizeofType, props, force, l->plans)) return nullptr;
     if (!estimateAll(l->plans, props)) return nullptr;
-    l->best = chooseHeuristic(l->plans);
+    l->best = chooseHeuristic(l->plans, props);
     return l.release();
   } catch (...) {  // nothing may cross the C boundary
     return nullptr;
@@ -1444,7 +1470,7 @@ extern "C" void* cuttCandidatesCreateStrided(int rank, const int* dim, const int
     cuttHipDeviceProps props = defaultMI355XProps();
     if (ldsPerBlock) props.ldsPerBlock = props.ldsPerCU = ldsPerBlock;
     if (!createPlans(pb, pb, props, plannerOptions(force), l->plans) || !estimateAll(l->plans, props)) return nullptr;
-    l->best = chooseHeuristic(l->plans);
+    l->best = chooseHeuristic(l->plans, props);
     return l.release();
   } catch (...) {  // nothing may cross the C boundary
     return nullptr;

@@ -1549,16 +1549,17 @@ void addPackedSplit(const Problem& pb, bool fromReduced, const cuttHipDeviceProp
       if (!any) break;
     }
   }
-  // Batches of small blocks: the slowest rank is the same on both sides, and what the others make is no more than 512 elements.  Several of
-  // these blocks, staged together, are one contiguous run on either side; one by one they leave lanes idle and lines partly written.  60 such
+  // Batches of small blocks: the slowest rank is the same on both sides, and the others make a block of which several fit a workgroup.  Staged
+  // together they are one contiguous run on either side; one by one they leave lanes idle and lines partly written.  60 such
   // tensors of 5-500 MB: 0.68 of the time in the mean, (2,2,10000000)/(1,0,2), 8 bytes, 1202 -> 104 us, (5,4,1374779)/(1,0,2), 8 bytes, 212 ->
-  // 74, (9,3,5,222222)/(2,1,0,3), 4 bytes, 84 -> 45; blocks of more elements take the same plans as before or gain nothing.
+  // 74, (9,3,5,222222)/(2,1,0,3), 4 bytes, 84 -> 45.  From 512 elements on, where little is left to gain, one size: (3,174,134555)/(1,0,2), 8 bytes,
+  // 228 -> 192, (15,54,2,85943)/(2,1,0,3), 4 bytes, 211 -> 200.
   const int last = pb.rank - 1;
   if (pb.perm[last] == last && pb.dense) {
     const int64_t below = pb.volume / pb.dim[last];
     for (int64_t t : targets) {
       const int ns = slabCount(pb.dim[last], t / below, below, pb.elemSize);
-      if (below <= 512 && t / below >= 2 && ns >= 2) tryPackedSplit(pb, fromReduced, props, opt, pb.rank, 1, last, ns, -1, 1, plans);
+      if ((below <= 512 || t == targets[1]) && t / below >= 2 && ns >= 2) tryPackedSplit(pb, fromReduced, props, opt, pb.rank, 1, last, ns, -1, 1, plans);
     }
   }
 }

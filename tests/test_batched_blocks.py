@@ -27,8 +27,9 @@ def test_where_they_exist(cutt):
         below = math.prod(dim[:-1])
         found = stretches(cutt, dim, perm, 8)
         assert found and all(i.volMmkInCont == i.volMmkOutCont >= 2 * below and i.volMbar == 1 for i in found)
+    assert len(stretches(cutt, (27, 19, 997), (1, 0, 2), 8)) == 1  # (one size only)
     # a slowest rank that moves, larger blocks, too few of them
-    for dim, perm in (((5, 4097, 4), (1, 0, 2)[::-1]), ((27, 19, 997), (1, 0, 2)), ((5, 4, 3), (1, 0, 2))):
+    for dim, perm in (((5, 4097, 4), (1, 0, 2)[::-1]), ((47, 49, 997), (1, 0, 2)), ((5, 4, 3), (1, 0, 2))):
         assert not stretches(cutt, dim, perm, 8)
 
 

@@ -108,6 +108,15 @@ def test_cache_policy_of_tensors_up_to_half_a_cache_size(planner, dim, perm, es,
     assert info.cachePolicy == policy, (info.method, info.wrPartialLines / (size / 128))
 
 
+def test_packed_plans_give_way_to_tiles_that_write_whole_lines(planner):
+    # beyond half a cache size, up to the margin; partly written lines, numberings by address bits, smaller tensors
+    assert planner.plan((8, 4, 262144, 24), (2, 1, 3, 0), 4).method == TILED
+    tiled, packed = (planner.plan((8, 4, 262144, 24), (2, 1, 3, 0), 4, m).usPredicted for m in (TILED, 3))
+    assert packed < tiled < 1.18 * packed
+    assert planner.plan((8, 4, 26214, 24), (2, 1, 3, 0), 4).method != TILED
+    assert planner.plan((5, 7, 11, 13, 17, 1093), (4, 2, 0, 5, 1, 3), 4).method != TILED
+
+
 def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
     # (counted as tiles of 64 elements they seem to issue a quarter of the requests)
     for dim, perm in (((8192, 8192), (1, 0)), ((4096, 256, 64), (1, 0, 2)), ((256, 400, 512), (2, 1, 0))):
