@@ -519,13 +519,14 @@ bool wideForm(const Plan& p, const cuttHipDeviceProps& props, Plan& q) {
   return true;
 }
 
-// 8-byte elements, blocks of 10 KB and more: one per workgroup.  More of them saved the kernel's way to its first load, which is short now, and a share
-// of the table reads, which weigh less than with 4-byte elements; one each evens out the end of the launch.  99 such plans of 90-800 MB per
-// buffer, two blocks before: 1.2 % faster in the mean, 8 % at best, 4 % slower at worst.  (4-byte elements, four blocks before: 4 % slower in the
+// 8-byte elements, blocks of 10 KB and more, up to twelve waves: one per workgroup.  More of them saved the kernel's way to its first load, which
+// is short now, and a share of the table reads, which weigh less than with 4-byte elements; one each evens out the end of the launch.  69 such plans of
+// 90-800 MB per buffer, two blocks before: 1.5 % faster in the mean, 8 % at best, 3 % slower at worst; 30 of 13-16 waves 0.5 %, but 4-5 % slower at
+// worst ((51,960,3,13,4,2,6,2)/(7,6,0,4,2,5,1,3) 537 -> 557 us).  (4-byte elements, four blocks before: 4 % slower in the
 // mean, 45 % at worst.)  Not applied when an option pins the number or the order.
 void oneBlockPerWorkgroup(Plan& p, const PlannerOptions& opt) {
   cuttHipPackedArgs& a = p.packed;
-  if ((p.method != kPacked && p.method != kPackedSplit) || a.itemsPerBlock == 1 || a.elemSize != 8 || a.elemsPerThread != 8 || p.ldsBytes < 10 * 1024 || a.wideOffsets ||
+  if ((p.method != kPacked && p.method != kPackedSplit) || a.itemsPerBlock == 1 || a.elemSize != 8 || a.elemsPerThread != 8 || p.ldsBytes < 10 * 1024 || a.numThreads > 768 || a.wideOffsets ||
       a.mbar.n > CUTT_PACKED_RANKS || opt.maxItemsPerBlock > 0 || opt.packedRounds > 0 || opt.itemOrder >= 0)
     return;
   cuttHipPackedArgs one = a;
