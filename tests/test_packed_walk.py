@@ -23,7 +23,7 @@ int main() {
   long items = 0, classes = 0;
   for (int t = 0; t < 3000; t++) {
     cuttHipPackedArgs a; std::memset(&a, 0, sizeof(a));
-    a.elemSize = r(0, 1) ? 4 : 8; a.elemsPerThread = 4; a.itemsPerBlock = r(0, 1) ? 1 : r(2, 9); a.itemOrder = r(0, 2); a.numThreads = 64 * r(1, 16); a.padShift = r(0, 3) ? 5 : 31;
+    a.elemSize = r(0, 1) ? 4 : 8; a.elemsPerThread = 4; a.itemsPerBlock = r(0, 1) ? 1 : r(2, 9); a.itemOrder = r(0, 2); a.numThreads = 64 * r(1, a.elemSize == 8 && a.itemsPerBlock > 1 ? 12 : 16); a.padShift = r(0, 3) ? 5 : 31;
     a.mbar.n = r(0, CUTT_PACKED_RANKS); a.volMbar = 1;
     for (int k = 0; k < a.mbar.n; k++) {
       a.mbar.d[k].extent = a.volMbar > 100 ? 1 : r(1, 7);
@@ -108,6 +108,7 @@ int main() {
     }
     for (char x : seen) CHECK(x);
     // forms that stay with the general kernel
+    if (a.elemSize == 8 && a.itemsPerBlock > 1) { cuttHipPackedArgs b = a; b.numThreads = 832; cuttHipFinishPackedWalk(&b); CHECK(b.walk.blocks == 0); }
     cuttHipPackedArgs b = a; b.itemsPerBlock = 3; b.elemsPerThread = 2; cuttHipFinishPackedWalk(&b); CHECK(b.walk.blocks == 0);
     b = a; b.wideOffsets = 1; cuttHipFinishPackedWalk(&b); CHECK(b.walk.blocks == 0);
     b = a; b.mbar.n = CUTT_PACKED_RANKS + 1; cuttHipFinishPackedWalk(&b); CHECK(b.walk.blocks == 0);
