@@ -469,7 +469,7 @@ int cuttHipLaunchTiled(const cuttHipTiledArgs* args, const void* in, void* out, 
 int cuttHipLaunchTiledCopy(const cuttHipTiledCopyArgs* args, const void* in, void* out, void* stream);
 int cuttHipLaunchPacked(const cuttHipPackedArgs* args, const void* in, void* out, void* stream);
 /*
- * Index tables of one slab class built on the device (for callers that may not allocate or copy):
+ * Index tables of a slab class built on the device (for callers that may not allocate or copy):
  * entry i of table l is the mixed-radix sum over list[l] (first entry fastest) of index * stride;
  * l = 0 fills rowIn (count[0] entries), l = 1 rowOut (count[1]), l = 2 the LDS gather slots
  * (count[2] entries, stored as position + (position >> padShift)).
@@ -489,7 +489,8 @@ typedef struct cuttHipTableBuildArgs {
   uint16_t* shIdx;
 } cuttHipTableBuildArgs;
 
-int cuttHipLaunchTableBuild(const cuttHipTableBuildArgs* args, void* stream);
+/* The tables of a plan's slab classes, 1 ... 4 of them: one launch where their lists allow it. */
+int cuttHipLaunchTableBuilds(const cuttHipTableBuildArgs* args, int classes, void* stream);
 
 /*
  * The library's static scratch memory on the current device (a __device__ array in the code

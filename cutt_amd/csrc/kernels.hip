@@ -1174,6 +1174,10 @@ struct BuildLists {
   int padShift;
   BuildRank rank[3][RANKS];
 };
+template <int RANKS, int CLASSES>
+struct BuildClasses {
+  BuildLists<RANKS> cls[CLASSES];
+};
 
 template <int RANKS>
 __device__ __forceinline__ uint32_t radixSum(const BuildRank (&r)[RANKS], uint32_t i) {
@@ -1190,8 +1194,11 @@ __device__ __forceinline__ uint32_t radixSum(const BuildRank (&r)[RANKS], uint32
 // Bound by the dispatch (1.8 us) and what one lane computes in turn.  With a division by a variable per rank and list, each waiting
 // for the one before and for its extent, a call with such a build took 16.5 us on
 // (24,32,16,36,9)/(4,1,3,2,0), 8 bytes (the transpose itself 13.0), 15.4 with these; (12,13,14,15,16)/(4,3,2,1,0), 8 bytes: 10.5 -> 8.9.
-template <int RANKS>
-__global__ __launch_bounds__(kBuildThreads) void buildTablesKernel(const BuildLists<RANKS> a) {
+// One launch for all slab classes (blockIdx.y), where a launch for each cost 2 us more per class: (11,5,196,31,4)/(4,1,3,2,0), 8 bytes, two classes,
+// 12.3 -> 10.0 us a call; (24,613,532)/(0,2,1), 4 bytes, four, 20.4 -> 14.1; (4,107,5,1475)/(2,0,3,1), 8 bytes, four, 22.0 -> 12.6.
+template <int RANKS, int CLASSES>
+__global__ __launch_bounds__(kBuildThreads) void buildTablesKernel(const BuildClasses<RANKS, CLASSES> classes) {
+  const BuildLists<RANKS>& a = classes.cls[CLASSES > 1 ? blockIdx.y : 0];
   const uint32_t i = blockIdx.x * kBuildThreads + threadIdx.x;
   const uint32_t in = radixSum(a.rank[0], i), out = radixSum(a.rank[1], i), pos = radixSum(a.rank[2], i);
   if (i < a.count[0]) a.rowIn[i] = in;
@@ -1199,43 +1206,66 @@ __global__ __launch_bounds__(kBuildThreads) void buildTablesKernel(const BuildLi
   if (i < a.count[2]) a.shIdx[i] = (uint16_t)(pos + (pos >> a.padShift));
 }
 
-template <int RANKS>
-hipError_t launchTableBuild(const cuttHipTableBuildArgs& a, uint32_t entries, hipStream_t s) {
-  BuildLists<RANKS> b = {a.rowIn, a.rowOut, a.shIdx, {a.count[0], a.count[1], a.count[2]}, a.padShift, {}};
-  for (int l = 0; l < 3; l++)
-    for (int k = 0; k < a.list[l].n; k++) {
-      b.rank[l][k].stride = a.list[l].stride[k];
-      if (k + 1 == a.list[l].n) break;
-      const cuttHipDivisor d = cuttHipMakeDivisor(a.list[l].extent[k]);
-      b.rank[l][k].mul = d.mul;
-      b.rank[l][k].shift = d.shift;
-      b.rank[l][k].add = d.add;
-      b.rank[l][k].extent = a.list[l].extent[k];
+template <int RANKS, int CLASSES>
+hipError_t launchTableBuild(const cuttHipTableBuildArgs* args, int classes, uint32_t entries, hipStream_t s) {
+  BuildClasses<RANKS, CLASSES> all = {};
+  for (int c = 0; c < classes; c++) {
+    const cuttHipTableBuildArgs& a = args[c];
+    BuildLists<RANKS>& b = all.cls[c];
+    b.rowIn = a.rowIn;
+    b.rowOut = a.rowOut;
+    b.shIdx = a.shIdx;
+    b.padShift = a.padShift;
+    for (int l = 0; l < 3; l++) {
+      b.count[l] = a.count[l];
+      for (int k = 0; k < a.list[l].n; k++) {
+        b.rank[l][k].stride = a.list[l].stride[k];
+        if (k + 1 == a.list[l].n) break;
+        const cuttHipDivisor d = cuttHipMakeDivisor(a.list[l].extent[k]);
+        b.rank[l][k].mul = d.mul;
+        b.rank[l][k].shift = d.shift;
+        b.rank[l][k].add = d.add;
+        b.rank[l][k].extent = a.list[l].extent[k];
+      }
     }
-  return launchKernel(buildTablesKernel<RANKS>, dim3((entries + kBuildThreads - 1) / kBuildThreads), dim3(kBuildThreads), 0, s, b);
+  }
+  return launchKernel(buildTablesKernel<RANKS, CLASSES>, dim3((entries + kBuildThreads - 1) / kBuildThreads, (uint32_t)classes), dim3(kBuildThreads), 0, s, all);
 }
 }  // namespace
 
-extern "C" int cuttHipLaunchTableBuild(const cuttHipTableBuildArgs* a, void* stream) {
-  if (!a || !a->rowIn || !a->rowOut || !a->shIdx || a->padShift < 1 || a->padShift > 31)
-    return (int)hipErrorInvalidValue;
+extern "C" int cuttHipLaunchTableBuilds(const cuttHipTableBuildArgs* args, int classes, void* stream) {
+  if (!args || classes < 1 || classes > 4) return (int)hipErrorInvalidValue;
   uint32_t most = 0;
-  for (int l = 0; l < 3; l++) {
-    if (a->count[l] < 1 || a->count[l] > 65536 || a->list[l].n < 0 || a->list[l].n > CUTT_MAX_RANK)
-      return (int)hipErrorInvalidValue;
-    uint64_t span = 1;  // the list must enumerate at least count entries
-    for (int k = 0; k < a->list[l].n; k++) {
-      if (a->list[l].extent[k] < 1) return (int)hipErrorInvalidValue;
-      span *= a->list[l].extent[k];
-      if (span > (1ull << 32)) return (int)hipErrorInvalidValue;
+  int ranks = 0;
+  for (int c = 0; c < classes; c++) {
+    const cuttHipTableBuildArgs& a = args[c];
+    if (!a.rowIn || !a.rowOut || !a.shIdx || a.padShift < 1 || a.padShift > 31) return (int)hipErrorInvalidValue;
+    for (int l = 0; l < 3; l++) {
+      if (a.count[l] < 1 || a.count[l] > 65536 || a.list[l].n < 0 || a.list[l].n > CUTT_MAX_RANK) return (int)hipErrorInvalidValue;
+      uint64_t span = 1;  // the list must enumerate at least count entries
+      for (int k = 0; k < a.list[l].n; k++) {
+        if (a.list[l].extent[k] < 1) return (int)hipErrorInvalidValue;
+        span *= a.list[l].extent[k];
+        if (span > (1ull << 32)) return (int)hipErrorInvalidValue;
+      }
+      if (span != a.count[l]) return (int)hipErrorInvalidValue;
+      most = std::max(most, a.count[l]);
+      ranks = std::max(ranks, a.list[l].n);
     }
-    if (span != a->count[l]) return (int)hipErrorInvalidValue;
-    most = std::max(most, a->count[l]);
   }
-  const int ranks = std::max({a->list[0].n, a->list[1].n, a->list[2].n});
-  if (ranks <= 4) return (int)launchTableBuild<4>(*a, most, (hipStream_t)stream);
-  if (ranks <= 8) return (int)launchTableBuild<8>(*a, most, (hipStream_t)stream);
-  return (int)launchTableBuild<CUTT_MAX_RANK>(*a, most, (hipStream_t)stream);
+  const hipStream_t s = (hipStream_t)stream;
+  if (classes == 1) {
+    if (ranks <= 4) return (int)launchTableBuild<4, 1>(args, 1, most, s);
+    if (ranks <= 8) return (int)launchTableBuild<8, 1>(args, 1, most, s);
+    if (ranks <= 12) return (int)launchTableBuild<12, 1>(args, 1, most, s);
+    return (int)launchTableBuild<CUTT_MAX_RANK, 1>(args, 1, most, s);
+  }
+  if (ranks <= 4) return (int)launchTableBuild<4, 4>(args, classes, most, s);
+  if (ranks <= 8) return (int)launchTableBuild<8, 4>(args, classes, most, s);
+  if (ranks <= 12) return (int)launchTableBuild<12, 4>(args, classes, most, s);
+  for (int c = 0; c < classes; c++)  // (four classes of 32 ranks each do not fit a launch's arguments)
+    if (int e = cuttHipLaunchTableBuilds(args + c, 1, stream); e != 0) return e;
+  return 0;
 }
 
 // Lets the packed kernels use more than the default 64 KB of dynamic LDS on the current device.

@@ -1752,11 +1752,13 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
   if (tableLayout(packed, off) > capacity) return -1;
   if (int e = cuttHipPreparePacked(); e != 0) return e;
   unsigned char* base = (unsigned char*)tables;
+  cuttHipTableBuildArgs builds[4];
+  int classes = 0;
   for (int c = 0; c < 4; c++) {
     if (!classUsed(packed, c)) continue;
     std::vector<RadixDim> lists[3];
     if (!classRadixLists(*this, c, lists[0], lists[1], lists[2])) return -1;
-    cuttHipTableBuildArgs b;
+    cuttHipTableBuildArgs& b = builds[classes++];
     std::memset(&b, 0, sizeof(b));
     const cuttHipPackedClass& k = packed.cls[c];
     b.count[0] = (uint32_t)(k.vol / k.inCont);
@@ -1774,11 +1776,11 @@ int Plan::activateInPlace(void* tables, size_t capacity) {
     b.rowIn = (uint32_t*)(base + off[c][0]);
     b.rowOut = (uint32_t*)(base + off[c][1]);
     b.shIdx = (uint16_t*)(base + off[c][2]);
-    if (int e = cuttHipLaunchTableBuild(&b, stream); e != 0) return e;
     packed.cls[c].rowIn = b.rowIn;
     packed.cls[c].rowOut = b.rowOut;
     packed.cls[c].shIdx = b.shIdx;
   }
+  if (int e = cuttHipLaunchTableBuilds(builds, classes, stream); e != 0) return e;
   cuttHipFinishPackedWalk(&packed);
   if (int v = cuttHipValidatePacked(&packed); v != 0) return v;
   launchable = true;

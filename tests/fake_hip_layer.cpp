@@ -95,7 +95,7 @@ int cuttHipScratch(void** ptr, size_t* bytes) {
   *bytes = sizeof(scratch);
   return 0;
 }
-int cuttHipLaunchTableBuild(const cuttHipTableBuildArgs* a, void*) {
+int cuttHipLaunchTableBuilds(const cuttHipTableBuildArgs* args, int classes, void*) {
   auto radix = [](const cuttHipRadixList& l, uint32_t i) {
     uint32_t off = 0;
     for (int k = 0; k < l.n; k++) {
@@ -104,11 +104,13 @@ int cuttHipLaunchTableBuild(const cuttHipTableBuildArgs* a, void*) {
     }
     return off;
   };
-  for (uint32_t i = 0; i < a->count[0]; i++) a->rowIn[i] = radix(a->list[0], i);
-  for (uint32_t i = 0; i < a->count[1]; i++) a->rowOut[i] = radix(a->list[1], i);
-  for (uint32_t i = 0; i < a->count[2]; i++) {
-    const uint32_t pos = radix(a->list[2], i);
-    a->shIdx[i] = (uint16_t)(pos + (pos >> a->padShift));
+  for (const cuttHipTableBuildArgs* a = args; a < args + classes; a++) {
+    for (uint32_t i = 0; i < a->count[0]; i++) a->rowIn[i] = radix(a->list[0], i);
+    for (uint32_t i = 0; i < a->count[1]; i++) a->rowOut[i] = radix(a->list[1], i);
+    for (uint32_t i = 0; i < a->count[2]; i++) {
+      const uint32_t pos = radix(a->list[2], i);
+      a->shIdx[i] = (uint16_t)(pos + (pos >> a->padShift));
+    }
   }
   return 0;
 }

@@ -33,3 +33,28 @@ def test_tables_built_on_the_device(dim, perm, es):
             assert rc == cutt.CUTT_SUCCESS and np.array_equal(gpu_util.to_host(d_out, es), expect), (dim, perm, es, method)
     finally:
         cutt.set_method_override(0)
+
+
+@pytest.mark.parametrize("es,dim,perm", [
+    (4, (331, 2, 270), (2, 1, 0)),                                   # two slab classes, lists of up to four ranks
+    (4, (6, 613, 252), (0, 2, 1)),                                   # four classes of different sizes
+    (8, (2, 3, 2, 2, 5, 2, 7, 2, 301), (8, 6, 4, 2, 0, 1, 7, 5, 3)),   # two, up to eight ranks
+    (4, (2, 2, 2, 5, 2, 2, 2, 2, 11, 2, 2, 2, 13, 2, 2), (6, 10, 2, 1, 12, 11, 3, 0, 14, 4, 7, 13, 9, 5, 8)),   # two, up to twelve
+])
+def test_the_tables_of_several_slab_classes(es, dim, perm):
+    import torch
+    import cutt_amd as cutt
+    import gpu_util
+    import oracle
+    data = gpu_util.seeded(int(np.prod(dim)), es, seed=len(dim))
+    d_in = gpu_util.to_device(data)
+    expect = oracle.transpose(list(dim), list(perm), data)
+    try:
+        cutt.set_method_override(cutt.METHOD_PACKEDSPLIT)
+        for call in range(3):  # (the tables of the call before are in the scratch memory)
+            d_out = torch.full_like(d_in, -1)
+            rc = cutt.cuttExecuteNoAlloc(len(dim), list(dim), list(perm), es, gpu_util.stream_handle(), d_in.data_ptr(), d_out.data_ptr())
+            torch.cuda.synchronize()
+            assert rc == cutt.CUTT_SUCCESS and np.array_equal(gpu_util.to_host(d_out, es), expect), (dim, perm, es, call)
+    finally:
+        cutt.set_method_override(0)
