@@ -560,9 +560,10 @@ bool estimateAndTune(Plan& p, const cuttHipDeviceProps& props) {
   if (!estimatePlan(p, props, 10)) return false;
   chooseTiledGrouping(p, props);
   if (lineWindowsPay(p, props)) p.model.usPredicted *= 0.92;
-  // The model's constants stem from plans whose stores all went through the caches up to half of the memory-side one.  450 tensors of 45-134 MB per buffer, forced to each method: packed plans that store past the caches ran at 0.72-0.78 of
-  // their estimates (buffers in rotation; 0.92 on new ones), Tiled plans with partly written lines at 0.93-1.0.  With 0.87, up to 100 MB, a fifth
-  // of the plans change: 7 % faster in rotation, the same on 4 GB of buffers, 1 % faster on inputs just written, 3.5 % with kernels before and behind.
+  // The model's constants stem from plans whose stores all went through the caches up to half of the memory-side one.  450 tensors of 45-134 MB per
+  // buffer, forced to each method: packed plans that store past the caches ran at 0.72-0.78 of their estimates (buffers in rotation; 0.92 on new
+  // ones), Tiled plans with partly written lines at 0.93-1.0.  With 0.87, up to 100 MB, 60 of 626 plans change: 0.81 of the time in rotation, 1.01
+  // on 4 GB of buffers, 0.96 on inputs just written, 0.94 with kernels before and behind.
   const double bytes = (double)p.pb.volume * p.pb.elemSize, cache = (double)props.infinityCacheBytes;
   const bool rows = p.method == kTiledCopy && p.tcopy.rowGather;  // (gathered rows store past the caches at every size: as they stood to packed plans)
   const bool blocks = (p.method == kTiled && p.tiled.lineWidth == 0) || p.method == kPacked || p.method == kPackedSplit;

@@ -413,7 +413,7 @@ long long cuttHipPackedItemNumbers(const cuttHipPackedArgs* args);
 int cuttHipDecodeItem(const cuttHipPackedArgs* args, uint32_t w, uint32_t* m, uint32_t* s0, uint32_t* s1, int* cls);
 /* Bytes of LDS the packed kernel needs for these arguments. */
 size_t cuttHipPackedLdsBytes(const cuttHipPackedArgs* a);
-/* Vector registers per lane of the packed kernel instance for this element size, elements per lane
+/* Vector registers per lane of the general packed kernel's instance for this element size, elements per lane
  * and offset width, as built (a table kept beside the kernel; needs no GPU).  The planner derives
  * the resident wavefronts per CU from it: min(8, 512 / roundup8(registers)) per SIMD, 4 SIMDs. */
 int cuttHipPackedRegsPerLane(int elemSize, int elemsPerThread, int wideOffsets);

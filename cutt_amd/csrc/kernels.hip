@@ -17,10 +17,10 @@
  *    clamping indices, not by branches, so the memory instructions stay back to back;
  *  - Packed/PackedSplit take their index remap from tables the planner precomputed in device
  *    memory (one input offset per contiguous input run, one output offset per contiguous output
- *    run, an LDS gather slot per staged element); a workgroup derives its lanes' offsets once and
- *    keeps them in registers while it loops over its work items, so the loop body is load, LDS
- *    write, LDS read, store; the LDS buffer is skewed by one slot per 2^padShift to break
- *    power-of-two bank strides;
+ *    run, an LDS gather slot per staged element); a workgroup takes one block (packedOnceKernel), or it derives
+ *    its lanes' offsets once and keeps them in registers while it loops over its blocks, so the loop body is load, LDS
+ *    write, LDS read, store (packedLoopKernel; packedKernel where the blocks cannot be decoded as a walk);
+ *    the LDS buffer is skewed by one slot per 2^padShift to break power-of-two bank strides;
  *  - workgroups are short-lived and small (a tile, or a few Mbar positions),
  *    thousands are in flight: on this chip that streams faster than a
  *    persistent grid-stride loop.
@@ -435,6 +435,8 @@ __global__ __launch_bounds__(kRowThreads) void rowGatherKernel(const cuttHipRowA
 // Packed / PackedSplit: stage a block of Mmk through LDS with remap tables.
 // ---------------------------------------------------------------------------
 
+// The general kernel: 64-bit offsets, more than twelve Mbar ranks, loops of fewer than four elements per lane and 8-byte loops of 13-16
+// waves (cuttHipFinishPackedWalk).  Bound by memory.
 // E = elements per lane.  Every lane keeps its E table entries in registers, so that the loop
 // over work items does no index arithmetic beyond adding the item's base offsets; the loop is
 // software-pipelined (an item's loads are in flight while the previous one is gathered and stored).
@@ -617,10 +619,10 @@ __global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ i
 constexpr uint32_t kPackedWalkAt = 3 * 8 + 8 * 4;
 static_assert(alignof(cuttHipPackedWalk) == 4, "no gap in front of it");
 
-// Several blocks per workgroup (4-byte elements beyond some 60 MB, where the table reads weigh most), in a software pipeline: a block's loads are issued before the LDS gather and the stores of the one before, so
-// they overlap, and the wait for them (the memory counter counts loads and stores in issue order) does not also wait for those stores to
-// complete.  Bound by memory.  Against packedKernel, 70 tensors of 90-700 MB per buffer: 0.7 % faster in the mean, (6,18,5,14,8,24,17)/(0,5,1,6,2,3,4), 4
-// bytes, 42.3 -> 39.2 us, (15,2842,3021)/(1,0,2), 4 bytes, 193 -> 188, (2,8,...) 8 bytes +2.6 % the worst.
+// Several blocks per workgroup (4-byte elements beyond some 60 MB, where the table reads weigh most), in a software pipeline: a block's loads
+// are issued before the LDS gather and the stores of the one before, so they overlap, and the wait for them (the memory counter counts loads and
+// stores in issue order) does not also wait for those stores to complete.  Bound by memory.  Against packedKernel, 70 tensors of 90-700 MB per
+// buffer: 0.7 % faster in the mean, (6,18,5,14,8,24,17)/(0,5,1,6,2,3,4), 4 bytes, 42.3 -> 39.2 us, (15,2842,3021)/(1,0,2), 4 bytes, 193 -> 188.
 // (The instances with 8 elements per lane are held to the 72 and 80 registers that let seven and six of their waves share a SIMD.  64, and eight
 // waves, cost the 4-byte one 1 % in the mean over 70 tensors, up to 7 %: what is in flight then crowds the L2, which has to hold the lines
 // that neighbouring blocks complete.)
