@@ -620,9 +620,11 @@ void refineMbarOrder(std::vector<Plan>& plans, const cuttHipDeviceProps& props, 
 // the later candidate (reference src/cuttplan.cpp:700-768).
 //
 // A packed plan gives way to the best Tiled one, beyond half a cache size, if that writes whole lines, in 64x64 tiles whose order is no
-// numbering by address bits, and is not estimated 1.18 (4 bytes) or 1.1 times as long: the model's constants stem from plans whose workgroups the
+// numbering by address bits, and is not estimated 1.18 (4 bytes, whole lines read too) or 1.1 times as long: the model's constants stem from plans whose workgroups the
 // XCDs took in chunks, and in groups such Tiled plans run at 0.89 and 0.93 of their estimates (130 tensors), packed ones at 0.95.  2 % of 1600 tensors
 // change their plan for it, 5 % faster in the mean: (8,4,262144,24)/(2,1,3,0), 4 bytes, 302 -> 249 us; (6,17,8,156,32,9)/(2,3,0,1,4,5), 4 bytes, 52 -> 55.
+// Where 4-byte tiles request each line read about twice, 1.18 gains nothing: (22,22,2,61,80,20)/(1,5,3,4,0,2) 171 -> 179, (83,976160)/(1,0) 123.5 -> 126.7
+// and 14 % on an input just written, (74,10,128,70,6)/(1,2,4,3,0) 66 -> 61 but 8 % more there.
 int chooseHeuristic(const std::vector<Plan>& plans, const cuttHipDeviceProps& props) {
   int best = -1, tiled = -1;
   for (int i = 0; i < (int)plans.size(); i++) {
@@ -635,7 +637,8 @@ int chooseHeuristic(const std::vector<Plan>& plans, const cuttHipDeviceProps& pr
   if (2.0 * (double)t.pb.volume * t.pb.elemSize <= (double)props.infinityCacheBytes || t.tiled.lineWidth > 0 || t.tiled.order == 7 ||
       lineWindowsPay(t, props) || !storesPastCaches(t, props))
     return best;
-  return t.model.usPredicted <= (t.pb.elemSize == 4 ? 1.18 : 1.1) * plans[best].model.usPredicted ? tiled : best;
+  const bool wholeReads = t.model.rdLines <= 1.02 * (double)t.pb.volume * t.pb.elemSize / 128.0;
+  return t.model.usPredicted <= (t.pb.elemSize == 4 && wholeReads ? 1.18 : 1.1) * plans[best].model.usPredicted ? tiled : best;
 }
 
 PlannerOptions plannerOptions(int forceMethod) {
