@@ -1183,7 +1183,8 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
   // faster one is kept, so that the measuring planner does not end behind the heuristic one by more than the
   // noise of these last runs.  Within 1 %, which two such timings differ by, that is the heuristic one: its cache policy is
   // chosen with other surroundings in view than its own runs, as the candidates are timed.  (1544,426,76,4)/(2,0,1,3), 8 bytes:
-  // loads past the caches 553 us, ordinary ones 552; with the output written by another kernel before 554 and 608.
+  // loads past the caches 553 us, ordinary ones 552; with the output written by another kernel before 554 and 608.  (So 1.8 % where the policies
+  // differ: (4,50000000)/(1,0), 8 bytes, 545 and 536 us, with such a kernel before 545 and 581.)
   if (plans[best].method != kTrivial && !std::getenv("CUTT_MEASURE_NO_PLAYOFF")) {
     std::vector<Plan> again;
     if (createPlans(orig, red, props, plannerOptions(force), again) && !again.empty() && estimateAll(again, props)) {
@@ -1201,7 +1202,7 @@ static cuttResult measureProblem(const Problem& orig, const Problem& red, int fo
           tw = std::min(tw, t);
         }
         if (failed) return CUTT_INTERNAL_ERROR;
-        if (th <= 1.01 * tw) {
+        if (th <= (cachePolicyOf(heur) != cachePolicyOf(plans[best]) ? 1.018 : 1.01) * tw) {
           plans[best].release();
           us.push_back(th);
           plans.push_back(std::move(heur));
