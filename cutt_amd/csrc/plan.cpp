@@ -522,7 +522,14 @@ bool numberItemsByDigits(cuttHipPackedArgs& a, const cuttHipTileDigits& dg) {
 // of the first cut rank, of the second, Mbar ranks), with the digits at bit 11 that would lie in that zone
 // moved to the very top.  `residentPerXcd` = workgroups one XCD holds at a time.  False if there is nothing
 // to move (or the numbering cannot be written as at most 16 digits).
-bool thawAddressBit11(const cuttHipPackedArgs& a, int elemSize, int64_t residentPerXcd, cuttHipTileDigits& dg) {
+//
+// Such a numbering goes with one chunk per XCD, where it is 10 % faster than the default one.  In groups (chooseXcdGroup, which all of 1700
+// such plans would take) the chip works at one place at a time, and the default numbering is as fast: 1337 tensors with power-of-two extents and mixed ones,
+// 0.13-1.1 GB per buffer, digits in chunks over default in groups 1.002 of the time in the mean, 0.68-1.48.  Digits are 3.2 (4 bytes) and 6.5 % (8 bytes)
+// faster where the digit lies right below the ones the XCDs split (at most 24 positions of it and above) and a lane moves at most 8 elements, 292 plans;
+// with more elements 3.1 % slower (53), further below 1.5 % (992).  350 others: 4.1 and 3.6 % faster there, 0.8 % slower elsewhere.  So only
+// there, unless `anywhere` (which the measuring planner tries).
+bool thawAddressBit11(const cuttHipPackedArgs& a, int elemSize, int64_t residentPerXcd, bool anywhere, cuttHipTileDigits& dg) {
   if (a.split[0].slabRem || a.split[1].slabRem) return false;
   auto log2Exact = [](int64_t v) {
     int l = 0;
@@ -567,11 +574,13 @@ bool thawAddressBit11(const cuttHipPackedArgs& a, int elemSize, int64_t resident
   double total = 0;
   for (const Part& p : seq) total += std::log2((double)p.radix);
   const double inFlight = std::log2((double)std::max<int64_t>(1, a.itemsPerBlock)) + std::log2((double)std::max<int64_t>(1, residentPerXcd));
+  if (!anywhere && a.elemsPerThread > 8) return false;
+  // (half a digit of margin on the fast side: a digit that only part of the resident workgroups differ in)
+  const double from = anywhere ? inFlight - 0.5 : std::max(inFlight - 0.5, total - 4.6);
   std::vector<Part> kept, moved;
   double pos = 0;
   for (const Part& p : seq) {
-    // (half a digit of margin on the fast side: a digit that only part of the resident workgroups differ in)
-    if (p.bit11 && pos >= inFlight - 0.5 && pos < total - 3.0) moved.push_back(p);
+    if (p.bit11 && pos >= from && pos < total - 3.0) moved.push_back(p);
     else kept.push_back(p);
     pos += std::log2((double)p.radix);
   }
@@ -703,7 +712,7 @@ bool setupPacked(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptio
     const double cacheBytes = props.infinityCacheBytes > 0 ? (double)props.infinityCacheBytes : 256.0 * 1024 * 1024;
     cuttHipTileDigits dg;
     if ((double)pb.volume * pb.elemSize > 0.75 * cacheBytes &&
-        thawAddressBit11(a, pb.elemSize, (int64_t)props.cuCount / kNumXcd * residentPerCU, dg) && numberItemsByDigits(a, dg))
+        thawAddressBit11(a, pb.elemSize, (int64_t)props.cuCount / kNumXcd * residentPerCU, opt.itemBitsAnywhere, dg) && numberItemsByDigits(a, dg))
       plan.itemDigits = dg;
   }
   const int64_t numbers = cuttHipPackedItemNumbers(&a);

@@ -161,6 +161,7 @@ struct PlannerOptions {
                             // size and whose extents the radices multiply to exactly
   int digitLanes = -1;      // tile order 7: decode the digits lane-parallel (1), digit by digit (0), planner's choice (-1)
   bool addressBits = true;  // Tiled: number the workgroups by the address bits their digits move where that rule applies (addressBitOrder)
+  bool itemBitsAnywhere = false;  // Packed/PackedSplit: number the work items by such bits also where the XCDs' groups are faster in the mean (thawAddressBit11)
   int tiledFuse = -1;       // Tiled over fused rank sets: -1 = planner's choice, 0 = one rank per side only
   int tiledAligned = -1;    // Tiled: line-aligned stores, -1 = planner's choice, 0 = off, 1 = on
   int tiledWide = -1;       // Tiled: 128x128 tiles where they fit (4-byte elements), -1 = planner's choice (finishPlan), 0 = off, 1 = on

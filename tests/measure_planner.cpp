@@ -14,6 +14,8 @@
 //   narrow    - wide tiles 100 us, 64x64 tiles in tile order 6 40 us in patches of 2 x 2 and 41 us in others, 60 us in any other order:
 //               prints how often one plan in order 6 other than the winner was launched
 //   tie98, tie99 - Packed plans: the one cuttPlan makes 100 us, all others 98 or 99.5 us; prints the policy of cuttPlan's plan
+//   bits      - PackedSplit plans: work items numbered by address bits 50 us, others 100 us, for a tensor that cuttPlan numbers the other way
+//   nobits    - the same for one whose plan cuttPlan numbers by address bits: these 100 us, others in groups of workgroups 50 us, 120 us in chunks
 //   drift     - line-aligned Tiled plans 100 us, others 200 us, every launch a little less than the one before
 #define cuttHipEventCreate fakeEventCreate
 #define cuttHipEventDestroy fakeEventDestroy
@@ -173,6 +175,18 @@ static int narrow() {
   return 0;
 }
 
+static int bits(std::vector<int> dim, std::vector<int> perm, int es, double numbered, double inGroups, double inChunks) {
+  cuttSetMethodOverride(CUTT_METHOD_PACKEDSPLIT);
+  cuttHandle h;
+  cuttPlanInfo own = {};
+  if (cuttPlan(&h, (int)dim.size(), dim.data(), perm.data(), es, 0) != CUTT_SUCCESS || cuttGetPlanInfo(h, &own) != CUTT_SUCCESS) return 1;
+  cuttDestroy(h);
+  std::printf("own numbered %d group %d\n", own.tileDigits[0] != 0, own.xcdGroup);
+  // (a numbering by digits leaves no cut ranks; blocks of another size are slower)
+  gPackedUs = [=](const cuttHipPackedArgs& a) { return cuttHipPackedLdsBytes(&a) != own.ldsBytes ? 150.0 : oneSlab(a) ? numbered : (a.xcdGroup ? inGroups : inChunks); };
+  return measure(dim, perm, es);
+}
+
 static int predicted() {
   int dim[7] = {18, 39, 13, 100, 2, 3, 25}, perm[7] = {0, 3, 1, 6, 5, 2, 4};
   for (const char* gather : {"1", "0"}) {
@@ -212,6 +226,8 @@ int main(int argc, char** argv) {
   if (what == "drift") return drift();
   if (what == "tie98") return tie(98.0);
   if (what == "tie99") return tie(99.5);
+  if (what == "bits") return bits({32, 4096, 2048}, {0, 2, 1}, 4, 50, 100, 100);
+  if (what == "nobits") return bits({2, 4096, 512, 64}, {0, 3, 1, 2}, 4, 100, 50, 120);
   if (what == "groups") return groups();
   if (what == "narrow") return narrow();
   return 2;

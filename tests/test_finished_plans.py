@@ -117,6 +117,19 @@ def test_packed_plans_give_way_to_tiles_that_write_whole_lines(planner):
     assert planner.plan((5, 7, 11, 13, 17, 1093), (4, 2, 0, 5, 1, 3), 4).method != TILED
 
 
+@pytest.mark.parametrize("dim,perm,es,numbered", [
+    # the digit at address bit 11 right below the three slowest binary ones, written and read side
+    ((2, 4096, 512, 64), (0, 3, 1, 2), 4, True), ((16, 2, 1024, 8, 4, 128), (5, 4, 2, 1, 3, 0), 8, True), ((4, 1024, 512, 64), (3, 1, 0, 2), 8, True),
+    # ... with sixteen elements per lane; further below
+    ((16, 12288, 512), (0, 2, 1), 4, False), ((16, 8, 4, 128, 512, 8), (5, 1, 4, 0, 3, 2), 4, False), ((4, 4, 32768, 512), (0, 1, 3, 2), 4, False), ((4, 2, 4, 1024, 512, 8), (3, 1, 2, 5, 4, 0), 8, False),
+])
+def test_packed_plans_are_numbered_by_address_bit_11_or_take_groups(planner, dim, perm, es, numbered):
+    info = planner.plan(dim, perm, es)
+    assert info.method in (2, 3) and (bool(info.tileDigits), info.xcdGroup) == ((True, 0) if numbered else (False, 5))
+    plain = planner.plan(dim, perm, es, CUTT_ADDRESS_BITS=0)
+    assert not plain.tileDigits and plain.xcdGroup == 5
+
+
 def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
     # (counted as tiles of 64 elements they seem to issue a quarter of the requests)
     for dim, perm in (((8192, 8192), (1, 0)), ((4096, 256, 64), (1, 0, 2)), ((256, 400, 512), (2, 1, 0))):

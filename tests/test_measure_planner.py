@@ -76,3 +76,12 @@ def test_no_plan_is_timed_again_as_a_variant_of_itself(program, scenario, launch
 def test_the_heuristic_plan_wins_ties(program, scenario, us):
     # half a per cent is what two timings of one plan differ by, two per cent are not
     assert measured(program, scenario)["us"] == us
+
+
+@pytest.mark.parametrize("scenario,own", [("bits", (0, 5)), ("nobits", (1, 0))])
+def test_both_numberings_of_packed_work_items_are_timed(program, scenario, own):
+    # by address bits in one chunk per XCD, and the default one in groups of workgroups, whichever cuttPlan takes
+    p = measured(program, scenario)
+    out = subprocess.check_output([program, scenario], text=True, timeout=120)
+    assert tuple(map(int, re.search(r"own numbered (\d) group (\d)", out).groups())) == own
+    assert p["us"] == 50.0
