@@ -524,7 +524,8 @@ bool wideForm(const Plan& p, const cuttHipDeviceProps& props, Plan& q) {
 // is short now, and a share of the table reads, which weigh less than with 4-byte elements; one each evens out the end of the launch.  69 such plans of
 // 90-800 MB per buffer, two blocks before: 1.5 % faster in the mean, 8 % at best, 3 % slower at worst; 30 of 13-16 waves 0.5 %, but 4-5 % slower at
 // worst ((51,960,3,13,4,2,6,2)/(7,6,0,4,2,5,1,3) 537 -> 557 us).  (4-byte elements, four blocks before: 4 % slower in the
-// mean, 45 % at worst.)  Not applied when an option pins the number or the order.
+// mean, 45 % at worst.)  Not applied when an option pins the number or the order.  Work items numbered by address bits keep their numbering: placed for
+// two blocks per workgroup it is the one for one block as well (all 85 numbered plans among 17500 tensors with power-of-two and mixed extents).
 void oneBlockPerWorkgroup(Plan& p, const PlannerOptions& opt) {
   cuttHipPackedArgs& a = p.packed;
   if ((p.method != kPacked && p.method != kPackedSplit) || a.itemsPerBlock == 1 || a.elemSize != 8 || a.elemsPerThread != 8 || p.ldsBytes < 10 * 1024 || a.numThreads > 768 || a.wideOffsets ||

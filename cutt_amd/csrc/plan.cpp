@@ -662,7 +662,8 @@ bool setupPacked(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptio
     const int64_t wanted = (int64_t)props.cuCount * residentPerCU * 4;
     // Measured on 200M-element tensors: with 8-byte elements and items of 10 KB and more, two items
     // per workgroup run about 2 % faster than four (the table is a smaller share of the traffic and
-    // more workgroups even out the tail); with 4-byte elements four is better.
+    // more workgroups even out the tail); with 4-byte elements four is better.  (The kernels have changed since: most such 8-byte plans
+    // are launched with one item per workgroup, cutt_api.cpp: oneBlockPerWorkgroup, but estimated with two.)
     const int64_t maxItems = opt.maxItemsPerBlock > 0 ? opt.maxItemsPerBlock
                              : (pb.elemSize == 8 && plan.ldsBytes >= 10 * 1024) ? 2 : 4;
     a.itemsPerBlock = (int)std::max<int64_t>(1, std::min<int64_t>(maxItems, items / std::max<int64_t>(wanted, 1)));

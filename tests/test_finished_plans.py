@@ -130,6 +130,29 @@ def test_packed_plans_are_numbered_by_address_bit_11_or_take_groups(planner, dim
     assert not plain.tileDigits and plain.xcdGroup == 5
 
 
+@pytest.mark.parametrize("dim,perm,es,waves,blocks", [
+    # 8-byte blocks of 10 KB and more: twelve waves and fewer, more; 4-byte elements
+    ((135, 3890, 2, 55, 2), (2, 4, 0, 3, 1), 8, 12, 1), ((2, 2, 24, 30521, 14), (0, 4, 2, 1, 3), 8, 3, 1), ((28, 1019, 9, 273), (1, 2, 0, 3), 8, 14, 2),
+    ((32, 32, 7, 9, 12, 29, 3), (2, 6, 4, 0, 5, 1, 3), 4, 16, 4),
+])
+def test_8_byte_packed_plans_take_one_block_per_workgroup(planner, dim, perm, es, waves, blocks):
+    info = planner.plan(dim, perm, es, CUTT_XCD_GROUP=0)
+    assert info.method in (2, 3) and info.ldsBytes >= 10240
+    assert (info.numThreads // 64, info.itemsPerBlock) == (waves, blocks)
+    items = info.volMbar * info.numSplit * info.numSplit2
+    assert info.numBlocks == ((items + blocks - 1) // blocks + 7) // 8 * 8
+    # options that pin the number or the order
+    more = blocks if blocks > 1 else 2
+    assert planner.plan(dim, perm, es, CUTT_MAX_ITEMS=more).itemsPerBlock == more
+    assert planner.plan(dim, perm, es, CUTT_ITEM_ORDER=0).itemsPerBlock == more
+
+
+def test_a_numbering_by_address_bits_fits_the_blocks_per_workgroup(planner):
+    dim, perm = (4, 1024, 512, 64), (3, 1, 0, 2)
+    info, one = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_MAX_ITEMS=1)
+    assert info.itemsPerBlock == one.itemsPerBlock == 1 and info.tileDigits == one.tileDigits != b"" and info.numBlocks == one.numBlocks
+
+
 def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
     # (counted as tiles of 64 elements they seem to issue a quarter of the requests)
     for dim, perm in (((8192, 8192), (1, 0)), ((4096, 256, 64), (1, 0, 2)), ((256, 400, 512), (2, 1, 0))):
