@@ -338,6 +338,7 @@ typedef struct cuttHipSplitRank {
  * long as n < items and that position is below volMbar.
  */
 #define CUTT_PACKED_RANKS 12
+#define CUTT_PACKED_LOOP_ELEMS 4       /* elements per lane, at least, of a loop over several blocks */
 typedef struct cuttHipPackedWalkClass {
   uint32_t last, inCont, outCont;      /* elements of the block - 1, run lengths */
   uint32_t inMul, outMul, shifts;      /* divisions by the run lengths: in | out << 5 */

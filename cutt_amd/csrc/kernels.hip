@@ -821,6 +821,15 @@ int allowLargeLds(K kernel, size_t bytes) {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// The same for the packed kernels whose arguments are decoded as a walk; loops over few elements per lane have none (cuttHipFinishPackedWalk).
+template <typename T, int E, int NT>
+int allowLargeLdsWalks(size_t bytes) {
+  int r = allowLargeLds(packedOnceKernel<T, E, NT>, bytes);
+  if constexpr (E >= CUTT_PACKED_LOOP_ELEMS)
+    if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, NT>, bytes);
+  return r;
+}
+
 // ---------------------------------------------------------------------------
 // Trivial method: a plain copy, 16 bytes per lane and one 4-KB piece per workgroup, so that the
 // hardware dispatcher spreads the pieces and every wave has exactly one load and one store in
@@ -1293,14 +1302,10 @@ extern "C" int cuttHipPreparePacked(void) {
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 1, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 2, true>, m);          \
   if (r == 0) r = allowLargeLds(packedKernel<T, E, 3, true>, m);          \
-  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 0>, m);            \
-  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 0>, m);            \
-  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 1>, m);            \
-  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 1>, m);            \
-  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 2>, m);            \
-  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 2>, m);            \
-  if (r == 0) r = allowLargeLds(packedLoopKernel<T, E, 3>, m);            \
-  if (r == 0) r = allowLargeLds(packedOnceKernel<T, E, 3>, m)
+  if (r == 0) r = allowLargeLdsWalks<T, E, 0>(m);                         \
+  if (r == 0) r = allowLargeLdsWalks<T, E, 1>(m);                         \
+  if (r == 0) r = allowLargeLdsWalks<T, E, 2>(m);                         \
+  if (r == 0) r = allowLargeLdsWalks<T, E, 3>(m)
     CUTT_ALLOW(uint32_t, 1); CUTT_ALLOW(uint32_t, 2); CUTT_ALLOW(uint32_t, 4); CUTT_ALLOW(uint32_t, 8);
     CUTT_ALLOW(uint32_t, 16);
     CUTT_ALLOW(uint64_t, 1); CUTT_ALLOW(uint64_t, 2); CUTT_ALLOW(uint64_t, 4); CUTT_ALLOW(uint64_t, 8);
@@ -1371,7 +1376,13 @@ extern "C" int cuttHipValidatePacked(const cuttHipPackedArgs* a) {
 template <typename T, int E, int NT>
 static int launchPackedWalk(const cuttHipPackedArgs& a, const void* in, void* out, hipStream_t s) {
   const cuttHipPackedWalk& o = a.walk;
-  return (int)launchKernel(o.perGroup > 1 ? packedLoopKernel<T, E, NT> : packedOnceKernel<T, E, NT>, dim3(o.blocks), dim3(a.numThreads), cuttHipPackedLdsBytes(&a), s, (const T*)in, (T*)out,
+  auto kernel = packedOnceKernel<T, E, NT>;
+  if constexpr (E >= CUTT_PACKED_LOOP_ELEMS) {
+    if (o.perGroup > 1) kernel = packedLoopKernel<T, E, NT>;
+  } else if (o.perGroup > 1) {  // (has no walk)
+    return (int)hipErrorInvalidValue;
+  }
+  return (int)launchKernel(kernel, dim3(o.blocks), dim3(a.numThreads), cuttHipPackedLdsBytes(&a), s, (const T*)in, (T*)out,
                            (const unsigned char*)a.cls[0].rowIn, o.chunk, o.shifts, o.items, o.num[0], o.mul[0], o.num[1], o.mul[1], o.padThreads, o);
 }
 

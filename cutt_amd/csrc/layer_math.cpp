@@ -196,7 +196,7 @@ extern "C" void cuttHipFinishPackedWalk(cuttHipPackedArgs* a) {
   // (a loop over blocks of few elements per lane is slower this way: (5,4,1374779)/(1,0,2), 8 bytes, one element per lane, 212 -> 254 us)
   // Nor does it help workgroups of 13-16 waves with 8-byte elements: 36 plans of 250-1600 MB per buffer 1.004 in
   // the mean, 0.975 ... 1.024, (1544,426,76,4)/(2,0,1,3) 556 -> 571 us.
-  if (a->itemsPerBlock > 1 && (a->elemsPerThread < 4 || (a->elemSize == 8 && a->numThreads > 768))) return;
+  if (a->itemsPerBlock > 1 && (a->elemsPerThread < CUTT_PACKED_LOOP_ELEMS || (a->elemSize == 8 && a->numThreads > 768))) return;
   if (a->itemsPerBlock < 1 || a->wideOffsets || a->mbar.n < 0 || a->mbar.n > CUTT_PACKED_RANKS || a->xcdGroup < 0 || a->xcdGroup > 20 || numbers < 1) return;
   const unsigned long long per = (unsigned long long)a->itemsPerBlock, groups = ((unsigned long long)numbers + per - 1) / per;
   unsigned long long blocks = groups;

@@ -4,6 +4,7 @@ A C++ program decodes every workgroup index of random launches with the kernel's
 slab class and offsets with the work items' definition, and the class's constants with its tables and run lengths.
 """
 import os
+import re
 import subprocess
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -128,3 +129,12 @@ def test_items_and_tables(tmp_path):
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-include", "algorithm", "-I" + csrc, str(src), os.path.join(csrc, "layer_math.cpp"), "-o", exe])
     out = subprocess.run([exe], capture_output=True, text=True)
     assert out.returncode == 0 and out.stdout.startswith("ok"), out.stdout + out.stderr
+
+
+def test_kernel_instances_that_can_be_launched():
+    # (a loop over blocks of fewer than four elements per lane has no walk: the general kernel takes it)
+    names = subprocess.check_output(["nm", "-C", os.path.join(ROOT, "cutt_amd", "libcutt.so")], text=True)
+    for kernel, elems in (("packedOnceKernel", {4: {1, 2, 4, 8, 16}, 8: {1, 2, 4, 8}}), ("packedLoopKernel", {4: {4, 8, 16}, 8: {4, 8}})):
+        for size, name in ((4, "unsigned int"), (8, "unsigned long")):
+            found = re.findall(kernel + "<%s, (\\d+), (\\d)>" % name, names)
+            assert set(found) == {(str(e), str(p)) for e in elems[size] for p in range(4)}, (kernel, size)
