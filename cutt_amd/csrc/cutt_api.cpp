@@ -278,8 +278,8 @@ bool storesPastCaches(const Plan& p, const cuttHipDeviceProps& props) {
 //    ordinary accesses: three pairs of buffers in rotation / as many pairs as make 4 GB / right after a kernel that writes the input /
 //    with such a kernel before and one that reads the result behind.  Packed plans 0.71 / 0.94 / 0.92 / 0.89 at 45-75 MB per buffer,
 //    0.77 / 0.94 / 0.88 / 0.93 at 75-95, 0.92 / 0.94 / 0.90 / 0.88 at 95-135; Tiled ones 0.77 / 0.93 / 1.01 / 0.92, 0.73 / 0.95 / 1.05 / 0.96,
-//    0.89 / 0.91 / 1.03 / 0.92.  The packed plans may cover up to 16 % of their lines partly there, any number below a third
-//    of the cache, and 4 % up to a whole cache size (0.95 / 0.96 / 0.91 / 0.92).  Other Tiled plans lose by such stores (0.81-1.1 / 1.03-1.13);
+//    0.89 / 0.91 / 1.03 / 0.92.  The packed plans may leave 16 partly covered lines per hundred lines of data there, two per line below a third
+//    of the cache per buffer, and 4 per hundred up to a whole cache size (0.95 / 0.96 / 0.91 / 0.92).  Other Tiled plans lose by such stores (0.81-1.1 / 1.03-1.13);
 //    with non-temporal loads they gain in rotation (0.96 at 45 MB, 0.84 at 75, 1.02 at 115), but a pass on an input just written takes 3-15 % longer;
 //  - outputs written in whole lines - at most one line in a hundred left partly covered by a workgroup -:
 //    non-temporal stores, 2-10 % faster than ordinary ones ((37,59,7,16,6,30) 146 -> 132 us, (985024,28,4) 345 ->
@@ -427,14 +427,16 @@ bool groupsLose(const Plan& p, const cuttHipDeviceProps& props) {
 // (2,1,3,0) 159 -> 157; 8192 x 8192, 4 bytes, 108 -> 102; (40,14881,4,6,14)/(3,2,0,1,4) 304 -> 293; (64,64,64,64,4)/(3,2,1,0,4)
 // 134 -> 99; 295 random Tiled plans of 0.16-1.3 GB per buffer outside the classes above 1.04 times as fast in the mean, 0.88 ... 1.22, 17 of them
 // below 0.98 ((4,30,783,592)/(2,3,0,1), 8 bytes, 168 -> 192 us); nothing found in their strides tells those from the others.  (Groups of 8 and 32 are as good; single workgroups lose what neighbours share in an L2.)  That holds where every line is
-// written whole and past the caches.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 such plans
-// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones +7 ... -9 %.
+// written past the caches, in Tiled plans whole ones.  Where workgroups complete each other's lines in the L2 they must stay on one XCD: 30 Tiled plans
+// lose 2-25 % ((129975,177)/(1,0), 4 bytes, 40 -> 55 us), packed ones with ordinary stores +7 ... -9 %.  Packed plans that store past the caches with
+// more than one line in a hundred covered partly (storesPastCaches) gain: 440 of 45-268 MB per buffer 1.01 times as fast in rotation, 0.87-1.32, and 1.05, 0.88-1.36,
+// on 24 pairs of buffers, the same for all shares of such lines.
 void chooseXcdGroup(Plan& p, const cuttHipDeviceProps& props) {
   if (const char* e = std::getenv("CUTT_XCD_GROUP")) {
     setXcdGroup(p, std::atoi(e));
     return;
   }
-  // (a packed workgroup moves several blocks: 512 of them are 8 MB and more)
+  // (packed plans that store past the caches are 45 MB and more, in 700 workgroups and more; of 1024-2048 they gain 2-4 %)
   if (!(cachePolicyOf(p) & 2) || groupsLose(p, props) || p.numBlocks < (p.method == kTiled ? 2048 : 512)) {
     setXcdGroup(p, 0);
     return;
