@@ -37,6 +37,7 @@ def test_tables_built_on_the_device(dim, perm, es):
 
 @pytest.mark.parametrize("es,dim,perm", [
     (4, (331, 2, 270), (2, 1, 0)),                                   # two slab classes, lists of up to four ranks
+    (8, (5, 4, 4097), (1, 0, 2)),                                    # two classes of a stretch of a batch
     (4, (6, 613, 252), (0, 2, 1)),                                   # four classes of different sizes
     (8, (2, 3, 2, 2, 5, 2, 7, 2, 301), (8, 6, 4, 2, 0, 1, 7, 5, 3)),   # two, up to eight ranks
     (4, (2, 2, 2, 5, 2, 2, 2, 2, 11, 2, 2, 2, 13, 2, 2), (6, 10, 2, 1, 12, 11, 3, 0, 14, 4, 7, 13, 9, 5, 8)),   # two, up to twelve
