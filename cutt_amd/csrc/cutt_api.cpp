@@ -522,9 +522,10 @@ bool wideForm(const Plan& p, const cuttHipDeviceProps& props, Plan& q) {
   return true;
 }
 
-// 8-byte elements, blocks of 10 KB and more, up to twelve waves: one per workgroup.  More of them saved the kernel's way to its first load, which
-// is short now, and a share of the table reads, which weigh less than with 4-byte elements; one each evens out the end of the launch.  69 such plans of
-// 90-800 MB per buffer, two blocks before: 1.5 % faster in the mean, 8 % at best, 3 % slower at worst; 30 of 13-16 waves 0.5 %, but 4-5 % slower at
+// 8-byte elements, blocks of 10 KB and more, up to twelve waves, at most 12000 of them: one per workgroup.  More of them save the kernel's way to its first
+// load, which is short, and a share of the table reads, which weigh less than with 4-byte elements; one each evens out the end of the launch, which
+// counts the more the shorter that is.  480 such plans of 0.13-1.6 GB per buffer, two blocks before: up to 12000 blocks 1.6 % faster in the mean, 0.95-1.10 times as
+// fast (190; up to 8000 2.4 %), beyond 0.7 % slower, 0.94-1.07 (290; workgroups of five to seven waves there 1-2 %).  30 of 13-16 waves 0.5 %, but 4-5 % slower at
 // worst ((51,960,3,13,4,2,6,2)/(7,6,0,4,2,5,1,3) 537 -> 557 us).  (4-byte elements, four blocks before: 4 % slower in the
 // mean, 45 % at worst.)  Not applied when an option pins the number or the order.  Work items numbered by address bits keep their numbering: placed for
 // two blocks per workgroup it is the one for one block as well (all 85 numbered plans among 17500 tensors with power-of-two and mixed extents).
@@ -537,12 +538,12 @@ void oneBlockPerWorkgroup(Plan& p, const PlannerOptions& opt) {
   one.itemsPerBlock = 1;
   one.itemOrder = 0;
   int64_t blocks = cuttHipPackedItemNumbers(&one);
+  if (blocks > 12000) return;
   if (one.xcdChunk) {
     one.xcdChunk = (uint32_t)((blocks + kNumXcd - 1) / kNumXcd);
     blocks = (int64_t)one.xcdChunk * kNumXcd;
   }
-  // (workgroups x lanes must fit a 32-bit count, with a group of workgroups per XCD more)
-  if (blocks < 1 || (uint64_t)(blocks + 16 * kNumXcd) * (uint64_t)a.numThreads > CUTT_HIP_MAX_GRID_LANES) return;
+  if (blocks < 1) return;
   a = one;
   p.numBlocks = blocks;
 }

@@ -416,7 +416,9 @@ int cuttHipDecodeItem(const cuttHipPackedArgs* args, uint32_t w, uint32_t* m, ui
 size_t cuttHipPackedLdsBytes(const cuttHipPackedArgs* a);
 /* Vector registers per lane of the general packed kernel's instance for this element size, elements per lane
  * and offset width, as built (a table kept beside the kernel; needs no GPU).  The planner derives
- * the resident wavefronts per CU from it: min(8, 512 / roundup8(registers)) per SIMD, 4 SIMDs. */
+ * the resident wavefronts per CU from it: min(8, 512 / roundup8(registers)) per SIMD, 4 SIMDs.  The kernels that most plans launch
+ * take other numbers (eight elements per lane: 56 and 70 with 4-byte ones, 60 and 78 with 8-byte ones, for one block per workgroup
+ * and several, where this says 68 and 73); the planner's constants and its blocks per workgroup were measured with these. */
 int cuttHipPackedRegsPerLane(int elemSize, int elemsPerThread, int wideOffsets);
 /* The same number asked of the HIP runtime for the loaded code object (needs a GPU); -1 on error. */
 int cuttHipPackedRegsPerLaneLoaded(int elemSize, int elemsPerThread, int wideOffsets);

@@ -407,7 +407,8 @@ void choosePackedThreads(int64_t vol, int elemSize, const cuttHipDeviceProps& pr
   elemsPerThread = e;
 }
 
-// Lanes of the packed kernel that fit a CU: 512 registers per SIMD lane in units of 8, 4 SIMDs of
+// Lanes of the general packed kernel that fit a CU (more or fewer of the others may: cuttHipPackedRegsPerLane; (24,32,16,36,9)/(4,1,3,2,0), 8 bytes, is
+// planned for three workgroups per CU and has four): 512 registers per SIMD lane in units of 8, 4 SIMDs of
 // 64-lane wavefronts, at most 8 wavefronts per SIMD.
 int64_t packedThreadsPerCU(const cuttHipDeviceProps& props, int elemSize, int elemsPerThread, int wide) {
   const int regs = cuttHipPackedRegsPerLane(elemSize, elemsPerThread, wide);
@@ -662,8 +663,8 @@ bool setupPacked(Plan& plan, const cuttHipDeviceProps& props, const PlannerOptio
     const int64_t wanted = (int64_t)props.cuCount * residentPerCU * 4;
     // Measured on 200M-element tensors: with 8-byte elements and items of 10 KB and more, two items
     // per workgroup run about 2 % faster than four (the table is a smaller share of the traffic and
-    // more workgroups even out the tail); with 4-byte elements four is better.  (The kernels have changed since: most such 8-byte plans
-    // are launched with one item per workgroup, cutt_api.cpp: oneBlockPerWorkgroup, but estimated with two.)
+    // more workgroups even out the tail); with 4-byte elements four is better.  (The kernels have changed since: such 8-byte plans of up to
+    // 12000 items are launched with one per workgroup, cutt_api.cpp: oneBlockPerWorkgroup, but estimated with two.)
     const int64_t maxItems = opt.maxItemsPerBlock > 0 ? opt.maxItemsPerBlock
                              : (pb.elemSize == 8 && plan.ldsBytes >= 10 * 1024) ? 2 : 4;
     a.itemsPerBlock = (int)std::max<int64_t>(1, std::min<int64_t>(maxItems, items / std::max<int64_t>(wanted, 1)));

@@ -131,9 +131,9 @@ def test_packed_plans_are_numbered_by_address_bit_11_or_take_groups(planner, dim
 
 
 @pytest.mark.parametrize("dim,perm,es,waves,blocks", [
-    # 8-byte blocks of 10 KB and more: twelve waves and fewer, more; 4-byte elements
-    ((135, 3890, 2, 55, 2), (2, 4, 0, 3, 1), 8, 12, 1), ((2, 2, 24, 30521, 14), (0, 4, 2, 1, 3), 8, 3, 1), ((28, 1019, 9, 273), (1, 2, 0, 3), 8, 14, 2),
-    ((32, 32, 7, 9, 12, 29, 3), (2, 6, 4, 0, 5, 1, 3), 4, 16, 4),
+    # 8-byte blocks of 10 KB and more, up to 12000: twelve waves and fewer, more waves; more blocks; 4-byte elements
+    ((2, 3, 6, 17, 5, 16, 3, 29, 15), (5, 4, 2, 7, 0, 6, 8, 1, 3), 8, 12, 1), ((122, 6, 25, 88, 11, 2), (2, 0, 3, 1, 4, 5), 8, 6, 1), ((28, 1019, 9, 273), (1, 2, 0, 3), 8, 14, 2),
+    ((14, 36, 38, 3, 669), (2, 1, 3, 0, 4), 8, 7, 2), ((135, 3890, 2, 55, 2), (2, 4, 0, 3, 1), 8, 12, 2), ((32, 32, 7, 9, 12, 29, 3), (2, 6, 4, 0, 5, 1, 3), 4, 16, 4),
 ])
 def test_8_byte_packed_plans_take_one_block_per_workgroup(planner, dim, perm, es, waves, blocks):
     info = planner.plan(dim, perm, es, CUTT_XCD_GROUP=0)
@@ -148,9 +148,9 @@ def test_8_byte_packed_plans_take_one_block_per_workgroup(planner, dim, perm, es
 
 
 def test_a_numbering_by_address_bits_fits_the_blocks_per_workgroup(planner):
-    dim, perm = (4, 1024, 512, 64), (3, 1, 0, 2)
-    info, one = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_MAX_ITEMS=1)
-    assert info.itemsPerBlock == one.itemsPerBlock == 1 and info.tileDigits == one.tileDigits != b"" and info.numBlocks == one.numBlocks
+    for dim, perm, blocks in (((4, 8192, 1024), (0, 2, 1), 1), ((4, 1024, 512, 64), (3, 1, 0, 2), 2)):
+        info, pinned = planner.plan(dim, perm, 8), planner.plan(dim, perm, 8, CUTT_MAX_ITEMS=blocks)
+        assert info.itemsPerBlock == pinned.itemsPerBlock == blocks and info.tileDigits == pinned.tileDigits != b"" and info.numBlocks == pinned.numBlocks
 
 
 def test_wide_tiles_are_estimated_as_the_small_ones_they_stand_for(planner):
