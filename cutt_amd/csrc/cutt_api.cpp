@@ -569,6 +569,8 @@ bool estimateAndTune(Plan& p, const cuttHipDeviceProps& props) {
   // buffer, forced to each method: packed plans that store past the caches ran at 0.72-0.78 of their estimates (buffers in rotation; 0.92 on new
   // ones), Tiled plans with partly written lines at 0.93-1.0.  With 0.87, up to 100 MB, 60 of 626 plans change: 0.81 of the time in rotation, 1.01
   // on 4 GB of buffers, 0.96 on inputs just written, 0.94 with kernels before and behind.
+  // (Not where CUTT_CACHE_POLICY pins the policy: all plans have the same one.)
+  if (std::getenv("CUTT_CACHE_POLICY")) return true;
   const double bytes = (double)p.pb.volume * p.pb.elemSize, cache = (double)props.infinityCacheBytes;
   const bool rows = p.method == kTiledCopy && p.tcopy.rowGather;  // (gathered rows store past the caches at every size: as they stood to packed plans)
   const bool blocks = (p.method == kTiled && p.tiled.lineWidth == 0) || p.method == kPacked || p.method == kPackedSplit;
@@ -626,7 +628,8 @@ void refineMbarOrder(std::vector<Plan>& plans, const cuttHipDeviceProps& props, 
 // A packed plan gives way to the best Tiled one, beyond half a cache size, if that writes whole lines, in 64x64 tiles whose order is no
 // numbering by address bits, and is not estimated 1.18 (4 bytes, whole lines read too) or 1.1 times as long: the model's constants stem from plans whose workgroups the
 // XCDs took in chunks, and in groups such Tiled plans run at 0.89 and 0.93 of their estimates (130 tensors), packed ones at 0.95.  2 % of 1600 tensors
-// change their plan for it, 5 % faster in the mean: (8,4,262144,24)/(2,1,3,0), 4 bytes, 302 -> 249 us; (6,17,8,156,32,9)/(2,3,0,1,4,5), 4 bytes, 52 -> 55.
+// change their plan for it, 4 % faster in the mean (0.75-1.27, 200 tensors in two rotations of buffers; right after a kernel that writes the input 1 %, and 8-byte ones that read
+// lines twice 3 % slower there): (8,4,262144,24)/(2,1,3,0), 4 bytes, 302 -> 249 us; (6,17,8,156,32,9)/(2,3,0,1,4,5), 4 bytes, 52 -> 55.
 // Where 4-byte tiles request each line read about twice, 1.18 gains nothing: (22,22,2,61,80,20)/(1,5,3,4,0,2) 171 -> 179, (83,976160)/(1,0) 123.5 -> 126.7
 // and 14 % on an input just written, (74,10,128,70,6)/(1,2,4,3,0) 66 -> 61 but 8 % more there.
 int chooseHeuristic(const std::vector<Plan>& plans, const cuttHipDeviceProps& props) {
@@ -638,6 +641,7 @@ int chooseHeuristic(const std::vector<Plan>& plans, const cuttHipDeviceProps& pr
   }
   if (best < 0 || tiled < 0 || (plans[best].method != kPacked && plans[best].method != kPackedSplit)) return best;
   const Plan& t = plans[tiled];
+  if (std::getenv("CUTT_CACHE_POLICY") && !(plannerOptions(0).cachePolicy & 2)) return best;  // (pinned to ordinary stores: no groups)
   if (2.0 * (double)t.pb.volume * t.pb.elemSize <= (double)props.infinityCacheBytes || t.tiled.lineWidth > 0 || t.tiled.order == 7 ||
       lineWindowsPay(t, props) || !storesPastCaches(t, props))
     return best;

@@ -108,6 +108,14 @@ def test_cache_policy_of_tensors_up_to_half_a_cache_size(planner, dim, perm, es,
     assert info.cachePolicy == policy, (info.method, info.wrPartialLines / (size / 128))
 
 
+def test_a_pinned_cache_policy_is_the_one_plans_are_chosen_for(planner):
+    # estimates of stores past the caches, and the preference for tiles in groups, only with such stores
+    dim, perm = (129975, 177), (1, 0)
+    assert [planner.plan(dim, perm, 4, **env).method for env in ({}, dict(CUTT_CACHE_POLICY=0), dict(CUTT_CACHE_POLICY=1))] == [3, TILED, TILED]
+    dim, perm = (8, 4, 262144, 24), (2, 1, 3, 0)
+    assert [planner.plan(dim, perm, 4, **env).method for env in ({}, dict(CUTT_CACHE_POLICY=3), dict(CUTT_CACHE_POLICY=0))] == [TILED, TILED, 3]
+
+
 def test_packed_plans_give_way_to_tiles_that_write_whole_lines(planner):
     # beyond half a cache size, up to the margin; partly written lines, numberings by address bits, smaller tensors
     assert planner.plan((8, 4, 262144, 24), (2, 1, 3, 0), 4).method == TILED

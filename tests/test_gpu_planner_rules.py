@@ -110,7 +110,8 @@ def test_workgroups_numbered_by_address_bits():
 def test_packed_items_with_address_bit_11_moving():
     # seeded tensors with power-of-two extents whose plan is a packed one with its bit-11 digit moved, against the default numbering in
     # groups of workgroups (found: +3.2 % with 4-byte elements, +6.5 % with 8-byte ones over 292 seeded plans of the class, -24 ... +48 %; +4.1 and
-    # +3.6 % over 52 others; this dozen +2.1 %, with three of the plans that lose 13-19 %)
+    # +3.6 % over 52 others; this dozen +2.1 and +1.6 % in two runs, with three of the plans that lose 13-20 %: the worst read 0.815 and 0.797,
+    # hence a bound of 0.75 for a single plan, 0.05 below)
     import torch  # noqa: F401  (before the library is loaded: both must share one HIP runtime)
     import cutt_amd as cutt
     rng = np.random.default_rng(515)
@@ -132,7 +133,7 @@ def test_packed_items_with_address_bit_11_moving():
                 cases.append(dict(dim=dim, perm=perm, es=es))
     assert len(cases) == 12, tries
     run_rule("address bit 11 (packed)", cases, {"CUTT_ADDRESS_BITS": "0"},
-             lambda on, off: bool(on.tileDigits) and on.method_name == off.method_name, 0.98, 0.78, 8)
+             lambda on, off: bool(on.tileDigits) and on.method_name == off.method_name, 0.98, 0.75, 8)
 
 
 def test_run_length_term_of_the_model_for_runs_on_the_line_grid(monkeypatch):
