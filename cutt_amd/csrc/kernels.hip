@@ -619,7 +619,7 @@ __global__ __launch_bounds__(1024) void packedOnceKernel(const T* __restrict__ i
 constexpr uint32_t kPackedWalkAt = 3 * 8 + 8 * 4;
 static_assert(alignof(cuttHipPackedWalk) == 4, "no gap in front of it");
 
-// Several blocks per workgroup (4-byte elements beyond some 60 MB, where the table reads weigh most), in a software pipeline: a block's loads
+// Several blocks per workgroup (4-byte elements beyond some 60 MB, where the table reads weigh most, and 8-byte ones in more than 12000 blocks), in a software pipeline: a block's loads
 // are issued before the LDS gather and the stores of the one before, so they overlap, and the wait for them (the memory counter counts loads and
 // stores in issue order) does not also wait for those stores to complete.  Bound by memory.  Against packedKernel, 70 tensors of 90-700 MB per
 // buffer: 0.7 % faster in the mean, (6,18,5,14,8,24,17)/(0,5,1,6,2,3,4), 4 bytes, 42.3 -> 39.2 us, (15,2842,3021)/(1,0,2), 4 bytes, 193 -> 188.
